@@ -60,6 +60,25 @@ def load():
     return _lib
 
 
+_host_module = None
+
+
+def host():
+    """The native host layer (csrc/host): operators that take tensors, prepare the call and enqueue the kernels without the
+    interpreter in between. Used for tensors on the GPU; missing is an error there, as the library itself missing is."""
+    global _host_module
+    if _host_module is None:
+        load()
+        try:
+            from . import _host
+        except ImportError as e:
+            raise NativeLibraryMissing(f"nmtgminor_amd/_host.so is not built or does not load ({e}). Build it with "
+                                       "`make -C nmtgminor_amd/csrc`.") from e
+        _host.bind(LIB_PATH)
+        _host_module = _host
+    return _host_module
+
+
 def dtype_code(t):
     try:
         return _DTYPE_CODES[t.dtype if isinstance(t, torch.Tensor) else t]

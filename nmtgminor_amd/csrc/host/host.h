@@ -1,0 +1,95 @@
+// Shared pieces of the native host layer (nmtgminor_amd/_host.so): the table of C entry points it calls, and the
+// operators as functions from tensors to tensors (allocate the results, enqueue the kernels). ops.cpp implements them,
+// autograd.cpp wraps them in autograd nodes, layers.cpp composes the transformer layers.
+//
+// Why it exists: a call through the Python stand-ins costs 25 to 80 us of interpreter, ctypes and autograd bookkeeping per
+// operator and direction, several times what the kernels of a small batch take. The same work here is 3 to 8 us.
+#pragma once
+#include <torch/extension.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <optional>
+#include <tuple>
+#include <vector>
+
+#include "../../../include/nmtg_hip.h"
+
+namespace nmtg_host {
+
+using at::Tensor;
+using std::optional;
+
+// The C entry points, resolved from the library that the Python side loaded (bind()).
+#define NMTG_HOST_API(X)                                                                                              \
+  X(last_error) X(ln_fwd) X(ln_bwd_parts) X(ln_bwd) X(dropout_add_fwd) X(dropout_add_bwd) X(xentropy_fwd)             \
+  X(xentropy_bwd) X(gemm) X(mlp_fwd) X(mlp_bwd_dtype_workspace_bytes) X(mlp_bwd) X(flash_attn_dropout_bits_bytes)     \
+  X(flash_attn_fwd) X(flash_attn_bwd) X(flash_attn_key_info_bytes) X(flash_attn_time_info_bytes)                      \
+  X(flash_attn_batched_fwd) X(flash_attn_batched_bwd)
+
+struct Api {
+#define X(name) decltype(&nmtg_##name) name = nullptr;
+  NMTG_HOST_API(X)
+#undef X
+};
+extern Api api;
+void bind(const std::string& path);
+
+// The stream of a tensor's device, with that device made current for the scope.
+struct Launch {
+  c10::OptionalDeviceGuard guard;
+  void* stream = nullptr;
+  explicit Launch(const Tensor& t) {
+    if (t.is_cuda()) {
+      guard.reset_device(t.device());
+      stream = c10::hip::getCurrentHIPStream(t.device().index()).stream();
+    }
+  }
+};
+
+void check(int rc, const char* what);
+int dtype_code(const Tensor& t);
+inline void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+inline void* ptr(const optional<Tensor>& t) { return t.has_value() ? ptr(*t) : nullptr; }
+inline Tensor contiguous(const Tensor& t) { return t.is_contiguous() ? t : t.contiguous(); }
+inline Tensor empty_like_sized(const Tensor& like, at::IntArrayRef sizes) { return at::empty(sizes, like.options().requires_grad(false)); }
+inline Tensor empty_as(const Tensor& like, at::IntArrayRef sizes, at::ScalarType type) {
+  return at::empty(sizes, like.options().dtype(type).requires_grad(false));
+}
+// (seed, offset) of the tensor's default generator, whose offset is advanced past `count` draws
+std::pair<uint64_t, uint64_t> draw(const Tensor& like, int64_t count);
+
+// ---- operators ------------------------------------------------------------------------------------------------------
+struct Norm { Tensor z, stats; };                        // stats: fp32 [2, rows], mean then 1 / sigma
+Norm ln_fwd(const Tensor& x, const Tensor& gamma, const Tensor& beta, double eps);
+struct NormGrads { Tensor dx, dgamma, dbeta; };
+NormGrads ln_bwd(const Tensor& dz, const Tensor& x_or_z, const Tensor& stats, const Tensor& gamma, const Tensor& beta, bool memory_efficient);
+
+Tensor linear_fwd(const Tensor& x, const Tensor& w, const Tensor& b);
+struct LinearGrads { Tensor dx, dw, db; };
+LinearGrads linear_bwd(const Tensor& dy, const Tensor& x, const Tensor& w, bool want_x, bool want_w, bool want_b);
+
+struct Mlp { Tensor out, post, pre, mask; };
+Mlp mlp_fwd(const Tensor& x, const Tensor& w1, const Tensor& w2, const Tensor& b1, const Tensor& b2, double p, int64_t act,
+            const optional<Tensor>& mask, bool save_pre);
+struct MlpGrads { Tensor dx, dw1, dw2, db1, db2; };
+MlpGrads mlp_bwd(const Tensor& dy, const Tensor& x, const Tensor& w1, const Tensor& w2, const Tensor& post, const Tensor& pre,
+                 const Tensor& mask, double p, int64_t act, bool want_x, bool want_w, bool want_b1, bool want_b2);
+
+// x <- residual + dropout(x) in place; returns the keep-mask (undefined without dropout)
+Tensor dropout_add_(const Tensor& x, const Tensor& residual, double p, bool training);
+Tensor dropout_bwd(const Tensor& g, const Tensor& mask, double p);
+
+struct Bits { int64_t mode = 0; uint64_t seed = 0, offset = 0; Tensor words; };
+// attention over a padded batch: q [Tq, B, H, D], k / v [Tk, B, H, D]
+struct Flash { Tensor out, lse; Bits bits; };
+Flash flash_fwd_batched(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& pad, const Tensor& time_mask, double p,
+                        double scale, bool causal);
+void flash_bwd_batched(const Tensor& dout, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& out, const Tensor& lse,
+                       const Tensor& dq, const Tensor& dk, const Tensor& dv, const Tensor& pad, const Tensor& time_mask, double p,
+                       double scale, bool causal, const Bits& bits);
+Tensor pad_bytes(const optional<Tensor>& mask, int64_t rows, int64_t cols);
+
+void define_autograd(pybind11::module_& m);
+void define_layers(pybind11::module_& m);
+
+}  // namespace nmtg_host

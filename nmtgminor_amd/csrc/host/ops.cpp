@@ -1,0 +1,239 @@
+// The operators of the host layer: argument preparation, result allocation and the call of the C entry point.
+#include "host.h"
+#include <dlfcn.h>
+
+namespace nmtg_host {
+
+Api api;
+
+void bind(const std::string& path) {
+  void* lib = dlopen(path.c_str(), RTLD_NOW | RTLD_LOCAL);
+  TORCH_CHECK(lib != nullptr, "cannot load ", path, ": ", dlerror());
+#define X(name)                                                                                     \
+  api.name = reinterpret_cast<decltype(&nmtg_##name)>(dlsym(lib, "nmtg_" #name));                   \
+  TORCH_CHECK(api.name != nullptr, path, " has no nmtg_" #name ": built from other sources");
+  NMTG_HOST_API(X)
+#undef X
+}
+
+void check(int rc, const char* what) {
+  if (rc == 0) return;
+  throw std::runtime_error(std::string(what) + ": " + api.last_error() + " (status " + std::to_string(rc) + ")");
+}
+
+int dtype_code(const Tensor& t) {
+  switch (t.scalar_type()) {
+    case at::kFloat: return NMTG_F32;
+    case at::kHalf: return NMTG_F16;
+    case at::kBFloat16: return NMTG_BF16;
+    default: TORCH_CHECK(false, "unsupported dtype ", t.scalar_type());
+  }
+}
+
+std::pair<uint64_t, uint64_t> draw(const Tensor& like, int64_t count) {
+  at::Generator gen = at::globalContext().defaultGenerator(like.device());
+  std::lock_guard<std::mutex> lock(gen.mutex());
+  const uint64_t seed = gen.current_seed(), offset = gen.get_offset();
+  gen.set_offset(offset + static_cast<uint64_t>((count + 3) / 4 * 4));
+  return {seed, offset};
+}
+
+// ---------------------------------------------------------------------------------------------------------- LayerNorm
+Norm ln_fwd(const Tensor& x, const Tensor& gamma, const Tensor& beta, double eps) {
+  const int64_t h = gamma.numel(), rows = h ? x.numel() / h : 0;
+  Launch on(x);
+  Norm r{at::empty_like(x, x.options().dtype(gamma.scalar_type())), empty_as(x, {2, rows}, at::kFloat)};
+  float* mu = r.stats.data_ptr<float>();
+  check(api.ln_fwd(ptr(x), ptr(gamma), ptr(beta), ptr(r.z), mu, mu + rows, rows, h, static_cast<float>(eps), dtype_code(x),
+                   dtype_code(gamma), on.stream), "nmtg_ln_fwd");
+  return r;
+}
+
+NormGrads ln_bwd(const Tensor& dz, const Tensor& x_or_z, const Tensor& stats, const Tensor& gamma, const Tensor& beta, bool memory_efficient) {
+  const int64_t h = gamma.numel(), rows = stats.size(1);
+  Launch on(dz);
+  NormGrads r{at::empty_like(x_or_z), at::empty_like(gamma), at::empty_like(gamma)};
+  const int64_t parts = api.ln_bwd_parts(rows, h);
+  Tensor part = empty_as(dz, {2, parts, h}, at::kFloat);
+  float* pp = part.data_ptr<float>();
+  const float* mu = stats.data_ptr<float>();
+  check(api.ln_bwd(ptr(dz), ptr(x_or_z), mu, mu + rows, ptr(gamma), memory_efficient ? ptr(beta) : nullptr, ptr(r.dx), ptr(r.dgamma),
+                   ptr(r.dbeta), pp, pp + parts * h, parts, rows, h, memory_efficient ? 1 : 0, dtype_code(x_or_z), dtype_code(gamma),
+                   on.stream), "nmtg_ln_bwd");
+  return r;
+}
+
+// -------------------------------------------------------------------------------------------------- products and MLP
+Tensor linear_fwd(const Tensor& x, const Tensor& w, const Tensor& b) {
+  const int64_t in = w.size(1), out = w.size(0), rows = x.numel() / in;
+  Launch on(x);
+  auto sizes = x.sizes().vec();
+  sizes.back() = out;
+  Tensor y = empty_like_sized(x, sizes);
+  check(api.gemm(0, 1, rows, out, in, 1.f, ptr(x), in, 0, ptr(w), in, 0, ptr(y), out, 0, 1, ptr(b), nullptr, 0, dtype_code(x), on.stream),
+        "nmtg_gemm");
+  return y;
+}
+
+static Tensor mlp_workspace(const Tensor& x, int layers, const int64_t* outs, int64_t rows, int64_t in) {
+  const int64_t bytes = api.mlp_bwd_dtype_workspace_bytes(layers, outs, rows, in, dtype_code(x));
+  return empty_as(x, {std::max<int64_t>(bytes, 256)}, at::kByte);
+}
+
+LinearGrads linear_bwd(const Tensor& dy, const Tensor& x, const Tensor& w, bool want_x, bool want_w, bool want_b) {
+  const int64_t out = w.size(0), in = w.size(1), rows = dy.numel() / out;
+  Launch on(dy);
+  LinearGrads r;
+  if (want_x) { auto sizes = dy.sizes().vec(); sizes.back() = in; r.dx = empty_like_sized(dy, sizes); }
+  if (want_w) r.dw = at::empty_like(w);
+  if (want_b) r.db = empty_like_sized(dy, {out});
+  Tensor ws = mlp_workspace(dy, 1, &out, rows, in);
+  const void* weights[1] = {ptr(w)};
+  void* dws[1] = {ptr(r.dw)};
+  void* dbs[1] = {ptr(r.db)};
+  check(api.mlp_bwd(1, ptr(x), weights, &out, rows, in, ptr(dy), nullptr, nullptr, nullptr, 0.f, NMTG_ACT_NONE, ptr(r.dx), dws, dbs, ptr(ws),
+                    ws.numel(), dtype_code(dy), on.stream), "nmtg_mlp_bwd");
+  return r;
+}
+
+Mlp mlp_fwd(const Tensor& x, const Tensor& w1, const Tensor& w2, const Tensor& b1, const Tensor& b2, double p, int64_t act,
+            const optional<Tensor>& mask, bool save_pre) {
+  const int64_t in = w1.size(1), rows = x.numel() / in, inner = w1.size(0), out = w2.size(0), hidden = rows * inner;
+  Launch on(x);
+  auto sizes = x.sizes().vec();
+  sizes.back() = out;
+  Mlp r;
+  r.out = empty_like_sized(x, sizes);
+  r.post = empty_like_sized(x, {hidden});
+  if (save_pre) r.pre = empty_like_sized(x, {hidden});
+  int mode = 0;
+  uint64_t seed = 0, offset = 0;
+  if (p > 0.0) {
+    if (mask.has_value()) {
+      TORCH_CHECK(mask->scalar_type() == at::kByte && mask->numel() == hidden, "mlp: mask must be uint8 with one byte per hidden activation");
+      r.mask = contiguous(*mask);
+      mode = 1;
+    } else {
+      r.mask = empty_as(x, {hidden}, at::kByte);
+      mode = 2;
+      std::tie(seed, offset) = draw(x, hidden);
+    }
+  }
+  const void* weights[2] = {ptr(w1), ptr(w2)};
+  const void* biases[2] = {ptr(b1), ptr(b2)};
+  const int64_t outs[2] = {inner, out};
+  if (rows > 0)
+    check(api.mlp_fwd(2, ptr(x), weights, biases, outs, rows, in, ptr(r.out), ptr(r.post), ptr(r.pre), static_cast<uint8_t*>(ptr(r.mask)), mode,
+                      static_cast<float>(p), seed, offset, static_cast<int>(act), dtype_code(x), on.stream), "nmtg_mlp_fwd");
+  return r;
+}
+
+MlpGrads mlp_bwd(const Tensor& dy, const Tensor& x, const Tensor& w1, const Tensor& w2, const Tensor& post, const Tensor& pre,
+                 const Tensor& mask, double p, int64_t act, bool want_x, bool want_w, bool want_b1, bool want_b2) {
+  const int64_t in = w1.size(1), rows = x.numel() / in, outs[2] = {w1.size(0), w2.size(0)};
+  Launch on(dy);
+  MlpGrads r;
+  if (want_x) r.dx = at::empty_like(x);
+  if (want_w) { r.dw1 = at::empty_like(w1); r.dw2 = at::empty_like(w2); }
+  if (want_b1) r.db1 = empty_like_sized(x, {outs[0]});
+  if (want_b2) r.db2 = empty_like_sized(x, {outs[1]});
+  if (rows == 0) {                                  // an empty batch contributes zero gradients
+    for (Tensor* t : {&r.dw1, &r.dw2, &r.db1, &r.db2}) if (t->defined()) t->zero_();
+    return r;
+  }
+  Tensor ws = mlp_workspace(x, 2, outs, rows, in);
+  const void* weights[2] = {ptr(w1), ptr(w2)};
+  void* dws[2] = {ptr(r.dw1), ptr(r.dw2)};
+  void* dbs[2] = {ptr(r.db1), ptr(r.db2)};
+  check(api.mlp_bwd(2, ptr(x), weights, outs, rows, in, ptr(dy), ptr(post), ptr(pre), p > 0.0 ? static_cast<const uint8_t*>(ptr(mask)) : nullptr,
+                    static_cast<float>(p), static_cast<int>(act), ptr(r.dx), dws, dbs, ptr(ws), ws.numel(), dtype_code(x), on.stream),
+        "nmtg_mlp_bwd");
+  return r;
+}
+
+// ------------------------------------------------------------------------------------------------ dropout + residual
+Tensor dropout_add_(const Tensor& x, const Tensor& residual, double p, bool training) {
+  Launch on(x);
+  Tensor mask;
+  int mode = 0;
+  uint64_t seed = 0, offset = 0;
+  if (training && p > 0.0) {
+    mask = empty_as(x, x.sizes(), at::kByte);
+    mode = 2;
+    std::tie(seed, offset) = draw(x, x.numel());
+  }
+  check(api.dropout_add_fwd(ptr(x), ptr(residual), static_cast<uint8_t*>(ptr(mask)), x.numel(), static_cast<float>(p), mode, seed, offset,
+                            dtype_code(x), on.stream), "nmtg_dropout_add_fwd");
+  return mask;
+}
+
+Tensor dropout_bwd(const Tensor& g, const Tensor& mask, double p) {
+  Launch on(g);
+  Tensor dx = at::empty_like(g);
+  check(api.dropout_add_bwd(ptr(g), static_cast<const uint8_t*>(mask.data_ptr()), ptr(dx), g.numel(), static_cast<float>(p), dtype_code(g),
+                            on.stream), "nmtg_dropout_add_bwd");
+  return dx;
+}
+
+// ------------------------------------------------------------------------------------------------------ tiled attention
+static Tensor bits_words(const Tensor& like, int64_t b, int64_t h, int64_t tq, int64_t tk) {
+  return empty_as(like, {std::max<int64_t>(api.flash_attn_dropout_bits_bytes(b, h, tq, tk), 16) / 4}, at::kInt);
+}
+static Tensor info_words(const Tensor& like, int64_t bytes) { return empty_as(like, {std::max<int64_t>(bytes, 4) / 4}, at::kInt); }
+
+Tensor pad_bytes(const optional<Tensor>& mask, int64_t rows, int64_t cols) {
+  if (!mask.has_value() || !mask->defined() || mask->numel() == 0) return Tensor();
+  TORCH_CHECK(mask->numel() == rows * cols, "mask must be [", rows, ", ", cols, "]");
+  Tensor m = contiguous(*mask);
+  if (m.scalar_type() == at::kBool) return m.view(at::kByte);          // a bool mask is its bytes
+  return m.scalar_type() == at::kByte ? m : m.to(at::kByte);
+}
+
+Flash flash_fwd_batched(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& pad, const Tensor& time_mask, double p,
+                        double scale, bool causal) {
+  const int64_t tq = q.size(0), b = q.size(1), h = q.size(2), d = q.size(3), tk = k.size(0);
+  Launch on(q);
+  Flash r;
+  r.out = empty_like_sized(q, {tq, b, h, d});
+  r.lse = empty_as(q, {b, h, tq}, at::kFloat);
+  Tensor kinfo, tinfo;
+  if (pad.defined()) kinfo = info_words(q, api.flash_attn_key_info_bytes(b, tk));
+  if (time_mask.defined()) tinfo = info_words(q, api.flash_attn_time_info_bytes(tq, tk));
+  if (p > 0.0) {
+    r.bits.words = bits_words(q, b, h, tq, tk);
+    r.bits.mode = 2;
+    std::tie(r.bits.seed, r.bits.offset) = draw(q, 4 * b * h * ((tq + 3) / 4) * ((tk + 3) / 4));
+  }
+  check(api.flash_attn_batched_fwd(ptr(q), ptr(k), ptr(v), ptr(r.out), static_cast<const uint8_t*>(ptr(pad)), ptr(kinfo),
+                                   static_cast<const uint8_t*>(ptr(time_mask)), ptr(tinfo), r.lse.data_ptr<float>(), b, h, d, tq, tk,
+                                   q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1),
+                                   v.stride(2), r.out.stride(0), r.out.stride(1), r.out.stride(2), static_cast<float>(scale), causal ? 1 : 0,
+                                   static_cast<int>(r.bits.mode), static_cast<float>(p), nullptr, nullptr, ptr(r.bits.words), r.bits.seed,
+                                   r.bits.offset, dtype_code(q), on.stream), "nmtg_flash_attn_batched_fwd");
+  return r;
+}
+
+void flash_bwd_batched(const Tensor& dout, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& out, const Tensor& lse,
+                       const Tensor& dq, const Tensor& dk, const Tensor& dv, const Tensor& pad, const Tensor& time_mask, double p,
+                       double scale, bool causal, const Bits& bits) {
+  const int64_t tq = q.size(0), b = q.size(1), h = q.size(2), d = q.size(3), tk = k.size(0);
+  Launch on(q);
+  Tensor kinfo, tinfo, sd = empty_as(q, {b, h, tq}, at::kFloat);
+  if (pad.defined()) kinfo = info_words(q, api.flash_attn_key_info_bytes(b, tk));
+  if (time_mask.defined()) tinfo = info_words(q, api.flash_attn_time_info_bytes(tq, tk));
+  check(api.flash_attn_batched_bwd(ptr(dout), ptr(q), ptr(k), ptr(v), ptr(out), lse.data_ptr<float>(), ptr(dq), ptr(dk), ptr(dv),
+                                   sd.data_ptr<float>(), static_cast<const uint8_t*>(ptr(pad)), ptr(kinfo),
+                                   static_cast<const uint8_t*>(ptr(time_mask)), ptr(tinfo), b, h, d, tq, tk, q.stride(0), q.stride(1),
+                                   q.stride(2), k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2), out.stride(0),
+                                   out.stride(1), out.stride(2), static_cast<float>(scale), causal ? 1 : 0, static_cast<int>(bits.mode),
+                                   static_cast<float>(p), nullptr, ptr(bits.words), bits.words.defined() ? 1 : 0, bits.seed, bits.offset,
+                                   dtype_code(q), on.stream), "nmtg_flash_attn_batched_bwd");
+}
+
+}  // namespace nmtg_host
+
+PYBIND11_MODULE(_host, m) {
+  m.def("bind", &nmtg_host::bind);
+  nmtg_host::define_autograd(m);
+  nmtg_host::define_layers(m);
+}

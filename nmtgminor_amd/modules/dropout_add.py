@@ -7,6 +7,7 @@ path for fp16; here fp32, fp16 and bf16 all do. An optional fifth argument repla
 keep-mask."""
 import torch
 
+from .. import _lib as L
 from ..native import fused_dropout_add_cuda
 from ._autocast import cast_if_autocast_enabled, no_autocast
 
@@ -34,6 +35,8 @@ class FusedDropoutAdd(torch.autograd.Function):
 
 
 def fused_dropout_add(*args):
+    if len(args) == 4 and args[0].is_cuda and not torch.is_autocast_enabled():
+        return L.host().dropout_add(*args)
     args = cast_if_autocast_enabled(*args)
     with no_autocast():
         return FusedDropoutAdd.apply(*args)

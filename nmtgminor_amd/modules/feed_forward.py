@@ -77,9 +77,8 @@ class PositionWiseFeedForward(nn.Module):
         else:
             if mask is not None:                                                       # the fused kernels replay a dense mask
                 mask = mask.repeat(seq_len, 1)
-            hidden = self.fused_function(dropout, recompute, input.reshape(seq_len * bsz, hidden_size), self.in_proj_weight,
-                                         self.out_proj_weight, self.in_proj_bias, self.out_proj_bias, mask=mask)
-            hidden = hidden.view(seq_len, bsz, hidden_size)
+            hidden = self.fused_function(dropout, recompute, input, self.in_proj_weight, self.out_proj_weight, self.in_proj_bias,
+                                         self.out_proj_bias, mask=mask)
         if self.dropout_residual:
             if self.variational:
                 # the reference's variational branch drops with the layer's own rate, not res_dropout (:203-205)

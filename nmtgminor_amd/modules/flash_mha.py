@@ -9,8 +9,11 @@ mirror FlashAttnQKVPackedFunc (flash_mha.py:104-140) and FlashAttnKVPackedFunc (
 same outputs (out, or (out, softmax_lse, S_dmask) with return_softmax, where S_dmask is the dropout keep-mask here),
 gradients written into the slots of one packed tensor. The backward regenerates the dropout mask from the Philox
 (seed, offset) pair that the forward drew, which the context carries instead of the reference's saved generator state."""
+import contextlib
+
 import torch
 
+from .. import _lib as L
 from ..native import flash_attn_cuda
 from ._autocast import cast_if_autocast_enabled, no_autocast
 
@@ -85,9 +88,22 @@ class FlashAttnKVPackedFunc(torch.autograd.Function):
         return dq, dkv, None, None, None, None, None, None, None, None
 
 
+def _host_takes(qkv, cu_seqlens, dropout_p, return_softmax):
+    return (not return_softmax and qkv.is_cuda and cu_seqlens.is_cuda and qkv.dim() == 4 and qkv.shape[1] == 3
+            and qkv.dtype in (torch.float16, torch.bfloat16) and qkv.stride(3) == 1 and qkv.shape[0] > 0
+            and cu_seqlens.dtype == torch.int32 and cu_seqlens.is_contiguous() and cu_seqlens.numel() > 1)
+
+
 def flash_bert_mha(*args):
-    args = cast_if_autocast_enabled(*args)
-    with no_autocast():
+    if torch.is_autocast_enabled():
+        args = cast_if_autocast_enabled(*args)
+    with no_autocast() if torch.is_autocast_enabled() else contextlib.nullcontext():
+        if len(args) == 7 and _host_takes(args[0], args[1], args[3], args[6]):
+            qkv, cu_seqlens, max_seqlen, dropout_p, softmax_scale, causal, _ = args
+            scale = qkv.shape[-1] ** (-0.5) if softmax_scale is None else softmax_scale
+            out, mode, seed, offset, bits = L.host().packed_attention(qkv, cu_seqlens, max_seqlen, dropout_p, scale, bool(causal))
+            flash_attn_cuda.last_rng = (mode, seed, offset, None, bits)
+            return out
         return FlashAttnQKVPackedFunc.apply(*args)
 
 

@@ -12,6 +12,7 @@ import torch
 from torch.nn import init
 from torch.nn.parameter import Parameter
 
+from .. import _lib as L
 from ..native import fast_layer_norm_cuda
 from ._autocast import cast_if_autocast_enabled, no_autocast
 
@@ -44,9 +45,11 @@ class FastLayerNormFN(torch.autograd.Function):
 
 
 def fast_layer_norm_affine(input, weight, bias, normalized_shape, eps=1e-5, memory_efficient=False):
+    if input.is_cuda and not torch.is_autocast_enabled():
+        return L.host().layer_norm(input, weight, bias, eps, memory_efficient)
     args = cast_if_autocast_enabled(input, weight, bias, eps, memory_efficient)
     with no_autocast():
-        return FastLayerNormFN.apply(*args)
+        return L.host().layer_norm(*args) if input.is_cuda else FastLayerNormFN.apply(*args)
 
 
 def _affine_or_identity(input, weight, bias, hidden):

@@ -7,6 +7,7 @@ mlp_gelu_function, mlp_agelu_function (autocast-aware). An optional keyword `mas
 callables replays an explicit dropout keep-mask (the reference draws its own)."""
 import torch
 
+from .. import _lib as L
 from ..native import fused_mlp_agelu, fused_mlp_gelu, fused_mlp_relu, fused_mlp_silu, mlp_gelu_blaslt
 from ._autocast import cast_if_autocast_enabled, no_autocast
 
@@ -92,15 +93,19 @@ class MlpGELUFunction(torch.autograd.Function):
         return (None, None, None, *grads)
 
 
-def _callable(fn):
+def _callable(fn, act):
+    act = L.ACT_CODES[act]
+
     def call(p, recompute, *args, mask=None):
+        if len(args) == 5 and not recompute and args[0].is_cuda and not torch.is_autocast_enabled():
+            return L.host().mlp(*args, mask, p, act)          # the transformer's two layers
         args = cast_if_autocast_enabled(*args)
         with no_autocast():
             return fn.apply(p, recompute, mask, *args)
     return call
 
 
-mlp_relu_function = _callable(MlpReluFunction)
-mlp_silu_function = _callable(MlpSiluFunction)
-mlp_gelu_function = _callable(MlpGELUFunction)
-mlp_agelu_function = _callable(MlpAGELUFunction)
+mlp_relu_function = _callable(MlpReluFunction, "relu")
+mlp_silu_function = _callable(MlpSiluFunction, "silu")
+mlp_gelu_function = _callable(MlpGELUFunction, "gelu")
+mlp_agelu_function = _callable(MlpAGELUFunction, "agelu")
