@@ -93,6 +93,34 @@ int nmtg_dropout_add_fwd(void* x, const void* residual, uint8_t* mask, int64_t n
 int nmtg_dropout_add_bwd(const void* grad_out, const uint8_t* mask, void* grad_x, int64_t n,
                          float p, int dtype, void* stream);
 
+/* The end of a layer: x <- residual + dropout(x) in place, with the layer's clamp of a stream that holds an inf or NaN to
+ * +-(largest finite value - 1000) applied on the way (onmt/models/transformer_layers.py:176-185). mask_mode 0 (no dropout) or
+ * 2 (drawn here). mask, one byte per element, may be NULL with mask_mode 0; bit 0 = kept, bit 1 = no gradient passes the
+ * element (clamped, or NaN). flag: a device int that is 0; fp16 only (may be NULL otherwise). */
+int nmtg_dropout_add_guard_fwd(void* x, const void* residual, uint8_t* mask, int64_t n, float p,
+                               int mask_mode, uint64_t seed, uint64_t offset, int* flag, int dtype,
+                               void* stream);
+/* grad_x <- grad_out / (1 - p) where the mask byte is 1, else 0. */
+int nmtg_dropout_add_guard_bwd(const void* grad_out, const uint8_t* mask, void* grad_x, int64_t n,
+                               float p, int dtype, void* stream);
+
+/* LayerNorm of a residual stream: h <- residual + dropout(x) (rounded and written), z <- LayerNorm(h). mask_mode 0 or 2 (the
+ * keep-mask [rows, hidden] is drawn as nmtg_dropout_add_fwd draws it, and written). clear_flag: a device int set to 0, or
+ * NULL. One dtype for all tensors; mu, rsigma fp32 [rows]. */
+int nmtg_add_ln_fwd(const void* x, const void* residual, void* h, uint8_t* mask, int mask_mode,
+                    float p, uint64_t seed, uint64_t offset, int* clear_flag, const void* gamma,
+                    const void* beta, void* z, float* mu, float* rsigma, int64_t rows, int64_t hidden,
+                    float eps, int dtype, void* stream);
+
+/* Backward of a LayerNorm whose input also went on as a residual stream: dx = round(d LayerNorm) + grad_residual (not added where
+ * bit 1 of guard_mask, which may be NULL, is set). keep_mask (or NULL): the stream was residual + dropout(y); then
+ * dy <- dx * keep / (1 - p) as well. The rest as nmtg_ln_bwd. */
+int nmtg_ln_bwd_add(const void* dz, const void* x, const float* mu, const float* rsigma,
+                    const void* gamma, const void* grad_residual, const uint8_t* guard_mask,
+                    const uint8_t* keep_mask, float p, void* dx, void* dy, void* dgamma, void* dbeta,
+                    float* dgamma_part, float* dbeta_part, int64_t n_part, int64_t rows,
+                    int64_t hidden, int dtype, void* stream);
+
 /* ------------------------------------------------------------------------------------------
  * Masked softmax over the last dimension with optional inverted dropout.
  * Reference: the softmax stage of the fused attention, dispatch_softmax_dropout /

@@ -22,6 +22,8 @@ using std::optional;
 // The C entry points, resolved from the library that the Python side loaded (bind()).
 #define NMTG_HOST_API(X)                                                                                              \
   X(last_error) X(ln_fwd) X(ln_bwd_parts) X(ln_bwd) X(dropout_add_fwd) X(dropout_add_bwd) X(xentropy_fwd)             \
+  X(add_ln_fwd) X(ln_bwd_add) X(dropout_add_guard_fwd) X(dropout_add_guard_bwd) X(encdec_attn_fwd)                    \
+  X(encdec_attn_bwd_workspace_bytes) X(encdec_attn_bwd_from_probs)                                                    \
   X(xentropy_bwd) X(gemm) X(mlp_fwd) X(mlp_bwd_dtype_workspace_bytes) X(mlp_bwd) X(flash_attn_dropout_bits_bytes)     \
   X(flash_attn_fwd) X(flash_attn_bwd) X(flash_attn_key_info_bytes) X(flash_attn_time_info_bytes)                      \
   X(flash_attn_batched_fwd) X(flash_attn_batched_bwd)
@@ -64,6 +66,14 @@ Norm ln_fwd(const Tensor& x, const Tensor& gamma, const Tensor& beta, double eps
 struct NormGrads { Tensor dx, dgamma, dbeta; };
 NormGrads ln_bwd(const Tensor& dz, const Tensor& x_or_z, const Tensor& stats, const Tensor& gamma, const Tensor& beta, bool memory_efficient);
 
+// h = residual + dropout(x), z = LayerNorm(h); mask undefined without dropout. clear: a device int set to 0, or undefined
+struct AddNorm { Tensor h, z, stats, mask; };
+AddNorm add_ln_fwd(const Tensor& x, const Tensor& residual, double p, const Tensor& clear, const Tensor& gamma, const Tensor& beta, double eps);
+// backward of a LayerNorm on a residual stream: dx includes the stream's gradient; keep defined: dy = dx * keep / (1 - p) too
+struct AddNormGrads { Tensor dx, dy, dgamma, dbeta; };
+AddNormGrads ln_bwd_add(const Tensor& dz, const Tensor& x, const Tensor& stats, const Tensor& gamma, const Tensor& grad_residual,
+                        const Tensor& guard, const Tensor& keep, double p);
+
 Tensor linear_fwd(const Tensor& x, const Tensor& w, const Tensor& b);
 struct LinearGrads { Tensor dx, dw, db; };
 LinearGrads linear_bwd(const Tensor& dy, const Tensor& x, const Tensor& w, bool want_x, bool want_w, bool want_b);
@@ -78,6 +88,10 @@ MlpGrads mlp_bwd(const Tensor& dy, const Tensor& x, const Tensor& w1, const Tens
 // x <- residual + dropout(x) in place; returns the keep-mask (undefined without dropout)
 Tensor dropout_add_(const Tensor& x, const Tensor& residual, double p, bool training);
 Tensor dropout_bwd(const Tensor& g, const Tensor& mask, double p);
+// the same at the end of a layer, with the clamp of a stream that holds an inf or NaN (nmtg_dropout_add_guard_fwd); the mask
+// comes back with want_mask or dropout. flag: a zeroed device int
+Tensor dropout_add_guard_(const Tensor& x, const Tensor& residual, double p, const Tensor& flag, bool want_mask);
+Tensor dropout_guard_bwd(const Tensor& g, const Tensor& mask, double p);
 
 struct Bits { int64_t mode = 0; uint64_t seed = 0, offset = 0; Tensor words; };
 // attention over a padded batch: q [Tq, B, H, D], k / v [Tk, B, H, D]

@@ -63,6 +63,38 @@ NormGrads ln_bwd(const Tensor& dz, const Tensor& x_or_z, const Tensor& stats, co
   return r;
 }
 
+AddNorm add_ln_fwd(const Tensor& x, const Tensor& residual, double p, const Tensor& clear, const Tensor& gamma, const Tensor& beta, double eps) {
+  const int64_t h = gamma.numel(), rows = x.numel() / h;
+  Launch on(x);
+  AddNorm r{at::empty_like(x), at::empty_like(x), empty_as(x, {2, rows}, at::kFloat), Tensor()};
+  uint64_t seed = 0, offset = 0;
+  if (p > 0.0) {
+    r.mask = empty_as(x, x.sizes(), at::kByte);
+    std::tie(seed, offset) = draw(x, x.numel());
+  }
+  float* mu = r.stats.data_ptr<float>();
+  check(api.add_ln_fwd(ptr(x), ptr(residual), ptr(r.h), static_cast<uint8_t*>(ptr(r.mask)), p > 0.0 ? 2 : 0, static_cast<float>(p), seed, offset,
+                       static_cast<int*>(ptr(clear)), ptr(gamma), ptr(beta), ptr(r.z), mu, mu + rows, rows, h, static_cast<float>(eps),
+                       dtype_code(x), on.stream), "nmtg_add_ln_fwd");
+  return r;
+}
+
+AddNormGrads ln_bwd_add(const Tensor& dz, const Tensor& x, const Tensor& stats, const Tensor& gamma, const Tensor& grad_residual,
+                        const Tensor& guard, const Tensor& keep, double p) {
+  const int64_t h = gamma.numel(), rows = stats.size(1);
+  Launch on(dz);
+  AddNormGrads r{at::empty_like(x), Tensor(), at::empty_like(gamma), at::empty_like(gamma)};
+  if (keep.defined()) r.dy = at::empty_like(x);
+  const int64_t parts = api.ln_bwd_parts(rows, h);
+  Tensor part = empty_as(dz, {2, parts, h}, at::kFloat);
+  float* pp = part.data_ptr<float>();
+  const float* mu = stats.data_ptr<float>();
+  check(api.ln_bwd_add(ptr(dz), ptr(x), mu, mu + rows, ptr(gamma), ptr(grad_residual), static_cast<const uint8_t*>(ptr(guard)),
+                       static_cast<const uint8_t*>(ptr(keep)), static_cast<float>(p), ptr(r.dx), ptr(r.dy), ptr(r.dgamma), ptr(r.dbeta), pp,
+                       pp + parts * h, parts, rows, h, dtype_code(x), on.stream), "nmtg_ln_bwd_add");
+  return r;
+}
+
 // -------------------------------------------------------------------------------------------------- products and MLP
 Tensor linear_fwd(const Tensor& x, const Tensor& w, const Tensor& b) {
   const int64_t in = w.size(1), out = w.size(0), rows = x.numel() / in;
@@ -175,6 +207,25 @@ Tensor dropout_bwd(const Tensor& g, const Tensor& mask, double p) {
   return dx;
 }
 
+Tensor dropout_add_guard_(const Tensor& x, const Tensor& residual, double p, const Tensor& flag, bool want_mask) {
+  Launch on(x);
+  Tensor mask;
+  uint64_t seed = 0, offset = 0;
+  if (p > 0.0) std::tie(seed, offset) = draw(x, x.numel());
+  if (p > 0.0 || want_mask) mask = empty_as(x, x.sizes(), at::kByte);
+  check(api.dropout_add_guard_fwd(ptr(x), ptr(residual), static_cast<uint8_t*>(ptr(mask)), x.numel(), static_cast<float>(p), p > 0.0 ? 2 : 0,
+                                  seed, offset, static_cast<int*>(ptr(flag)), dtype_code(x), on.stream), "nmtg_dropout_add_guard_fwd");
+  return mask;
+}
+
+Tensor dropout_guard_bwd(const Tensor& g, const Tensor& mask, double p) {
+  Launch on(g);
+  Tensor dx = at::empty_like(g);
+  check(api.dropout_add_guard_bwd(ptr(g), static_cast<const uint8_t*>(mask.data_ptr()), ptr(dx), g.numel(), static_cast<float>(p),
+                                  dtype_code(g), on.stream), "nmtg_dropout_add_guard_bwd");
+  return dx;
+}
+
 // ------------------------------------------------------------------------------------------------------ tiled attention
 static Tensor bits_words(const Tensor& like, int64_t b, int64_t h, int64_t tq, int64_t tk) {
   return empty_as(like, {std::max<int64_t>(api.flash_attn_dropout_bits_bytes(b, h, tq, tk), 16) / 4}, at::kInt);
@@ -184,13 +235,26 @@ static Tensor info_words(const Tensor& like, int64_t bytes) { return empty_as(li
 Tensor pad_bytes(const optional<Tensor>& mask, int64_t rows, int64_t cols) {
   if (!mask.has_value() || !mask->defined() || mask->numel() == 0) return Tensor();
   TORCH_CHECK(mask->numel() == rows * cols, "mask must be [", rows, ", ", cols, "]");
-  Tensor m = contiguous(*mask);
+  Tensor m = contiguous(*mask).view({rows, cols});
   if (m.scalar_type() == at::kBool) return m.view(at::kByte);          // a bool mask is its bytes
   return m.scalar_type() == at::kByte ? m : m.to(at::kByte);
 }
 
 Flash flash_fwd_batched(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& pad, const Tensor& time_mask, double p,
                         double scale, bool causal) {
+  TORCH_CHECK((q.scalar_type() == at::kHalf || q.scalar_type() == at::kBFloat16) && k.scalar_type() == q.scalar_type() &&
+              v.scalar_type() == q.scalar_type(), "flash_attn: q, k and v must share a 16-bit dtype");
+  TORCH_CHECK(q.dim() == 4 && k.dim() == 4 && k.sizes() == v.sizes(), "flash_attn: q [len_q, B, H, D], k and v [len_k, B, H, D]");
+  TORCH_CHECK(k.sizes().slice(1) == q.sizes().slice(1), "flash_attn: k and v must have q's batch, heads and head_dim");
+  for (const Tensor* t : {&q, &k, &v}) {
+    TORCH_CHECK(t->device() == q.device(), "expected a tensor in device memory (HIP); this op has no CPU path");
+    TORCH_CHECK(t->stride(3) == 1, "flash_attn: the head dimension must be contiguous");
+  }
+  auto byte_mask = [&](const Tensor& m, int64_t rows, int64_t cols) {
+    return m.device() == q.device() && m.scalar_type() == at::kByte && m.dim() == 2 && m.size(0) == rows && m.size(1) == cols && m.is_contiguous();
+  };
+  TORCH_CHECK(!pad.defined() || byte_mask(pad, q.size(1), k.size(0)), "flash_attn: key_padding_mask must be contiguous uint8 [batch, len_k]");
+  TORCH_CHECK(!time_mask.defined() || byte_mask(time_mask, q.size(0), k.size(0)), "flash_attn: time_mask must be contiguous uint8 [len_q, len_k]");
   const int64_t tq = q.size(0), b = q.size(1), h = q.size(2), d = q.size(3), tk = k.size(0);
   Launch on(q);
   Flash r;

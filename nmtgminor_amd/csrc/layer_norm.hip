@@ -15,6 +15,7 @@
 //             fp32 partials once written and once read)
 #include "common.hip.h"
 #include <algorithm>
+#include <type_traits>
 
 namespace nmtg {
 namespace {
@@ -59,11 +60,50 @@ __device__ __forceinline__ void row_sum2(float& a, float& b, float* smem, int wa
 // ---------------------------------------------------------------------------------------------
 // Forward: one row per WPR wavefronts, row held in registers.
 // ---------------------------------------------------------------------------------------------
-template <typename TI, typename TW, int VPL, int WPR>
+// ADD: x is the output of the sub-layer in front; the row that is normalised is h = residual + dropout(x), rounded to TI and
+// written on the way (the residual stream goes on from it). ADD 1: no dropout; 2: the keep-mask is drawn here and stored,
+// one byte per element. Against an addition and a LayerNorm of their own the row is not read back: 2 tensors fewer.
+enum { LN_PLAIN = 0, LN_ADD = 1, LN_ADD_RNG = 2 };
+template <typename TI> struct LnAdd {
+  const TI* residual;
+  TI* h;
+  uint8_t* mask;
+  float keep_p, scale;
+  uint64_t seed, offset;
+  int* clear;                // set to 0 (the flag of a guard further down the stream), or null
+};
+
+template <typename TI, int EPV, int ADD>
+__device__ __forceinline__ void ln_add_row(const LnAdd<TI>& add, int64_t first, const pack<TI, EPV>& res, float (&xf)[EPV]) {
+  float rf[EPV];
+  unpack_raw<TI, EPV>(res, rf);
+  if constexpr (ADD == LN_ADD_RNG) {
+    uint8_t keep[EPV];
+    philox_keep<EPV>(Philox(add.seed), static_cast<uint64_t>(first), add.offset, add.keep_p, keep);
+    store_bytes<EPV>(add.mask + first, keep);
+#pragma unroll
+    for (int j = 0; j < EPV; ++j) xf[j] = rf[j] + (keep[j] ? xf[j] * add.scale : 0.f);
+  } else {
+#pragma unroll
+    for (int j = 0; j < EPV; ++j) xf[j] += rf[j];
+  }
+  pack<TI, EPV> out;
+#pragma unroll
+  for (int j = 0; j < EPV; ++j) {
+    out.v[j] = elem<TI>::from_float(xf[j]);
+    xf[j] = elem<TI>::to_float(out.v[j]);
+  }
+  *reinterpret_cast<pack<TI, EPV>*>(add.h + first) = out;
+}
+
+template <typename TI, typename TW, int VPL, int WPR, int ADD>
 __global__ __launch_bounds__(LN_THREADS) void ln_fwd_kernel(
     const TI* __restrict__ x, const TW* __restrict__ gamma, const TW* __restrict__ beta,
     TW* __restrict__ z, float* __restrict__ mu, float* __restrict__ rsigma, int64_t rows, int hidden,
-    float eps) {
+    float eps, LnAdd<TI> add) {
+  if constexpr (ADD != LN_PLAIN) {
+    if (add.clear != nullptr && blockIdx.x == 0 && threadIdx.x == 0) *add.clear = 0;
+  }
   constexpr int EPV = ln_vec<TI>::EPV;
   constexpr int RPB = LN_WAVES / WPR;  // rows per block per iteration
   __shared__ float smem[2 * LN_WAVES];
@@ -89,14 +129,18 @@ __global__ __launch_bounds__(LN_THREADS) void ln_fwd_kernel(
     const int64_t row = g * RPB + wave / WPR;
     const bool row_ok = row < rows;
     const int64_t rowc = row_ok ? row : 0;
-    pack<TI, EPV> xr[VPL];
+    pack<TI, EPV> xr[VPL], rr[ADD != LN_PLAIN ? VPL : 1];
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {
       const int col = ((sub * VPL + i) * kWave + lane) * EPV;
       xr[i] = load_raw<TI, EPV>(x + rowc * hidden + (col < hidden ? col : 0));
+      if constexpr (ADD != LN_PLAIN) rr[i] = load_raw<TI, EPV>(add.residual + rowc * hidden + (col < hidden ? col : 0));
     }
 #pragma unroll
-    for (int i = 0; i < VPL; ++i) pin_raw(xr[i]);
+    for (int i = 0; i < VPL; ++i) {
+      pin_raw(xr[i]);
+      if constexpr (ADD != LN_PLAIN) pin_raw(rr[i]);
+    }
     float xf[VPL][EPV];
     float s = 0.f;
 #pragma unroll
@@ -104,6 +148,7 @@ __global__ __launch_bounds__(LN_THREADS) void ln_fwd_kernel(
       const int col = ((sub * VPL + i) * kWave + lane) * EPV;
       if (row_ok && col < hidden) {
         unpack_raw<TI, EPV>(xr[i], xf[i]);
+        if constexpr (ADD != LN_PLAIN) ln_add_row<TI, EPV, ADD>(add, row * hidden + col, rr[i], xf[i]);
 #pragma unroll
         for (int j = 0; j < EPV; ++j) s += xf[i][j];
       } else {
@@ -141,16 +186,26 @@ __global__ __launch_bounds__(LN_THREADS) void ln_fwd_kernel(
 
 // Fallback for hidden sizes that are not a multiple of the vector width or exceed what the
 // register kernel holds: one block per row, three passes over the row (the re-reads hit cache).
-template <typename TI, typename TW>
+template <typename TI, typename TW, int ADD>
 __global__ __launch_bounds__(LN_THREADS) void ln_fwd_generic_kernel(
-    const TI* __restrict__ x, const TW* __restrict__ gamma, const TW* __restrict__ beta,
+    const TI* x, const TW* __restrict__ gamma, const TW* __restrict__ beta,
     TW* __restrict__ z, float* __restrict__ mu, float* __restrict__ rsigma, int64_t rows, int hidden,
-    float eps) {
+    float eps, LnAdd<TI> add) {
   __shared__ float smem[2 * LN_WAVES];
   const int wave = threadIdx.x / kWave;
   const float rn = 1.f / static_cast<float>(hidden);
+  if constexpr (ADD != LN_PLAIN) {
+    if (add.clear != nullptr && blockIdx.x == 0 && threadIdx.x == 0) *add.clear = 0;
+  }
   for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
     const TI* xr = x + row * hidden;
+    if constexpr (ADD != LN_PLAIN) {          // a thread reads back only the elements of h that it wrote itself
+      for (int c = threadIdx.x; c < hidden; c += LN_THREADS) {
+        float xf[1] = {elem<TI>::to_float(xr[c])};
+        ln_add_row<TI, 1, ADD>(add, row * hidden + c, load_raw<TI, 1>(add.residual + row * hidden + c), xf);
+      }
+      xr = add.h + row * hidden;
+    }
     float s = 0.f;
     for (int c = threadIdx.x; c < hidden; c += LN_THREADS) s += elem<TI>::to_float(xr[c]);
     const float mean = row_sum<LN_WAVES>(s, smem, wave) * rn;
@@ -176,12 +231,38 @@ __global__ __launch_bounds__(LN_THREADS) void ln_fwd_generic_kernel(
 // Each lane keeps running sums of dz and dz*y for its own columns over all rows the block
 // visits; the block folds its wavefronts through LDS and writes one partial row.
 // ---------------------------------------------------------------------------------------------
-template <typename TI, typename TW, int VPL, int WPR, bool MEMEFF>
+// RES: the row went on into a residual stream as well, whose gradient `res.add` is added to the LayerNorm's (which is rounded
+// first, as a stored one would be; RES 2: not where bit 1 of the element's guard byte is set, dropout_add.hip). DROP: the row is h = residual +
+// dropout(y), and dy = dh * keep / (1 - p), the gradient of the dropped sub-layer output, is written from the same registers.
+// Against the separate passes (LayerNorm backward, addition, mask) one read and one write of the tensor each are gone.
+template <typename TI> struct LnRes {
+  const TI* add;
+  const uint8_t* guard;
+  const uint8_t* keep;
+  float scale;
+  TI* dy;
+};
+template <typename TI, int EPV, int RES, bool DROP>
+__device__ __forceinline__ void ln_res_row(const LnRes<TI>& res, int64_t first, const pack<TI, EPV>& add, const uint8_t (&guard)[EPV],
+                                           const uint8_t (&keep)[EPV], float (&dxf)[EPV]) {
+  float af[EPV];
+  unpack_raw<TI, EPV>(add, af);
+#pragma unroll
+  for (int j = 0; j < EPV; ++j) dxf[j] = elem<TI>::to_float(elem<TI>::from_float(dxf[j])) + (RES == 2 && (guard[j] & 2) ? 0.f : af[j]);
+  if constexpr (DROP) {
+    float dyf[EPV];
+#pragma unroll
+    for (int j = 0; j < EPV; ++j) dyf[j] = keep[j] ? elem<TI>::to_float(elem<TI>::from_float(dxf[j])) * res.scale : 0.f;
+    store_pack<TI, EPV>(res.dy + first, dyf);
+  }
+}
+
+template <typename TI, typename TW, int VPL, int WPR, bool MEMEFF, int RES, bool DROP>
 __global__ __launch_bounds__(LN_THREADS) void ln_bwd_kernel(
     const TW* __restrict__ dz, const TI* __restrict__ x_or_z, const float* __restrict__ mu,
     const float* __restrict__ rsigma, const TW* __restrict__ gamma, const TW* __restrict__ beta,
     TI* __restrict__ dx, float* __restrict__ dgamma_part, float* __restrict__ dbeta_part,
-    int64_t rows, int hidden) {
+    int64_t rows, int hidden, LnRes<TI> res) {
   constexpr int EPV = ln_vec<TI>::EPV;
   constexpr int RPB = LN_WAVES / WPR;
   __shared__ float smem[2 * LN_WAVES];
@@ -218,16 +299,25 @@ __global__ __launch_bounds__(LN_THREADS) void ln_bwd_kernel(
     float rs = rsigma[rowc], mean = 0.f;
     if constexpr (!MEMEFF) mean = mu[rowc];
     pack<TW, EPV> dzr[VPL];
-    pack<TI, EPV> xr[VPL];
+    pack<TI, EPV> xr[VPL], ar[RES != 0 ? VPL : 1];
+    pack<uint8_t, EPV> gr[RES == 2 ? VPL : 1], kr[DROP ? VPL : 1];
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {
       const int col = ((sub * VPL + i) * kWave + lane) * EPV;
       const int cc = col < hidden ? col : 0;
       dzr[i] = load_raw<TW, EPV>(dz + rowc * hidden + cc);
       xr[i] = load_raw<TI, EPV>(x_or_z + rowc * hidden + cc);
+      if constexpr (RES != 0) ar[i] = load_raw<TI, EPV>(res.add + rowc * hidden + cc);
+      if constexpr (RES == 2) gr[i] = load_raw<uint8_t, EPV>(res.guard + rowc * hidden + cc);
+      if constexpr (DROP) kr[i] = load_raw<uint8_t, EPV>(res.keep + rowc * hidden + cc);
     }
 #pragma unroll
-    for (int i = 0; i < VPL; ++i) { pin_raw(dzr[i]); pin_raw(xr[i]); }
+    for (int i = 0; i < VPL; ++i) {
+      pin_raw(dzr[i]); pin_raw(xr[i]);
+      if constexpr (RES != 0) pin_raw(ar[i]);
+      if constexpr (RES == 2) pin_raw(gr[i]);
+      if constexpr (DROP) pin_raw(kr[i]);
+    }
     if (!row_ok) { rs = 0.f; mean = 0.f; }
     float sdy = 0.f, sdyy = 0.f;
 #pragma unroll
@@ -264,6 +354,8 @@ __global__ __launch_bounds__(LN_THREADS) void ln_bwd_kernel(
         float dxf[EPV];
 #pragma unroll
         for (int j = 0; j < EPV; ++j) dxf[j] = rs * (dy[i][j] - (mdyy * y[i][j] + mdy));
+        if constexpr (RES != 0)
+          ln_res_row<TI, EPV, RES, DROP>(res, row * hidden + col, ar[i], gr[RES == 2 ? i : 0].v, kr[DROP ? i : 0].v, dxf);
         store_pack<TI, EPV>(dx + row * hidden + col, dxf);
       }
     }
@@ -316,12 +408,12 @@ __global__ __launch_bounds__(LN_THREADS) void ln_bwd_kernel(
 
 // Generic backward: one block per row slot, scalar columns, three passes; partial sums are kept
 // per thread for the columns c = threadIdx.x + k*LN_THREADS in the partial buffers themselves.
-template <typename TI, typename TW, bool MEMEFF>
+template <typename TI, typename TW, bool MEMEFF, int RES, bool DROP>
 __global__ __launch_bounds__(LN_THREADS) void ln_bwd_generic_kernel(
     const TW* __restrict__ dz, const TI* __restrict__ x_or_z, const float* __restrict__ mu,
     const float* __restrict__ rsigma, const TW* __restrict__ gamma, const TW* __restrict__ beta,
     TI* __restrict__ dx, float* __restrict__ dgamma_part, float* __restrict__ dbeta_part,
-    int64_t rows, int hidden) {
+    int64_t rows, int hidden, LnRes<TI> res) {
   __shared__ float smem[2 * LN_WAVES];
   const int wave = threadIdx.x / kWave;
   const float rn = 1.f / static_cast<float>(hidden);
@@ -350,7 +442,15 @@ __global__ __launch_bounds__(LN_THREADS) void ln_bwd_generic_kernel(
       const float xv = elem<TI>::to_float(x_or_z[row * hidden + c]);
       const float yv = MEMEFF ? (xv - elem<TW>::to_float(beta[c])) / gm : rs * (xv - mean);
       const float dyv = elem<TW>::to_float(dz[row * hidden + c]) * gm;
-      dx[row * hidden + c] = elem<TI>::from_float(rs * (dyv - (mdyy * yv + mdy)));
+      float dxf[1] = {rs * (dyv - (mdyy * yv + mdy))};
+      if constexpr (RES != 0) {
+        const int64_t e = row * hidden + c;
+        uint8_t guard[1] = {0}, keep[1] = {0};
+        if constexpr (RES == 2) guard[0] = res.guard[e];
+        if constexpr (DROP) keep[0] = res.keep[e];
+        ln_res_row<TI, 1, RES, DROP>(res, e, load_raw<TI, 1>(res.add + e), guard, keep, dxf);
+      }
+      dx[row * hidden + c] = elem<TI>::from_float(dxf[0]);
     }
   }
 }
@@ -435,10 +535,11 @@ LnPlan ln_plan(int64_t hidden, int max_vpl) {
 
 int ln_grid_limit() { return num_cus() * 8; }  // 8 blocks of 4 wavefronts per CU = full occupancy
 
-template <typename TI, typename TW>
+template <typename TI, typename TW, int ADD = LN_PLAIN>
 int ln_fwd_launch(const void* x, const void* gamma, const void* beta, void* z, float* mu,
-                  float* rsigma, int64_t rows, int64_t hidden, float eps, hipStream_t st) {
-  const bool al = aligned16(x) && aligned16(z) && aligned16(gamma) && aligned16(beta);
+                  float* rsigma, int64_t rows, int64_t hidden, float eps, hipStream_t st, LnAdd<TI> add = {}) {
+  const bool al = aligned16(x) && aligned16(z) && aligned16(gamma) && aligned16(beta) && aligned16(add.residual) && aligned16(add.h) &&
+                  aligned8(add.mask);
   LnPlan p = al ? ln_plan<TI>(hidden, 8) : LnPlan{false, 0, 0};
   auto X = static_cast<const TI*>(x);
   auto G = static_cast<const TW*>(gamma);
@@ -448,8 +549,8 @@ int ln_fwd_launch(const void* x, const void* gamma, const void* beta, void* z, f
   TraceScope trace("ln_fwd", st);
   if (!p.vectorised) {
     const int grid = static_cast<int>(std::min<int64_t>(rows, ln_grid_limit()));
-    hipLaunchKernelGGL((ln_fwd_generic_kernel<TI, TW>), dim3(grid), dim3(LN_THREADS), 0, st, X, G, B,
-                       Z, mu, rsigma, rows, H, eps);
+    hipLaunchKernelGGL((ln_fwd_generic_kernel<TI, TW, ADD>), dim3(grid), dim3(LN_THREADS), 0, st, X, G, B,
+                       Z, mu, rsigma, rows, H, eps, add);
     return 0;
   }
   const int rpb = LN_WAVES / p.wpr;
@@ -457,8 +558,8 @@ int ln_fwd_launch(const void* x, const void* gamma, const void* beta, void* z, f
   const int grid = static_cast<int>(std::min<int64_t>(groups, ln_grid_limit()));
 #define LN_FWD_CASE(V, W)                                                                       \
   if (p.vpl == V && p.wpr == W) {                                                               \
-    hipLaunchKernelGGL((ln_fwd_kernel<TI, TW, V, W>), dim3(grid), dim3(LN_THREADS), 0, st, X, G, \
-                       B, Z, mu, rsigma, rows, H, eps);                                         \
+    hipLaunchKernelGGL((ln_fwd_kernel<TI, TW, V, W, ADD>), dim3(grid), dim3(LN_THREADS), 0, st, X, G, \
+                       B, Z, mu, rsigma, rows, H, eps, add);                                    \
     return 0;                                                                                   \
   }
   LN_FWD_CASE(1, 1) LN_FWD_CASE(2, 1) LN_FWD_CASE(4, 1) LN_FWD_CASE(8, 1)
@@ -477,11 +578,11 @@ int64_t ln_bwd_parts_for(int64_t rows) {
   return std::max<int64_t>(1, std::min<int64_t>(groups, cap));
 }
 
-template <typename TI, typename TW>
+template <typename TI, typename TW, int RES = 0, bool DROP = false>
 int ln_bwd_launch(const void* dz, const void* x_or_z, const float* mu, const float* rsigma,
                   const void* gamma, const void* beta, void* dx, void* dgamma, void* dbeta,
                   float* dgp, float* dbp, int64_t n_part, int64_t rows, int64_t hidden, bool memeff,
-                  hipStream_t st) {
+                  hipStream_t st, LnRes<TI> res = {}) {
   auto DZ = static_cast<const TW*>(dz);
   auto X = static_cast<const TI*>(x_or_z);
   auto G = static_cast<const TW*>(gamma);
@@ -489,7 +590,8 @@ int ln_bwd_launch(const void* dz, const void* x_or_z, const float* mu, const flo
   auto DX = static_cast<TI*>(dx);
   const int H = static_cast<int>(hidden);
   const bool al = aligned16(dz) && aligned16(x_or_z) && aligned16(dx) && aligned16(gamma) &&
-                  (!memeff || aligned16(beta)) && aligned16(dgp) && aligned16(dbp);
+                  (!memeff || aligned16(beta)) && aligned16(dgp) && aligned16(dbp) && aligned16(res.add) && aligned16(res.dy) &&
+                  aligned8(res.guard) && aligned8(res.keep);
   LnPlan p = ln_plan<TI>(hidden, LN_BWD_MAX_VPL);
   const int grid = static_cast<int>(n_part);
   bool done = false;
@@ -502,24 +604,24 @@ int ln_bwd_launch(const void* dz, const void* x_or_z, const float* mu, const flo
         rpb > 1 ? static_cast<size_t>(rpb - 1) * 2 * p.wpr * p.vpl * kWave * EPV * sizeof(float) : 0;
 #define LN_BWD_CASE(V, W)                                                                          \
   if (!done && p.vpl == V && p.wpr == W) {                                                         \
-    if (memeff)                                                                                    \
-      hipLaunchKernelGGL((ln_bwd_kernel<TI, TW, V, W, true>), dim3(grid), dim3(LN_THREADS),        \
-                         fold_bytes, st, DZ, X, mu, rsigma, G, B, DX, dgp, dbp, rows, H);          \
+    if (RES == 0 && memeff)                                                                        \
+      hipLaunchKernelGGL((ln_bwd_kernel<TI, TW, V, W, RES == 0, RES, DROP>), dim3(grid), dim3(LN_THREADS), \
+                         fold_bytes, st, DZ, X, mu, rsigma, G, B, DX, dgp, dbp, rows, H, res);     \
     else                                                                                           \
-      hipLaunchKernelGGL((ln_bwd_kernel<TI, TW, V, W, false>), dim3(grid), dim3(LN_THREADS),       \
-                         fold_bytes, st, DZ, X, mu, rsigma, G, B, DX, dgp, dbp, rows, H);          \
+      hipLaunchKernelGGL((ln_bwd_kernel<TI, TW, V, W, false, RES, DROP>), dim3(grid), dim3(LN_THREADS), \
+                         fold_bytes, st, DZ, X, mu, rsigma, G, B, DX, dgp, dbp, rows, H, res);     \
     done = true;                                                                                   \
   }
     LN_BWD_CASE(1, 1) LN_BWD_CASE(2, 1) LN_BWD_CASE(4, 1) LN_BWD_CASE(4, 2) LN_BWD_CASE(4, 4)
 #undef LN_BWD_CASE
   }
   if (!done) {
-    if (memeff)
-      hipLaunchKernelGGL((ln_bwd_generic_kernel<TI, TW, true>), dim3(grid), dim3(LN_THREADS), 0, st,
-                         DZ, X, mu, rsigma, G, B, DX, dgp, dbp, rows, H);
+    if (RES == 0 && memeff)
+      hipLaunchKernelGGL((ln_bwd_generic_kernel<TI, TW, RES == 0, RES, DROP>), dim3(grid), dim3(LN_THREADS), 0, st,
+                         DZ, X, mu, rsigma, G, B, DX, dgp, dbp, rows, H, res);
     else
-      hipLaunchKernelGGL((ln_bwd_generic_kernel<TI, TW, false>), dim3(grid), dim3(LN_THREADS), 0, st,
-                         DZ, X, mu, rsigma, G, B, DX, dgp, dbp, rows, H);
+      hipLaunchKernelGGL((ln_bwd_generic_kernel<TI, TW, false, RES, DROP>), dim3(grid), dim3(LN_THREADS), 0, st,
+                         DZ, X, mu, rsigma, G, B, DX, dgp, dbp, rows, H, res);
   }
   }
   TraceScope trace("ln_bwd_finalize", st);
@@ -602,5 +704,52 @@ extern "C" int nmtg_ln_bwd(const void* dz, const void* x_or_z, const float* mu, 
   }
   if (rc) return rc;
   NMTG_CHECK_LAUNCH("ln_bwd");
+  return 0;
+}
+
+extern "C" int nmtg_add_ln_fwd(const void* x, const void* residual, void* h, uint8_t* mask, int mask_mode, float p, uint64_t seed,
+                               uint64_t offset, int* clear_flag, const void* gamma, const void* beta, void* z, float* mu, float* rsigma,
+                               int64_t rows, int64_t hidden, float eps, int dtype, void* stream) {
+  NMTG_REQUIRE(rows >= 0 && hidden > 0 && hidden <= (1 << 30), "add_ln_fwd: bad shape rows=%lld hidden=%lld", (long long)rows, (long long)hidden);
+  NMTG_REQUIRE(rows == 0 || (x && residual && h && gamma && beta && z && mu && rsigma), "add_ln_fwd: null pointer argument");
+  NMTG_REQUIRE(eps >= 0.f, "add_ln_fwd: epsilon must be >= 0");
+  NMTG_REQUIRE(mask_mode == 0 || (mask_mode == 2 && mask != nullptr && p >= 0.f && p < 1.f), "add_ln_fwd: bad dropout arguments");
+  if (rows == 0) return 0;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  int rc = 0;
+  NMTG_DISPATCH_DTYPE(dtype, T, {
+    LnAdd<T> add{static_cast<const T*>(residual), static_cast<T*>(h), mask_mode != 0 ? mask : nullptr, 1.f - p, 1.f / (1.f - p), seed, offset, clear_flag};
+    rc = mask_mode != 0 ? ln_fwd_launch<T, T, LN_ADD_RNG>(x, gamma, beta, z, mu, rsigma, rows, hidden, eps, st, add)
+                        : ln_fwd_launch<T, T, LN_ADD>(x, gamma, beta, z, mu, rsigma, rows, hidden, eps, st, add);
+  });
+  if (rc) return rc;
+  NMTG_CHECK_LAUNCH("add_ln_fwd");
+  return 0;
+}
+
+extern "C" int nmtg_ln_bwd_add(const void* dz, const void* x, const float* mu, const float* rsigma, const void* gamma, const void* grad_residual,
+                               const uint8_t* guard_mask, const uint8_t* keep_mask, float p, void* dx, void* dy, void* dgamma, void* dbeta,
+                               float* dgamma_part, float* dbeta_part, int64_t n_part, int64_t rows, int64_t hidden, int dtype, void* stream) {
+  NMTG_REQUIRE(gamma && dgamma && dbeta && dgamma_part && dbeta_part, "ln_bwd_add: null pointer argument");
+  NMTG_REQUIRE(rows == 0 || (dz && x && mu && rsigma && dx && grad_residual), "ln_bwd_add: null pointer argument");
+  NMTG_REQUIRE((keep_mask == nullptr) == (dy == nullptr), "ln_bwd_add: keep_mask and dy go together");
+  NMTG_REQUIRE(keep_mask == nullptr || (p >= 0.f && p < 1.f), "ln_bwd_add: dropout probability %f outside [0, 1)", p);
+  NMTG_REQUIRE(rows >= 0 && hidden > 0 && hidden <= (1 << 30), "ln_bwd_add: bad shape rows=%lld hidden=%lld", (long long)rows, (long long)hidden);
+  NMTG_REQUIRE(n_part >= 1 && n_part <= (1 << 20), "ln_bwd_add: n_part=%lld out of range", (long long)n_part);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  int rc = 0;
+  NMTG_DISPATCH_DTYPE(dtype, T, {
+    LnRes<T> res{static_cast<const T*>(grad_residual), guard_mask, keep_mask, 1.f / (1.f - p), static_cast<T*>(dy)};
+    auto go = [&](auto res_tag, auto drop_tag) {
+      return ln_bwd_launch<T, T, decltype(res_tag)::value, decltype(drop_tag)::value>(dz, x, mu, rsigma, gamma, nullptr, dx, dgamma, dbeta, dgamma_part,
+                                                                                      dbeta_part, n_part, rows, hidden, false, st, res);
+    };
+    using one = std::integral_constant<int, 1>;
+    using two = std::integral_constant<int, 2>;
+    if (guard_mask != nullptr) rc = keep_mask != nullptr ? go(two{}, std::true_type{}) : go(two{}, std::false_type{});
+    else rc = keep_mask != nullptr ? go(one{}, std::true_type{}) : go(one{}, std::false_type{});
+  });
+  if (rc) return rc;
+  NMTG_CHECK_LAUNCH("ln_bwd_add");
   return 0;
 }

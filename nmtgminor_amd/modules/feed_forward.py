@@ -16,6 +16,7 @@ import torch
 from torch import nn
 from torch.nn import Parameter
 
+from .. import _lib as L
 from . import mlp as fused
 from .dropout_add import fused_dropout_add
 from .glu import gated_activation_dropout
@@ -39,6 +40,7 @@ class PositionWiseFeedForward(nn.Module):
         self.bias, self.glu, self.variational, self.weight_drop = True, glu, variational, weight_drop
         self.dropout_residual, self.res_dropout = dropout_residual, res_dropout
         self.fused, self.fused_function = not glu, fns.get(activation)
+        self.activation_code = L.ACT_CODES.get("silu" if activation == "swish" else activation)
         self.in_proj_weight = Parameter(torch.empty(inner_size * (2 if glu else 1), model_size))
         self.out_proj_weight = Parameter(torch.empty(model_size, inner_size))
         self.in_proj_bias = Parameter(torch.empty(inner_size * (2 if glu else 1)))

@@ -21,10 +21,14 @@ from ..native import flash_attn_cuda as fa
 from .rotary import _linear, _linear_bwd
 
 
+def switched_on():
+    return os.environ.get("NMTG_ATTN_FLASH_TRAIN", "1") != "0"
+
+
 def eligible(is_training, return_coverage, recompute, x, heads):
     if not is_training or return_coverage or recompute:
         return False
-    if os.environ.get("NMTG_ATTN_FLASH_TRAIN", "1") == "0":
+    if not switched_on():
         return False
     e = x.shape[-1]
     return x.dtype in (torch.float16, torch.bfloat16) and x.dim() == 3 and e % heads == 0 and e // heads in (64, 128)

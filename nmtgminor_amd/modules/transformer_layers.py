@@ -16,9 +16,13 @@ of this package and asking for them raises.
 import torch
 from torch import nn
 
+from .. import _lib as L
+from ..native import flash_attn_cuda
+from . import feed_forward, flash_core
 from .encdec_attention import EncdecMultiheadAttn
 from .feed_forward import PositionWiseFeedForward
-from .pre_post_processing import PrePostProcessing
+from .layer_norm import LayerNorm
+from .pre_post_processing import Bottle, PrePostProcessing
 from .self_attention import SelfMultiheadAttn
 
 
@@ -102,6 +106,55 @@ class _Layer(nn.Module):
         return self.postprocess_ffn(self._times(out, self._scaled_ffn_scale()), input)
 
 
+    # -- the layer as one node of the host layer (csrc/host/layers.cpp) -------------------------------------------------
+    # Taken by the plain form: 16-bit tensors on the GPU, LayerNorm with affine parameters in front, dropout + add behind,
+    # no gate, no variational dropout, no stochastic depth, no macaron block, no hooks on the sub-modules, and either
+    # training with a backward to come or evaluation without one. Everything else runs operator by operator below.
+    _PRE, _POST = ["n"], ["d", "a"]
+
+    def _sub_parameters(self, pre, mods):
+        """The parameters of the sub-modules in the order of the native layer, or None where one is not of the plain form."""
+        t, out = self.training, []
+        for name in mods:
+            m = self._modules.get(name)
+            if m is None or m.training is not t or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks:
+                return None
+            kind = type(m)
+            if kind is PrePostProcessing:
+                if name in pre:
+                    n = m._modules["layer_norm"] if m.steps == self._PRE else None
+                    n = n._modules["function"] if type(n) is Bottle else None
+                    if type(n) is not LayerNorm or n.eps != 1e-5 or n.memory_efficient or n._forward_hooks or n._forward_pre_hooks:
+                        return None
+                    out += [n._parameters["weight"], n._parameters["bias"]]
+                elif m.steps != self._POST or m.variational or type(m._modules["dropout"]) is not nn.Dropout \
+                        or m._modules["dropout"].p != m.dropout_p or m.dropout_p != self.postprocess_ffn.dropout_p:
+                    return None
+            elif kind is SelfMultiheadAttn:
+                if m.rotary_pos_enc or m.head_dim not in (64, 128):
+                    return None
+                p = m._parameters
+                out += [p["in_proj_weight"], p["in_proj_bias"], p["out_proj_weight"], p["out_proj_bias"]]
+            elif kind is EncdecMultiheadAttn:
+                p = m._parameters
+                out += [p["in_proj_weight_q"], p["in_proj_weight_kv"], p["out_proj_weight"]]
+            elif kind is PositionWiseFeedForward:
+                if m.glu or m.variational or m.dropout_residual or m.fused_function is None:
+                    return None
+                p = m._parameters
+                out += [p["in_proj_weight"], p["in_proj_bias"], p["out_proj_weight"], p["out_proj_bias"]]
+            else:
+                return None
+        return out
+
+    def _native_mode(self, x, inputs, params):
+        if params is None or self.macaron or self.death_rate > 0 or feed_forward.recompute or torch.is_autocast_enabled() \
+                or not flash_core.switched_on():
+            return 0
+        mode = L.host().layer_mode(x, inputs, params)
+        return mode if (mode == 2) is self.training else 0
+
+
 class EncoderLayer(_Layer):
     """forward(input [T, B, model_size], attn_mask: key-padding mask [B, T], nonzero = padded) -> [T, B, model_size]."""
 
@@ -112,8 +165,29 @@ class EncoderLayer(_Layer):
         self._ffn_blocks(opt)
         self.multihead = SelfMultiheadAttn(opt.model_size, opt.n_heads, opt.attn_dropout)
 
+    _SUB = ("preprocess_attn", "multihead", "postprocess_attn", "preprocess_ffn", "feedforward", "postprocess_ffn")
+
+    def _native_forward(self, x, attn_mask):
+        params = self._sub_parameters(("preprocess_attn", "preprocess_ffn"), self._SUB)
+        mode = self._native_mode(x, (), params)
+        if mode == 0:
+            return None
+        host, train = L.host(), self.training
+        mh, ff = self._modules["multihead"], self._modules["feedforward"]
+        heads = mh.num_heads
+        p_attn, p_res, p_ffn = (mh.dropout, self._modules["postprocess_ffn"].dropout_p, ff.dropout) if train else (0.0, 0.0, 0.0)
+        x = x.contiguous()
+        pad = host.mask_bytes(attn_mask, x.shape[1], x.shape[0])
+        z, stats, lin, q, k, v = host.layer_begin(x, *params[:4], heads)
+        ctx, lse, state = flash_attn_cuda.fwd_batched(q, k, v, pad, p_attn, mh.head_dim ** -0.5, False)
+        return host.encoder_end(x, z, stats, lin, ctx, lse, state, pad, params, heads, ff.activation_code, p_attn, p_res, p_ffn, mode == 2)
+
     def forward(self, input, attn_mask):
         if self._alive():
+            if input.is_cuda:
+                out = self._native_forward(input, attn_mask)
+                if out is not None:
+                    return out
             input = self._macaron_step(input)
             query = self.preprocess_attn(input)
             out, _ = self.multihead(query, None, attn_mask, None, return_coverage=False)    # the coverage is dropped here
@@ -141,11 +215,40 @@ class DecoderLayer(_Layer):
             self.multihead_src = EncdecMultiheadAttn(opt.n_heads, opt.model_size, opt.attn_dropout)
         self._ffn_blocks(opt)
 
+    _SUB = ("preprocess_attn", "multihead_tgt", "postprocess_attn", "preprocess_src_attn", "multihead_src", "postprocess_src_attn",
+            "preprocess_ffn", "feedforward", "postprocess_ffn")
+
+    def _native_forward(self, x, context, mask_tgt, mask_src):
+        params = self._sub_parameters(("preprocess_attn", "preprocess_src_attn", "preprocess_ffn"), self._SUB)
+        mode = self._native_mode(x, (context,), params)
+        if mode == 0 or context.dim() != 3 or context.shape[0] > 4096 or context.shape[1:] != x.shape[1:]:
+            return None
+        host, train = L.host(), self.training
+        mh, mc, ff = self._modules["multihead_tgt"], self._modules["multihead_src"], self._modules["feedforward"]
+        heads = mh.num_heads
+        if mc.num_heads != heads:
+            return None
+        p_attn, p_cross, p_res, p_ffn = ((mh.dropout, mc.dropout, self._modules["postprocess_ffn"].dropout_p, ff.dropout) if train
+                                         else (0.0, 0.0, 0.0, 0.0))
+        x = x.contiguous()
+        time = None
+        if mask_tgt is not None:
+            time = host.mask_bytes(mask_tgt if mask_tgt.dtype in (torch.bool, torch.uint8) else mask_tgt.to(torch.bool), x.shape[0], x.shape[0])
+        pad = host.mask_bytes(mask_src, context.shape[1], context.shape[0])
+        z, stats, lin, q, k, v = host.layer_begin(x, *params[:4], heads)
+        ctx, lse, state = flash_attn_cuda.fwd_batched(q, k, v, None, p_attn, mh.head_dim ** -0.5, False, time_mask=time)
+        return host.decoder_end(x, context, z, stats, lin, ctx, lse, state, time, pad, params, heads, ff.activation_code, p_attn, p_cross,
+                                p_res, p_ffn, mode == 2)
+
     def forward(self, input, context, mask_tgt, mask_src, incremental=False, incremental_cache=None, reuse_source=True):
         if incremental and incremental_cache is None:
             incremental_cache = dict()
         coverage = None
         if self._alive():
+            if input.is_cuda and not incremental and not self.ignore_source and context is not None:
+                native = self._native_forward(input, context, mask_tgt, mask_src)
+                if native is not None:
+                    return native[0], native[1], incremental_cache
             input = self._macaron_step(input)
             query = self.preprocess_attn(input)
             out, _ = self.multihead_tgt(query, None, None, mask_tgt, incremental=incremental,

@@ -178,6 +178,8 @@ def fwd_batched(q, k, v, key_padding_mask, dropout_p, softmax_scale, causal, *, 
     time_mask uint8 [len_q, len_k] or None (one of the two at most)
     -> (out [len_q, B, H, D] contiguous, softmax_lse [B, H, len_q], state); `state` goes to bwd_batched as it is (dropout
     mode, Philox pair, explicit mask, keep bits, drawn mask when want_mask)."""
+    if q.is_cuda and dropout_mask is None and rng is None and not want_mask:
+        return L.host().flash_fwd_batched(q, k, v, key_padding_mask, time_mask, dropout_p, softmax_scale, bool(causal))
     L.require_cuda(q, k, v)
     _check(q.dtype in (torch.float16, torch.bfloat16) and k.dtype == q.dtype and v.dtype == q.dtype,
            "flash_attn: q, k and v must share a 16-bit dtype")

@@ -1,0 +1,186 @@
+"""The layers as one native node (csrc/host/layers.cpp) against the same layer run operator by operator (a forward hook on a
+sub-module keeps a layer on that path), and the kernels it adds (LayerNorm over a residual sum and its backward, the guarded
+dropout + add) against the separate ones, at the edges of their shapes."""
+import math
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from nmtgminor_amd import _lib as L
+from nmtgminor_amd.modules.transformer_layers import DecoderLayer, EncoderLayer
+from nmtgminor_amd.native import fast_layer_norm_cuda as ln
+from util import assert_close, rel_err
+
+pytestmark = pytest.mark.gpu
+F16, BF16, F32 = torch.float16, torch.bfloat16, torch.float32
+
+
+def options(e, p, act):
+    return SimpleNamespace(model_size=e, inner_size=2 * e, n_heads=e // 64, dropout=p, attn_dropout=p, variational_dropout=False,
+                           macaron=False, rezero=False, ffn_activation=act, ffn_glu=False, fast_self_attention=True,
+                           fast_xattention=True, fast_feed_forward=True, ignore_source=False)
+
+
+def randomised(layer, dev, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    with torch.no_grad():
+        for p in layer.parameters():
+            p.add_((0.1 if p.dim() == 1 else 0.02) * torch.randn(p.shape, generator=g))
+    return layer.to(dev).to(dtype)
+
+
+def both_paths(layer, hooked, call, inputs, dy):
+    """[outputs and gradients] of the native path and of the operator-by-operator one, with the same dropout masks"""
+    res = []
+    for by_operator in (False, True):
+        handle = hooked.register_forward_hook(lambda m, i, o: None) if by_operator else None
+        torch.manual_seed(3)
+        torch.cuda.manual_seed(5)
+        for t in list(inputs) + list(layer.parameters()):
+            t.grad = None
+        out = call()
+        out = out if isinstance(out, tuple) else (out,)
+        if dy is not None:
+            out[0].backward(dy)
+        res.append([o for o in out if torch.is_tensor(o)] + ([t.grad for t in inputs] + [p.grad for p in layer.parameters()] if dy is not None else []))
+        if handle is not None:
+            handle.remove()
+    return res
+
+
+def same(pair, dtype):
+    """The two paths round at the same points; where their kernels sum in another order a rounding may fall the other way."""
+    for a, b in zip(*pair):
+        assert (a is None) == (b is None)
+        if a is not None:
+            assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(torch.isnan(a), torch.isnan(b))
+            assert rel_err(torch.nan_to_num(a), torch.nan_to_num(b)) < (1e-2 if dtype == BF16 else 2e-3)
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("t,b,e,p,act,train", [(1, 1, 128, 0.1, "relu", True), (37, 13, 512, 0.1, "gelu", True), (130, 3, 256, 0.0, "silu", True),
+                                               (64, 2, 1024, 0.1, "relu", True), (33, 5, 512, 0.1, "relu", False)])
+def test_encoder_layer(dev, dtype, t, b, e, p, act, train):
+    layer = randomised(EncoderLayer(options(e, p, act)), dev, dtype, 1).train(train)
+    x = torch.randn(t, b, e, device=dev).to(dtype).requires_grad_(train)
+    pad = torch.arange(t, device=dev)[None] >= torch.randint((t + 1) // 2, t + 1, (b,), device=dev)[:, None]
+    dy = torch.randn(t, b, e, device=dev).to(dtype)
+    with torch.set_grad_enabled(train):
+        same(both_paths(layer, layer.feedforward, lambda: layer(x, pad), [x] if train else [], dy if train else None), dtype)
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("tq,tk,b,e,p,train", [(1, 4, 1, 128, 0.1, True), (61, 73, 6, 512, 0.1, True), (129, 64, 3, 256, 0.0, True),
+                                               (31, 100, 4, 512, 0.1, False), (5, 61, 2, 128, 0.0, False)])
+def test_decoder_layer(dev, dtype, tq, tk, b, e, p, train):
+    layer = randomised(DecoderLayer(options(e, p, "gelu")), dev, dtype, 2).train(train)
+    x = torch.randn(tq, b, e, device=dev).to(dtype).requires_grad_(train)
+    c = torch.randn(tk, b, e, device=dev).to(dtype).requires_grad_(train)
+    pad = torch.arange(tk, device=dev)[None] >= torch.randint((tk + 1) // 2, tk + 1, (b,), device=dev)[:, None]
+    causal = torch.triu(torch.ones(tq, tq, device=dev), 1).bool()
+    dy = torch.randn(tq, b, e, device=dev).to(dtype)
+    with torch.set_grad_enabled(train):
+        same(both_paths(layer, layer.feedforward, lambda: layer(x, c, causal, pad), [x, c] if train else [], dy if train else None), dtype)
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("bad", [math.inf, -math.inf, math.nan])
+def test_a_stream_that_is_not_finite_is_clamped_and_its_gradient_stops(dev, dtype, bad):
+    layer = randomised(EncoderLayer(options(128, 0.1, "relu")), dev, dtype, 4).train()
+    x = torch.randn(9, 3, 128, device=dev).to(dtype)
+    x[2, 1, 5] = 65000.0 if dtype == F16 else 3e38            # above fp16's bound: clamped with the rest of the tensor
+    with torch.no_grad():
+        layer.feedforward.out_proj_bias[7] = bad
+    x.requires_grad_()
+    pad = torch.zeros(3, 9, dtype=torch.bool, device=dev)
+    pair = both_paths(layer, layer.feedforward, lambda: layer(x, pad), [x], torch.randn(9, 3, 128, device=dev).to(dtype))
+    out = pair[0][0]
+    assert torch.equal(torch.nan_to_num(out, nan=0.5), torch.nan_to_num(pair[1][0], nan=0.5))
+    if not math.isnan(bad):
+        assert torch.isfinite(out).all() and out.abs().max().item() >= 64512
+    same([pair[0][1:], pair[1][1:]], dtype)
+
+
+def add_ln(x, r, gamma, beta, p, seed):
+    rows, hidden = x.shape
+    h, z = torch.empty_like(x), torch.empty_like(x)
+    mask = torch.full((rows, hidden), 9, dtype=torch.uint8, device=x.device)
+    mu, rs = torch.empty(rows, device=x.device), torch.empty(rows, device=x.device)
+    flag = torch.ones(1, dtype=torch.int32, device=x.device)
+    import ctypes
+    L.call("nmtg_add_ln_fwd", L.ptr(x), L.ptr(r), L.ptr(h), L.ptr(mask), L.i32(2 if p else 0), L.f32(p), ctypes.c_uint64(seed), ctypes.c_uint64(8),
+           L.ptr(flag), L.ptr(gamma), L.ptr(beta), L.ptr(z), L.ptr(mu), L.ptr(rs), L.i64(rows), L.i64(hidden), L.f32(1e-5),
+           L.i32(L.dtype_code(x)), L.stream_of(x))
+    assert flag.item() == 0
+    return h, mask, z, mu, rs
+
+
+@pytest.mark.parametrize("dtype", [F32, F16, BF16])
+@pytest.mark.parametrize("rows,hidden", [(1, 8), (5, 7), (3, 520), (67, 512), (9, 2056), (2, 8200)])
+@pytest.mark.parametrize("p", [0.0, 0.25])
+def test_layer_norm_over_a_residual_sum(dev, dtype, rows, hidden, p):
+    import ctypes
+    g = torch.Generator().manual_seed(rows * hidden)
+    mk = lambda *s: torch.randn(*s, generator=g).to(dtype).to(dev)
+    x, r, gamma, beta, dz, dr = mk(rows, hidden), mk(rows, hidden), mk(hidden), mk(hidden), mk(rows, hidden), mk(rows, hidden)
+    h, mask, z, mu, rs = add_ln(x, r, gamma, beta, p, 77)
+    want_h, want_mask = x.clone(), torch.ones(rows, hidden, dtype=torch.uint8, device=dev)
+    L.call("nmtg_dropout_add_fwd", L.ptr(want_h), L.ptr(r), L.ptr(want_mask), L.i64(x.numel()), L.f32(p), L.i32(2 if p else 0), ctypes.c_uint64(77),
+           ctypes.c_uint64(8), L.i32(L.dtype_code(x)), L.stream_of(x))
+    assert torch.equal(h, want_h)
+    if p:
+        assert torch.equal(mask, want_mask)
+    want_z, want_mu, want_rs = ln.ln_fwd(want_h, gamma, beta, 1e-5)
+    for a, b in ((z, want_z), (mu, want_mu), (rs, want_rs)):         # the compiler fuses a multiply-add here or there
+        assert rel_err(a, b) < 1e-4
+    # backward: the LayerNorm's gradient plus the stream's (not where the guard byte says so), and the dropped branch's
+    guard = (torch.rand(rows, hidden, generator=g) < 0.2).to(torch.uint8).mul_(2).to(dev)
+    keep = (torch.rand(rows, hidden, generator=g) < 0.7).to(torch.uint8).to(dev)
+    plain = ln.ln_bwd(dz, h, mu, rs, gamma, None, False)
+    parts = plain[3].shape[0]
+    for use_guard in (False, True):
+        for drop in (False, True):
+            dx, dy, dg, db = torch.empty_like(x), torch.empty_like(x), torch.empty_like(gamma), torch.empty_like(gamma)
+            part = torch.empty(2, parts, hidden, device=dev)
+            L.call("nmtg_ln_bwd_add", L.ptr(dz), L.ptr(h), L.ptr(mu), L.ptr(rs), L.ptr(gamma), L.ptr(dr), L.ptr(guard if use_guard else None),
+                   L.ptr(keep if drop else None), L.f32(0.25), L.ptr(dx), L.ptr(dy if drop else None), L.ptr(dg), L.ptr(db), L.ptr(part[0]),
+                   L.ptr(part[1]), L.i64(parts), L.i64(rows), L.i64(hidden), L.i32(L.dtype_code(x)), L.stream_of(x))
+            want = plain[0] + (dr.masked_fill(guard != 0, 0.0) if use_guard else dr)
+            assert torch.equal(dg, plain[1]) and torch.equal(db, plain[2])
+            assert rel_err(dx, want) < 1e-4                            # a fused multiply-add here or there
+            assert_close(dx, want.double().cpu(), dtype, "dx", atol=1e-5)
+            if drop:
+                assert_close(dy, want.double().cpu() * keep.cpu() / 0.75, dtype, "dy", atol=1e-5 if dtype == F32 else None)
+
+
+@pytest.mark.parametrize("dtype", [F32, F16, BF16])
+@pytest.mark.parametrize("n", [1, 7, 4096, 70003])
+def test_guarded_dropout_add(dev, dtype, n):
+    import ctypes
+    g = torch.Generator().manual_seed(n)
+    x, r = torch.randn(n, generator=g).to(dtype).to(dev), torch.randn(n, generator=g).to(dtype).to(dev)
+    for p in (0.0, 0.5):
+        for bad in (None, math.inf, math.nan):
+            src = r.clone()
+            if bad is not None:
+                src[n // 2] = bad
+                if dtype == F16:
+                    src[n - 1] = 65504.0 if n > 1 else bad
+            want, mask = x.clone(), torch.ones(n, dtype=torch.uint8, device=dev)
+            L.call("nmtg_dropout_add_fwd", L.ptr(want), L.ptr(src), L.ptr(mask), L.i64(n), L.f32(p), L.i32(2 if p else 0), ctypes.c_uint64(5),
+                   ctypes.c_uint64(4), L.i32(L.dtype_code(x)), L.stream_of(x))
+            ref = want.clone().requires_grad_()
+            out = ref * 1.0
+            if not bool(torch.isfinite(out).all()):
+                out = out.clamp(-(torch.finfo(dtype).max - 1000), torch.finfo(dtype).max - 1000)
+            out.backward(torch.ones_like(out))
+            got, gm = x.clone(), torch.empty(n, dtype=torch.uint8, device=dev)
+            flag = torch.zeros(1, dtype=torch.int32, device=dev)
+            L.call("nmtg_dropout_add_guard_fwd", L.ptr(got), L.ptr(src), L.ptr(gm), L.i64(n), L.f32(p), L.i32(2 if p else 0), ctypes.c_uint64(5),
+                   ctypes.c_uint64(4), L.ptr(flag), L.i32(L.dtype_code(x)), L.stream_of(x))
+            assert torch.equal(torch.nan_to_num(got, nan=0.25), torch.nan_to_num(out.detach(), nan=0.25))
+            assert torch.equal(gm & 1, mask) and torch.equal((gm & 2) == 0, ref.grad != 0)
+            dx = torch.empty_like(x)
+            L.call("nmtg_dropout_add_guard_bwd", L.ptr(r), L.ptr(gm), L.ptr(dx), L.i64(n), L.f32(p), L.i32(L.dtype_code(x)), L.stream_of(x))
+            assert_close(dx, r.double().cpu() * (gm == 1).cpu() / (1 - p), dtype, "dx")
