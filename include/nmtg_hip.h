@@ -508,6 +508,15 @@ int nmtg_attn_decode(const void* q, int64_t q_stride_b, const void* keys, int64_
                      int64_t batch, int64_t heads, int64_t head_dim, int64_t tk, float scale,
                      int dtype, void* stream);
 
+/* The self-attention of a decoding step in one launch: projection [batch, heads, 3, head_dim] of the new position (q, k, v) is
+ * attended over cache rows 0 .. position - 1 and itself, and its key / value are written into cache row `position`. The
+ * probabilities are not returned. The rest as nmtg_attn_decode. */
+int nmtg_attn_decode_append(const void* projection, int64_t projection_stride_b, void* keys,
+                            int64_t k_stride_t, int64_t k_stride_b, void* values, int64_t v_stride_t,
+                            int64_t v_stride_b, void* context, int64_t ctx_stride_b, int64_t batch,
+                            int64_t heads, int64_t head_dim, int64_t position, float scale, int dtype,
+                            void* stream);
+
 /* ------------------------------------------------------------------------------------------
  * Gated feed-forward activation with dropout.
  * Reference: the gated branch of PositionWiseFeedForward.forward, PyTorch ops there

@@ -24,6 +24,8 @@ struct DecArgs {
   int64_t q_sb, k_st, k_sb, v_st, v_sb, c_sb;   // element strides: per sentence (sb) and per key position (st)
   int heads, tk;
   float scale;
+  const void* fresh;      // append form: the new position's projection [batch, heads, 3, head_dim] (q, k, v), else null
+  int64_t fresh_sb;
 };
 
 template <typename T>
@@ -41,8 +43,10 @@ __device__ __forceinline__ float block_reduce(float v, bool is_max, float* red) 
   return r;
 }
 
-// LPR lanes share one key row: head_dim = 8 * LPR
-template <typename T, int LPR>
+// LPR lanes share one key row: head_dim = 8 * LPR.
+// APPEND: the step's own position comes straight from its projection (query, and key / value of cache row tk - 1), and the
+// block that owns the head writes that row into the cache: two copies and the query's re-layout are no launches of their own.
+template <typename T, int LPR, bool APPEND>
 __global__ __launch_bounds__(DEC_THREADS) void attn_decode_kernel(DecArgs a) {
   extern __shared__ __align__(16) float lds[];
   float* sc = lds;                       // [tk]
@@ -52,9 +56,15 @@ __global__ __launch_bounds__(DEC_THREADS) void attn_decode_kernel(DecArgs a) {
   const int tid = threadIdx.x, slot = tid / LPR, c = tid % LPR;
   const int64_t head_off = static_cast<int64_t>(h) * D + 8 * c;
   uint32_t qw[4];
+  const T* fresh = APPEND ? static_cast<const T*>(a.fresh) + b * a.fresh_sb + static_cast<int64_t>(h) * 3 * D + 8 * c : nullptr;
   {
-    const pack<T, 8> qraw = load_raw<T, 8>(static_cast<const T*>(a.q) + b * a.q_sb + head_off);
+    const pack<T, 8> qraw = load_raw<T, 8>(APPEND ? fresh : static_cast<const T*>(a.q) + b * a.q_sb + head_off);
     __builtin_memcpy(qw, &qraw, 16);
+  }
+  if (APPEND && slot == 0) {
+    const int64_t row = static_cast<int64_t>(a.tk - 1);
+    *reinterpret_cast<pack<T, 8>*>(const_cast<T*>(static_cast<const T*>(a.keys)) + row * a.k_st + b * a.k_sb + head_off) = load_raw<T, 8>(fresh + D);
+    *reinterpret_cast<pack<T, 8>*>(const_cast<T*>(static_cast<const T*>(a.values)) + row * a.v_st + b * a.v_sb + head_off) = load_raw<T, 8>(fresh + 2 * D);
   }
   const T* kb = static_cast<const T*>(a.keys) + b * a.k_sb + head_off;
   const T* vb = static_cast<const T*>(a.values) + b * a.v_sb + head_off;
@@ -77,7 +87,8 @@ __global__ __launch_bounds__(DEC_THREADS) void attn_decode_kernel(DecArgs a) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int j = j0 + u * RPS + slot;
-      raw[u] = load_raw<T, 8>(kb + static_cast<int64_t>(j < live ? j : 0) * a.k_st);
+      const T* src = kb + static_cast<int64_t>(j < live ? j : 0) * a.k_st;
+      raw[u] = load_raw<T, 8>(APPEND && (j >= a.tk - 1) ? fresh + D : src);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -111,7 +122,7 @@ __global__ __launch_bounds__(DEC_THREADS) void attn_decode_kernel(DecArgs a) {
   T* pr = static_cast<T*>(a.probs) + static_cast<int64_t>(bh) * a.tk;
   for (int j = tid; j < a.tk; j += DEC_THREADS) {
     const T p = elem<T>::from_float(sc[j] * inv);
-    pr[j] = p;
+    if (a.probs != nullptr) pr[j] = p;
     sc[j] = elem<T>::to_float(p);
   }
   __syncthreads();
@@ -123,7 +134,8 @@ __global__ __launch_bounds__(DEC_THREADS) void attn_decode_kernel(DecArgs a) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int j = j0 + u * RPS + slot;
-      raw[u] = load_raw<T, 8>(vb + static_cast<int64_t>(j < live ? j : 0) * a.v_st);
+      const T* src = vb + static_cast<int64_t>(j < live ? j : 0) * a.v_st;
+      raw[u] = load_raw<T, 8>(APPEND && (j >= a.tk - 1) ? fresh + 2 * D : src);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -154,18 +166,18 @@ __global__ __launch_bounds__(DEC_THREADS) void attn_decode_kernel(DecArgs a) {
   }
 }
 
-template <typename T>
+template <typename T, bool APPEND>
 int decode_launch(const DecArgs& a, int head_dim, int64_t blocks, hipStream_t st) {
   const int lds = (a.tk + 4 + 4 * head_dim) * static_cast<int>(sizeof(float));
   TraceScope trace("attn_decode", st);
 #define DEC_LAUNCH(LPR)                                                                                                   \
   {                                                                                                                       \
     if (lds > 64 * 1024) {                                                                                                \
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(attn_decode_kernel<T, LPR>),                      \
+      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(attn_decode_kernel<T, LPR, APPEND>),              \
                                          hipFuncAttributeMaxDynamicSharedMemorySize, lds);                                \
       if (e != hipSuccess) return fail(NMTG_ERR_LAUNCH, "attn_decode: cannot reserve %d bytes of LDS", lds);              \
     }                                                                                                                     \
-    hipLaunchKernelGGL((attn_decode_kernel<T, LPR>), dim3(static_cast<unsigned>(blocks)), dim3(DEC_THREADS), lds, st, a); \
+    hipLaunchKernelGGL((attn_decode_kernel<T, LPR, APPEND>), dim3(static_cast<unsigned>(blocks)), dim3(DEC_THREADS), lds, st, a); \
   }
   if (head_dim == 32) DEC_LAUNCH(4)
   else if (head_dim == 64) DEC_LAUNCH(8)
@@ -199,9 +211,36 @@ extern "C" int nmtg_attn_decode(const void* q, int64_t q_stride_b, const void* k
   a.q_sb = q_stride_b; a.k_st = k_stride_t; a.k_sb = k_stride_b; a.v_st = v_stride_t; a.v_sb = v_stride_b; a.c_sb = ctx_stride_b;
   a.heads = static_cast<int>(heads); a.tk = static_cast<int>(tk); a.scale = scale;
   int rc;
-  if (dtype == NMTG_F16) rc = decode_launch<f16_t>(a, static_cast<int>(head_dim), batch * heads, static_cast<hipStream_t>(stream));
-  else rc = decode_launch<bf16_t>(a, static_cast<int>(head_dim), batch * heads, static_cast<hipStream_t>(stream));
+  if (dtype == NMTG_F16) rc = decode_launch<f16_t, false>(a, static_cast<int>(head_dim), batch * heads, static_cast<hipStream_t>(stream));
+  else rc = decode_launch<bf16_t, false>(a, static_cast<int>(head_dim), batch * heads, static_cast<hipStream_t>(stream));
   if (rc) return rc;
   NMTG_CHECK_LAUNCH("attn_decode");
+  return 0;
+}
+
+extern "C" int nmtg_attn_decode_append(const void* projection, int64_t projection_stride_b, void* keys, int64_t k_stride_t, int64_t k_stride_b,
+                                       void* values, int64_t v_stride_t, int64_t v_stride_b, void* context, int64_t ctx_stride_b, int64_t batch,
+                                       int64_t heads, int64_t head_dim, int64_t position, float scale, int dtype, void* stream) {
+  NMTG_REQUIRE(batch >= 0 && heads >= 1 && position >= 0 && batch * heads <= 0x7fffffff, "attn_decode_append: bad shape batch=%lld heads=%lld position=%lld",
+               (long long)batch, (long long)heads, (long long)position);
+  NMTG_REQUIRE(head_dim == 32 || head_dim == 64 || head_dim == 128, "attn_decode_append: head dimension %lld (32, 64 and 128 are built)",
+               (long long)head_dim);
+  NMTG_REQUIRE(dtype == NMTG_F16 || dtype == NMTG_BF16, "attn_decode_append: fp16 or bf16 tensors required");
+  NMTG_REQUIRE(position < DEC_MAX_KEYS, "attn_decode_append: position %lld, at most %d keys (the scores of a row are kept in LDS)", (long long)position,
+               DEC_MAX_KEYS);
+  if (batch == 0) return 0;
+  NMTG_REQUIRE(projection && keys && values && context, "attn_decode_append: null pointer argument");
+  const int64_t strides[] = {projection_stride_b, k_stride_t, k_stride_b, v_stride_t, v_stride_b, ctx_stride_b};
+  for (int64_t s : strides) NMTG_REQUIRE(s % 8 == 0 && s >= 0, "attn_decode_append: strides must be non-negative multiples of 8 elements");
+  NMTG_REQUIRE(aligned16(projection) && aligned16(keys) && aligned16(values) && aligned16(context), "attn_decode_append: 16-byte aligned tensors required");
+  DecArgs a = {};
+  a.keys = keys; a.values = values; a.ctx = context; a.fresh = projection; a.fresh_sb = projection_stride_b;
+  a.k_st = k_stride_t; a.k_sb = k_stride_b; a.v_st = v_stride_t; a.v_sb = v_stride_b; a.c_sb = ctx_stride_b;
+  a.heads = static_cast<int>(heads); a.tk = static_cast<int>(position) + 1; a.scale = scale;
+  int rc;
+  if (dtype == NMTG_F16) rc = decode_launch<f16_t, true>(a, static_cast<int>(head_dim), batch * heads, static_cast<hipStream_t>(stream));
+  else rc = decode_launch<bf16_t, true>(a, static_cast<int>(head_dim), batch * heads, static_cast<hipStream_t>(stream));
+  if (rc) return rc;
+  NMTG_CHECK_LAUNCH("attn_decode_append");
   return 0;
 }

@@ -76,6 +76,10 @@ __global__ __launch_bounds__(DA_THREADS) void dropout_add_fwd_kernel(
 // NaN). Bandwidth bound like the plain form: 16.4 us at [512 x 32 x 1024] bf16 against 39 us for the two reductions it
 // replaces, and no host round trip.
 // ---------------------------------------------------------------------------------------------------------------------
+template <typename T> __device__ __forceinline__ float guard_limit();
+template <> __device__ __forceinline__ float guard_limit<float>() { return INFINITY; }
+template <> __device__ __forceinline__ float guard_limit<bf16_t>() { return 3.3895313892515355e38f; }
+template <> __device__ __forceinline__ float guard_limit<f16_t>() { return 65504.f; }
 __device__ __forceinline__ bool guard_element(bf16_t& o) {
   if ((o.bits & 0x7f80u) != 0x7f80u) return false;
   if ((o.bits & 0x7fu) == 0) o.bits = static_cast<uint16_t>((o.bits & 0x8000u) | 0x7f7fu);
@@ -90,20 +94,10 @@ __device__ __forceinline__ bool guard_element(float& o) {
 __device__ __forceinline__ bool guard_element(f16_t& o) { return (o.bits & 0x7c00u) == 0x7c00u; }
 
 template <typename T, int EPV, int MODE>
-__global__ __launch_bounds__(DA_THREADS) void dropout_add_guard_kernel(
-    T* __restrict__ x, const T* __restrict__ residual, uint8_t* __restrict__ mask, int64_t n, float keep_p,
-    float scale, uint64_t seed, uint64_t offset, int* __restrict__ flag) {
-  const int64_t first = (static_cast<int64_t>(blockIdx.x) * DA_THREADS + threadIdx.x) * EPV;
-  if (first >= n) return;
-  const int count = static_cast<int>(min(static_cast<int64_t>(EPV), n - first));
-  pack<T, EPV> rawx, rawr;
-  if (count == EPV) {
-    rawx = load_raw<T, EPV>(x + first);
-    rawr = load_raw<T, EPV>(residual + first);
-    pin_raw(rawx); pin_raw(rawr);
-  } else {
-    for (int j = 0; j < EPV; ++j) { rawx.v[j] = x[first + (j < count ? j : 0)]; rawr.v[j] = residual[first + (j < count ? j : 0)]; }
-  }
+__device__ __forceinline__ void guard_pack(T* __restrict__ x, const T* __restrict__ residual, uint8_t* __restrict__ mask, int64_t first,
+                                           float keep_p, float scale, uint64_t seed, uint64_t offset, int* __restrict__ flag) {
+  pack<T, EPV> rawx = load_raw<T, EPV>(x + first), rawr = load_raw<T, EPV>(residual + first);
+  pin_raw(rawx); pin_raw(rawr);
   float xv[EPV], rv[EPV];
   unpack_raw<T, EPV>(rawx, xv);
   unpack_raw<T, EPV>(rawr, rv);
@@ -114,20 +108,38 @@ __global__ __launch_bounds__(DA_THREADS) void dropout_add_guard_kernel(
 #pragma unroll
     for (int j = 0; j < EPV; ++j) keep[j] = 1;
   }
-  pack<T, EPV> out;
+#pragma unroll
+  for (int j = 0; j < EPV; ++j) xv[j] = rv[j] + (keep[j] ? xv[j] * scale : 0.f);
+  // one comparison per element (false for NaN); only a pack with an element at or beyond the largest finite value looks closer
   bool any = false;
 #pragma unroll
-  for (int j = 0; j < EPV; ++j) {
-    const float v = rv[j] + (keep[j] ? xv[j] * scale : 0.f);
-    out.v[j] = elem<T>::from_float(v);
-    if (guard_element(out.v[j])) { keep[j] |= 2; any = true; }
+  for (int j = 0; j < EPV; ++j) any = any || !(fabsf(xv[j]) < guard_limit<T>());
+  if (any) {
+    for (int j = 0; j < EPV; ++j) {
+      T o = elem<T>::from_float(xv[j]);
+      if (guard_element(o)) {
+        keep[j] |= 2;
+        if (flag != nullptr) *flag = 1;
+      }
+      x[first + j] = o;
+      if (mask != nullptr) mask[first + j] = keep[j];
+    }
+    return;
   }
-  if (sizeof(T) == 2 && any && flag != nullptr) *flag = 1;
-  if (count == EPV) {
-    *reinterpret_cast<pack<T, EPV>*>(x + first) = out;
-    if (mask != nullptr) store_bytes<EPV>(mask + first, keep);
-  } else {
-    for (int j = 0; j < count; ++j) { x[first + j] = out.v[j]; if (mask != nullptr) mask[first + j] = keep[j]; }
+  store_pack<T, EPV>(x + first, xv);
+  if (mask != nullptr) store_bytes<EPV>(mask + first, keep);
+}
+
+template <typename T, int EPV, int MODE>
+__global__ __launch_bounds__(DA_THREADS) void dropout_add_guard_kernel(
+    T* __restrict__ x, const T* __restrict__ residual, uint8_t* __restrict__ mask, int64_t n, float keep_p,
+    float scale, uint64_t seed, uint64_t offset, int* __restrict__ flag) {
+  const int64_t first = (static_cast<int64_t>(blockIdx.x) * DA_THREADS + threadIdx.x) * EPV;
+  if (first >= n) return;
+  if (first + EPV <= n) {
+    guard_pack<T, EPV, MODE>(x, residual, mask, first, keep_p, scale, seed, offset, flag);
+  } else {  // ragged tail: scalar
+    for (int64_t e = first; e < n; ++e) guard_pack<T, 1, MODE>(x, residual, mask, e, keep_p, scale, seed, offset, flag);
   }
 }
 

@@ -15,6 +15,8 @@ namespace nmtg {
 namespace {
 
 constexpr int SK_ROWS = 32, SK_COLS = 32, SK_WAVES = 8, SK_THREADS = 64 * SK_WAVES, SK_CHUNK = 128;
+// Two row blocks (a batch of 64 hypotheses) re-read W from L2 and still leave the 128 x 128 tile far behind.
+constexpr int SK_MAX_ROWS = 64;
 
 template <typename T>
 __global__ __launch_bounds__(SK_THREADS) void gemm_skinny_kernel(const GemmArgs g) {
@@ -27,7 +29,8 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_skinny_kernel(const GemmArgs 
   // this wavefront's share of k: whole 16-k steps, dealt out in chunks of 128 so that the loads in flight stay bounded
   const int steps = (g.K + 15) / 16, per = (steps + SK_WAVES - 1) / SK_WAVES;
   const int k_begin = wave * per * 16, k_end = min(g.K, (wave + 1) * per * 16);
-  const int m = lane & 31, n = n0 + (lane & 31);
+  const int m0 = static_cast<int>(blockIdx.y) * SK_ROWS;
+  const int m = m0 + (lane & 31), n = n0 + (lane & 31);
   const T* xrow = X + static_cast<int64_t>(m) * g.lda + 8 * half;
   const T* wrow = W + static_cast<int64_t>(n) * g.ldb + 8 * half;
   acc16_t acc;
@@ -54,7 +57,7 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_skinny_kernel(const GemmArgs 
     float v = 0.f;
 #pragma unroll
     for (int w = 0; w < SK_WAVES; ++w) v += part[w][r][l];
-    const int row = 8 * (r / 4) + 4 * (l >> 5) + r % 4, col = n0 + (l & 31);
+    const int row = m0 + 8 * (r / 4) + 4 * (l >> 5) + r % 4, col = n0 + (l & 31);
     if (row < g.M && col < g.N) {
       v *= g.alpha;
       if (g.bias != nullptr) v += elem<T>::to_float(static_cast<const T*>(g.bias)[col]);
@@ -70,15 +73,15 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_skinny_kernel(const GemmArgs 
 bool gemm_skinny_ok(int dtype, int layout, int epi, const GemmArgs& a) {
   if (switched_off("NMTG_GEMM_SKINNY")) return false;
   return (dtype == NMTG_F16 || dtype == NMTG_BF16) && layout == LAYOUT_NT && epi == EPI_PLAIN && a.batch == 1 && a.M >= 1 &&
-         a.M <= SK_ROWS && a.N >= 64 && a.K >= 8 && a.K % 8 == 0 && a.lda % 8 == 0 && a.ldb % 8 == 0 && aligned16(a.A) &&
+         a.M <= SK_MAX_ROWS && a.N >= 64 && a.K >= 8 && a.K % 8 == 0 && a.lda % 8 == 0 && a.ldb % 8 == 0 && aligned16(a.A) &&
          aligned16(a.B);
 }
 
 int gemm_skinny_run(int dtype, const GemmArgs& a, hipStream_t st) {
-  const unsigned grid = static_cast<unsigned>((a.N + SK_COLS - 1) / SK_COLS);
+  const dim3 grid(static_cast<unsigned>((a.N + SK_COLS - 1) / SK_COLS), static_cast<unsigned>((a.M + SK_ROWS - 1) / SK_ROWS));
   TraceScope trace("gemm_nt_skinny", st);
-  if (dtype == NMTG_F16) hipLaunchKernelGGL((gemm_skinny_kernel<f16_t>), dim3(grid), dim3(SK_THREADS), 0, st, a);
-  else hipLaunchKernelGGL((gemm_skinny_kernel<bf16_t>), dim3(grid), dim3(SK_THREADS), 0, st, a);
+  if (dtype == NMTG_F16) hipLaunchKernelGGL((gemm_skinny_kernel<f16_t>), grid, dim3(SK_THREADS), 0, st, a);
+  else hipLaunchKernelGGL((gemm_skinny_kernel<bf16_t>), grid, dim3(SK_THREADS), 0, st, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(NMTG_ERR_LAUNCH, "gemm: launch failed: %s", hipGetErrorString(e));
   return 0;

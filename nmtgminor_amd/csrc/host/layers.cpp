@@ -233,6 +233,28 @@ struct DecoderNode : Function<DecoderNode> {
   }
 };
 
+// One step of incremental decoding: x [1, B, E], self-attention over the n cached positions and the new one (which is written
+// into row n of the buffers), cross-attention over the cached encoder keys / values, feed-forward block.
+std::tuple<Tensor, Tensor> decoder_step(const Tensor& x, const Tensor& kbuf, const Tensor& vbuf, int64_t n, const Tensor& ck, const Tensor& cv,
+                                        const Tensor& pad, const std::vector<Tensor>& w, int64_t heads, int64_t act) {
+  const int64_t b = x.size(1), e = x.size(2), d = e / heads, tk = ck.size(0);
+  const float scale = static_cast<float>(1.0 / std::sqrt(static_cast<double>(d)));
+  Launch on(x);
+  Norm n1 = ln_fwd(x, w[0], w[1], kEps);
+  Tensor lin = linear_fwd(n1.z, w[2], w[3]);
+  Tensor cx = at::empty_like(x);
+  check(api.attn_decode_append(ptr(lin), 3 * e, ptr(kbuf), kbuf.stride(0), kbuf.stride(1), ptr(vbuf), vbuf.stride(0), vbuf.stride(1), ptr(cx), e, b,
+                               heads, d, n, scale, dtype_code(x), on.stream), "nmtg_attn_decode_append");
+  AddNorm n2 = add_ln_fwd(linear_fwd(cx, w[4], w[5]), x, 0.0, Tensor(), w[6], w[7], kEps);
+  Tensor q = linear_fwd(n2.z, w[8], Tensor());
+  Tensor coverage = empty_like_sized(x, {b * heads, 1, tk});
+  check(api.attn_decode(ptr(q), e, ptr(ck), ck.stride(0), ck.stride(1), ptr(cv), cv.stride(0), cv.stride(1),
+                        static_cast<const uint8_t*>(ptr(pad)), ptr(coverage), ptr(cx), e, b, heads, d, tk, scale, dtype_code(x), on.stream),
+        "nmtg_attn_decode");
+  FfnState f = ffn_fwd(linear_fwd(cx, w[10], Tensor()), n2.h, 0.0, w[11], w[12], w[13], w[14], w[15], w[16], act, 0.0, 0.0, false);
+  return {f.out, coverage};
+}
+
 using State = std::tuple<int64_t, uint64_t, uint64_t, optional<Tensor>, optional<Tensor>, optional<Tensor>>;
 using Params = std::vector<Tensor>;
 
@@ -282,6 +304,12 @@ void define_layers(pybind11::module_& m) {
       return EncoderNode::compute(in, x, w[4], w[5], w[6], w[7], w[8], w[9], w[10], w[11], &keep).out;
     }
     return EncoderNode::apply(&in, x, w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7], w[8], w[9], w[10], w[11]);
+  });
+  m.def("decoder_step", [](const Tensor& x, const Tensor& kbuf, const Tensor& vbuf, int64_t n, const Tensor& ck, const Tensor& cv,
+                           const optional<Tensor>& pad, const Params& w, int64_t heads, int64_t act) {
+    at::AutoDispatchBelowADInplaceOrView off;
+    auto r = decoder_step(contiguous(x), kbuf, vbuf, n, ck, cv, defined_or(pad), w, heads, act);
+    return std::make_tuple(std::get<0>(r), std::get<1>(r), kbuf.narrow(0, 0, n + 1), vbuf.narrow(0, 0, n + 1));
   });
   // -> (output, coverage)
   m.def("decoder_end", [](const Tensor& x, const Tensor& context, const Tensor& z1, const Tensor& stats1, const Tensor& lin, const Tensor& cx,

@@ -95,7 +95,13 @@ def _append(cache, name, row):
     caller leaves that tensor in place, a step writes one row. A caller that replaces cache[name] (beam search re-indexes
     every entry along dimension 1, which yields new tensors) gets a fresh buffer filled from it: the reference's copy,
     with room for the steps that follow."""
-    old = cache[name]
+    buf, n = _room(cache[name])
+    buf[n:n + 1].view(row.shape).copy_(row)       # `row` may be the strided [1, B*H, D] slice of the projection
+    return _grown(buf, buf[:n + 1])
+
+
+def _room(old):
+    """(buffer, n): the buffer that holds the n rows of cache entry `old` and has room for one more"""
     n = old.shape[0]
     buf = getattr(old, "_nmtg_buffer", None)
     in_place = (buf is not None and buf.shape[0] > n and buf.shape[1:] == old.shape[1:] and buf.dtype == old.dtype
@@ -103,10 +109,35 @@ def _append(cache, name, row):
     if not in_place:
         buf = old.new_empty((max(2 * n, n + 64),) + tuple(old.shape[1:]))
         buf[:n].copy_(old)
-    buf[n:n + 1].view(row.shape).copy_(row)       # `row` may be the strided [1, B*H, D] slice of the projection
-    grown = buf[:n + 1]
-    grown._nmtg_buffer = buf
-    return grown
+    return buf, n
+
+
+def _grown(buf, rows):
+    rows._nmtg_buffer = buf
+    return rows
+
+
+def layer_step(layer_step_fn, x, params, heads, act, mask, cache):
+    """One position through a whole decoder layer on the cache-streaming kernels (csrc/host/layers.cpp, decoder_step), or None
+    where an operand is not of the form they take. mask: key padding of the encoder positions."""
+    k, v, ck, cv = (cache.get(name) for name in ("k", "v", "c_k", "c_v"))
+    if k is None or v is None or ck is None or cv is None or x.shape[0] != 1:
+        return None
+    e, b = x.shape[2], x.shape[1]
+    if any(t.dtype != x.dtype or t.dim() != 3 or t.shape[1:] != x.shape[1:] for t in (k, v, ck, cv)) or v.shape != k.shape \
+            or not (k.is_contiguous() and v.is_contiguous()) or not _decode_ok(x, ck, cv, heads) or not _decode_ok(x, k, v, heads):
+        return None
+    if mask is not None:
+        mask = mask.squeeze(1) if mask.dim() == 3 else mask
+        if mask.shape != (b, ck.shape[0]):
+            return None
+        mask = mask.contiguous()
+        mask = mask.view(torch.uint8) if mask.dtype == torch.bool else mask.to(torch.uint8)
+    kbuf, n = _room(k)
+    vbuf, _ = _room(v)
+    out, coverage, k, v = layer_step_fn(x, kbuf, vbuf, n, ck, cv, mask, params, heads, act)
+    cache["k"], cache["v"] = _grown(kbuf, k), _grown(vbuf, v)
+    return out, coverage
 
 
 @torch.no_grad()

@@ -18,7 +18,7 @@ from torch import nn
 
 from .. import _lib as L
 from ..native import flash_attn_cuda
-from . import feed_forward, flash_core
+from . import feed_forward, flash_core, incremental as incremental_steps
 from .encdec_attention import EncdecMultiheadAttn
 from .feed_forward import PositionWiseFeedForward
 from .layer_norm import LayerNorm
@@ -240,11 +240,24 @@ class DecoderLayer(_Layer):
         return host.decoder_end(x, context, z, stats, lin, ctx, lse, state, time, pad, params, heads, ff.activation_code, p_attn, p_cross,
                                 p_res, p_ffn, mode == 2)
 
+    def _native_step(self, x, mask_tgt, mask_src, cache):
+        params = self._sub_parameters(("preprocess_attn", "preprocess_src_attn", "preprocess_ffn"), self._SUB)
+        if mask_tgt is not None or self._native_mode(x, (), params) != 1:
+            return None
+        heads = self._modules["multihead_tgt"].num_heads
+        if self._modules["multihead_src"].num_heads != heads:
+            return None
+        return incremental_steps.layer_step(L.host().decoder_step, x, params, heads, self._modules["feedforward"].activation_code, mask_src, cache)
+
     def forward(self, input, context, mask_tgt, mask_src, incremental=False, incremental_cache=None, reuse_source=True):
         if incremental and incremental_cache is None:
             incremental_cache = dict()
         coverage = None
         if self._alive():
+            if input.is_cuda and incremental and not self.ignore_source:
+                native = self._native_step(input, mask_tgt, mask_src, incremental_cache)
+                if native is not None:
+                    return native[0], native[1], incremental_cache
             if input.is_cuda and not incremental and not self.ignore_source and context is not None:
                 native = self._native_forward(input, context, mask_tgt, mask_src)
                 if native is not None:

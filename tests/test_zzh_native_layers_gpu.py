@@ -85,6 +85,34 @@ def test_decoder_layer(dev, dtype, tq, tk, b, e, p, train):
 
 
 @pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("b,tk,prev,e", [(1, 1, 2, 128), (5, 61, 24, 512), (33, 130, 64, 256), (64, 300, 70, 1024), (3, 1500, 255, 128)])
+def test_decoding_step(dev, dtype, b, tk, prev, e):
+    """Three steps in a row: the cache grows inside its buffer, into a new buffer, and from entries the caller replaced."""
+    layer = randomised(DecoderLayer(options(e, 0.1, "relu")), dev, dtype, 6).eval()
+    c = torch.randn(tk, b, e, device=dev).to(dtype)
+    pad = torch.arange(tk, device=dev)[None] >= torch.randint((tk + 1) // 2, tk + 1, (b,), device=dev)[:, None]
+    steps = torch.randn(3, 1, b, e, device=dev).to(dtype)
+    prefix = torch.randn(prev, b, e, device=dev).to(dtype)
+    res = []
+    for by_operator in (False, True):
+        handle = layer.feedforward.register_forward_hook(lambda m, i, o: None) if by_operator else None
+        cache, outs = {}, []
+        with torch.no_grad():
+            layer(prefix, c, torch.triu(torch.ones(prev, prev, device=dev), 1).bool(), pad, incremental=True, incremental_cache=cache)
+            for i in range(3):
+                if i == 2:
+                    order = torch.randperm(b, generator=torch.Generator().manual_seed(1)).to(dev)
+                    for name in list(cache):
+                        cache[name] = cache[name].index_select(1, order)
+                out, coverage, cache = layer(steps[i], c, None, pad, incremental=True, incremental_cache=cache)
+                outs += [out, coverage, cache["k"].clone(), cache["v"].clone()]
+        res.append(outs)
+        if handle is not None:
+            handle.remove()
+    same(res, dtype)
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
 @pytest.mark.parametrize("bad", [math.inf, -math.inf, math.nan])
 def test_a_stream_that_is_not_finite_is_clamped_and_its_gradient_stops(dev, dtype, bad):
     layer = randomised(EncoderLayer(options(128, 0.1, "relu")), dev, dtype, 4).train()
