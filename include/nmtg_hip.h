@@ -638,6 +638,8 @@ int nmtg_rel_softmax_dropout_bwd(const void* grad_dropped, const void* scores, c
  * nmtg_multi_tensor_l2norm: norm[0] = sqrt(sum over all tensors of x^2); per_tensor[t] (may be NULL)
  *   = the norm of tensor t; both fp32 on the device; deterministic (fixed-order sums). workspace: fp32
  *   scratch of nmtg_multi_tensor_l2norm_workspace_bytes(n_tensors, sizes) bytes.
+ * nmtg_multi_tensor_clip: x *= min(1, max_norm / (norm[0] + 1e-6)) in place, norm in device memory (as
+ *   nmtg_multi_tensor_l2norm leaves it); nothing is written where the factor is 1.
  * nmtg_multi_tensor_l2norm_scale: the same norms of `in` (unscaled) while writing out = in * scale in
  *   the same pass (multi_tensor_l2norm_scale_kernel.cu:28-125); same workspace.
  * ------------------------------------------------------------------------------------------ */
@@ -658,6 +660,9 @@ int64_t nmtg_multi_tensor_l2norm_workspace_bytes(int n_tensors, const int64_t* s
 int nmtg_multi_tensor_l2norm(int n_tensors, const void* const* x, const int64_t* sizes, float* norm,
                              float* per_tensor, void* workspace, int64_t workspace_bytes, int dtype,
                              void* stream);
+
+int nmtg_multi_tensor_clip(int n_tensors, void* const* x, const int64_t* sizes, const float* norm, float max_norm,
+                           int dtype, void* stream);
 
 int nmtg_multi_tensor_l2norm_scale(int n_tensors, const void* const* in, void* const* out,
                                    const int64_t* sizes, float scale, float* norm, float* per_tensor,

@@ -1,6 +1,6 @@
 // Shared pieces of the native host layer (nmtgminor_amd/_host.so): the table of C entry points it calls, and the
 // operators as functions from tensors to tensors (allocate the results, enqueue the kernels). ops.cpp implements them,
-// autograd.cpp wraps them in autograd nodes, layers.cpp composes the transformer layers.
+// autograd.cpp wraps them in autograd nodes, layers.cpp composes the transformer layers, optim.cpp prepares the optimizer's passes.
 //
 // Why it exists: a call through the Python stand-ins costs 25 to 80 us of interpreter, ctypes and autograd bookkeeping per
 // operator and direction, several times what the kernels of a small batch take. The same work here is 3 to 8 us.
@@ -26,7 +26,8 @@ using std::optional;
   X(attn_decode) X(attn_decode_append) X(encdec_attn_bwd_workspace_bytes) X(encdec_attn_bwd_from_probs)                                                    \
   X(xentropy_bwd) X(gemm) X(mlp_fwd) X(mlp_bwd_dtype_workspace_bytes) X(mlp_bwd) X(flash_attn_dropout_bits_bytes)     \
   X(flash_attn_fwd) X(flash_attn_bwd) X(flash_attn_key_info_bytes) X(flash_attn_time_info_bytes)                      \
-  X(flash_attn_batched_fwd) X(flash_attn_batched_bwd)
+  X(flash_attn_batched_fwd) X(flash_attn_batched_bwd) X(multi_tensor_adam) X(multi_tensor_clip)                       \
+  X(multi_tensor_l2norm) X(multi_tensor_l2norm_workspace_bytes)
 
 struct Api {
 #define X(name) decltype(&nmtg_##name) name = nullptr;
@@ -105,5 +106,6 @@ Tensor pad_bytes(const optional<Tensor>& mask, int64_t rows, int64_t cols);
 
 void define_autograd(pybind11::module_& m);
 void define_layers(pybind11::module_& m);
+void define_optim(pybind11::module_& m);
 
 }  // namespace nmtg_host

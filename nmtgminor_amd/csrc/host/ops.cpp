@@ -300,4 +300,5 @@ PYBIND11_MODULE(_host, m) {
   m.def("bind", &nmtg_host::bind);
   nmtg_host::define_autograd(m);
   nmtg_host::define_layers(m);
+  nmtg_host::define_optim(m);
 }

@@ -4,6 +4,7 @@ instead of one small kernel per parameter. Same result as torch.nn.utils.clip_gr
 gradients that are not on the GPU have no HIP path and raise (the reference falls back to a per-tensor loop there)."""
 import torch
 
+from .. import _lib as L
 from ..native import fused_optim
 from .fused_adam import multi_tensor_applier
 
@@ -13,8 +14,13 @@ def fused_clip_grad_norm(parameters, max_norm, norm_type=2.0, error_if_nonfinite
     max_norm <= 0). -> the joint norm before clipping (fp32 tensor on the gradients' device)."""
     if isinstance(parameters, torch.Tensor):
         parameters = [parameters]
-    parameters = [p for p in parameters if p.grad is not None]
     max_norm, norm_type = float(max_norm), float(norm_type)
+    parameters = list(parameters)
+    if norm_type == 2.0 and not error_if_nonfinite and parameters and parameters[0].is_cuda:
+        total_norm = L.host().clip_grad_norm(parameters, max_norm)      # None: gradients of several dtypes, or ones it refuses
+        if total_norm is not None:
+            return total_norm
+    parameters = [p for p in parameters if p.grad is not None]
     if len(parameters) == 0:
         return torch.tensor(0.)
     if norm_type != 2.0:
@@ -39,9 +45,7 @@ def fused_clip_grad_norm(parameters, max_norm, norm_type=2.0, error_if_nonfinite
                            'clipped. To disable this error and scale the gradients by the non-finite norm anyway, set '
                            '`error_if_nonfinite=False`')
     if max_norm > 0:
-        # the clipping factor is computed in fp32 like the reference's tensor expression; reading it back is the one
-        # host synchronisation of the function (the reference's float conversion of the same tensor)
-        clip_coef = float(torch.clamp(max_norm / (total_norm + 1e-6), max=1.0))
+        # the clipping factor is computed in fp32 like the reference's tensor expression, in the kernel
         for grads in by_dtype.values():
-            multi_tensor_applier(fused_optim.multi_tensor_scale, dummy_overflow_buf, [grads, grads], clip_coef)
+            multi_tensor_applier(fused_optim.multi_tensor_clip, dummy_overflow_buf, [grads], total_norm, max_norm)
     return total_norm

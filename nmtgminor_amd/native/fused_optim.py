@@ -1,6 +1,6 @@
 """Stand-in for the reference's extension module `fused_optim` (onmt/modules/extensions/fused_optim/frontend.cpp:45-53):
 multi_tensor_adam, multi_tensor_scale, multi_tensor_axpby, multi_tensor_l2norm and multi_tensor_l2norm_scale with the
-reference's argument lists (chunk_size, noop_flag, tensor_lists, ...). `chunk_size` is accepted and not used: the kernels
+reference's argument lists (chunk_size, noop_flag, tensor_lists, ...), and multi_tensor_clip of the same form. `chunk_size` is accepted and not used: the kernels
 work in chunks of 32768 elements."""
 import ctypes
 
@@ -77,6 +77,19 @@ def multi_tensor_l2norm(chunk_size, noop_flag, tensor_lists, per_tensor=False):
     L.call("nmtg_multi_tensor_l2norm", L.i32(n), _ptr_array(xs), sizes, L.ptr(norm), L.ptr(each if per_tensor else None), L.ptr(ws),
            L.i64(ws_bytes), L.i32(L.dtype_code(xs[0])), L.stream_of(xs[0]))
     return norm, each
+
+
+def multi_tensor_clip(chunk_size, noop_flag, tensor_lists, norm, max_norm):
+    """tensor_lists = [tensors], scaled in place by min(1, max_norm / (norm + 1e-6)); norm (fp32 device tensor) is read by the
+    kernel, so the host waits for nothing."""
+    n = _lists(tensor_lists, 1, "multi_tensor_clip")
+    if n == 0:
+        return
+    xs = tensor_lists[0]
+    _check(norm.dtype == torch.float32 and norm.numel() >= 1, "multi_tensor_clip: norm must be an fp32 tensor")
+    L.require_cuda(norm)
+    L.call("nmtg_multi_tensor_clip", L.i32(n), _ptr_array(xs), _size_array(xs), L.ptr(norm), L.f32(max_norm), L.i32(L.dtype_code(xs[0])),
+           L.stream_of(xs[0]))
 
 
 def multi_tensor_axpby(chunk_size, noop_flag, tensor_lists, a, b, arg_to_check):
