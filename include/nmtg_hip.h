@@ -190,6 +190,16 @@ int nmtg_xentropy_bwd(const float* grad_loss, const void* logits, const float* l
                       int64_t total_classes, float smoothing, int64_t padding_idx, int dtype,
                       void* stream);
 
+/* nmtg_xentropy_bwd over whole rows (fp16 / bf16) that also writes colsum [vocab] (dtype), the sums of the rounded
+ * gradients over the rows: the bias gradient of the projection in front. 16-byte aligned bases and pitches.
+ * grad_stride: 1, or 0 where one gradient value serves all rows. part: fp32 scratch of
+ * nmtg_xentropy_bwd_colsum_parts(rows) x vocab floats. */
+int64_t nmtg_xentropy_bwd_colsum_parts(int64_t rows);
+int nmtg_xentropy_bwd_colsum(const float* grad_loss, int64_t grad_stride, const void* logits, const float* lse,
+                             const int64_t* labels, void* grad_logits, void* colsum, float* part, int64_t rows,
+                             int64_t vocab, int64_t ld_logits, int64_t ld_grad, float smoothing, int64_t padding_idx,
+                             int dtype, void* stream);
+
 /* ------------------------------------------------------------------------------------------
  * Strided-batched GEMM on the MFMA units (fp16 / bf16 in and out, fp32 accumulation), row-major:
  *   C[b] = alpha * op(A[b]) * op(B[b]) (+ bias[n]),   op(A) is m x k, op(B) is k x n.
@@ -202,7 +212,7 @@ int nmtg_xentropy_bwd(const float* grad_loss, const void* logits, const float* l
  *   (multihead_attn_blaslt/strided_batched_gemm_blaslt.cuh:9-126); also linear_blaslt
  *   (mlp_blaslt/linear.cpp:142-144).
  * workspace (may be NULL): fp32 scratch of nmtg_gemm_workspace_bytes(m, n, k, batch) bytes; with
- *   it a (1,0) product with a long reduction is split over the chip (deterministic reduction).
+ *   it a (1,0) or (0,0) product with a long reduction and no bias is split over the chip (deterministic reduction).
  * ------------------------------------------------------------------------------------------ */
 int64_t nmtg_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k, int64_t batch);
 

@@ -12,7 +12,7 @@ bool gemm_has(int layout, int tile, int epi) {
     return (tile == TILE_L || tile == TILE_M) && (epi == EPI_PLAIN || epi == EPI_ACT_FWD || epi == EPI_SCORES);
   if (layout == LAYOUT_NN) {
     if (epi == EPI_PLAIN) return true;
-    return epi == EPI_ACT_BWD && (tile == TILE_L || tile == TILE_M);
+    return (epi == EPI_ACT_BWD || epi == EPI_SPLITK) && (tile == TILE_L || tile == TILE_M);
   }
   if (layout == LAYOUT_TN) {
     if (epi == EPI_PLAIN) return true;
@@ -39,7 +39,8 @@ struct SplitPlan {
   int tile, splits, k_per_split;
 };
 
-// Weight-gradient style products (small output, long reduction): spread the reduction over
+// Products of a small output and a long reduction (weight gradients over the tokens, the gradient of the states over a
+// vocabulary): spread the reduction over
 // enough blocks to occupy the chip; partial tiles go through an fp32 workspace.
 SplitPlan plan_splitk(int M, int N, int K, int batch) {
   const int cus = num_cus();
@@ -116,7 +117,7 @@ int gemm_run(int dtype, int layout, int epi, GemmArgs a, void* workspace, size_t
   a.splits = 1;
   a.k_per_split = ceil_div(std::max(a.K, 1), GEMM_BK) * GEMM_BK;
 
-  if (layout == LAYOUT_TN && epi == EPI_PLAIN && workspace != nullptr) {
+  if (layout != LAYOUT_NT && epi == EPI_PLAIN && workspace != nullptr && a.bias == nullptr) {
     const SplitPlan p = plan_splitk(a.M, a.N, a.K, a.batch);
     if (p.splits > 1 && (p.tile != TILE_L || vec == 8) && splitk_ws_bytes(p, a.M, a.N, a.batch) <= workspace_bytes &&
         (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0) {
@@ -149,12 +150,13 @@ int gemm_run(int dtype, int layout, int epi, GemmArgs a, void* workspace, size_t
   }
   if (!gemm_has(layout, tile, epi))
     return fail(NMTG_ERR_UNSUPPORTED, "gemm: layout %d has no kernel for epilogue %d", layout, epi);
-  // The slot-ring kernel (direct global -> LDS loads) needs whole 64-k steps (k_per_split is a multiple of 64 already),
-  // 16-byte accesses, and 32-bit lane offsets inside one tile of an operand: 256 rows of a reduction-contiguous one, 64
+  // The slot-ring kernel (direct global -> LDS loads) needs whole 64-k steps where gemm_ring_ragged<> (gemm_inst.hip.h) has
+  // no kernel for a last partial one (k_per_split is a multiple of 64), 16-byte accesses, and 32-bit lane offsets inside one tile of an operand: 256 rows of a reduction-contiguous one, 64
   // k-rows plus a row of the other kind. Every other call takes the two-buffer loop.
   const int64_t a_span = a_kc ? 256 * a.lda * 2 : 64 * a.lda * 2 + static_cast<int64_t>(a.M) * 2;
   const int64_t b_span = b_kc ? 256 * a.ldb * 2 : 64 * a.ldb * 2 + static_cast<int64_t>(a.N) * 2;
-  a.ring = (a.K > 0 && a.K % GEMM_BK == 0 && vec == 8 && a_span < (int64_t{1} << 32) && b_span < (int64_t{1} << 32)) ? 1 : 0;
+  const bool whole = a.K % GEMM_BK == 0 || (layout != LAYOUT_NT && (epi == EPI_PLAIN || epi == EPI_SPLITK));
+  a.ring = (a.K > 0 && whole && vec == 8 && a_span < (int64_t{1} << 32) && b_span < (int64_t{1} << 32)) ? 1 : 0;
   // gelu and gelu' of the activation epilogues come from a table in LDS in the ring kernels (they have the LDS room)
   a.act_lut = (a.ring && (epi == EPI_ACT_FWD || epi == EPI_ACT_BWD)) ? 1 : 0;
   int bm, bn;

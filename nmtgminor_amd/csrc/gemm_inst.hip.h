@@ -57,14 +57,20 @@ template <int TILE, bool A_KC, bool B_KC, int EPI> struct ring_rider {
   static constexpr bool value = TILE == TILE_M && A_KC && !B_KC && EPI == EPI_PLAIN;
 };
 
-template <typename T, int TILE, bool A_KC, bool B_KC, int EPI>
+// Which kernels exist for a reduction that ends inside a 64-k step too: the weight and data gradients, whose reduction is the
+// token count or the vocabulary (the forward's is a model dimension).
+template <bool B_KC, int EPI> struct gemm_ring_ragged {
+  static constexpr bool value = !B_KC && (EPI == EPI_PLAIN || EPI == EPI_SPLITK);
+};
+
+template <typename T, int TILE, bool A_KC, bool B_KC, int EPI, bool RAGGED = false>
 int gemm_launch_ring(const GemmArgs& a, hipStream_t st) {
   using C = tile_cfg<TILE>;
   constexpr int RING = ring_slots<TILE>::value;
   constexpr bool RIDER = ring_rider<TILE, A_KC, B_KC, EPI>::value;
   auto kern = [] {
-    if constexpr (RIDER) return gemm_ring_rider_kernel<T, C::BM, C::BN, C::WM, C::WN, A_KC, B_KC, EPI, RING, ring_stepbuf<TILE>::value>;
-    else return gemm_ring_kernel<T, C::BM, C::BN, C::WM, C::WN, A_KC, B_KC, EPI, RING, ring_stepbuf<TILE>::value>;
+    if constexpr (RIDER) return gemm_ring_rider_kernel<T, C::BM, C::BN, C::WM, C::WN, A_KC, B_KC, EPI, RING, ring_stepbuf<TILE>::value, RAGGED>;
+    else return gemm_ring_kernel<T, C::BM, C::BN, C::WM, C::WN, A_KC, B_KC, EPI, RING, ring_stepbuf<TILE>::value, RAGGED>;
   }();
   constexpr int lds = gemm_ring_lds_bytes<C::BM, C::BN, RING>();
   static bool attr_done = false;
@@ -96,7 +102,12 @@ int gemm_launch_ring(const GemmArgs& a, hipStream_t st) {
 // The 256x256 tile exists for 16-byte accesses only; narrower calls are routed to the smaller tiles.
 template <typename T, int TILE, bool A_KC, bool B_KC, int EPI>
 int gemm_launch_one(const GemmArgs& a, hipStream_t st) {
-  if (a.vec == 8 && a.ring) return gemm_launch_ring<T, TILE, A_KC, B_KC, EPI>(a, st);
+  if (a.vec == 8 && a.ring) {
+    if constexpr (gemm_ring_ragged<B_KC, EPI>::value) {
+      if (a.K % GEMM_BK != 0) return gemm_launch_ring<T, TILE, A_KC, B_KC, EPI, true>(a, st);
+    }
+    return gemm_launch_ring<T, TILE, A_KC, B_KC, EPI>(a, st);
+  }
   if (a.vec == 8) return gemm_launch_vec<T, TILE, A_KC, B_KC, EPI, 8>(a, st);
   if constexpr (TILE != TILE_L) {
     if (a.vec == 4) return gemm_launch_vec<T, TILE, A_KC, B_KC, EPI, 4>(a, st);

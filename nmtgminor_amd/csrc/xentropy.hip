@@ -18,6 +18,9 @@
 // Bandwidth bound: forward reads N*V elements once; backward reads them once and writes N*V
 // (rows whose label is the padding index are written as zeros without reading the logits).
 #include "common.hip.h"
+#include "reduce.hip.h"
+
+#include <algorithm>
 
 namespace nmtg {
 namespace {
@@ -266,6 +269,67 @@ __global__ __launch_bounds__(XE_THREADS) void xentropy_bwd_kernel(
   for (int64_t c = tail0 + tid; c < vocab; c += XE_THREADS) one(c);
 }
 
+// The backward with the column sums of its result (the bias gradient of the output projection). A block owns XC_COLS
+// columns of `rows_per_block` rows and walks down the rows, a lane's eight columns summed in registers, so the gradient is
+// not read again for the sums; per-row values are wavefront-uniform loads. 16-bit types, 16-byte aligned rows.
+// 4096 rows of 250 054 classes in bf16: 815 + 11 us (5.0 TB/s); the row kernel above took 795 and the column sums of its
+// result another 575.
+constexpr int XC_THREADS = 256;
+constexpr int XC_COLS = XC_THREADS * 8;
+constexpr int XC_INFLIGHT = 8;          // rows in flight per lane: 16 bytes each
+constexpr int XC_ROWS = 128;            // rows per block; few enough that the partial rows are a 64th of the gradient's bytes
+
+template <typename T>
+__global__ __launch_bounds__(XC_THREADS) void xentropy_bwd_colsum_kernel(
+    const float* __restrict__ grad_loss, int64_t grad_stride, const T* logits, const float* __restrict__ lse_in,
+    const int64_t* __restrict__ labels, T* grad_logits, float* __restrict__ part, int rows, int rows_per_block, int64_t vocab,
+    int64_t ld, int64_t ld_grad, float smoothing, int64_t padding_idx) {
+  static_assert(sizeof(T) == 2, "a lane moves eight 16-bit elements");
+  const int r0 = blockIdx.y * rows_per_block, r1 = min(rows, r0 + rows_per_block);
+  const int64_t c0 = static_cast<int64_t>(blockIdx.x) * XC_COLS + threadIdx.x * 8;
+  if (c0 >= vocab) return;
+  const int valid = static_cast<int>(min(static_cast<int64_t>(8), vocab - c0));   // the last lane's vector ends in the pitch
+  const float sm = smoothing / static_cast<float>(vocab), onem = 1.f - smoothing;
+  float sum[8] = {};
+  const T* x = logits + c0;
+  T* dx = grad_logits + c0;
+  auto row = [&](int r, const pack<T, 8>& raw) {
+    const int64_t label = labels[r];
+    const bool padded = label == padding_idx;
+    const float g = padded ? 0.f : grad_loss[r * grad_stride], nlse = -lse_in[r] * LOG2E;
+    float v[8];
+    unpack_raw<T, 8>(raw, v);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = __builtin_amdgcn_exp2f(fmaf(v[j], LOG2E, nlse)) - sm;
+    if (label >= c0 && label < c0 + 8) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) if (c0 + j == label) v[j] -= onem;
+    }
+    pack<T, 8> out;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      out.v[j] = elem<T>::from_float(padded ? 0.f : g * v[j]);      // exact zeros, whatever the logits hold
+      sum[j] += elem<T>::to_float(out.v[j]);
+    }
+    T* to = dx + static_cast<int64_t>(r) * ld_grad;
+    if (valid == 8) *reinterpret_cast<pack<T, 8>*>(to) = out;
+    else for (int j = 0; j < valid; ++j) to[j] = out.v[j];
+  };
+  int r = r0;
+  for (; r + XC_INFLIGHT <= r1; r += XC_INFLIGHT) {
+    pack<T, 8> raw[XC_INFLIGHT];
+#pragma unroll
+    for (int u = 0; u < XC_INFLIGHT; ++u) raw[u] = load_raw<T, 8>(x + static_cast<int64_t>(r + u) * ld);
+#pragma unroll
+    for (int u = 0; u < XC_INFLIGHT; ++u) pin_raw(raw[u]);
+#pragma unroll
+    for (int u = 0; u < XC_INFLIGHT; ++u) row(r + u, raw[u]);
+  }
+  for (; r < r1; ++r) row(r, load_raw<T, 8>(x + static_cast<int64_t>(r) * ld));
+  float* to = part + static_cast<int64_t>(blockIdx.y) * vocab + c0;
+  for (int j = 0; j < valid; ++j) to[j] = sum[j];
+}
+
 }  // namespace
 }  // namespace nmtg
 
@@ -340,4 +404,36 @@ extern "C" int nmtg_xentropy_bwd(const float* grad_loss, const void* logits, con
                               ld_logits, ld_grad, class_offset, total_classes, smoothing, padding_idx));
   NMTG_CHECK_LAUNCH("xentropy_bwd");
   return 0;
+}
+
+extern "C" int64_t nmtg_xentropy_bwd_colsum_parts(int64_t rows) { return rows > 0 ? (rows + XC_ROWS - 1) / XC_ROWS : 0; }
+
+extern "C" int nmtg_xentropy_bwd_colsum(const float* grad_loss, int64_t grad_stride, const void* logits, const float* lse,
+                                        const int64_t* labels, void* grad_logits, void* colsum, float* part, int64_t rows,
+                                        int64_t vocab, int64_t ld_logits, int64_t ld_grad, float smoothing, int64_t padding_idx,
+                                        int dtype, void* stream) {
+  NMTG_REQUIRE(rows > 0 && rows <= INT32_MAX && vocab > 0 && vocab <= INT32_MAX, "xentropy_bwd_colsum: bad sizes %lld x %lld",
+               (long long)rows, (long long)vocab);
+  NMTG_REQUIRE(dtype == NMTG_F16 || dtype == NMTG_BF16, "xentropy_bwd_colsum: fp16 or bf16 logits");
+  NMTG_REQUIRE(grad_loss && logits && lse && labels && grad_logits && colsum && part, "xentropy_bwd_colsum: null pointer argument");
+  NMTG_REQUIRE(grad_stride == 0 || grad_stride == 1, "xentropy_bwd_colsum: one gradient per row or one for all");
+  // whole 16-byte vectors up to the pitch
+  NMTG_REQUIRE(aligned16(logits) && aligned16(grad_logits) && ld_logits % 8 == 0 && ld_grad % 8 == 0 && ld_logits >= vocab && ld_grad >= vocab,
+               "xentropy_bwd_colsum: rows must be 16-byte aligned");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const int parts = static_cast<int>(nmtg_xentropy_bwd_colsum_parts(rows));
+  {
+    TraceScope trace("xentropy_bwd_colsum", st);
+    const dim3 grid(static_cast<unsigned>((vocab + XC_COLS - 1) / XC_COLS), static_cast<unsigned>(parts));
+    auto go = [&](auto tag) {
+      using T = decltype(tag);
+      hipLaunchKernelGGL((xentropy_bwd_colsum_kernel<T>), grid, dim3(XC_THREADS), 0, st, grad_loss, grad_stride, static_cast<const T*>(logits),
+                         lse, labels, static_cast<T*>(grad_logits), part, static_cast<int>(rows), XC_ROWS, vocab, ld_logits, ld_grad,
+                         smoothing, padding_idx);
+    };
+    if (dtype == NMTG_F16) go(f16_t{});
+    else go(bf16_t{});
+    NMTG_CHECK_LAUNCH("xentropy_bwd_colsum");
+  }
+  return colsum_finish(dtype, part, parts, static_cast<int>(vocab), colsum, st);
 }

@@ -94,14 +94,10 @@ class LinearSoftmaxCrossEntropy(torch.autograd.Function):
             pitch = (v + 63) // 64 * 64
             keep = any(ctx.needs_input_grad[:3]) and n * pitch * hidden.element_size() <= int(keep_logits_bytes)
             if keep:
-                # the columns between V and the pitch are multiplied by nothing, but the contraction over the classes
-                # reads whole 16-byte groups: keep them finite
+                # the columns between V and the pitch are never written: whatever reads them drops what it read
                 full = torch.empty(n, pitch, dtype=hidden.dtype, device=hidden.device)
-                full[:, v:].zero_()
                 z = linear_gemm.gemm(hidden, weight, trans_b=True, bias=bias, out=full[:, :v])
-                part, m = xentropy_cuda.forward(z, labels, smoothing, True, padding_idx=padding_idx)
-                losses.copy_(part)
-                lse.copy_(m)
+                losses, lse = xentropy_cuda.forward(z, labels, smoothing, True, padding_idx=padding_idx)
                 ctx.kept = full
             else:
                 buf = _chunk_buffer(min(n, chunk_rows), v, hidden)
@@ -119,22 +115,15 @@ class LinearSoftmaxCrossEntropy(torch.autograd.Function):
         """The kept logits become their gradient in place; one contraction with the states, one with the weights."""
         n, v = hidden.size(0), weight.size(0)
         z = full[:, :v]
-        dz = xentropy_cuda.backward(grad_loss, z, lse, labels, ctx.smoothing, padding_idx=ctx.padding_idx, out=z)
         dh = dw = db = None
+        if need_b:                                          # the column sums come out of the pass that makes the gradient
+            dz, db = xentropy_cuda.backward_with_colsum(grad_loss, z, lse, labels, ctx.smoothing, ctx.padding_idx, z)
+        else:
+            dz = xentropy_cuda.backward(grad_loss, z, lse, labels, ctx.smoothing, padding_idx=ctx.padding_idx, out=z)
         if need_w:
             dw = linear_gemm.gemm(dz, hidden, trans_a=True)                          # [V, N] x [N, E]
-        if need_b:
-            db = linear_gemm.colsum(dz)                                              # fixed-order fp32 column sums
         if need_h:
-            # the contraction over the classes in whole 64-class steps (the matrix-core loop fed from LDS directly), and
-            # the last V % 64 classes as a product of their own; summed in fp32
-            v0 = v // 64 * 64
-            if v0 == v or v0 == 0:
-                dh = linear_gemm.gemm(dz, weight)
-            else:
-                dh32 = linear_gemm.gemm(full[:, :v0], weight[:v0]).float()
-                dh32.add_(linear_gemm.gemm(full[:, v0:v], weight[v0:]))
-                dh = dh32.to(hidden.dtype)
+            dh = linear_gemm.gemm(dz, weight)                                        # classes split over the chip
         return dh, dw, db
 
     @staticmethod

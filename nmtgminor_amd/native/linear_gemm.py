@@ -36,7 +36,7 @@ def gemm(a, b, trans_a=False, trans_b=False, alpha=1.0, bias=None, out=None, spl
         return out if a.dim() == 3 else o3[0]
     ws = None
     ws_bytes = 0
-    if split_k and trans_a and not trans_b and a3.dtype != torch.float32:      # the fp32 kernel never splits K
+    if split_k and not trans_b and bias is None and a3.dtype != torch.float32:      # the fp32 kernel never splits K
         ws_bytes = int(L.load().nmtg_gemm_workspace_bytes(L.i64(m), L.i64(n), L.i64(k), L.i64(batch)))
         if ws_bytes:
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a3.device)

@@ -85,3 +85,19 @@ def backward(grad_loss, logits, max_log_sum_exp, labels, smoothing, *, padding_i
            L.i64(class_offset), L.i64(v if total_classes is None else total_classes), L.f32(smoothing),
            L.i64(_NO_PAD if padding_idx is None else padding_idx), L.i32(L.dtype_code(logits)), L.stream_of(logits))
     return grad_logits
+
+
+def backward_with_colsum(grad_loss, logits, lse, labels, smoothing, padding_idx, out):
+    """backward() of whole rows in place of `out`, and the sum of its rows ([classes], logits dtype) from the same pass: the
+    bias gradient of the projection in front. grad_loss: fp32 [N], or one value for all rows ([1] or a scalar)."""
+    L.require_cuda(grad_loss, logits, lse, labels, out)
+    n, v = logits.shape
+    _check(out.shape == logits.shape and out.dtype == logits.dtype and labels.numel() == n and lse.numel() == n and
+           grad_loss.numel() in (1, n) and grad_loss.dtype == torch.float32 and lse.dtype == torch.float32, "shape mismatch")
+    grad_loss, lse, labels = grad_loss.contiguous(), lse.contiguous(), labels.contiguous()
+    colsum = torch.empty(v, dtype=logits.dtype, device=logits.device)
+    part = torch.empty(int(L.load().nmtg_xentropy_bwd_colsum_parts(L.i64(n))), v, dtype=torch.float32, device=logits.device)
+    L.call("nmtg_xentropy_bwd_colsum", L.ptr(grad_loss), L.i64(int(grad_loss.numel() == n and n > 1)), L.ptr(logits), L.ptr(lse),
+           L.ptr(labels), L.ptr(out), L.ptr(colsum), L.ptr(part), L.i64(n), L.i64(v), L.i64(logits.stride(0)), L.i64(out.stride(0)),
+           L.f32(smoothing), L.i64(_NO_PAD if padding_idx is None else padding_idx), L.i32(L.dtype_code(logits)), L.stream_of(logits))
+    return out, colsum
