@@ -221,6 +221,11 @@ int nmtg_gemm(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float a
               int64_t ldc, int64_t stride_c, int64_t batch, const void* bias, void* workspace,
               int64_t workspace_bytes, int dtype, void* stream);
 
+/* y = x W^T (+ bias), x [rows, in], W [out, in], dense: nmtg_gemm(0, 1, ...) for the projections of a decoding step, whose
+ * batches of up to 64 rows take the few-row kernel (nmtg_gemm: up to 32). */
+int nmtg_linear_step(int64_t rows, int64_t out, int64_t in, const void* x, const void* w, const void* bias, void* y,
+                     int dtype, void* stream);
+
 /* nmtg_gemm without a workspace argument, for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc). No counterpart in the reference. The split-K
  * partial sums go to an array of nmtg_gemm_static_max_workspace_bytes() (32 MiB) that the library keeps in device
@@ -462,7 +467,8 @@ int nmtg_flash_attn_bwd(const void* dout, const void* q, const void* k, const vo
  * the same kernel packs the mask to bits in both orientations (len_q * len_k / 4 bytes), and the
  * attention kernels read one packed word per lane in patches that hold masked elements.
  * causal, dropout_*, seed, offset, softmax_lse [batch, heads, len_q], softmax_d: as above, with
- * max_seqlen_* = len_*.
+ * max_seqlen_* = len_*. dropout_mode 3 draws the mask in the numbering of the extension modules (element e of
+ * [batch, heads, len_q, len_k] from word e % 4 of the generator's block e / 4, kept with probability 1 - p exactly).
  * nmtg_flash_attn_batched_bwd: dout has the strides of out; dq, dk, dv have the strides of q, k, v
  * and are written whole (zeros at masked keys). Deterministic: no atomics.
  * ------------------------------------------------------------------------------------------ */
@@ -482,6 +488,22 @@ int nmtg_flash_attn_batched_fwd(const void* q, const void* k, const void* v, voi
                                 int dropout_mode, float dropout_p, const uint8_t* dropout_mask,
                                 uint8_t* dropout_mask_out, void* dropout_bits, uint64_t seed,
                                 uint64_t offset, int dtype, void* stream);
+
+/* nmtg_flash_attn_batched_fwd that also writes probs [batch * heads, len_q, len_k] (dtype): the softmax of the scores,
+ * after dropout with probs_dropped (the extension modules' dropout_results), 0 at masked keys. */
+int nmtg_flash_attn_batched_fwd_probs(const void* q, const void* k, const void* v, void* out,
+                                      const uint8_t* key_padding_mask, void* key_info,
+                                      const uint8_t* time_mask, void* time_info, float* softmax_lse,
+                                      int64_t batch, int64_t heads, int64_t head_dim, int64_t len_q,
+                                      int64_t len_k, int64_t q_stride_t, int64_t q_stride_b,
+                                      int64_t q_stride_h, int64_t k_stride_t, int64_t k_stride_b,
+                                      int64_t k_stride_h, int64_t v_stride_t, int64_t v_stride_b,
+                                      int64_t v_stride_h, int64_t out_stride_t, int64_t out_stride_b,
+                                      int64_t out_stride_h, float softmax_scale, int causal,
+                                      int dropout_mode, float dropout_p, const uint8_t* dropout_mask,
+                                      uint8_t* dropout_mask_out, void* dropout_bits, uint64_t seed,
+                                      uint64_t offset, int dtype, void* stream, void* probs,
+                                      int probs_dropped);
 
 int nmtg_flash_attn_batched_bwd(const void* dout, const void* q, const void* k, const void* v,
                                 const void* out, const float* softmax_lse, void* dq, void* dk,

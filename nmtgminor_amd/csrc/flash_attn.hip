@@ -23,7 +23,9 @@
 // query-major kernels (forward, dQ) a lane pair is a query and an accumulator register a key, so the pair of words
 // of the two keys that a register holds in the two halves of the wavefront IS the lane mask of a select: it is loaded
 // into scalar registers and costs no vector instruction besides the select. The key-major kernel (dK / dV) loads its
-// key's word per group of queries and tests bits. An explicit byte mask is turned into the same words.
+// key's word per group of queries and tests bits. An explicit byte mask is turned into the same words, and so are the
+// decisions of the extension modules' numbering (mode 3: element (i, j) uses word e % 4 of the Philox block e / 4,
+// e = ((b H + h) max_q + i) max_k + j, and is kept when word / 2^32 < 1 - p), for calls that return the probabilities.
 #include "gemm.hip.h"
 
 namespace nmtg {
@@ -60,7 +62,7 @@ struct FaArgs {
   int causal;
   const uint8_t* mask;   // explicit keep-mask [B, H, max_q, max_k] (bit kernel, mode 1)
   uint8_t* mask_out;     // where the drawn mask is written as bytes, or null (bit kernel, mode 2)
-  uint32_t thr;          // keep when byte < thr (bit kernel, mode 2)
+  uint32_t thr;          // keep when byte < thr (bit kernel, mode 2) or when the word's upper 24 bits are (mode 3)
   float drop_scale;
   uint64_t seed, offset;
   // keep bits [B H, q32 groups of 32 queries, kp keys]: bit (i % 32) of word bit_slot(j) of row (b H + h, i / 32)
@@ -399,6 +401,42 @@ __global__ __launch_bounds__(256) void flash_bits_rng_kernel(FaArgs a, int64_t t
   }
 }
 
+// Keep bits in the extension modules' numbering (mode 3): one thread per (head of a sequence, group of 32 queries, group of
+// four keys), one generator call per query where rows start on a multiple of four elements and two where they do not.
+__global__ __launch_bounds__(256) void flash_bits_linear_kernel(FaArgs a, int64_t total) {
+  const int64_t id = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (id >= total) return;
+  const int k4n = a.kp / 4;
+  const int j4 = static_cast<int>(id % k4n);
+  const int64_t row = id / k4n;                      // (b H + h) q32 + group
+  const int grp = static_cast<int>(row % a.q32);
+  const int bh = static_cast<int>(row / a.q32), b = bh / a.heads;
+  const SeqSpan sp = seq_span(a, b);
+  if (32 * grp >= sp.lq || 4 * j4 >= sp.lk) return;  // never read
+  const Philox gen(a.seed);
+  const uint64_t e0 = (static_cast<uint64_t>(bh) * a.max_q + 32u * grp) * a.max_k + 4u * j4;
+  const bool aligned = (a.max_k & 3) == 0;
+  uint32_t word[4] = {0, 0, 0, 0};
+#pragma unroll 4
+  for (int i = 0; i < 32; ++i) {
+    const uint64_t e = e0 + static_cast<uint64_t>(i) * a.max_k;
+    const uint4 r = gen(e >> 2, a.offset);
+    uint32_t w[4] = {r.x, r.y, r.z, r.w};
+    if (!aligned) {
+      const uint4 n = gen((e >> 2) + 1, a.offset);
+      const uint32_t both[8] = {r.x, r.y, r.z, r.w, n.x, n.y, n.z, n.w};
+      const int shift = static_cast<int>(e & 3);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) w[k] = shift == 0 ? both[k] : shift == 1 ? both[k + 1] : shift == 2 ? both[k + 2] : both[k + 3];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) word[k] |= ((w[k] >> 8) < a.thr ? 1u : 0u) << i;
+  }
+  uint32_t* out = a.bits + row * a.kp;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) out[bit_slot(4 * j4 + k)] = word[k];
+}
+
 // Keep bits from an explicit byte mask [B, H, max_q, max_k]: one thread per (head of a sequence, group of 32 queries, key).
 __global__ __launch_bounds__(256) void flash_bits_mask_kernel(FaArgs a, int64_t total) {
   const int64_t id = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
@@ -536,6 +574,14 @@ __global__ __launch_bounds__(FA_THREADS, D == 64 ? 3 : 1) void flash_fwd_kernel(
       sv.load(vb, a.v_st, (t + 1) * FA_TILE, lk);
       if constexpr (PAD != 0) mdead_next = tile_mask_bits<PAD>(a, b, qr, t + 1, half);
     }
+    // the lane masks of the tile: asked for ahead of the products, which cover the scalar cache's latency (packed forward of
+    // the benchmark 61 -> 56 us, padded 82 -> 70 us)
+    [[maybe_unused]] uint64_t lane_mask[32];
+    if constexpr (DROP != 0) {
+      const uint64_t* lm = tile_lane_masks(a, bh, group, t);
+#pragma unroll
+      for (int r = 0; r < 32; ++r) lane_mask[r] = lm[r];
+    }
     acc16_t s[2];
 #pragma unroll
     for (int n = 0; n < 2; ++n)
@@ -622,7 +668,6 @@ __global__ __launch_bounds__(FA_THREADS, D == 64 ? 3 : 1) void flash_fwd_kernel(
     }
     l += lsum;
     if constexpr (DROP != 0) {
-      const uint64_t* lane_mask = tile_lane_masks(a, bh, group, t);
 #pragma unroll
       for (int n = 0; n < 2; ++n)
 #pragma unroll
@@ -1311,6 +1356,153 @@ __global__ __launch_bounds__(FA_THREADS * G, (D == 64 && G == 1) ? 2 : 1) void a
   store_rows_out<T, D>(o, 1.f, lds_raw + wave_all * (32 * D * 2), cb, a.c_st, q0 + 32 * wave, group == 0 ? a.tq : 0, lane);
 }
 
+// -------------------------------------------------------------------------------------------------------------------
+// training: the probabilities of a call that returns them
+// -------------------------------------------------------------------------------------------------------------------
+// probs [B H, max_q, max_k] = exp(scores - log-sum-exp) of the forward that ran before, DROP: times keep / (1 - p). The
+// scores are computed again from queries and keys instead of being stored for this and for the backward (both recompute
+// them): the one tensor of that size is written once and never read. Bound by those stores. A block owns 128 queries and
+// a run of key tiles (`tiles_per_block`); nothing is summed, so the keys are dealt out freely. [512 x 512] x 512 heads in
+// bf16: scores, probabilities after dropout and mask bytes in one kernel and their product with the values took 336 us; the
+// keep bits (75), the context (70) and these probabilities (76) take 221, and the backward, which read 670 MB of them in
+// 436 us, takes 245. (Keys straight from memory instead of through LDS, without the barrier: 102 us, bound by the vector
+// memory pipe. The lane masks through a pointer that may alias `probs`: 94 us, they come in vector registers then.)
+constexpr int FP_PITCH = FA_TILE * 2 + 16;   // bytes per row of a wavefront's strip
+template <typename T, int D, int DROP, int PAD>
+__global__ __launch_bounds__(FA_THREADS, 2) void flash_probs_kernel(FaArgs a, T* __restrict__ probs, const uint64_t* __restrict__ keep,
+                                                                const int32_t* __restrict__ tile_info, int chunks, int tiles_per_block, int wide) {
+  extern __shared__ __align__(16) uint8_t lds_raw[];
+  constexpr int IMG = FA_TILE * D * 2;
+  const int b = blockIdx.z, h = blockIdx.y, qblock = static_cast<int>(blockIdx.x) / chunks, chunk = static_cast<int>(blockIdx.x) % chunks;
+  const int q0 = qblock * FA_ROWS;
+  const SeqSpan sp = seq_span(a, b);
+  const int lq = sp.lq, lk = sp.lk;
+  const int lane = static_cast<int>(threadIdx.x) & 63, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  const int bh = b * a.heads + h, group = qblock * (FA_ROWS / 32) + wave;
+  const int qrow = q0 + 32 * wave + (lane & 31);
+  const T* qb = static_cast<const T*>(a.q) + static_cast<int64_t>(b) * a.q_sb + static_cast<int64_t>(h) * a.q_sh;
+  const T* kb = static_cast<const T*>(a.k) + static_cast<int64_t>(b) * a.k_sb + static_cast<int64_t>(h) * a.k_sh;
+  uint4 qf[D / 16];
+  load_resident<T, D>(qf, qb, a.q_st, qrow, lq, lane);
+  float lse2 = -FA_NEG;   // a row without a live key: probability 0
+  if (qrow < lq) {
+    const float v = a.lse[static_cast<int64_t>(bh) * a.max_q + qrow];
+    if (v != -INFINITY) lse2 = v * FA_LOG2E - log2f(a.drop_scale);      // the dropout scale rides in the exponent
+  }
+  [[maybe_unused]] const int qr = min(qrow, lq - 1);
+  const int limit = a.causal ? min(lk, qrow + 1) : lk;      // keys from here on are dead for this lane's query
+  const int t0 = chunk * tiles_per_block, t1 = min(t0 + tiles_per_block, (a.max_k + FA_TILE - 1) / FA_TILE);
+  T* prow = probs + (static_cast<int64_t>(bh) * a.max_q + q0 + 32 * wave) * a.max_k;
+  uint8_t* strip = lds_raw + 2 * IMG + wave * (32 * FP_PITCH);
+  // one tile of the wavefront's rows from its strip (or zeros) to memory
+  // FULL (all of the block's rows and keys exist, 16-byte rows): unconditional stores, so that the compiler can count them and
+  // the wait for the next tile's keys, requested before them, does not wait for the stores as well
+  auto store_tile = [&](auto full_tag, int t, bool live) {
+    constexpr bool FULL = decltype(full_tag)::value;
+    const int rows = lq - (q0 + 32 * wave);
+    if (FULL || wide) {                                     // 16 bytes per lane, eight rows of 64 keys per step
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = 8 * i + (lane >> 3), key = t * FA_TILE + 8 * (lane & 7);
+        if (FULL || (r < rows && key < a.max_k)) {
+          const uint4 v = live ? *reinterpret_cast<const uint4*>(strip + r * FP_PITCH + 16 * (lane & 7)) : make_uint4(0, 0, 0, 0);
+          *reinterpret_cast<uint4*>(prow + static_cast<int64_t>(r) * a.max_k + key) = v;
+        }
+      }
+    } else {                                        // rows of any length: a row of 64 keys per step
+      const int key = t * FA_TILE + lane;
+#pragma unroll 8
+      for (int r = 0; r < 32; ++r) {
+        uint16_t v = 0;
+        if (live) v = *reinterpret_cast<const uint16_t*>(strip + r * FP_PITCH + 2 * lane);
+        if (r < rows && key < a.max_k) *reinterpret_cast<uint16_t*>(prow + static_cast<int64_t>(r) * a.max_k + key) = v;
+      }
+    }
+  };
+  auto tile = [&](auto full_tag, int t, Staged<D>& sk, uint32_t mdead, uint32_t& mdead_next) {
+    const uint8_t* kimg = lds_raw + ((t - t0) & 1) * IMG;
+    const bool live = t * FA_TILE < lk;
+    if (t + 1 < t1) {
+      sk.load(kb, a.k_st, (t + 1) * FA_TILE, lk);
+      if constexpr (PAD != 0) mdead_next = tile_mask_bits<PAD>(a, b, qr, t + 1, half);
+    }
+    if (live) {
+      [[maybe_unused]] uint64_t lane_mask[32];      // requested ahead of the products
+      if constexpr (DROP != 0) {
+        // (through an argument of its own that cannot alias `probs`: read back behind a store that might, the masks would come
+        // in vector registers, 64 of them)
+        const uint64_t* lm = keep + ((static_cast<int64_t>(bh) * a.q32 + group) * a.kp + FA_TILE * t) / 2;
+#pragma unroll
+        for (int i = 0; i < 32; ++i) lane_mask[i] = lm[i];
+      }
+      acc16_t s[2];
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[n][r] = 0.f;
+#pragma unroll
+      for (int ss = 0; ss < D / 16; ++ss)
+#pragma unroll
+        for (int n = 0; n < 2; ++n) mfma<T>::run(read_rows<D>(kimg, n, ss, lane), qf[ss], s[n]);
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[n][r] = fast_exp2(__builtin_fmaf(s[n][r], a.scale_log2, -lse2));
+      // masked keys only where the tile has any (uniform over the wavefront)
+      bool edge = (t + 1) * FA_TILE > lk || (a.causal && t * FA_TILE + FA_TILE - 1 > q0 + 32 * wave);
+      if constexpr (PAD == 1) edge = edge || tile_info[static_cast<int64_t>(b) * a.kinfo_pitch + 1 + t] != 0;
+      if constexpr (PAD == 2) edge = edge || tile_info[static_cast<int64_t>(min(group, (a.max_q + 31) / 32 - 1)) * a.qinfo_pitch + 1 + t] != 0;
+      if (edge) {
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int key = t * FA_TILE + 32 * n + 8 * (r / 4) + 4 * half + r % 4;
+            bool dead = key >= limit;
+            if constexpr (PAD != 0) dead = dead | (((mdead >> (16 * n + r)) & 1u) != 0);
+            s[n][r] = dead ? 0.f : s[n][r];
+          }
+      }
+      if constexpr (DROP != 0) {
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) s[n][r] = __builtin_amdgcn_inverse_ballot_w64(lane_mask[16 * n + r]) ? s[n][r] : 0.f;
+      }
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) {
+          uint2 w;
+          w.x = pack2<T>(s[n][4 * g4 + 0], s[n][4 * g4 + 1]);
+          w.y = pack2<T>(s[n][4 * g4 + 2], s[n][4 * g4 + 3]);
+          *reinterpret_cast<uint2*>(strip + (lane & 31) * FP_PITCH + (32 * n + 8 * g4 + 4 * half) * 2) = w;
+        }
+      wave_lds_fence();
+    }
+    store_tile(full_tag, t, live);
+    wave_lds_fence();
+    if (t + 1 < t1) sk.store_rows(lds_raw + ((t + 1 - t0) & 1) * IMG);
+    __syncthreads();
+  };
+  auto tiles = [&](auto full_tag) {
+    uint32_t mdead = 0, mdead_next = 0;             // a tile's mask word is requested with its keys, one tile ahead
+    if constexpr (PAD != 0) mdead_next = tile_mask_bits<PAD>(a, b, qr, t0, half);
+    Staged<D> sk;
+    sk.load(kb, a.k_st, t0 * FA_TILE, lk);
+    sk.store_rows(lds_raw);
+    __syncthreads();
+    for (int t = t0; t < t1; ++t) {
+      mdead = mdead_next;
+      tile(full_tag, t, sk, mdead, mdead_next);
+    }
+  };
+  if (wide && q0 + FA_ROWS <= lq && t1 * FA_TILE <= a.max_k) tiles(std::true_type{});
+  else tiles(std::false_type{});
+}
+template <int D> constexpr int fprobs_lds() { return 2 * FA_TILE * D * 2 + 4 * 32 * FP_PITCH; }
+
 template <int D, int G> constexpr int probs_lds() { return G * (4 * FA_TILE * D * 2 + 4 * 32 * PA_PITCH + 128 * 2 * 4); }
 
 template <int D> constexpr int fwd_lds() { return 2 * 2 * FA_TILE * D * 2; }
@@ -1376,11 +1568,12 @@ int bits_launch(const char* what, FaArgs& a, int drop_mode, int64_t batch, void*
   if (ready || a.max_q == 0 || a.max_k == 0) return 0;
   const int64_t rows = batch * a.heads * a.q32;
   const bool words = drop_mode == 1 && a.max_k % 4 == 0 && reinterpret_cast<uintptr_t>(a.mask) % 4 == 0;   // four keys per thread
-  const int64_t total = rows * (drop_mode == 2 || words ? a.kp / 4 : a.kp);
+  const int64_t total = rows * (drop_mode >= 2 || words ? a.kp / 4 : a.kp);
   NMTG_REQUIRE((total + 255) / 256 <= 0x7fffffff, "%s: keep-bit workspace beyond one launch", what);
   TraceScope trace("flash_attn_keep_bits", st);
   const dim3 grid(static_cast<unsigned>((total + 255) / 256));
   if (drop_mode == 2) hipLaunchKernelGGL(flash_bits_rng_kernel, grid, dim3(256), 0, st, a, total);
+  else if (drop_mode == 3) hipLaunchKernelGGL(flash_bits_linear_kernel, grid, dim3(256), 0, st, a, total);
   else if (words) hipLaunchKernelGGL(flash_bits_mask4_kernel, grid, dim3(256), 0, st, a, total);
   else hipLaunchKernelGGL(flash_bits_mask_kernel, grid, dim3(256), 0, st, a, total);
   return 0;
@@ -1398,7 +1591,7 @@ int check_common(const char* what, int64_t batch, int64_t heads, int64_t d, int6
                what, (long long)batch, (long long)heads, (long long)max_q, (long long)max_k);
   NMTG_REQUIRE(d == 64 || d == 128, "%s: head dimension %lld (64 and 128 are built)", what, (long long)d);
   NMTG_REQUIRE(dtype == NMTG_F16 || dtype == NMTG_BF16, "%s: fp16 or bf16 tensors required (matrix-core kernel)", what);
-  NMTG_REQUIRE(drop_mode >= 0 && drop_mode <= 2, "%s: dropout mode %d", what, drop_mode);
+  NMTG_REQUIRE(drop_mode >= 0 && drop_mode <= 3, "%s: dropout mode %d", what, drop_mode);
   NMTG_REQUIRE(drop_mode == 0 || (p >= 0.f && p < 1.f), "%s: dropout probability %g outside [0, 1)", what, (double)p);
   NMTG_REQUIRE(heads <= 65535 && batch <= 65535, "%s: more than 65535 heads or sequences in one launch", what);
   NMTG_REQUIRE(batch * heads * (max_q + 3) / 4 * ((max_k + 3) / 4) < (1ll << 62) && max_q <= (1 << 24) && max_k <= (1 << 24),
@@ -1409,7 +1602,9 @@ int check_common(const char* what, int64_t batch, int64_t heads, int64_t d, int6
 void set_dropout(FaArgs& a, int drop_mode, float p, uint64_t seed, uint64_t offset) {
   a.thr = 256;
   a.drop_scale = 1.f;
-  if (drop_mode == 1) a.drop_scale = 1.f / (1.f - p);
+  if (drop_mode == 1 || drop_mode == 3) a.drop_scale = 1.f / (1.f - p);
+  // (word >> 8) 2^-24 < 1 - p, compared as integers (the product is exact)
+  if (drop_mode == 3) a.thr = static_cast<uint32_t>(std::ceil((1.f - p) * 16777216.f));
   if (drop_mode == 2) {
     long thr = lroundf(256.f * (1.f - p));
     a.thr = static_cast<uint32_t>(thr < 1 ? 1 : thr > 256 ? 256 : thr);
@@ -1441,6 +1636,29 @@ int bwd_run(const char* what, FaArgs& a, int64_t batch, int64_t d, int drop_mode
   if (rc) return rc;
   NMTG_CHECK_LAUNCH(what);
   return 0;
+}
+
+// The probabilities of a batch-strided forward that has run with these arguments (key / time summaries and keep bits in
+// place). dropped: after dropout.
+template <typename T, int D>
+int fprobs_launch(FaArgs a, int64_t batch, bool dropped, void* probs, hipStream_t st) {
+  const int qblocks = (a.max_q + FA_ROWS - 1) / FA_ROWS, tiles = (a.max_k + FA_TILE - 1) / FA_TILE;
+  if (tiles == 0) return 0;
+  // eight tiles per block amortise the resident queries; fewer where the blocks would not fill the chip four times over
+  int per = 8;
+  while (per > 1 && static_cast<int64_t>(qblocks) * ((tiles + per - 1) / per) * a.heads * batch < 4 * num_cus()) per /= 2;
+  const int chunks = (tiles + per - 1) / per, wide = aligned16(probs) && a.max_k % 8 == 0 ? 1 : 0;
+  if (!dropped) a.drop_scale = 1.f;
+  const dim3 grid(static_cast<unsigned>(qblocks * chunks), static_cast<unsigned>(a.heads), static_cast<unsigned>(batch));
+  TraceScope trace("flash_attn_probs", st);
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, dim3(FA_THREADS), fprobs_lds<D>(), st, a, static_cast<T*>(probs), reinterpret_cast<const uint64_t*>(a.bits),
+                       a.tmask != nullptr ? a.qinfo : a.kinfo, chunks, per, wide);
+    return 0;
+  };
+  if (a.tmask != nullptr) return dropped ? go(flash_probs_kernel<T, D, 1, 2>) : go(flash_probs_kernel<T, D, 0, 2>);
+  if (a.pad != nullptr) return dropped ? go(flash_probs_kernel<T, D, 1, 1>) : go(flash_probs_kernel<T, D, 0, 1>);
+  return dropped ? go(flash_probs_kernel<T, D, 1, 0>) : go(flash_probs_kernel<T, D, 0, 0>);
 }
 
 // a [len, batch, heads, head_dim] view: as view_ok, and a batch stride that keeps the alignment
@@ -1637,15 +1855,16 @@ extern "C" int64_t nmtg_flash_attn_time_info_bytes(int64_t len_q, int64_t len_k)
   return time_info_words(len_q, len_k) * 4;
 }
 
-extern "C" int nmtg_flash_attn_batched_fwd(const void* q, const void* k, const void* v, void* out, const uint8_t* key_padding_mask,
-                                           void* key_info, const uint8_t* time_mask, void* time_info, float* softmax_lse, int64_t batch, int64_t heads, int64_t head_dim,
-                                           int64_t len_q, int64_t len_k, int64_t q_stride_t, int64_t q_stride_b, int64_t q_stride_h,
-                                           int64_t k_stride_t, int64_t k_stride_b, int64_t k_stride_h, int64_t v_stride_t,
-                                           int64_t v_stride_b, int64_t v_stride_h, int64_t out_stride_t, int64_t out_stride_b,
-                                           int64_t out_stride_h, float softmax_scale, int causal, int dropout_mode, float dropout_p,
-                                           const uint8_t* dropout_mask, uint8_t* dropout_mask_out, void* dropout_bits,
-                                           uint64_t seed, uint64_t offset, int dtype, void* stream) {
-  const char* what = "flash_attn_batched_fwd";
+static int flash_batched_fwd(const void* q, const void* k, const void* v, void* out, const uint8_t* key_padding_mask,
+                             void* key_info, const uint8_t* time_mask, void* time_info, float* softmax_lse, int64_t batch, int64_t heads, int64_t head_dim,
+                             int64_t len_q, int64_t len_k, int64_t q_stride_t, int64_t q_stride_b, int64_t q_stride_h,
+                             int64_t k_stride_t, int64_t k_stride_b, int64_t k_stride_h, int64_t v_stride_t,
+                             int64_t v_stride_b, int64_t v_stride_h, int64_t out_stride_t, int64_t out_stride_b,
+                             int64_t out_stride_h, float softmax_scale, int causal, int dropout_mode, float dropout_p,
+                             const uint8_t* dropout_mask, uint8_t* dropout_mask_out, void* dropout_bits,
+                             uint64_t seed, uint64_t offset, int dtype, void* stream,
+                             void* probs, int probs_dropped) {
+  const char* what = probs != nullptr ? "flash_attn_batched_fwd_probs" : "flash_attn_batched_fwd";
   if (int rc = check_common(what, batch, heads, head_dim, len_q, len_k, dropout_mode, dropout_p, softmax_scale, dtype)) return rc;
   if (batch == 0 || len_q == 0) return 0;
   NMTG_REQUIRE(q && k && v && out && softmax_lse, "%s: null pointer argument", what);
@@ -1667,7 +1886,40 @@ extern "C" int nmtg_flash_attn_batched_fwd(const void* q, const void* k, const v
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (int rc = key_info_launch(what, a, batch, key_padding_mask, key_info, st)) return rc;
   if (int rc = time_info_launch(what, a, time_mask, time_info, st)) return rc;
-  return fwd_run(what, a, batch, head_dim, dropout_mode, dropout_bits, dtype, st);
+  if (int rc = fwd_run(what, a, batch, head_dim, dropout_mode, dropout_bits, dtype, st)) return rc;
+  if (probs == nullptr) return 0;
+  const bool dropped = probs_dropped != 0 && dropout_mode != 0;
+  if (dtype == NMTG_F16) {
+    if (int rc = head_dim == 64 ? fprobs_launch<f16_t, 64>(a, batch, dropped, probs, st) : fprobs_launch<f16_t, 128>(a, batch, dropped, probs, st)) return rc;
+  } else {
+    if (int rc = head_dim == 64 ? fprobs_launch<bf16_t, 64>(a, batch, dropped, probs, st) : fprobs_launch<bf16_t, 128>(a, batch, dropped, probs, st)) return rc;
+  }
+  NMTG_CHECK_LAUNCH(what);
+  return 0;
+}
+
+extern "C" int nmtg_flash_attn_batched_fwd(const void* q, const void* k, const void* v, void* out, const uint8_t* key_padding_mask,
+                                           void* key_info, const uint8_t* time_mask, void* time_info, float* softmax_lse, int64_t batch, int64_t heads, int64_t head_dim,
+                                           int64_t len_q, int64_t len_k, int64_t q_stride_t, int64_t q_stride_b, int64_t q_stride_h,
+                                           int64_t k_stride_t, int64_t k_stride_b, int64_t k_stride_h, int64_t v_stride_t,
+                                           int64_t v_stride_b, int64_t v_stride_h, int64_t out_stride_t, int64_t out_stride_b,
+                                           int64_t out_stride_h, float softmax_scale, int causal, int dropout_mode, float dropout_p,
+                                           const uint8_t* dropout_mask, uint8_t* dropout_mask_out, void* dropout_bits,
+                                           uint64_t seed, uint64_t offset, int dtype, void* stream) {
+  return flash_batched_fwd(q, k, v, out, key_padding_mask, key_info, time_mask, time_info, softmax_lse, batch, heads, head_dim, len_q, len_k, q_stride_t, q_stride_b, q_stride_h, k_stride_t, k_stride_b, k_stride_h, v_stride_t, v_stride_b, v_stride_h, out_stride_t, out_stride_b, out_stride_h, softmax_scale, causal, dropout_mode, dropout_p, dropout_mask, dropout_mask_out, dropout_bits, seed, offset, dtype, stream, nullptr, 0);
+}
+
+extern "C" int nmtg_flash_attn_batched_fwd_probs(const void* q, const void* k, const void* v, void* out, const uint8_t* key_padding_mask,
+                                                 void* key_info, const uint8_t* time_mask, void* time_info, float* softmax_lse, int64_t batch, int64_t heads, int64_t head_dim,
+                                                 int64_t len_q, int64_t len_k, int64_t q_stride_t, int64_t q_stride_b, int64_t q_stride_h,
+                                                 int64_t k_stride_t, int64_t k_stride_b, int64_t k_stride_h, int64_t v_stride_t,
+                                                 int64_t v_stride_b, int64_t v_stride_h, int64_t out_stride_t, int64_t out_stride_b,
+                                                 int64_t out_stride_h, float softmax_scale, int causal, int dropout_mode, float dropout_p,
+                                                 const uint8_t* dropout_mask, uint8_t* dropout_mask_out, void* dropout_bits,
+                                                 uint64_t seed, uint64_t offset, int dtype, void* stream,
+                                                 void* probs, int probs_dropped) {
+  NMTG_REQUIRE(probs, "flash_attn_batched_fwd_probs: null pointer argument");
+  return flash_batched_fwd(q, k, v, out, key_padding_mask, key_info, time_mask, time_info, softmax_lse, batch, heads, head_dim, len_q, len_k, q_stride_t, q_stride_b, q_stride_h, k_stride_t, k_stride_b, k_stride_h, v_stride_t, v_stride_b, v_stride_h, out_stride_t, out_stride_b, out_stride_h, softmax_scale, causal, dropout_mode, dropout_p, dropout_mask, dropout_mask_out, dropout_bits, seed, offset, dtype, stream, probs, probs_dropped);
 }
 
 extern "C" int nmtg_flash_attn_batched_bwd(const void* dout, const void* q, const void* k, const void* v, const void* out,

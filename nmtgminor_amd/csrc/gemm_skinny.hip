@@ -1,4 +1,4 @@
-// C[m][n] = alpha * sum_k X[m][k] W[n][k] (+ bias[n]) for at most 32 rows m: the projections of a decoding step
+// C[m][n] = alpha * sum_k X[m][k] W[n][k] (+ bias[n]) for at most 64 rows m: the projections of a decoding step
 // (one new position of a few dozen hypotheses against a [1024 x 1024] weight), which the reference runs as cuBLASLt
 // calls like any other linear layer (onmt/modules/extensions/mlp_blaslt/linear.cpp:142-144).
 //
@@ -11,11 +11,16 @@
 // the eight of them up in a fixed order. A [1024 x 1024] weight is 32 blocks of one load latency each.
 #include "gemm.hip.h"
 
+#include <algorithm>
+
 namespace nmtg {
 namespace {
 
 constexpr int SK_ROWS = 32, SK_COLS = 32, SK_WAVES = 8, SK_THREADS = 64 * SK_WAVES, SK_CHUNK = 128;
-// Two row blocks (a batch of 64 hypotheses) re-read W from L2 and still leave the 128 x 128 tile far behind.
+// Up to two row blocks where the caller allows it (GemmArgs::skinny_rows): a batch of 64 hypotheses re-reads W from L2 and
+// still leaves the 128 x 128 tile far behind. Other calls of more than 32 rows stay with the tiles: the two sum the reduction
+// in different orders, and in training a hidden activation within rounding of zero would pass the relu with the one and not
+// with the other.
 constexpr int SK_MAX_ROWS = 64;
 
 template <typename T>
@@ -73,7 +78,7 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_skinny_kernel(const GemmArgs 
 bool gemm_skinny_ok(int dtype, int layout, int epi, const GemmArgs& a) {
   if (switched_off("NMTG_GEMM_SKINNY")) return false;
   return (dtype == NMTG_F16 || dtype == NMTG_BF16) && layout == LAYOUT_NT && epi == EPI_PLAIN && a.batch == 1 && a.M >= 1 &&
-         a.M <= SK_MAX_ROWS && a.N >= 64 && a.K >= 8 && a.K % 8 == 0 && a.lda % 8 == 0 && a.ldb % 8 == 0 && aligned16(a.A) &&
+         a.M <= (a.skinny_rows != 0 ? std::min(a.skinny_rows, SK_MAX_ROWS) : SK_ROWS) && a.N >= 64 && a.K >= 8 && a.K % 8 == 0 && a.lda % 8 == 0 && a.ldb % 8 == 0 && aligned16(a.A) &&
          aligned16(a.B);
 }
 
@@ -88,3 +93,18 @@ int gemm_skinny_run(int dtype, const GemmArgs& a, hipStream_t st) {
 }
 
 }  // namespace nmtg
+
+using namespace nmtg;
+
+extern "C" int nmtg_linear_step(int64_t rows, int64_t out, int64_t in, const void* x, const void* w, const void* bias, void* y, int dtype,
+                                void* stream) {
+  NMTG_REQUIRE(rows >= 0 && out >= 0 && in >= 0 && rows <= INT32_MAX && out <= INT32_MAX && in <= INT32_MAX, "linear_step: bad shape");
+  GemmArgs g{};
+  g.A = x; g.B = w; g.C = y; g.bias = bias;
+  g.lda = in; g.ldb = in; g.ldc = out;
+  g.M = static_cast<int>(rows); g.N = static_cast<int>(out); g.K = static_cast<int>(in);
+  g.batch = 1;
+  g.alpha = 1.f;
+  g.skinny_rows = SK_MAX_ROWS;
+  return gemm_run(dtype, LAYOUT_NT, EPI_PLAIN, g, nullptr, 0, static_cast<hipStream_t>(stream));
+}

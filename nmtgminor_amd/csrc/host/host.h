@@ -1,6 +1,7 @@
 // Shared pieces of the native host layer (nmtgminor_amd/_host.so): the table of C entry points it calls, and the
 // operators as functions from tensors to tensors (allocate the results, enqueue the kernels). ops.cpp implements them,
-// autograd.cpp wraps them in autograd nodes, layers.cpp composes the transformer layers, optim.cpp prepares the optimizer's passes.
+// autograd.cpp wraps them in autograd nodes, layers.cpp composes the transformer layers, attention.cpp the attention modules, optim.cpp prepares the
+// optimizer's passes.
 //
 // Why it exists: a call through the Python stand-ins costs 25 to 80 us of interpreter, ctypes and autograd bookkeeping per
 // operator and direction, several times what the kernels of a small batch take. The same work here is 3 to 8 us.
@@ -27,7 +28,7 @@ using std::optional;
   X(xentropy_bwd) X(gemm) X(mlp_fwd) X(mlp_bwd_dtype_workspace_bytes) X(mlp_bwd) X(flash_attn_dropout_bits_bytes)     \
   X(flash_attn_fwd) X(flash_attn_bwd) X(flash_attn_key_info_bytes) X(flash_attn_time_info_bytes)                      \
   X(flash_attn_batched_fwd) X(flash_attn_batched_bwd) X(multi_tensor_adam) X(multi_tensor_clip)                       \
-  X(multi_tensor_l2norm) X(multi_tensor_l2norm_workspace_bytes)
+  X(multi_tensor_l2norm) X(multi_tensor_l2norm_workspace_bytes) X(flash_attn_batched_fwd_probs) X(linear_step)
 
 struct Api {
 #define X(name) decltype(&nmtg_##name) name = nullptr;
@@ -76,6 +77,7 @@ AddNormGrads ln_bwd_add(const Tensor& dz, const Tensor& x, const Tensor& stats, 
                         const Tensor& guard, const Tensor& keep, double p);
 
 Tensor linear_fwd(const Tensor& x, const Tensor& w, const Tensor& b);
+Tensor linear_step(const Tensor& x, const Tensor& w, const Tensor& b);          // of a decoding step: few rows, no gradient
 struct LinearGrads { Tensor dx, dw, db; };
 LinearGrads linear_bwd(const Tensor& dy, const Tensor& x, const Tensor& w, bool want_x, bool want_w, bool want_b);
 
@@ -96,16 +98,22 @@ Tensor dropout_guard_bwd(const Tensor& g, const Tensor& mask, double p);
 
 struct Bits { int64_t mode = 0; uint64_t seed = 0, offset = 0; Tensor words; };
 // attention over a padded batch: q [Tq, B, H, D], k / v [Tk, B, H, D]
-struct Flash { Tensor out, lse; Bits bits; };
+// coverage: the probabilities come back too ([B * H, Tq, Tk], before or after dropout), and the dropout mask is drawn in the
+// extension modules' numbering
+enum class Coverage { none, softmax, dropped };
+struct Flash { Tensor out, lse, probs; Bits bits; };
 Flash flash_fwd_batched(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& pad, const Tensor& time_mask, double p,
-                        double scale, bool causal);
+                        double scale, bool causal, Coverage coverage = Coverage::none);
 void flash_bwd_batched(const Tensor& dout, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& out, const Tensor& lse,
                        const Tensor& dq, const Tensor& dk, const Tensor& dv, const Tensor& pad, const Tensor& time_mask, double p,
                        double scale, bool causal, const Bits& bits);
+// q / k / v slots of a projection [T, B, H, parts, D]
+Tensor slot(const Tensor& lin, int64_t heads, int64_t parts, int64_t which);
 Tensor pad_bytes(const optional<Tensor>& mask, int64_t rows, int64_t cols);
 
 void define_autograd(pybind11::module_& m);
 void define_layers(pybind11::module_& m);
 void define_optim(pybind11::module_& m);
+void define_attention(pybind11::module_& m);
 
 }  // namespace nmtg_host

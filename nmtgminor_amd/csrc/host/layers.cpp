@@ -23,12 +23,6 @@ Tensor defined_or(const optional<Tensor>& t) { return t.has_value() ? *t : Tenso
 
 struct Rates { double attn, residual, ffn; };                     // dropout: attention weights, sub-layer outputs, feed-forward
 
-// q / k / v slots of a projection [T, B, H, parts, D]
-Tensor slot(const Tensor& lin, int64_t heads, int64_t parts, int64_t which) {
-  const int64_t d = lin.size(2) / (heads * parts);
-  return lin.as_strided({lin.size(0), lin.size(1), heads, d}, {lin.stride(0), lin.stride(1), parts * d, 1}, lin.storage_offset() + which * d);
-}
-
 // the flag of the fp16 clamp: cleared by the LayerNorm in front of the feed-forward block, see add_ln_fwd
 Tensor guard_flag(const Tensor& x) { return x.scalar_type() == at::kHalf ? empty_as(x, {1}, at::kInt) : Tensor(); }
 
@@ -197,10 +191,12 @@ struct DecoderNode : Function<DecoderNode> {
     ctx->save_for_backward({x, context, in->z1, in->stats1, in->lin, in->ctx, in->lse, in->words, in->time, r.keep1, r.h1, r.z2, r.stats2, r.c.q_lin,
                             r.c.kv_lin, r.c.softmax, r.c.dropped, r.c.mask, r.c.ctx, r.f.h, r.f.z, r.f.stats, r.f.keep, r.f.post, r.f.pre, r.f.mask,
                             r.f.guard, g1, wi, wo, g2, wq, wkv, wc, g3, w1, w2});
+    ctx->set_materialize_grads(false);                              // no zero-filled gradient of the coverage
     ctx->mark_non_differentiable({r.c.softmax});
     return {r.f.out, r.c.softmax};
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    if (!grads[0].defined()) return variable_list(20);
     auto s = ctx->get_saved_variables();
     const Tensor &x = s[0], &context = s[1], &z1 = s[2], &stats1 = s[3], &lin = s[4], &cx = s[5], &lse = s[6], &words = s[7], &time = s[8],
                  &keep1 = s[9], &h1 = s[10], &z2 = s[11], &stats2 = s[12];
@@ -241,17 +237,17 @@ std::tuple<Tensor, Tensor> decoder_step(const Tensor& x, const Tensor& kbuf, con
   const float scale = static_cast<float>(1.0 / std::sqrt(static_cast<double>(d)));
   Launch on(x);
   Norm n1 = ln_fwd(x, w[0], w[1], kEps);
-  Tensor lin = linear_fwd(n1.z, w[2], w[3]);
+  Tensor lin = linear_step(n1.z, w[2], w[3]);
   Tensor cx = at::empty_like(x);
   check(api.attn_decode_append(ptr(lin), 3 * e, ptr(kbuf), kbuf.stride(0), kbuf.stride(1), ptr(vbuf), vbuf.stride(0), vbuf.stride(1), ptr(cx), e, b,
                                heads, d, n, scale, dtype_code(x), on.stream), "nmtg_attn_decode_append");
-  AddNorm n2 = add_ln_fwd(linear_fwd(cx, w[4], w[5]), x, 0.0, Tensor(), w[6], w[7], kEps);
-  Tensor q = linear_fwd(n2.z, w[8], Tensor());
+  AddNorm n2 = add_ln_fwd(linear_step(cx, w[4], w[5]), x, 0.0, Tensor(), w[6], w[7], kEps);
+  Tensor q = linear_step(n2.z, w[8], Tensor());
   Tensor coverage = empty_like_sized(x, {b * heads, 1, tk});
   check(api.attn_decode(ptr(q), e, ptr(ck), ck.stride(0), ck.stride(1), ptr(cv), cv.stride(0), cv.stride(1),
                         static_cast<const uint8_t*>(ptr(pad)), ptr(coverage), ptr(cx), e, b, heads, d, tk, scale, dtype_code(x), on.stream),
         "nmtg_attn_decode");
-  FfnState f = ffn_fwd(linear_fwd(cx, w[10], Tensor()), n2.h, 0.0, w[11], w[12], w[13], w[14], w[15], w[16], act, 0.0, 0.0, false);
+  FfnState f = ffn_fwd(linear_step(cx, w[10], Tensor()), n2.h, 0.0, w[11], w[12], w[13], w[14], w[15], w[16], act, 0.0, 0.0, false);
   return {f.out, coverage};
 }
 

@@ -96,14 +96,26 @@ AddNormGrads ln_bwd_add(const Tensor& dz, const Tensor& x, const Tensor& stats, 
 }
 
 // -------------------------------------------------------------------------------------------------- products and MLP
+static Tensor linear_result(const Tensor& x, int64_t out) {
+  auto sizes = x.sizes().vec();
+  sizes.back() = out;
+  return empty_like_sized(x, sizes);
+}
+
 Tensor linear_fwd(const Tensor& x, const Tensor& w, const Tensor& b) {
   const int64_t in = w.size(1), out = w.size(0), rows = x.numel() / in;
   Launch on(x);
-  auto sizes = x.sizes().vec();
-  sizes.back() = out;
-  Tensor y = empty_like_sized(x, sizes);
+  Tensor y = linear_result(x, out);
   check(api.gemm(0, 1, rows, out, in, 1.f, ptr(x), in, 0, ptr(w), in, 0, ptr(y), out, 0, 1, ptr(b), nullptr, 0, dtype_code(x), on.stream),
         "nmtg_gemm");
+  return y;
+}
+
+Tensor linear_step(const Tensor& x, const Tensor& w, const Tensor& b) {
+  const int64_t in = w.size(1), out = w.size(0);
+  Launch on(x);
+  Tensor y = linear_result(x, out);
+  check(api.linear_step(x.numel() / in, out, in, ptr(x), ptr(w), ptr(b), ptr(y), dtype_code(x), on.stream), "nmtg_linear_step");
   return y;
 }
 
@@ -232,6 +244,11 @@ static Tensor bits_words(const Tensor& like, int64_t b, int64_t h, int64_t tq, i
 }
 static Tensor info_words(const Tensor& like, int64_t bytes) { return empty_as(like, {std::max<int64_t>(bytes, 4) / 4}, at::kInt); }
 
+Tensor slot(const Tensor& lin, int64_t heads, int64_t parts, int64_t which) {
+  const int64_t d = lin.size(2) / (heads * parts);
+  return lin.as_strided({lin.size(0), lin.size(1), heads, d}, {lin.stride(0), lin.stride(1), parts * d, 1}, lin.storage_offset() + which * d);
+}
+
 Tensor pad_bytes(const optional<Tensor>& mask, int64_t rows, int64_t cols) {
   if (!mask.has_value() || !mask->defined() || mask->numel() == 0) return Tensor();
   TORCH_CHECK(mask->numel() == rows * cols, "mask must be [", rows, ", ", cols, "]");
@@ -241,7 +258,7 @@ Tensor pad_bytes(const optional<Tensor>& mask, int64_t rows, int64_t cols) {
 }
 
 Flash flash_fwd_batched(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& pad, const Tensor& time_mask, double p,
-                        double scale, bool causal) {
+                        double scale, bool causal, Coverage coverage) {
   TORCH_CHECK((q.scalar_type() == at::kHalf || q.scalar_type() == at::kBFloat16) && k.scalar_type() == q.scalar_type() &&
               v.scalar_type() == q.scalar_type(), "flash_attn: q, k and v must share a 16-bit dtype");
   TORCH_CHECK(q.dim() == 4 && k.dim() == 4 && k.sizes() == v.sizes(), "flash_attn: q [len_q, B, H, D], k and v [len_k, B, H, D]");
@@ -265,8 +282,19 @@ Flash flash_fwd_batched(const Tensor& q, const Tensor& k, const Tensor& v, const
   if (time_mask.defined()) tinfo = info_words(q, api.flash_attn_time_info_bytes(tq, tk));
   if (p > 0.0) {
     r.bits.words = bits_words(q, b, h, tq, tk);
-    r.bits.mode = 2;
-    std::tie(r.bits.seed, r.bits.offset) = draw(q, 4 * b * h * ((tq + 3) / 4) * ((tk + 3) / 4));
+    r.bits.mode = coverage == Coverage::none ? 2 : 3;
+    std::tie(r.bits.seed, r.bits.offset) = draw(q, coverage == Coverage::none ? 4 * b * h * ((tq + 3) / 4) * ((tk + 3) / 4) : b * h * tq * tk);
+  }
+  if (coverage != Coverage::none) {
+    r.probs = empty_like_sized(q, {b * h, tq, tk});
+    check(api.flash_attn_batched_fwd_probs(
+              ptr(q), ptr(k), ptr(v), ptr(r.out), static_cast<const uint8_t*>(ptr(pad)), ptr(kinfo), static_cast<const uint8_t*>(ptr(time_mask)),
+              ptr(tinfo), r.lse.data_ptr<float>(), b, h, d, tq, tk, q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1),
+              k.stride(2), v.stride(0), v.stride(1), v.stride(2), r.out.stride(0), r.out.stride(1), r.out.stride(2), static_cast<float>(scale),
+              causal ? 1 : 0, static_cast<int>(r.bits.mode), static_cast<float>(p), nullptr, nullptr, ptr(r.bits.words), r.bits.seed,
+              r.bits.offset, dtype_code(q), on.stream, ptr(r.probs), coverage == Coverage::dropped ? 1 : 0),
+          "nmtg_flash_attn_batched_fwd_probs");
+    return r;
   }
   check(api.flash_attn_batched_fwd(ptr(q), ptr(k), ptr(v), ptr(r.out), static_cast<const uint8_t*>(ptr(pad)), ptr(kinfo),
                                    static_cast<const uint8_t*>(ptr(time_mask)), ptr(tinfo), r.lse.data_ptr<float>(), b, h, d, tq, tk,
@@ -301,4 +329,5 @@ PYBIND11_MODULE(_host, m) {
   nmtg_host::define_autograd(m);
   nmtg_host::define_layers(m);
   nmtg_host::define_optim(m);
+  nmtg_host::define_attention(m);
 }

@@ -102,6 +102,7 @@ extern "C" int nmtg_mlp_fwd(int num_layers, const void* x, const void* const* we
     int rc;
     if (last) {
       g.C = out;
+      g.skinny_rows = 64;     // nothing that could gate follows in this block
       rc = gemm_run(dtype, LAYOUT_NT, EPI_PLAIN, g, nullptr, 0, st);
     } else {
       g.C = static_cast<uint8_t*>(post_acts) + elt_off * esz;

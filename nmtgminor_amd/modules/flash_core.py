@@ -34,6 +34,13 @@ def eligible(is_training, return_coverage, recompute, x, heads):
     return x.dtype in (torch.float16, torch.bfloat16) and x.dim() == 3 and e % heads == 0 and e // heads in (64, 128)
 
 
+def with_coverage(return_coverage, p, dropout_mask):
+    """Whether a call that would be eligible without its coverage runs on the tiled core in the host layer, which writes the
+    coverage besides: on the GPU, with dropout and no explicit keep-mask. (A call without dropout stays on the extension's
+    path, whose probabilities round where the reference's stored scores do; it has no mask to write or read either.)"""
+    return bool(return_coverage) and dropout_mask is None and p > 0.0
+
+
 def _pad(mask, batch, len_k):
     if mask is None or mask.numel() == 0:
         return None

@@ -7,10 +7,12 @@ optional, T <= 4096). Rotary position encodings take the composed path of nmtgmi
 GEMM, rotation kernel, compact core); rotary together with incremental decoding raises. Incremental decoding (inference, `incremental=True` with a cache dict) runs in
 nmtgminor_amd/modules/incremental.py. As in the reference's fused branch the result is always
 the pair (outputs, dropout_results). An 18th optional argument replays an explicit dropout
-keep-mask. A training call with return_coverage false (key padding mask, time mask or none) runs the tiled attention core
-of nmtgminor_amd/modules/flash_core.py instead and returns an empty tensor as dropout_results."""
+keep-mask. A training call (key padding mask, time mask or none) runs the tiled attention core instead: with return_coverage
+false nmtgminor_amd/modules/flash_core.py, an empty tensor standing in for dropout_results; with it and dropout, on the GPU,
+the host layer (csrc/host/attention.cpp)."""
 import torch
 
+from .. import _lib as L
 from ..native import self_multihead_attn_blaslt as native
 from ._autocast import cast_if_autocast_enabled, no_autocast
 
@@ -45,10 +47,13 @@ class SelfAttnFunc(torch.autograd.Function):
         else:
             ctx.save_for_backward(inputs, input_weights, output_weights, ctx_t, dropped, scores, lin, dmask)
         ctx.mark_non_differentiable(dropped)
+        ctx.set_materialize_grads(False)                   # no zero-filled gradient of the coverage
         return outputs, dropped
 
     @staticmethod
     def backward(ctx, output_grads, coverage_grads=None):
+        if output_grads is None:
+            return (None,) * 18
         p, heads = ctx.p, ctx.heads
         output_grads = output_grads.contiguous()
         if ctx.recompute:
@@ -92,9 +97,12 @@ def self_attn_func(*args):
             cos, sin = pos_emb
             return SelfAttnRotaryFunc.apply(use_time_mask, is_training, heads, inputs, w_in, w_out, b_in, b_out, mask, p, cos,
                                             sin, args[17] if len(args) > 17 else None)
-        if len(args) >= 17:                           # training call whose coverage nobody reads: no [B*H, T, T] tensor
+        if len(args) >= 17:                           # training call: the tiled core; no [B*H, T, T] tensor besides the coverage
             from . import flash_core
             (use_time_mask, is_training, heads, inputs, w_in, w_out, b_in, b_out, mask, p) = args[:10]
+            if inputs.is_cuda and flash_core.with_coverage(args[15], p, args[17] if len(args) > 17 else None) and \
+                    flash_core.eligible(is_training, False, args[16], inputs, heads):
+                return tuple(L.host().self_attention(inputs, w_in, w_out, b_in, b_out, mask, bool(use_time_mask), heads, p))
             if flash_core.eligible(is_training, args[15], args[16], inputs, heads):
                 outputs = flash_core.SelfAttnFlashFunc.apply(bool(use_time_mask), heads, inputs, w_in, w_out, b_in, b_out, mask, p,
                                                              args[17] if len(args) > 17 else None)
