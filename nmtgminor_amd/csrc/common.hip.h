@@ -235,6 +235,16 @@ template <> __device__ __forceinline__ float dot2<bf16_t>(uint32_t a, uint32_t b
 // counter and a 64-bit key into four 32-bit words. Dropout draws u = (word >> 8) * 2^-24 in
 // [0, 1) and keeps an element when u < keep_probability.
 // ---------------------------------------------------------------------------------------------
+// a ^ b ^ c: one instruction on gfx950, which the compiler does not form by itself (two thirds of the generator's vector
+// instructions were exclusive-ors and multiplies in equal parts; keep bits of 512 x [512 x 512] elements 75 -> 57 us)
+__device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+#if __has_builtin(__builtin_amdgcn_bitop3_b32)
+  return static_cast<uint32_t>(__builtin_amdgcn_bitop3_b32(static_cast<int>(a), static_cast<int>(b), static_cast<int>(c), 0x96));
+#else
+  return a ^ b ^ c;
+#endif
+}
+
 struct Philox {
   uint32_t key0, key1;
   __device__ __forceinline__ Philox(uint64_t seed) : key0(static_cast<uint32_t>(seed)), key1(static_cast<uint32_t>(seed >> 32)) {}
@@ -248,7 +258,7 @@ struct Philox {
       const uint64_t p0 = static_cast<uint64_t>(0xD2511F53u) * c0, p1 = static_cast<uint64_t>(0xCD9E8D57u) * c2;
       const uint32_t hi0 = static_cast<uint32_t>(p0 >> 32), lo0 = static_cast<uint32_t>(p0);
       const uint32_t hi1 = static_cast<uint32_t>(p1 >> 32), lo1 = static_cast<uint32_t>(p1);
-      const uint32_t n0 = hi1 ^ c1 ^ k0, n2 = hi0 ^ c3 ^ k1;
+      const uint32_t n0 = xor3(hi1, c1, k0), n2 = xor3(hi0, c3, k1);
       c0 = n0; c1 = lo1; c2 = n2; c3 = lo0;
       k0 += 0x9E3779B9u; k1 += 0xBB67AE85u;
     }

@@ -62,7 +62,7 @@ struct FaArgs {
   int causal;
   const uint8_t* mask;   // explicit keep-mask [B, H, max_q, max_k] (bit kernel, mode 1)
   uint8_t* mask_out;     // where the drawn mask is written as bytes, or null (bit kernel, mode 2)
-  uint32_t thr;          // keep when byte < thr (bit kernel, mode 2) or when the word's upper 24 bits are (mode 3)
+  uint32_t thr;          // keep when byte < thr (bit kernel, mode 2) or when word <= thr (mode 3)
   float drop_scale;
   uint64_t seed, offset;
   // keep bits [B H, q32 groups of 32 queries, kp keys]: bit (i % 32) of word bit_slot(j) of row (b H + h, i / 32)
@@ -430,7 +430,7 @@ __global__ __launch_bounds__(256) void flash_bits_linear_kernel(FaArgs a, int64_
       for (int k = 0; k < 4; ++k) w[k] = shift == 0 ? both[k] : shift == 1 ? both[k + 1] : shift == 2 ? both[k + 2] : both[k + 3];
     }
 #pragma unroll
-    for (int k = 0; k < 4; ++k) word[k] |= ((w[k] >> 8) < a.thr ? 1u : 0u) << i;
+    for (int k = 0; k < 4; ++k) word[k] |= (w[k] <= a.thr ? 1u : 0u) << i;
   }
   uint32_t* out = a.bits + row * a.kp;
 #pragma unroll
@@ -1603,8 +1603,8 @@ void set_dropout(FaArgs& a, int drop_mode, float p, uint64_t seed, uint64_t offs
   a.thr = 256;
   a.drop_scale = 1.f;
   if (drop_mode == 1 || drop_mode == 3) a.drop_scale = 1.f / (1.f - p);
-  // (word >> 8) 2^-24 < 1 - p, compared as integers (the product is exact)
-  if (drop_mode == 3) a.thr = static_cast<uint32_t>(std::ceil((1.f - p) * 16777216.f));
+  // (word >> 8) 2^-24 < 1 - p, compared as integers (the product is exact) and without the shift
+  if (drop_mode == 3) a.thr = static_cast<uint32_t>((static_cast<uint64_t>(std::ceil((1.f - p) * 16777216.f)) << 8) - 1);
   if (drop_mode == 2) {
     long thr = lroundf(256.f * (1.f - p));
     a.thr = static_cast<uint32_t>(thr < 1 ? 1 : thr > 256 ? 256 : thr);
