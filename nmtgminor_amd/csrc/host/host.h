@@ -1,7 +1,7 @@
 // Shared pieces of the native host layer (nmtgminor_amd/_host.so): the table of C entry points it calls, and the
 // operators as functions from tensors to tensors (allocate the results, enqueue the kernels). ops.cpp implements them,
-// autograd.cpp wraps them in autograd nodes, layers.cpp composes the transformer layers, attention.cpp the attention modules, optim.cpp prepares the
-// optimizer's passes.
+// autograd.cpp wraps them in autograd nodes, layers.cpp composes the transformer layers, attention.cpp the attention modules, loss.cpp the output
+// projection with its loss, optim.cpp prepares the optimizer's passes.
 //
 // Why it exists: a call through the Python stand-ins costs 25 to 80 us of interpreter, ctypes and autograd bookkeeping per
 // operator and direction, several times what the kernels of a small batch take. The same work here is 3 to 8 us.
@@ -28,7 +28,8 @@ using std::optional;
   X(xentropy_bwd) X(gemm) X(mlp_fwd) X(mlp_bwd_dtype_workspace_bytes) X(mlp_bwd) X(flash_attn_dropout_bits_bytes)     \
   X(flash_attn_fwd) X(flash_attn_bwd) X(flash_attn_key_info_bytes) X(flash_attn_time_info_bytes)                      \
   X(flash_attn_batched_fwd) X(flash_attn_batched_bwd) X(multi_tensor_adam) X(multi_tensor_clip)                       \
-  X(multi_tensor_l2norm) X(multi_tensor_l2norm_workspace_bytes) X(flash_attn_batched_fwd_probs) X(linear_step)
+  X(multi_tensor_l2norm) X(multi_tensor_l2norm_workspace_bytes) X(flash_attn_batched_fwd_probs) X(linear_step) X(gemm_workspace_bytes)            \
+  X(xentropy_bwd_colsum) X(xentropy_bwd_colsum_parts)
 
 struct Api {
 #define X(name) decltype(&nmtg_##name) name = nullptr;
@@ -115,5 +116,6 @@ void define_autograd(pybind11::module_& m);
 void define_layers(pybind11::module_& m);
 void define_optim(pybind11::module_& m);
 void define_attention(pybind11::module_& m);
+void define_loss(pybind11::module_& m);
 
 }  // namespace nmtg_host

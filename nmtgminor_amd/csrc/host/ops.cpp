@@ -330,4 +330,5 @@ PYBIND11_MODULE(_host, m) {
   nmtg_host::define_layers(m);
   nmtg_host::define_optim(m);
   nmtg_host::define_attention(m);
+  nmtg_host::define_loss(m);
 }

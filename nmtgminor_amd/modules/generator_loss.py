@@ -31,6 +31,7 @@ per-slice gradients of the states (`add_` in fp32, [N, E]): a device-side PyTorc
 import torch
 import torch.nn as nn
 
+from .. import _lib as L
 from ..native import linear_gemm, xentropy_cuda
 
 DEFAULT_CHUNK_ROWS = 4096
@@ -234,8 +235,14 @@ class GeneratorLoss(nn.Module):
             correct, total = int(((preds == y) & real).sum().item()), int(real.sum().item())
         else:
             smoothing = self.label_smoothing if self.training else 0.0
-            rows = LinearSoftmaxCrossEntropy.apply(h, self.linear.weight, self.linear.bias, y, smoothing,
-                                                   self.padding_idx, self.chunk_rows)
+            w, c = self.linear.weight, self.linear.bias
+            kept = L.host().generator_loss(h, w, c, y, float(smoothing), int(self.padding_idx), DEFAULT_KEEP_LOGITS_BYTES) if h.is_cuda else None
+            if kept is not None:
+                rows, total_loss = kept
+                if sum_loss and not loss_constraint and loss_weights is None:
+                    return dict(loss=total_loss, data=total_loss.detach().item(), correct=correct, total=total)
+            else:
+                rows = LinearSoftmaxCrossEntropy.apply(h, w, c, y, smoothing, self.padding_idx, self.chunk_rows)
         data = rows.detach().sum().item() if sum_loss else rows.detach()
         # the constraint is subtracted on real rows only: padded rows are not part of the reference's batch
         loss = rows - loss_constraint * (y != self.padding_idx).to(rows.dtype) if loss_constraint else rows
