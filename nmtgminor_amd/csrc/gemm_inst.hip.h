@@ -63,14 +63,14 @@ template <bool B_KC, int EPI> struct gemm_ring_ragged {
   static constexpr bool value = !B_KC && (EPI == EPI_PLAIN || EPI == EPI_SPLITK);
 };
 
-template <typename T, int TILE, bool A_KC, bool B_KC, int EPI, bool RAGGED = false>
+template <typename T, int TILE, bool A_KC, bool B_KC, int EPI, bool RAGGED = false, bool STREAM = false>
 int gemm_launch_ring(const GemmArgs& a, hipStream_t st) {
   using C = tile_cfg<TILE>;
   constexpr int RING = ring_slots<TILE>::value;
   constexpr bool RIDER = ring_rider<TILE, A_KC, B_KC, EPI>::value;
   auto kern = [] {
-    if constexpr (RIDER) return gemm_ring_rider_kernel<T, C::BM, C::BN, C::WM, C::WN, A_KC, B_KC, EPI, RING, ring_stepbuf<TILE>::value, RAGGED>;
-    else return gemm_ring_kernel<T, C::BM, C::BN, C::WM, C::WN, A_KC, B_KC, EPI, RING, ring_stepbuf<TILE>::value, RAGGED>;
+    if constexpr (RIDER) return gemm_ring_rider_kernel<T, C::BM, C::BN, C::WM, C::WN, A_KC, B_KC, EPI, RING, ring_stepbuf<TILE>::value, RAGGED, STREAM>;
+    else return gemm_ring_kernel<T, C::BM, C::BN, C::WM, C::WN, A_KC, B_KC, EPI, RING, ring_stepbuf<TILE>::value, RAGGED, STREAM>;
   }();
   constexpr int lds = gemm_ring_lds_bytes<C::BM, C::BN, RING>();
   static bool attr_done = false;
@@ -79,11 +79,11 @@ int gemm_launch_ring(const GemmArgs& a, hipStream_t st) {
     if (e != hipSuccess) return fail(NMTG_ERR_LAUNCH, "gemm: cannot reserve %d bytes of LDS: %s", lds, hipGetErrorString(e));
     attr_done = true;
   }
-  dim3 grid(a.m_tiles * a.n_tiles, a.batch, a.splits);
+  dim3 grid(STREAM ? static_cast<unsigned>(num_cus()) : static_cast<unsigned>(a.m_tiles * a.n_tiles), a.batch, a.splits);
   static const std::string name = std::string("gemm_") + (A_KC ? (B_KC ? "nt" : "nn") : "tn") + "_" +
                                   (TILE == TILE_L ? "256x256" : TILE == TILE_M ? "128x128" : "256x64") + "_" +
                                   (EPI == EPI_PLAIN ? "plain" : EPI == EPI_ACT_FWD ? "actfwd" : EPI == EPI_ACT_BWD ? "actbwd"
-                                   : EPI == EPI_SCORES ? "scores" : "splitk") + "_ring";
+                                   : EPI == EPI_SCORES ? "scores" : "splitk") + (STREAM ? "_stream" : "_ring");
   TraceScope trace(name.c_str(), st);
   if constexpr (RIDER) {
     const bool ride = a.riders != nullptr && a.rider_blocks > 0;
@@ -103,6 +103,12 @@ int gemm_launch_ring(const GemmArgs& a, hipStream_t st) {
 template <typename T, int TILE, bool A_KC, bool B_KC, int EPI>
 int gemm_launch_one(const GemmArgs& a, hipStream_t st) {
   if (a.vec == 8 && a.ring) {
+    // more 256x256 tiles than compute units: one block per unit walks its share of them (at least three steps of k, the ring's
+    // worth of transfers)
+    if constexpr (TILE == TILE_L && EPI == EPI_PLAIN) {
+      if (a.K % GEMM_BK == 0 && a.K >= 3 * GEMM_BK && a.batch == 1 && a.splits == 1 && a.m_tiles * a.n_tiles > num_cus())
+        return gemm_launch_ring<T, TILE, A_KC, B_KC, EPI, false, true>(a, st);
+    }
     if constexpr (gemm_ring_ragged<B_KC, EPI>::value) {
       if (a.K % GEMM_BK != 0) return gemm_launch_ring<T, TILE, A_KC, B_KC, EPI, true>(a, st);
     }

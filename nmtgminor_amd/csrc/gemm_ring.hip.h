@@ -91,6 +91,90 @@ constexpr int gemm_ring_lds_bytes() {
   return main_loop > c_tile ? main_loop : c_tile;
 }
 
+// A vector store occupies a place in the same in-order counter as the transfers; a CPU build of this source counts the
+// transfers alone.
+constexpr int counted_stores(int n) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return n;
+#else
+  return 0 * n;
+#endif
+}
+
+// The way out of a tile while the next one's first stages are on their way into the ring: the wavefront's rows go through a
+// patch of its own, 32 rows x 64 columns at a time (no barrier), and leave as whole 128-byte lines.
+constexpr int STREAM_PATCH_BYTES = 32 * 128;
+template <typename T, int TM, int TN>
+struct StreamEpilogue {
+  uint2 braw[TN][4];
+  // requested a stage before the end of the tile
+  __device__ __forceinline__ void load_bias(const GemmArgs& g, int nw, int lane) {
+    const T* bias = static_cast<const T*>(g.bias);
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int n = nw + j * 32 + q * 8 + (lane >> 5) * 4;
+        braw[j][q] = make_uint2(0, 0);
+        if (bias != nullptr) {
+          if (n + 4 <= g.N) {
+            braw[j][q] = *reinterpret_cast<const uint2*>(bias + n);
+          } else {
+            T* e = reinterpret_cast<T*>(&braw[j][q]);
+            for (int k = 0; k < 4; ++k) if (n + k < g.N) e[k] = bias[n + k];
+          }
+        }
+      }
+  }
+  // a use, so that the compiler waits for the bias here and not behind transfers it does not know of
+  __device__ __forceinline__ void bias_landed() {
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        asm volatile("" : "+v"(braw[j][q].x));
+        asm volatile("" : "+v"(braw[j][q].y));
+      }
+  }
+  // -> whether exactly TM * 4 stores went out (the tile lies inside C)
+  __device__ __forceinline__ bool store(const GemmArgs& g, const acc16_t (&acc)[TM][TN], uint8_t* patch, int mw, int nw, int lane) {
+    static_assert(TN == 2, "a patch row is 64 columns");
+    const bool whole = mw + 32 * TM <= g.M && nw + 64 <= g.N;
+    uint16_t* C = reinterpret_cast<uint16_t*>(g.C);
+    const int row = lane & 31, half = lane >> 5;
+    auto rows = [&](auto whole_tag) {
+      constexpr bool WHOLE = decltype(whole_tag)::value;
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const T* b4 = reinterpret_cast<const T*>(&braw[j][q]);
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = acc[i][j][q * 4 + e] * g.alpha + elem<T>::to_float(b4[e]);
+            store_pack<T, 4>(reinterpret_cast<T*>(patch + row * 128 + (((4 * j + q) ^ (row & 7)) * 16) + half * 8), v);
+          }
+        wave_lds_fence();
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int r = 8 * u + (lane >> 3), c = lane & 7;
+          const uint4 v = *reinterpret_cast<const uint4*>(patch + r * 128 + ((c ^ (r & 7)) * 16));
+          const int m = mw + 32 * i + r, n = nw + 8 * c;
+          uint16_t* to = C + static_cast<int64_t>(m) * g.ldc + n;
+          if constexpr (WHOLE) store8<8>(to, v, 8);
+          else store8<8>(to, v, m < g.M ? g.N - n : 0);
+        }
+        wave_lds_fence();
+      }
+    };
+    if (whole) rows(std::true_type{});
+    else rows(std::false_type{});
+    return whole;
+  }
+};
+
 // STEPBUF = false: a step reads its operand fragments from LDS k-group by k-group, one k-group ahead of the MFMAs
 // that use them, and ends with the wait for the next stage and the barrier: the matrix pipe drains there, which two
 // wavefronts per SIMD (the 256x256 tile) cover in part and a single one (the 128x128 tile) does not.
@@ -101,7 +185,7 @@ constexpr int gemm_ring_lds_bytes() {
 // out between the MFMAs of the remaining k-groups. The matrix pipe has work on both sides of the barrier. Phase 0
 // only reads, one more phase without reads follows the last stage; the ring positions and the vmcnt bookkeeping are
 // those of the plain loop.
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, bool A_KC, bool B_KC, int EPI, int RING, bool STEPBUF = false, bool RAGGED = false>
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, bool A_KC, bool B_KC, int EPI, int RING, bool STEPBUF = false, bool RAGGED = false, bool STREAM = false>
 __device__ __forceinline__ void gemm_ring_body(const GemmArgs& g, int block_x) {
   constexpr int NT = 64 * WAVES_M * WAVES_N, NW = NT / 64;
   constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N;
@@ -122,15 +206,20 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs& g, int block_x) {
   const int wm0 = (wave / WAVES_N) * WTM, wn0 = (wave % WAVES_N) * WTN;
 
   // tile order: see gemm_kernel
-  int bid = block_x;
   const int ntile = g.m_tiles * g.n_tiles;
-  if ((ntile & 7) == 0) bid = (bid & 7) * (ntile >> 3) + (bid >> 3);
-  constexpr int GM = 4;
-  const int in_group = GM * g.n_tiles;
-  const int first_m = (bid / in_group) * GM;
-  const int gsize = min(g.m_tiles - first_m, GM);
-  const int tile_m = first_m + (bid % in_group) % gsize, tile_n = (bid % in_group) / gsize;
-  const int m0 = tile_m * BM, n0 = tile_n * BN;
+  int tile_m, tile_n, m0, n0;
+  auto place = [&](int bid) {
+    if ((ntile & 7) == 0) bid = (bid & 7) * (ntile >> 3) + (bid >> 3);
+    constexpr int GM = 4;
+    const int in_group = GM * g.n_tiles;
+    const int first_m = (bid / in_group) * GM;
+    const int gsize = min(g.m_tiles - first_m, GM);
+    tile_m = first_m + (bid % in_group) % gsize;
+    tile_n = (bid % in_group) / gsize;
+    m0 = tile_m * BM;
+    n0 = tile_n * BN;
+  };
+  place(block_x);
   const int bz = blockIdx.y, split = blockIdx.z;
 
   const int kbeg = split * g.k_per_split;
@@ -142,10 +231,14 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs& g, int block_x) {
   const int64_t lda_b = g.lda * 2, ldb_b = g.ldb * 2;  // bytes
   // A reduction-contiguous operand is addressed from the first row of this block's tile (64-bit, scalar), so that the
   // per-lane offsets span one tile's rows and fit 32 bits whatever the size of the operand.
-  const char* a_base = static_cast<const char*>(g.A) + static_cast<int64_t>(bz) * g.sA * 2 + static_cast<int64_t>(kbeg) * (A_KC ? 2 : lda_b) +
-                       (A_KC ? static_cast<int64_t>(m0) * lda_b : 0);
-  const char* b_base = static_cast<const char*>(g.B) + static_cast<int64_t>(bz) * g.sB * 2 + static_cast<int64_t>(kbeg) * (B_KC ? 2 : ldb_b) +
-                       (B_KC ? static_cast<int64_t>(n0) * ldb_b : 0);
+  const char *a_base, *b_base;
+  auto operand_bases = [&]() {
+    a_base = static_cast<const char*>(g.A) + static_cast<int64_t>(bz) * g.sA * 2 + static_cast<int64_t>(kbeg) * (A_KC ? 2 : lda_b) +
+             (A_KC ? static_cast<int64_t>(m0) * lda_b : 0);
+    b_base = static_cast<const char*>(g.B) + static_cast<int64_t>(bz) * g.sB * 2 + static_cast<int64_t>(kbeg) * (B_KC ? 2 : ldb_b) +
+             (B_KC ? static_cast<int64_t>(n0) * ldb_b : 0);
+  };
+  operand_bases();
   const int64_t step_a = A_KC ? GEMM_BK * 2 : GEMM_BK * lda_b;
   const int64_t step_b = B_KC ? GEMM_BK * 2 : GEMM_BK * ldb_b;
 
@@ -165,14 +258,17 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs& g, int block_x) {
       return static_cast<uint32_t>(static_cast<int64_t>(k) * ld_b + row * 2);
     }
   };
+  auto transfer_offsets = [&]() {
 #pragma unroll
-  for (int j = 0; j < SA; ++j)
+    for (int j = 0; j < SA; ++j)
 #pragma unroll
-    for (int i = 0; i < IPS; ++i) dA[j][i] = lane_offsets(std::integral_constant<bool, A_KC>{}, g.M, m0, lda_b, j, i);
+      for (int i = 0; i < IPS; ++i) dA[j][i] = lane_offsets(std::integral_constant<bool, A_KC>{}, g.M, m0, lda_b, j, i);
 #pragma unroll
-  for (int j = 0; j < SB; ++j)
+    for (int j = 0; j < SB; ++j)
 #pragma unroll
-    for (int i = 0; i < IPS; ++i) dB[j][i] = lane_offsets(std::integral_constant<bool, B_KC>{}, g.N, n0, ldb_b, j, i);
+      for (int i = 0; i < IPS; ++i) dB[j][i] = lane_offsets(std::integral_constant<bool, B_KC>{}, g.N, n0, ldb_b, j, i);
+  };
+  transfer_offsets();
 
   // LDS address of the ring (the transfers name their destination by address, not through a pointer)
   const uint32_t lds_base = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds_raw)));
@@ -219,12 +315,15 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs& g, int block_x) {
     for (int kk = 0; kk < (B_KC ? 4 : 1); ++kk) fb[j][kk] = frag_offsets(std::integral_constant<bool, B_KC>{}, wn0 % 128, j, kk);
 
   acc16_t acc[TM][TN];
+  auto clear = [&]() {
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
+      for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  };
+  clear();
 
   NMTG_PROF_MARK(0);
   // ---- prologue: fill the ring ----
@@ -335,6 +434,8 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs& g, int block_x) {
       if constexpr (MFMAS > PAIRS) __builtin_amdgcn_sched_group_barrier(0x008, MFMAS - PAIRS, 0);
     };
     static_assert(KG % 2 == 0, "the fragment buffers alternate by k-group and the loop carries buffer 0 across steps");
+    [[maybe_unused]] StreamEpilogue<T, TM, TN> out;
+    for (int next = block_x + static_cast<int>(gridDim.x);; next += static_cast<int>(gridDim.x)) {   // once, unless STREAM
     auto slots_of = [&](int pos, const uint8_t*& sa, const uint8_t*& sb) {
       int pa = pos + ja, pb = pos + SA + jb;
       if (pa >= RING) pa -= RING;
@@ -374,10 +475,46 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs& g, int block_x) {
       pin_pairs();
       refill(s + 1);   // into the slots of stage s, behind the MFMAs that keep the pipe busy right after the barrier
     }
+    if constexpr (STREAM) out.load_bias(g, n0 + wn0, lane);
     if (nk > 0) {
       leading_groups();
       mfmas(std::integral_constant<int, (KG - 1) & 1>{});
       ring_barrier();   // every wavefront is done reading the ring: the epilogue stages the output tile there
+    }
+    if constexpr (!STREAM) {
+      break;
+    } else {
+      const int om0 = m0, on0 = n0;
+      const bool more = next < ntile;
+      out.bias_landed();
+      if (more) {
+        // the first two stages of the next tile travel while this one is written out
+        place(next);
+        operand_bases();
+        transfer_offsets();
+        static_for<0, 2 * SPS>([&](auto tt) {
+          constexpr int t = decltype(tt)::value;
+          issue(std::integral_constant<int, t % SPS>{}, a_base + (t / SPS) * step_a, b_base + (t / SPS) * step_b, t, t / SPS);
+        });
+      }
+      const bool counted = out.store(g, acc, lds_raw + 2 * SPS * RING_SLOT_BYTES + wave * STREAM_PATCH_BYTES, om0 + wm0, on0 + wn0, lane);
+      if (!more) return;
+      ring_barrier();   // every wavefront is done with its patch: the slots there belong to the ring again
+      static_for<2 * SPS, RING>([&](auto tt) {
+        constexpr int t = decltype(tt)::value;
+        issue(std::integral_constant<int, t % SPS>{}, a_base + (t / SPS) * step_a, b_base + (t / SPS) * step_b, t, t / SPS);
+      });
+      clear();
+      pos_r = pos_w = 0;
+      a_cur = a_base - step_a;
+      b_cur = b_base - step_b;
+      // stage 0 has landed when only what was issued behind it is outstanding: stage 1, this tile's stores (at least none,
+      // and all of them where the tile is whole) and the last RING - 2 SPS slots
+      constexpr int behind = (RING - SPS) * IPS;
+      if (counted) wait_vmcnt<behind + counted_stores(TM * 4)>();
+      else wait_vmcnt<behind>();
+      ring_barrier();
+    }
     }
   } else {
     // Two register sets of a whole stage's fragments; phases alternate between them. Phase 0 only reads, the phase
@@ -490,9 +627,9 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs& g, int block_x) {
   gemm_epilogue<T, BM, BN, WAVES_M, WAVES_N, EPI, 8, true>(g, acc, lds_raw, tile_m, tile_n, bz, split);
 }
 
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, bool A_KC, bool B_KC, int EPI, int RING, bool STEPBUF = false, bool RAGGED = false>
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, bool A_KC, bool B_KC, int EPI, int RING, bool STEPBUF = false, bool RAGGED = false, bool STREAM = false>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_ring_kernel(const GemmArgs g) {
-  gemm_ring_body<T, BM, BN, WAVES_M, WAVES_N, A_KC, B_KC, EPI, RING, STEPBUF, RAGGED>(g, static_cast<int>(blockIdx.x));
+  gemm_ring_body<T, BM, BN, WAVES_M, WAVES_N, A_KC, B_KC, EPI, RING, STEPBUF, RAGGED, STREAM>(g, static_cast<int>(blockIdx.x));
 }
 
 // The same kernel with riders: the first g.rider_blocks blocks of the grid's x extent (first batch and split only) run
@@ -500,7 +637,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_ring_kernel(const
 // for a second one there; the riders' loads and adds fill the memory pipes that the main loop leaves idle, and the
 // launches those jobs would otherwise need fall away. The jobs are independent of this product. The riders come
 // first, one per CU, so that the tiles that follow spread over the CUs as they would without them.
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, bool A_KC, bool B_KC, int EPI, int RING, bool STEPBUF = false, bool RAGGED = false>
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, bool A_KC, bool B_KC, int EPI, int RING, bool STEPBUF = false, bool RAGGED = false, bool STREAM = false>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_ring_rider_kernel(const GemmArgs g, const TailArgs riders) {
   static_assert(64 * WAVES_M * WAVES_N == 256, "the reduction jobs are written for blocks of 256 threads");
   if (static_cast<int>(blockIdx.x) < g.rider_blocks) {
@@ -509,7 +646,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_ring_rider_kernel
       tail_ride<T>(riders, static_cast<int>(blockIdx.x), g.rider_blocks, reinterpret_cast<float*>(lds_raw));
     return;
   }
-  gemm_ring_body<T, BM, BN, WAVES_M, WAVES_N, A_KC, B_KC, EPI, RING, STEPBUF, RAGGED>(g, static_cast<int>(blockIdx.x) - g.rider_blocks);
+  gemm_ring_body<T, BM, BN, WAVES_M, WAVES_N, A_KC, B_KC, EPI, RING, STEPBUF, RAGGED, STREAM>(g, static_cast<int>(blockIdx.x) - g.rider_blocks);
 }
 
 }  // namespace nmtg

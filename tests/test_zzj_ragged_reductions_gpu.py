@@ -48,3 +48,21 @@ def test_loss_backward_with_column_sums(dev, dtype, rows, vocab, one_grad):
     got, sums = xentropy_cuda.backward_with_colsum(grad, z, lse, labels, 0.1, 1, z)
     assert_close(got, want.cpu().to(D), dtype, "gradient", scale_atol=True)
     assert_close(sums, want.cpu().to(D).sum(0), dtype, "column sums", scale_atol=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(4200, 4100, 192), (4096, 4352, 256), (256 * 300 + 8, 256, 320), (264, 256 * 260 + 24, 1024)])
+@pytest.mark.parametrize("layout", ["nt", "nn", "tn"])
+def test_more_tiles_than_compute_units(dev, dtype, m, n, k, layout):
+    """One block per unit walks several 256 x 256 tiles: whole ones, ragged ends in both directions, uneven shares."""
+    g = torch.Generator(device=dev).manual_seed(m + k)
+    make = lambda r, c: torch.randn(r, c, generator=g, device=dev).to(dtype)
+    a, b = make(k, m) if layout == "tn" else make(m, k), make(n, k) if layout == "nt" else make(k, n)
+    bias = make(1, n)[0] if layout == "nt" else None
+    pitched = torch.full((m, n + 8), 7.0, dtype=dtype, device=dev)
+    got = linear_gemm.gemm(a, b, trans_a=layout == "tn", trans_b=layout == "nt", bias=bias, out=pitched[:, :n], split_k=False)
+    want = (a.t() if layout == "tn" else a).float() @ (b.t() if layout == "nt" else b).float() + (0 if bias is None else bias.float())
+    bound = (5e-3 if dtype == torch.float16 else 4e-2) * k ** 0.5
+    for r in range(0, m, 8192):
+        assert float((got[r:r + 8192].float() - want[r:r + 8192]).abs().max()) < bound
+    assert bool((pitched[:, n:] == 7.0).all())
