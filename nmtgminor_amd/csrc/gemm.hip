@@ -8,6 +8,7 @@
 namespace nmtg {
 
 bool gemm_has(int layout, int tile, int epi) {
+  if (tile == TILE_X) return epi == EPI_PLAIN || epi == (layout == LAYOUT_NT ? EPI_ACT_FWD : layout == LAYOUT_NN ? EPI_ACT_BWD : EPI_PLAIN);
   if (layout == LAYOUT_NT)
     return (tile == TILE_L || tile == TILE_M) && (epi == EPI_PLAIN || epi == EPI_ACT_FWD || epi == EPI_SCORES);
   if (layout == LAYOUT_NN) {
@@ -130,7 +131,7 @@ int gemm_run(int dtype, int layout, int epi, GemmArgs a, void* workspace, size_t
   }
   // NMTG_GEMM_TILE=0|1|2 (256x256 | 128x128 | 256x64) overrides the tile choice: a tuning aid.
   const int forced_tile = [] { const char* e = getenv("NMTG_GEMM_TILE"); return e ? atoi(e) : -1; }();
-  if (tile < 0 && forced_tile >= 0 && gemm_has(layout, forced_tile, epi) && (forced_tile != TILE_L || vec == 8)) tile = forced_tile;
+  if (tile < 0 && forced_tile >= 0 && forced_tile != TILE_X && gemm_has(layout, forced_tile, epi) && (forced_tile != TILE_L || vec == 8)) tile = forced_tile;
   if (tile < 0) {
     const int cus = num_cus();
     const int64_t cnt_l = static_cast<int64_t>(ceil_div(a.M, 256)) * ceil_div(a.N, 256) * a.batch;
@@ -148,6 +149,10 @@ int gemm_run(int dtype, int layout, int epi, GemmArgs a, void* workspace, size_t
     else if (l_ok) tile = TILE_L;
     else tile = TILE_S;
   }
+  // 64x64 tiles where 128x128 ones would leave more than half of the chip idle: four times the blocks, each a quarter of the
+  // work, and the same sums in the same order. Chosen below, once the call is known to suit the ring kernel.
+  const bool few_tiles = tile == TILE_M && forced_tile < 0 && gemm_has(layout, TILE_X, epi) &&
+                         static_cast<int64_t>(ceil_div(a.M, 128)) * ceil_div(a.N, 128) * a.batch * 2 <= num_cus();
   if (!gemm_has(layout, tile, epi))
     return fail(NMTG_ERR_UNSUPPORTED, "gemm: layout %d has no kernel for epilogue %d", layout, epi);
   // The slot-ring kernel (direct global -> LDS loads) needs whole 64-k steps where gemm_ring_ragged<> (gemm_inst.hip.h) has
@@ -157,6 +162,7 @@ int gemm_run(int dtype, int layout, int epi, GemmArgs a, void* workspace, size_t
   const int64_t b_span = b_kc ? 256 * a.ldb * 2 : 64 * a.ldb * 2 + static_cast<int64_t>(a.N) * 2;
   const bool whole = a.K % GEMM_BK == 0 || (layout != LAYOUT_NT && (epi == EPI_PLAIN || epi == EPI_SPLITK));
   a.ring = (a.K > 0 && whole && vec == 8 && a_span < (int64_t{1} << 32) && b_span < (int64_t{1} << 32)) ? 1 : 0;
+  if (few_tiles && a.ring) tile = TILE_X;
   // gelu and gelu' of the activation epilogues come from a table in LDS in the ring kernels (they have the LDS room)
   a.act_lut = (a.ring && (epi == EPI_ACT_FWD || epi == EPI_ACT_BWD)) ? 1 : 0;
   int bm, bn;
@@ -171,7 +177,7 @@ int gemm_run(int dtype, int layout, int epi, GemmArgs a, void* workspace, size_t
   a.tile_used = tile;
   if (epi != EPI_SPLITK) a.defer_reduce = 0;
   // riders travel with the kernels that ring_rider<> (gemm_inst.hip.h) names, and only in an unbatched launch
-  const bool can_ride = tile == TILE_M && a.vec == 8 && a.ring && a.batch == 1 && layout == LAYOUT_NN && epi == EPI_PLAIN;
+  const bool can_ride = (tile == TILE_M || tile == TILE_X) && a.vec == 8 && a.ring && a.batch == 1 && layout == LAYOUT_NN && epi == EPI_PLAIN;
   a.riders_taken = (a.riders != nullptr && a.rider_blocks > 0 && can_ride) ? 1 : 0;
   if (!a.riders_taken) { a.riders = nullptr; a.rider_blocks = 0; }
   if (planned_out) *planned_out = a;

@@ -3,6 +3,7 @@
 //   L: 256x256 tile, 2x4 wavefronts (each 128x64), 512 threads  — large outputs
 //   M: 128x128 tile, 2x2 wavefronts (each 64x64),  256 threads  — outputs too small to fill the chip with L
 //   S: 256x64  tile, 4x1 wavefronts (each 64x64),  256 threads  — N <= 64 (per-head attention products)
+//   X: 64x64 tile, 2x2 wavefronts (each 32x32),    256 threads  — outputs too small to fill the chip with M (ring kernel only)
 //   R: 128x512 tile, 4x2 wavefronts (each 32x256), 512 threads  — whole score rows (fused softmax epilogue only)
 #pragma once
 #include "gemm.hip.h"
@@ -17,6 +18,7 @@ inline void tile_dims(int tile, int& bm, int& bn) {
   if (tile == TILE_L) { bm = 256; bn = 256; }
   else if (tile == TILE_M) { bm = 128; bn = 128; }
   else if (tile == TILE_R) { bm = 128; bn = 512; }
+  else if (tile == TILE_X) { bm = 64; bn = 64; }
   else { bm = 256; bn = 64; }
 }
 
@@ -48,13 +50,13 @@ int gemm_launch_vec(const GemmArgs& a, hipStream_t st) {
 // tile takes 5 slots so that two blocks share a CU and one block's epilogue overlaps the other's
 // main loop.
 template <int TILE> struct ring_slots { static constexpr int value = TILE == TILE_M ? 5 : 10; };
-// The 128x128 tile runs one wavefront per SIMD: its main loop keeps a whole stage's fragments in registers (STEPBUF).
-template <int TILE> struct ring_stepbuf { static constexpr bool value = TILE == TILE_M; };
+// The 128x128 and 64x64 tiles run one wavefront per SIMD: their main loop keeps a whole stage's fragments in registers (STEPBUF).
+template <int TILE> struct ring_stepbuf { static constexpr bool value = TILE == TILE_M || TILE == TILE_X; };
 
-// Which kernels carry riders (GemmArgs::riders): the plain 128x128 data-gradient product, the last kernel of a backward
+// Which kernels carry riders (GemmArgs::riders): the plain 128x128 and 64x64 data-gradient products, the last kernel of a backward
 // pass, which leaves one block on a CU at the shapes of a feed-forward block.
 template <int TILE, bool A_KC, bool B_KC, int EPI> struct ring_rider {
-  static constexpr bool value = TILE == TILE_M && A_KC && !B_KC && EPI == EPI_PLAIN;
+  static constexpr bool value = (TILE == TILE_M || TILE == TILE_X) && A_KC && !B_KC && EPI == EPI_PLAIN;
 };
 
 // Which kernels exist for a reduction that ends inside a 64-k step too: the weight and data gradients, whose reduction is the
@@ -81,7 +83,7 @@ int gemm_launch_ring(const GemmArgs& a, hipStream_t st) {
   }
   dim3 grid(STREAM ? static_cast<unsigned>(num_cus()) : static_cast<unsigned>(a.m_tiles * a.n_tiles), a.batch, a.splits);
   static const std::string name = std::string("gemm_") + (A_KC ? (B_KC ? "nt" : "nn") : "tn") + "_" +
-                                  (TILE == TILE_L ? "256x256" : TILE == TILE_M ? "128x128" : "256x64") + "_" +
+                                  (TILE == TILE_L ? "256x256" : TILE == TILE_M ? "128x128" : TILE == TILE_X ? "64x64" : "256x64") + "_" +
                                   (EPI == EPI_PLAIN ? "plain" : EPI == EPI_ACT_FWD ? "actfwd" : EPI == EPI_ACT_BWD ? "actbwd"
                                    : EPI == EPI_SCORES ? "scores" : "splitk") + (STREAM ? "_stream" : "_ring");
   TraceScope trace(name.c_str(), st);
@@ -114,8 +116,10 @@ int gemm_launch_one(const GemmArgs& a, hipStream_t st) {
     }
     return gemm_launch_ring<T, TILE, A_KC, B_KC, EPI>(a, st);
   }
-  if (a.vec == 8) return gemm_launch_vec<T, TILE, A_KC, B_KC, EPI, 8>(a, st);
-  if constexpr (TILE != TILE_L) {
+  if constexpr (TILE == TILE_X) return fail(NMTG_ERR_UNSUPPORTED, "gemm: the 64x64 tile has a ring kernel only");
+  else if (a.vec == 8) return gemm_launch_vec<T, TILE, A_KC, B_KC, EPI, 8>(a, st);
+  if constexpr (TILE == TILE_X) return 0;
+  else if constexpr (TILE != TILE_L) {
     if (a.vec == 4) return gemm_launch_vec<T, TILE, A_KC, B_KC, EPI, 4>(a, st);
     return gemm_launch_vec<T, TILE, A_KC, B_KC, EPI, 1>(a, st);
   } else {

@@ -15,7 +15,7 @@
 //     slot = [128 rows][8 chunks of 16 B], chunk position c' of row r holds k-chunk c' ^ swz(r);
 //     MFMA fragments are read with ds_read_b128.
 //   row-contiguous operand ("MC", element (row, k) at base[k * ld + row]):
-//     slot = [64 k][16 chunks of 16 B], chunk position c' of k-row k holds row-chunk c' ^ 4 (k & 3);
+//     slot = [64 k][16 chunks of 16 B], chunk position c' of k-row k holds row-chunk c' ^ 4 (k & 3) (of 8 chunks: 2 (k & 3));
 //     MFMA fragments are read with the LDS transpose read (ds_read_b64_tr_b16): the 16 lanes of a
 //     group read 4 k-rows x 16 rows and each lane receives the 4 consecutive k of its own row.
 // Both are filled by one-kilobyte transfers (64 lanes x 16 B, LDS destination contiguous, the
@@ -42,7 +42,9 @@
 
 namespace nmtg {
 
-constexpr int RING_SLOT_BYTES = 128 * GEMM_BK * 2;
+// rows of a slot: 128, or 64 for the 64x64 tile (the layout below with half the rows: 8 KB, 8 transfers)
+template <int BM> constexpr int ring_slot_rows() { return BM >= 128 ? 128 : 64; }
+template <int BM> constexpr int ring_slot_bytes() { return ring_slot_rows<BM>() * GEMM_BK * 2; }
 
 typedef short short4_t __attribute__((ext_vector_type(4)));
 
@@ -86,7 +88,7 @@ __device__ __forceinline__ void ring_barrier() { asm volatile("s_waitcnt lgkmcnt
 
 template <int BM, int BN, int RING>
 constexpr int gemm_ring_lds_bytes() {
-  constexpr int main_loop = RING * RING_SLOT_BYTES;
+  constexpr int main_loop = RING * ring_slot_bytes<BM>();
   constexpr int c_tile = ((BM * (BN * 2 + 8) + 15) & ~15) + ACT_LUT_BYTES;   // staged output tile + activation table
   return main_loop > c_tile ? main_loop : c_tile;
 }
@@ -190,13 +192,14 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs& g, int block_x) {
   constexpr int NT = 64 * WAVES_M * WAVES_N, NW = NT / 64;
   constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N;
   constexpr int TM = WTM / 32, TN = WTN / 32;
-  constexpr int SA = BM / 128, SB = (BN + 127) / 128, SPS = SA + SB;
-  constexpr int IPS = 16 / NW;  // transfers per wavefront per slot
+  constexpr int SR = ring_slot_rows<BM>(), RING_SLOT_BYTES = ring_slot_bytes<BM>();
+  constexpr int SA = BM / SR, SB = (BN + SR - 1) / SR, SPS = SA + SB;
+  constexpr int IPS = SR / 8 / NW;  // transfers per wavefront per slot
   // BN = 64 (the per-head products) fills a whole B slot too: its upper 64 rows hold clamped duplicates no
   // fragment reads, which keeps the transfer count per slot uniform for the vmcnt bookkeeping.
-  static_assert(BM % 128 == 0 && (BN % 128 == 0 || BN == 64), "block tile is a whole number of slots (or a 64-row B tile)");
-  static_assert(WTM % 32 == 0 && WTN % 32 == 0 && 128 % WTM == 0 && 128 % WTN == 0, "a wave tile lies inside one slot");
-  static_assert(16 % NW == 0, "slots are dealt evenly to the wavefronts");
+  static_assert(BM % SR == 0 && (BN % SR == 0 || BN == 64), "block tile is a whole number of slots (or a 64-row B tile)");
+  static_assert(WTM % 32 == 0 && WTN % 32 == 0 && SR % WTM == 0 && SR % WTN == 0, "a wave tile lies inside one slot");
+  static_assert(SR / 8 % NW == 0, "slots are dealt evenly to the wavefronts");
   static_assert(RING >= 2 * SPS, "the ring must hold the stage being read and the next one");
   static_assert((RING - SPS) * IPS < 64, "vmcnt range");
   extern __shared__ __align__(16) uint8_t lds_raw[];
@@ -249,12 +252,13 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs& g, int block_x) {
     if constexpr (decltype(kc_tag)::value) {
       const int r = 8 * ii + (lane >> 3);
       const int c = min((lane & 7) ^ lds_swz(r), kmax >> 3);
-      const int row = min(row0 + 128 * j + r, rows_total - 1) - row0;      // from the tile's first row (see a_base)
+      const int row = min(row0 + SR * j + r, rows_total - 1) - row0;      // from the tile's first row (see a_base)
       return static_cast<uint32_t>(static_cast<int64_t>(row) * ld_b + c * 16);
     } else {
-      const int k = min(4 * ii + (lane >> 4), kmax);
-      const int c = (lane & 15) ^ (4 * ((lane >> 4) & 3));
-      const int row = min(row0 + 128 * j + 8 * c, (rows_total - 1) & ~7);   // last (possibly partial) aligned group of 8 rows
+      constexpr int CPK = SR / 8;                          // 16-byte chunks of a k-row
+      const int k = min((64 / CPK) * ii + lane / CPK, kmax);
+      const int c = (lane % CPK) ^ ((CPK / 4) * ((lane / CPK) & 3));
+      const int row = min(row0 + SR * j + 8 * c, (rows_total - 1) & ~7);   // last (possibly partial) aligned group of 8 rows
       return static_cast<uint32_t>(static_cast<int64_t>(k) * ld_b + row * 2);
     }
   };
@@ -292,7 +296,7 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs& g, int block_x) {
   };
 
   // per-lane LDS offsets of the MFMA fragments inside a slot
-  const int ja = wm0 / 128, jb = wn0 / 128;
+  const int ja = wm0 / SR, jb = wn0 / SR;
   uint32_t fa[TM][A_KC ? 4 : 1], fb[TN][B_KC ? 4 : 1];
   auto frag_offsets = [&](auto kc_tag, int r0, int i, int kk) -> uint32_t {
     if constexpr (decltype(kc_tag)::value) {
@@ -301,18 +305,18 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs& g, int block_x) {
     } else {
       const int kq = 8 * (lane >> 5) + ((lane >> 2) & 3);
       const int c = r0 / 8 + 4 * i + 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1);
-      const int cp = c ^ (4 * ((lane >> 2) & 3));
-      return static_cast<uint32_t>(kq * 256 + cp * 16 + (lane & 1) * 8);
+      const int cp = c ^ ((SR / 32) * ((lane >> 2) & 3));
+      return static_cast<uint32_t>(kq * (2 * SR) + cp * 16 + (lane & 1) * 8);
     }
   };
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int kk = 0; kk < (A_KC ? 4 : 1); ++kk) fa[i][kk] = frag_offsets(std::integral_constant<bool, A_KC>{}, wm0 % 128, i, kk);
+    for (int kk = 0; kk < (A_KC ? 4 : 1); ++kk) fa[i][kk] = frag_offsets(std::integral_constant<bool, A_KC>{}, wm0 % SR, i, kk);
 #pragma unroll
   for (int j = 0; j < TN; ++j)
 #pragma unroll
-    for (int kk = 0; kk < (B_KC ? 4 : 1); ++kk) fb[j][kk] = frag_offsets(std::integral_constant<bool, B_KC>{}, wn0 % 128, j, kk);
+    for (int kk = 0; kk < (B_KC ? 4 : 1); ++kk) fb[j][kk] = frag_offsets(std::integral_constant<bool, B_KC>{}, wn0 % SR, j, kk);
 
   acc16_t acc[TM][TN];
   auto clear = [&]() {
@@ -351,7 +355,7 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs& g, int block_x) {
           else if (left < 8) *p = keep_first(*p, left);
         }
       } else {
-        for (int o = k_last * 16 + tid; o < RING_SLOT_BYTES / 16; o += NT) reinterpret_cast<uint4*>(slot)[o] = make_uint4(0, 0, 0, 0);
+        for (int o = k_last * (SR / 8) + tid; o < RING_SLOT_BYTES / 16; o += NT) reinterpret_cast<uint4*>(slot)[o] = make_uint4(0, 0, 0, 0);
       }
     });
     ring_barrier();
@@ -369,9 +373,9 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs& g, int block_x) {
       if constexpr (A_KC) {
         fm_[i] = *reinterpret_cast<const uint4*>(sa + fa[i][kk]);
       } else {
-        const uint8_t* p = sa + fa[i][0] + kk * 16 * 256;
+        const uint8_t* p = sa + fa[i][0] + kk * 16 * 2 * SR;
         const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)(p));
-        const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)(p + 4 * 256));
+        const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)(p + 4 * 2 * SR));
         union { short4_t s[2]; uint4 u; } cv;
         cv.s[0] = lo;
         cv.s[1] = hi;
@@ -383,9 +387,9 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs& g, int block_x) {
       if constexpr (B_KC) {
         fn_[j] = *reinterpret_cast<const uint4*>(sb + fb[j][kk]);
       } else {
-        const uint8_t* p = sb + fb[j][0] + kk * 16 * 256;
+        const uint8_t* p = sb + fb[j][0] + kk * 16 * 2 * SR;
         const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)(p));
-        const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)(p + 4 * 256));
+        const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)(p + 4 * 2 * SR));
         union { short4_t s[2]; uint4 u; } cv;
         cv.s[0] = lo;
         cv.s[1] = hi;

@@ -48,7 +48,7 @@ BwdPlan plan_bwd(int num_layers, const int64_t* out_features, int64_t batch, int
                                                                           static_cast<int>(batch), 1));
   }
   p.dh_bytes = align_up(static_cast<size_t>(batch) * max_hidden * esz);
-  const size_t parts = static_cast<size_t>(std::max<int64_t>(colsum_parts(static_cast<int>(batch)), (batch + 127) / 128));
+  const size_t parts = static_cast<size_t>(std::max<int64_t>(colsum_parts(static_cast<int>(batch)), (batch + 63) / 64));    // row tiles of 64 at most
   p.colsum_bytes = align_up(parts * max_out * sizeof(float));
   p.splitk_bytes = align_up(p.splitk_bytes);
   return p;
@@ -195,7 +195,9 @@ extern "C" int nmtg_mlp_bwd(int num_layers, const void* x, const void* const* we
     // bias gradient (its partial rows: written by the data-gradient GEMM of the layer above, or by a kernel of its own)
     float* colsum_ws = colsum_region(i);
     if (grad_biases && grad_biases[i]) {
-      if (!tail.full()) {
+      if (!bias_from_parts && tail_add_colsum_whole(tail, dtype, g_cur, out_i, static_cast<int>(batch), static_cast<int>(out_i), grad_biases[i])) {
+        rc = 0;
+      } else if (!tail.full()) {
         int parts = parts_rows;
         rc = 0;
         if (!bias_from_parts) {

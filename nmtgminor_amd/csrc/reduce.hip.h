@@ -64,7 +64,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
 // Block = 32 column lanes (8 columns each = one 16-byte load for 16-bit T) x 8 row lanes.
 template <typename T, bool VEC>
 __device__ __forceinline__ void colsum_partial_block(int bx, int by, const T* __restrict__ X, int64_t ld, int M, int N,
-                                                     int rows_per_block, float* __restrict__ part, float* red_lds) {
+                                                     int rows_per_block, float* __restrict__ part, float* red_lds, T* __restrict__ direct = nullptr) {
   constexpr int CPT = VEC ? 8 : 1;
   float (*red)[32 * CPT + 1] = reinterpret_cast<float (*)[32 * CPT + 1]>(red_lds);   // [8][32 * CPT + 1] floats of LDS
   const int cl = threadIdx.x & 31, rl = threadIdx.x >> 5;
@@ -124,7 +124,8 @@ __device__ __forceinline__ void colsum_partial_block(int bx, int by, const T* __
       float t = 0.f;
 #pragma unroll
       for (int k = 0; k < 8; ++k) t += red[k][c];
-      part[static_cast<int64_t>(by) * N + col] = t;
+      if (direct != nullptr) direct[col] = elem<T>::from_float(t);
+      else part[static_cast<int64_t>(by) * N + col] = t;
     }
   }
   __syncthreads();   // a caller that runs several of these blocks one after the other reuses `red`
@@ -174,15 +175,17 @@ __global__ __launch_bounds__(256) void colsum_final_kernel(const float* __restri
 // four launches of a few microseconds each. A block finds its job from the block ranges (uniform per block) and
 // then does exactly what the stand-alone kernel's block would have done: results are bit-identical.
 // ---------------------------------------------------------------------------------------------
-enum GemmTile { TILE_L = 0, TILE_M = 1, TILE_S = 2, TILE_R = 3 };
+enum GemmTile { TILE_L = 0, TILE_M = 1, TILE_S = 2, TILE_R = 3, TILE_X = 4 };
 
 template <int TILE> struct tile_cfg;
 template <> struct tile_cfg<TILE_L> { static constexpr int BM = 256, BN = 256, WM = 2, WN = 4; };
 template <> struct tile_cfg<TILE_M> { static constexpr int BM = 128, BN = 128, WM = 2, WN = 2; };
 template <> struct tile_cfg<TILE_S> { static constexpr int BM = 256, BN = 64, WM = 4, WN = 1; };
+template <> struct tile_cfg<TILE_X> { static constexpr int BM = 64, BN = 64, WM = 2, WN = 2; };
 template <> struct tile_cfg<TILE_R> { static constexpr int BM = 128, BN = 512, WM = 4, WN = 2; };
 
-enum TailKind { TAIL_SPLITK_M = 1, TAIL_SPLITK_L = 2, TAIL_COLSUM = 3, TAIL_COLSUM_PARTIAL = 4, TAIL_COLSUM_PARTIAL_VEC = 5 };
+enum TailKind { TAIL_SPLITK_M = 1, TAIL_SPLITK_L = 2, TAIL_COLSUM = 3, TAIL_COLSUM_PARTIAL = 4, TAIL_COLSUM_PARTIAL_VEC = 5,
+                TAIL_COLSUM_WHOLE_VEC = 6 };
 struct TailJob {
   int kind;
   int first_block;       // the job's blocks are [first_block, next job's first_block)
@@ -218,6 +221,9 @@ __device__ __forceinline__ void tail_block(const TailArgs& a, int vb, float* lds
     } else {
       colsum_partial_block<T, false>(bx, by, static_cast<const T*>(t.x), t.ldc, t.M, t.N, t.rows_per_block, static_cast<float*>(t.dst), lds);
     }
+  } else if (t.kind == TAIL_COLSUM_WHOLE_VEC) {
+    if constexpr (sizeof(T) == 2)
+      colsum_partial_block<T, true>(vb - t.first_block, 0, static_cast<const T*>(t.x), t.ldc, t.M, t.N, t.M, nullptr, lds, static_cast<T*>(t.dst));
   } else if (t.kind == TAIL_SPLITK_M) {
     using C = tile_cfg<TILE_M>;
     splitk_reduce_slot<T, C::BM, C::BN, C::WM, C::WN>(local, t.src, static_cast<T*>(t.dst), t.ldc, t.M, t.N, t.m_tiles, t.n_tiles,
@@ -258,6 +264,8 @@ int tail_add_splitk(ReduceTail& t, int tile, const float* ws, void* C, int64_t l
 int tail_add_colsum(ReduceTail& t, const float* part, int parts, int N, void* out);
 // the partial phase of a column sum as a job (what colsum_partial_run launches on its own)
 int tail_add_colsum_partial(ReduceTail& t, int dtype, const void* X, int64_t ld, int M, int N, float* part);
+// the whole column sum as one job, for few rows: false if it is not one (the partial and the final phase are queued then)
+bool tail_add_colsum_whole(ReduceTail& t, int dtype, const void* X, int64_t ld, int M, int N, void* out);
 int tail_launch(const ReduceTail& t, int dtype, hipStream_t st);
 // the partial phase of colsum_run alone (its final sum is then queued with tail_add_colsum)
 int colsum_partial_run(int dtype, const void* X, int64_t ld, int M, int N, float* part, hipStream_t st);
