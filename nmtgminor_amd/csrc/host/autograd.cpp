@@ -133,13 +133,13 @@ struct PackedNode : Function<PackedNode> {
     Launch on(qkv);
     Tensor dout = g[0].stride(-1) == 1 ? g[0] : g[0].contiguous();
     Tensor dqkv = empty_like_sized(qkv, qkv.sizes());
-    Tensor sd = empty_as(qkv, {b, h, max_len}, at::kFloat);
+    const Scratch sd(qkv, b * h * max_len * static_cast<int64_t>(sizeof(float)));
     const int64_t st = qkv.stride(0), sh = qkv.stride(2), slot = qkv.stride(1) * 2;
     const int64_t gt = dqkv.stride(0), gh = dqkv.stride(2), gslot = dqkv.stride(1) * 2;
     const char* q = static_cast<const char*>(qkv.data_ptr());
     char* dq = static_cast<char*>(dqkv.data_ptr());
     check(api.flash_attn_bwd(ptr(dout), q, q + slot, q + 2 * slot, ptr(out), lse.data_ptr<float>(), dq, dq + gslot, dq + 2 * gslot,
-                             sd.data_ptr<float>(), cu.data_ptr<int32_t>(), cu.data_ptr<int32_t>(), b, h, d, max_len, max_len, dout.stride(0),
+                             sd.get<float>(), cu.data_ptr<int32_t>(), cu.data_ptr<int32_t>(), b, h, d, max_len, max_len, dout.stride(0),
                              dout.stride(1), st, sh, st, sh, st, sh, h * d, d, gt, gh, gt, gh, gt, gh,
                              static_cast<float>(ctx->saved_data["s"].toDouble()), ctx->saved_data["c"].toBool() ? 1 : 0,
                              words.defined() ? 2 : 0, static_cast<float>(ctx->saved_data["p"].toDouble()), nullptr, ptr(words),

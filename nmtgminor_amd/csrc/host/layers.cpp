@@ -88,12 +88,12 @@ struct EncoderNode : Function<EncoderNode> {
     AddNormGrads n2 = ln_bwd_add(m.dx, h, stats2, g2, g, guard, keep, pr);
     const Tensor& dy = keep.defined() ? n2.dy : n2.dx;
     LinearGrads o = linear_bwd(dy, cx, wo, true, need(5), need(6));
-    Tensor dlin = at::empty_like(lin);
+    Tensor dlin = new_like(lin);
     const int64_t t = x.size(0), b = x.size(1), d = x.size(2) / heads;
     Bits bits{ctx->saved_data["mode"].toInt(), static_cast<uint64_t>(ctx->saved_data["seed"].toInt()),
               static_cast<uint64_t>(ctx->saved_data["offset"].toInt()), words};
-    flash_bwd_batched(o.dx.view({t, b, heads, d}), slot(lin, heads, 3, 0), slot(lin, heads, 3, 1), slot(lin, heads, 3, 2), cx, lse,
-                      slot(dlin, heads, 3, 0), slot(dlin, heads, 3, 1), slot(dlin, heads, 3, 2), pad, Tensor(), pa,
+    flash_bwd_batched({t, t, b, heads, d}, o.dx, slot_view(lin, heads, 3, 0), slot_view(lin, heads, 3, 1), slot_view(lin, heads, 3, 2), cx, lse,
+                      slot_view(dlin, heads, 3, 0), slot_view(dlin, heads, 3, 1), slot_view(dlin, heads, 3, 2), pad, Tensor(), pa,
                       1.0 / std::sqrt(static_cast<double>(d)), false, bits);
     LinearGrads i = linear_bwd(dlin, z1, wi, true, need(3), need(4));
     AddNormGrads n1 = ln_bwd_add(i.dx, x, stats1, g1, n2.dx, Tensor(), Tensor(), 0.0);
@@ -119,15 +119,15 @@ Cross cross_fwd(const Tensor& xq, const Tensor& xkv, const Tensor& wq, const Ten
   const int64_t tq = xq.size(0), tk = xkv.size(0), b = xq.size(1), e = xq.size(2), d = e / heads;
   Launch on(xq);
   Cross r;
-  r.q_lin = at::empty_like(xq);
+  r.q_lin = new_like(xq);
   r.kv_lin = empty_like_sized(xkv, {tk, b, 2 * e});
-  r.ctx = at::empty_like(xq);
-  r.out = at::empty_like(xq);
+  r.ctx = new_like(xq);
+  r.out = new_like(xq);
   r.dropped = empty_like_sized(xq, {b * heads, tq, tk});
   // an inference call writes the probabilities only where one kernel makes them and the context (nmtg_encdec_attn_fwd)
   const bool probs_only = !grad && p == 0.0 && tk % 4 == 0 && (d == 64 || d == 128);
-  Tensor scores;
-  if (!probs_only) scores = empty_like_sized(xq, {b * heads, tq, tk});
+  Scratch scores;
+  if (!probs_only) scores = Scratch(xq, b * heads * tq * tk * static_cast<int64_t>(xq.element_size()));
   uint64_t seed = 0, offset = 0;
   if (grad) r.softmax = empty_like_sized(xq, {b * heads, tq, tk});
   if (p > 0.0) {
@@ -135,7 +135,7 @@ Cross cross_fwd(const Tensor& xq, const Tensor& xkv, const Tensor& wq, const Ten
     std::tie(seed, offset) = draw(xq, r.mask.numel());
   }
   check(api.encdec_attn_fwd(ptr(xq), ptr(xkv), ptr(wq), ptr(wkv), ptr(wo), nullptr, nullptr, nullptr, static_cast<const uint8_t*>(ptr(pad)),
-                            ptr(r.q_lin), ptr(r.kv_lin), ptr(scores), ptr(r.softmax), ptr(r.dropped), static_cast<uint8_t*>(ptr(r.mask)),
+                            ptr(r.q_lin), ptr(r.kv_lin), scores.get(), ptr(r.softmax), ptr(r.dropped), static_cast<uint8_t*>(ptr(r.mask)),
                             p > 0.0 ? 2 : 0, static_cast<float>(p), seed, offset, ptr(r.ctx), ptr(r.out), tq, tk, b, e,
                             static_cast<int>(heads), dtype_code(xq), on.stream), "nmtg_encdec_attn_fwd");
   if (!grad) r.softmax = r.dropped;
@@ -147,11 +147,11 @@ CrossGrads cross_bwd(const Tensor& dy, const Cross& c, const Tensor& xq, const T
                      int64_t heads, double p) {
   const int64_t tq = xq.size(0), tk = xkv.size(0), b = xq.size(1), e = xq.size(2);
   Launch on(xq);
-  CrossGrads r{at::empty_like(xq), at::empty_like(xkv), at::empty_like(wq), at::empty_like(wkv), at::empty_like(wo)};
-  Tensor ws = empty_as(xq, {std::max<int64_t>(api.encdec_attn_bwd_workspace_bytes(tq, tk, b, e, static_cast<int>(heads)), 256)}, at::kByte);
+  CrossGrads r{new_like(xq), new_like(xkv), new_like(wq), new_like(wkv), new_like(wo)};
+  const Scratch ws(xq, std::max<int64_t>(api.encdec_attn_bwd_workspace_bytes(tq, tk, b, e, static_cast<int>(heads)), 256));
   check(api.encdec_attn_bwd_from_probs(ptr(dy), ptr(c.ctx), ptr(c.dropped), ptr(c.softmax), ptr(c.q_lin), ptr(c.kv_lin), ptr(xq), ptr(xkv), ptr(wq),
                                        ptr(wkv), ptr(wo), static_cast<const uint8_t*>(ptr(c.mask)), static_cast<float>(p), ptr(r.dxq), ptr(r.dxkv),
-                                       ptr(r.dwq), ptr(r.dwkv), ptr(r.dwo), nullptr, nullptr, ptr(ws), ws.numel(), tq, tk, b, e,
+                                       ptr(r.dwq), ptr(r.dwkv), ptr(r.dwo), nullptr, nullptr, ws.get(), ws.bytes, tq, tk, b, e,
                                        static_cast<int>(heads), dtype_code(xq), on.stream), "nmtg_encdec_attn_bwd_from_probs");
   return r;
 }
@@ -215,12 +215,12 @@ struct DecoderNode : Function<DecoderNode> {
     CrossGrads r = cross_bwd(keep2.defined() ? n3.dy : n3.dx, c, z2, context, wq, wkv, wc, heads, pc);
     AddNormGrads n2 = ln_bwd_add(r.dxq, h1, stats2, g2, n3.dx, Tensor(), keep1, pr);
     LinearGrads o = linear_bwd(keep1.defined() ? n2.dy : n2.dx, cx, wo, true, need(6), need(7));
-    Tensor dlin = at::empty_like(lin);
+    Tensor dlin = new_like(lin);
     const int64_t t = x.size(0), b = x.size(1), d = x.size(2) / heads;
     Bits bits{ctx->saved_data["mode"].toInt(), static_cast<uint64_t>(ctx->saved_data["seed"].toInt()),
               static_cast<uint64_t>(ctx->saved_data["offset"].toInt()), words};
-    flash_bwd_batched(o.dx.view({t, b, heads, d}), slot(lin, heads, 3, 0), slot(lin, heads, 3, 1), slot(lin, heads, 3, 2), cx, lse,
-                      slot(dlin, heads, 3, 0), slot(dlin, heads, 3, 1), slot(dlin, heads, 3, 2), Tensor(), time, pa,
+    flash_bwd_batched({t, t, b, heads, d}, o.dx, slot_view(lin, heads, 3, 0), slot_view(lin, heads, 3, 1), slot_view(lin, heads, 3, 2), cx, lse,
+                      slot_view(dlin, heads, 3, 0), slot_view(dlin, heads, 3, 1), slot_view(dlin, heads, 3, 2), Tensor(), time, pa,
                       1.0 / std::sqrt(static_cast<double>(d)), false, bits);
     LinearGrads i = linear_bwd(dlin, z1, wi, true, need(4), need(5));
     AddNormGrads n1 = ln_bwd_add(i.dx, x, stats1, g1, n2.dx, Tensor(), Tensor(), 0.0);
@@ -238,7 +238,7 @@ std::tuple<Tensor, Tensor> decoder_step(const Tensor& x, const Tensor& kbuf, con
   Launch on(x);
   Norm n1 = ln_fwd(x, w[0], w[1], kEps);
   Tensor lin = linear_step(n1.z, w[2], w[3]);
-  Tensor cx = at::empty_like(x);
+  Tensor cx = new_like(x);
   check(api.attn_decode_append(ptr(lin), 3 * e, ptr(kbuf), kbuf.stride(0), kbuf.stride(1), ptr(vbuf), vbuf.stride(0), vbuf.stride(1), ptr(cx), e, b,
                                heads, d, n, scale, dtype_code(x), on.stream), "nmtg_attn_decode_append");
   AddNorm n2 = add_ln_fwd(linear_step(cx, w[4], w[5]), x, 0.0, Tensor(), w[6], w[7], kEps);

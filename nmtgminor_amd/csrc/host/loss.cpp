@@ -70,9 +70,9 @@ struct GeneratorNode : Function<GeneratorNode> {
     const int dtype = dtype_code(hidden);
     if (need_b) {
       r[2] = empty_like_sized(weight, {v});
-      Tensor part = empty_as(hidden, {api.xentropy_bwd_colsum_parts(n), v}, at::kFloat);
+      const Scratch part(hidden, api.xentropy_bwd_colsum_parts(n) * v * static_cast<int64_t>(sizeof(float)));
       check(api.xentropy_bwd_colsum(g.data_ptr<float>(), one ? 0 : 1, ptr(full), lse.data_ptr<float>(), labels.data_ptr<int64_t>(), ptr(full),
-                                    ptr(r[2]), part.data_ptr<float>(), n, v, pitch, pitch, smoothing, padding_idx, dtype, on.stream),
+                                    ptr(r[2]), part.get<float>(), n, v, pitch, pitch, smoothing, padding_idx, dtype, on.stream),
             "nmtg_xentropy_bwd_colsum");
     } else {
       if (one) g = g.expand({n}).contiguous();
@@ -81,16 +81,16 @@ struct GeneratorNode : Function<GeneratorNode> {
     }
     auto product = [&](int trans_a, int64_t m, int64_t k, const Tensor& b, const Tensor& c) {
       const int64_t bytes = api.gemm_workspace_bytes(m, e, k, 1);
-      Tensor ws = bytes > 0 ? empty_as(hidden, {bytes}, at::kByte) : Tensor();
-      check(api.gemm(trans_a, 0, m, e, k, 1.f, ptr(full), pitch, 0, ptr(b), e, 0, ptr(c), e, 0, 1, nullptr, ptr(ws), bytes, dtype, on.stream),
+      const Scratch ws(hidden, bytes);
+      check(api.gemm(trans_a, 0, m, e, k, 1.f, ptr(full), pitch, 0, ptr(b), e, 0, ptr(c), e, 0, 1, nullptr, ws.get(), bytes, dtype, on.stream),
             "nmtg_gemm");
     };
     if (ctx->needs_input_grad(1)) {
-      r[1] = at::empty_like(weight);
+      r[1] = new_like(weight);
       product(1, v, n, hidden, r[1]);                              // [V, N] x [N, E]
     }
     if (ctx->needs_input_grad(0)) {
-      r[0] = at::empty_like(hidden);
+      r[0] = new_like(hidden);
       product(0, n, v, weight, r[0]);                              // [N, V] x [V, E], the classes split over the chip
     }
     return r;

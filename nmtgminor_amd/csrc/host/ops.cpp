@@ -42,7 +42,7 @@ std::pair<uint64_t, uint64_t> draw(const Tensor& like, int64_t count) {
 Norm ln_fwd(const Tensor& x, const Tensor& gamma, const Tensor& beta, double eps) {
   const int64_t h = gamma.numel(), rows = h ? x.numel() / h : 0;
   Launch on(x);
-  Norm r{at::empty_like(x, x.options().dtype(gamma.scalar_type())), empty_as(x, {2, rows}, at::kFloat)};
+  Norm r{x.is_contiguous() ? empty_as(x, x.sizes(), gamma.scalar_type()) : at::empty_like(x, x.options().dtype(gamma.scalar_type())), empty_as(x, {2, rows}, at::kFloat)};
   float* mu = r.stats.data_ptr<float>();
   check(api.ln_fwd(ptr(x), ptr(gamma), ptr(beta), ptr(r.z), mu, mu + rows, rows, h, static_cast<float>(eps), dtype_code(x),
                    dtype_code(gamma), on.stream), "nmtg_ln_fwd");
@@ -52,10 +52,10 @@ Norm ln_fwd(const Tensor& x, const Tensor& gamma, const Tensor& beta, double eps
 NormGrads ln_bwd(const Tensor& dz, const Tensor& x_or_z, const Tensor& stats, const Tensor& gamma, const Tensor& beta, bool memory_efficient) {
   const int64_t h = gamma.numel(), rows = stats.size(1);
   Launch on(dz);
-  NormGrads r{at::empty_like(x_or_z), at::empty_like(gamma), at::empty_like(gamma)};
+  NormGrads r{new_like(x_or_z), new_like(gamma), new_like(gamma)};
   const int64_t parts = api.ln_bwd_parts(rows, h);
-  Tensor part = empty_as(dz, {2, parts, h}, at::kFloat);
-  float* pp = part.data_ptr<float>();
+  const Scratch part(dz, 2 * parts * h * static_cast<int64_t>(sizeof(float)));
+  float* pp = part.get<float>();
   const float* mu = stats.data_ptr<float>();
   check(api.ln_bwd(ptr(dz), ptr(x_or_z), mu, mu + rows, ptr(gamma), memory_efficient ? ptr(beta) : nullptr, ptr(r.dx), ptr(r.dgamma),
                    ptr(r.dbeta), pp, pp + parts * h, parts, rows, h, memory_efficient ? 1 : 0, dtype_code(x_or_z), dtype_code(gamma),
@@ -66,7 +66,7 @@ NormGrads ln_bwd(const Tensor& dz, const Tensor& x_or_z, const Tensor& stats, co
 AddNorm add_ln_fwd(const Tensor& x, const Tensor& residual, double p, const Tensor& clear, const Tensor& gamma, const Tensor& beta, double eps) {
   const int64_t h = gamma.numel(), rows = x.numel() / h;
   Launch on(x);
-  AddNorm r{at::empty_like(x), at::empty_like(x), empty_as(x, {2, rows}, at::kFloat), Tensor()};
+  AddNorm r{new_like(x), new_like(x), empty_as(x, {2, rows}, at::kFloat), Tensor()};
   uint64_t seed = 0, offset = 0;
   if (p > 0.0) {
     r.mask = empty_as(x, x.sizes(), at::kByte);
@@ -83,11 +83,11 @@ AddNormGrads ln_bwd_add(const Tensor& dz, const Tensor& x, const Tensor& stats, 
                         const Tensor& guard, const Tensor& keep, double p) {
   const int64_t h = gamma.numel(), rows = stats.size(1);
   Launch on(dz);
-  AddNormGrads r{at::empty_like(x), Tensor(), at::empty_like(gamma), at::empty_like(gamma)};
-  if (keep.defined()) r.dy = at::empty_like(x);
+  AddNormGrads r{new_like(x), Tensor(), new_like(gamma), new_like(gamma)};
+  if (keep.defined()) r.dy = new_like(x);
   const int64_t parts = api.ln_bwd_parts(rows, h);
-  Tensor part = empty_as(dz, {2, parts, h}, at::kFloat);
-  float* pp = part.data_ptr<float>();
+  const Scratch part(dz, 2 * parts * h * static_cast<int64_t>(sizeof(float)));
+  float* pp = part.get<float>();
   const float* mu = stats.data_ptr<float>();
   check(api.ln_bwd_add(ptr(dz), ptr(x), mu, mu + rows, ptr(gamma), ptr(grad_residual), static_cast<const uint8_t*>(ptr(guard)),
                        static_cast<const uint8_t*>(ptr(keep)), static_cast<float>(p), ptr(r.dx), ptr(r.dy), ptr(r.dgamma), ptr(r.dbeta), pp,
@@ -119,9 +119,8 @@ Tensor linear_step(const Tensor& x, const Tensor& w, const Tensor& b) {
   return y;
 }
 
-static Tensor mlp_workspace(const Tensor& x, int layers, const int64_t* outs, int64_t rows, int64_t in) {
-  const int64_t bytes = api.mlp_bwd_dtype_workspace_bytes(layers, outs, rows, in, dtype_code(x));
-  return empty_as(x, {std::max<int64_t>(bytes, 256)}, at::kByte);
+static Scratch mlp_workspace(const Tensor& x, int layers, const int64_t* outs, int64_t rows, int64_t in) {
+  return Scratch(x, std::max<int64_t>(api.mlp_bwd_dtype_workspace_bytes(layers, outs, rows, in, dtype_code(x)), 256));
 }
 
 LinearGrads linear_bwd(const Tensor& dy, const Tensor& x, const Tensor& w, bool want_x, bool want_w, bool want_b) {
@@ -129,14 +128,14 @@ LinearGrads linear_bwd(const Tensor& dy, const Tensor& x, const Tensor& w, bool 
   Launch on(dy);
   LinearGrads r;
   if (want_x) { auto sizes = dy.sizes().vec(); sizes.back() = in; r.dx = empty_like_sized(dy, sizes); }
-  if (want_w) r.dw = at::empty_like(w);
+  if (want_w) r.dw = new_like(w);
   if (want_b) r.db = empty_like_sized(dy, {out});
-  Tensor ws = mlp_workspace(dy, 1, &out, rows, in);
+  const Scratch ws = mlp_workspace(dy, 1, &out, rows, in);
   const void* weights[1] = {ptr(w)};
   void* dws[1] = {ptr(r.dw)};
   void* dbs[1] = {ptr(r.db)};
-  check(api.mlp_bwd(1, ptr(x), weights, &out, rows, in, ptr(dy), nullptr, nullptr, nullptr, 0.f, NMTG_ACT_NONE, ptr(r.dx), dws, dbs, ptr(ws),
-                    ws.numel(), dtype_code(dy), on.stream), "nmtg_mlp_bwd");
+  check(api.mlp_bwd(1, ptr(x), weights, &out, rows, in, ptr(dy), nullptr, nullptr, nullptr, 0.f, NMTG_ACT_NONE, ptr(r.dx), dws, dbs, ws.get(),
+                    ws.bytes, dtype_code(dy), on.stream), "nmtg_mlp_bwd");
   return r;
 }
 
@@ -177,20 +176,20 @@ MlpGrads mlp_bwd(const Tensor& dy, const Tensor& x, const Tensor& w1, const Tens
   const int64_t in = w1.size(1), rows = x.numel() / in, outs[2] = {w1.size(0), w2.size(0)};
   Launch on(dy);
   MlpGrads r;
-  if (want_x) r.dx = at::empty_like(x);
-  if (want_w) { r.dw1 = at::empty_like(w1); r.dw2 = at::empty_like(w2); }
+  if (want_x) r.dx = new_like(x);
+  if (want_w) { r.dw1 = new_like(w1); r.dw2 = new_like(w2); }
   if (want_b1) r.db1 = empty_like_sized(x, {outs[0]});
   if (want_b2) r.db2 = empty_like_sized(x, {outs[1]});
   if (rows == 0) {                                  // an empty batch contributes zero gradients
     for (Tensor* t : {&r.dw1, &r.dw2, &r.db1, &r.db2}) if (t->defined()) t->zero_();
     return r;
   }
-  Tensor ws = mlp_workspace(x, 2, outs, rows, in);
+  const Scratch ws = mlp_workspace(x, 2, outs, rows, in);
   const void* weights[2] = {ptr(w1), ptr(w2)};
   void* dws[2] = {ptr(r.dw1), ptr(r.dw2)};
   void* dbs[2] = {ptr(r.db1), ptr(r.db2)};
   check(api.mlp_bwd(2, ptr(x), weights, outs, rows, in, ptr(dy), ptr(post), ptr(pre), p > 0.0 ? static_cast<const uint8_t*>(ptr(mask)) : nullptr,
-                    static_cast<float>(p), static_cast<int>(act), ptr(r.dx), dws, dbs, ptr(ws), ws.numel(), dtype_code(x), on.stream),
+                    static_cast<float>(p), static_cast<int>(act), ptr(r.dx), dws, dbs, ws.get(), ws.bytes, dtype_code(x), on.stream),
         "nmtg_mlp_bwd");
   return r;
 }
@@ -213,7 +212,7 @@ Tensor dropout_add_(const Tensor& x, const Tensor& residual, double p, bool trai
 
 Tensor dropout_bwd(const Tensor& g, const Tensor& mask, double p) {
   Launch on(g);
-  Tensor dx = at::empty_like(g);
+  Tensor dx = new_like(g);
   check(api.dropout_add_bwd(ptr(g), static_cast<const uint8_t*>(mask.data_ptr()), ptr(dx), g.numel(), static_cast<float>(p), dtype_code(g),
                             on.stream), "nmtg_dropout_add_bwd");
   return dx;
@@ -232,7 +231,7 @@ Tensor dropout_add_guard_(const Tensor& x, const Tensor& residual, double p, con
 
 Tensor dropout_guard_bwd(const Tensor& g, const Tensor& mask, double p) {
   Launch on(g);
-  Tensor dx = at::empty_like(g);
+  Tensor dx = new_like(g);
   check(api.dropout_add_guard_bwd(ptr(g), static_cast<const uint8_t*>(mask.data_ptr()), ptr(dx), g.numel(), static_cast<float>(p),
                                   dtype_code(g), on.stream), "nmtg_dropout_add_guard_bwd");
   return dx;
@@ -242,7 +241,7 @@ Tensor dropout_guard_bwd(const Tensor& g, const Tensor& mask, double p) {
 static Tensor bits_words(const Tensor& like, int64_t b, int64_t h, int64_t tq, int64_t tk) {
   return empty_as(like, {std::max<int64_t>(api.flash_attn_dropout_bits_bytes(b, h, tq, tk), 16) / 4}, at::kInt);
 }
-static Tensor info_words(const Tensor& like, int64_t bytes) { return empty_as(like, {std::max<int64_t>(bytes, 4) / 4}, at::kInt); }
+static Scratch info_words(const Tensor& like, int64_t bytes) { return Scratch(like, std::max<int64_t>(bytes, 4)); }
 
 Tensor slot(const Tensor& lin, int64_t heads, int64_t parts, int64_t which) {
   const int64_t d = lin.size(2) / (heads * parts);
@@ -277,7 +276,7 @@ Flash flash_fwd_batched(const Tensor& q, const Tensor& k, const Tensor& v, const
   Flash r;
   r.out = empty_like_sized(q, {tq, b, h, d});
   r.lse = empty_as(q, {b, h, tq}, at::kFloat);
-  Tensor kinfo, tinfo;
+  Scratch kinfo, tinfo;
   if (pad.defined()) kinfo = info_words(q, api.flash_attn_key_info_bytes(b, tk));
   if (time_mask.defined()) tinfo = info_words(q, api.flash_attn_time_info_bytes(tq, tk));
   if (p > 0.0) {
@@ -288,16 +287,16 @@ Flash flash_fwd_batched(const Tensor& q, const Tensor& k, const Tensor& v, const
   if (coverage != Coverage::none) {
     r.probs = empty_like_sized(q, {b * h, tq, tk});
     check(api.flash_attn_batched_fwd_probs(
-              ptr(q), ptr(k), ptr(v), ptr(r.out), static_cast<const uint8_t*>(ptr(pad)), ptr(kinfo), static_cast<const uint8_t*>(ptr(time_mask)),
-              ptr(tinfo), r.lse.data_ptr<float>(), b, h, d, tq, tk, q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1),
+              ptr(q), ptr(k), ptr(v), ptr(r.out), static_cast<const uint8_t*>(ptr(pad)), kinfo.get(), static_cast<const uint8_t*>(ptr(time_mask)),
+              tinfo.get(), r.lse.data_ptr<float>(), b, h, d, tq, tk, q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1),
               k.stride(2), v.stride(0), v.stride(1), v.stride(2), r.out.stride(0), r.out.stride(1), r.out.stride(2), static_cast<float>(scale),
               causal ? 1 : 0, static_cast<int>(r.bits.mode), static_cast<float>(p), nullptr, nullptr, ptr(r.bits.words), r.bits.seed,
               r.bits.offset, dtype_code(q), on.stream, ptr(r.probs), coverage == Coverage::dropped ? 1 : 0),
           "nmtg_flash_attn_batched_fwd_probs");
     return r;
   }
-  check(api.flash_attn_batched_fwd(ptr(q), ptr(k), ptr(v), ptr(r.out), static_cast<const uint8_t*>(ptr(pad)), ptr(kinfo),
-                                   static_cast<const uint8_t*>(ptr(time_mask)), ptr(tinfo), r.lse.data_ptr<float>(), b, h, d, tq, tk,
+  check(api.flash_attn_batched_fwd(ptr(q), ptr(k), ptr(v), ptr(r.out), static_cast<const uint8_t*>(ptr(pad)), kinfo.get(),
+                                   static_cast<const uint8_t*>(ptr(time_mask)), tinfo.get(), r.lse.data_ptr<float>(), b, h, d, tq, tk,
                                    q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1),
                                    v.stride(2), r.out.stride(0), r.out.stride(1), r.out.stride(2), static_cast<float>(scale), causal ? 1 : 0,
                                    static_cast<int>(r.bits.mode), static_cast<float>(p), nullptr, nullptr, ptr(r.bits.words), r.bits.seed,
@@ -305,21 +304,26 @@ Flash flash_fwd_batched(const Tensor& q, const Tensor& k, const Tensor& v, const
   return r;
 }
 
-void flash_bwd_batched(const Tensor& dout, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& out, const Tensor& lse,
-                       const Tensor& dq, const Tensor& dk, const Tensor& dv, const Tensor& pad, const Tensor& time_mask, double p,
-                       double scale, bool causal, const Bits& bits) {
-  const int64_t tq = q.size(0), b = q.size(1), h = q.size(2), d = q.size(3), tk = k.size(0);
-  Launch on(q);
-  Tensor kinfo, tinfo, sd = empty_as(q, {b, h, tq}, at::kFloat);
-  if (pad.defined()) kinfo = info_words(q, api.flash_attn_key_info_bytes(b, tk));
-  if (time_mask.defined()) tinfo = info_words(q, api.flash_attn_time_info_bytes(tq, tk));
-  check(api.flash_attn_batched_bwd(ptr(dout), ptr(q), ptr(k), ptr(v), ptr(out), lse.data_ptr<float>(), ptr(dq), ptr(dk), ptr(dv),
-                                   sd.data_ptr<float>(), static_cast<const uint8_t*>(ptr(pad)), ptr(kinfo),
-                                   static_cast<const uint8_t*>(ptr(time_mask)), ptr(tinfo), b, h, d, tq, tk, q.stride(0), q.stride(1),
-                                   q.stride(2), k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2), out.stride(0),
-                                   out.stride(1), out.stride(2), static_cast<float>(scale), causal ? 1 : 0, static_cast<int>(bits.mode),
-                                   static_cast<float>(p), nullptr, ptr(bits.words), bits.words.defined() ? 1 : 0, bits.seed, bits.offset,
-                                   dtype_code(q), on.stream), "nmtg_flash_attn_batched_bwd");
+View head_view(const Tensor& x, int64_t heads) { return {ptr(x), x.stride(0), x.stride(1), x.size(2) / heads}; }
+View slot_view(const Tensor& lin, int64_t heads, int64_t parts, int64_t which) {
+  const int64_t d = lin.size(2) / (heads * parts);
+  return {static_cast<char*>(ptr(lin)) + which * d * static_cast<int64_t>(lin.element_size()), lin.stride(0), lin.stride(1), parts * d};
+}
+
+void flash_bwd_batched(const FlashShape& s, const Tensor& dout, const View& q, const View& k, const View& v, const Tensor& out, const Tensor& lse,
+                       const View& dq, const View& dk, const View& dv, const Tensor& pad, const Tensor& time_mask, double p, double scale,
+                       bool causal, const Bits& bits) {
+  Launch on(out);
+  Scratch kinfo, tinfo, sd(out, s.b * s.h * s.tq * static_cast<int64_t>(sizeof(float)));
+  if (pad.defined()) kinfo = info_words(out, api.flash_attn_key_info_bytes(s.b, s.tk));
+  if (time_mask.defined()) tinfo = info_words(out, api.flash_attn_time_info_bytes(s.tq, s.tk));
+  check(api.flash_attn_batched_bwd(ptr(dout), q.data, k.data, v.data, ptr(out), lse.data_ptr<float>(), dq.data, dk.data, dv.data, sd.get<float>(),
+                                   static_cast<const uint8_t*>(ptr(pad)), kinfo.get(), static_cast<const uint8_t*>(ptr(time_mask)), tinfo.get(),
+                                   s.b, s.h, s.d, s.tq, s.tk, q.stride_t, q.stride_b, q.stride_h, k.stride_t, k.stride_b, k.stride_h, v.stride_t,
+                                   v.stride_b, v.stride_h, out.stride(0), out.stride(1), out.stride(2), static_cast<float>(scale),
+                                   causal ? 1 : 0, static_cast<int>(bits.mode), static_cast<float>(p), nullptr, ptr(bits.words),
+                                   bits.words.defined() ? 1 : 0, bits.seed, bits.offset, dtype_code(out), on.stream),
+        "nmtg_flash_attn_batched_bwd");
 }
 
 }  // namespace nmtg_host

@@ -42,8 +42,8 @@ optional<Tensor> clip_grad_norm(const py::list& params, double max_norm) {
   Launch on(l.first);
   const int n = static_cast<int>(l.size.size()), type = dtype_code(l.first);
   Tensor norm = empty_as(l.first, {}, at::kFloat);
-  Tensor ws = empty_as(l.first, {std::max<int64_t>(api.multi_tensor_l2norm_workspace_bytes(n, l.size.data()), 256)}, at::kByte);
-  check(api.multi_tensor_l2norm(n, l.addr[0].data(), l.size.data(), norm.data_ptr<float>(), nullptr, ptr(ws), ws.numel(), type, on.stream),
+  const Scratch ws(l.first, std::max<int64_t>(api.multi_tensor_l2norm_workspace_bytes(n, l.size.data()), 256));
+  check(api.multi_tensor_l2norm(n, l.addr[0].data(), l.size.data(), norm.data_ptr<float>(), nullptr, ws.get(), ws.bytes, type, on.stream),
         "nmtg_multi_tensor_l2norm");
   if (max_norm > 0.0)
     check(api.multi_tensor_clip(n, l.addr[0].data(), l.size.data(), norm.data_ptr<float>(), static_cast<float>(max_norm), type, on.stream),
