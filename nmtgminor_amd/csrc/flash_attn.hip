@@ -1863,11 +1863,11 @@ static int flash_batched_fwd(const void* q, const void* k, const void* v, void* 
                              int64_t out_stride_h, float softmax_scale, int causal, int dropout_mode, float dropout_p,
                              const uint8_t* dropout_mask, uint8_t* dropout_mask_out, void* dropout_bits,
                              uint64_t seed, uint64_t offset, int dtype, void* stream,
-                             void* probs, int probs_dropped) {
-  const char* what = probs != nullptr ? "flash_attn_batched_fwd_probs" : "flash_attn_batched_fwd";
+                             bool want_probs, void* probs, int probs_dropped) {
+  const char* what = want_probs ? "flash_attn_batched_fwd_probs" : "flash_attn_batched_fwd";
   if (int rc = check_common(what, batch, heads, head_dim, len_q, len_k, dropout_mode, dropout_p, softmax_scale, dtype)) return rc;
-  if (batch == 0 || len_q == 0) return 0;
-  NMTG_REQUIRE(q && k && v && out && softmax_lse, "%s: null pointer argument", what);
+  if (batch == 0 || len_q == 0) return 0;        // nothing to write; tensors without elements have no address
+  NMTG_REQUIRE(q && k && v && out && softmax_lse && (probs || !want_probs), "%s: null pointer argument", what);
   NMTG_REQUIRE(dropout_mode != 1 || dropout_mask, "%s: dropout mode 1 replays a keep-mask and none was given", what);
   NMTG_REQUIRE(batched_view_ok(q, q_stride_t, q_stride_b, q_stride_h, heads, head_dim) &&
                    batched_view_ok(k, k_stride_t, k_stride_b, k_stride_h, heads, head_dim) &&
@@ -1887,7 +1887,7 @@ static int flash_batched_fwd(const void* q, const void* k, const void* v, void* 
   if (int rc = key_info_launch(what, a, batch, key_padding_mask, key_info, st)) return rc;
   if (int rc = time_info_launch(what, a, time_mask, time_info, st)) return rc;
   if (int rc = fwd_run(what, a, batch, head_dim, dropout_mode, dropout_bits, dtype, st)) return rc;
-  if (probs == nullptr) return 0;
+  if (!want_probs) return 0;
   const bool dropped = probs_dropped != 0 && dropout_mode != 0;
   if (dtype == NMTG_F16) {
     if (int rc = head_dim == 64 ? fprobs_launch<f16_t, 64>(a, batch, dropped, probs, st) : fprobs_launch<f16_t, 128>(a, batch, dropped, probs, st)) return rc;
@@ -1906,7 +1906,7 @@ extern "C" int nmtg_flash_attn_batched_fwd(const void* q, const void* k, const v
                                            int64_t out_stride_h, float softmax_scale, int causal, int dropout_mode, float dropout_p,
                                            const uint8_t* dropout_mask, uint8_t* dropout_mask_out, void* dropout_bits,
                                            uint64_t seed, uint64_t offset, int dtype, void* stream) {
-  return flash_batched_fwd(q, k, v, out, key_padding_mask, key_info, time_mask, time_info, softmax_lse, batch, heads, head_dim, len_q, len_k, q_stride_t, q_stride_b, q_stride_h, k_stride_t, k_stride_b, k_stride_h, v_stride_t, v_stride_b, v_stride_h, out_stride_t, out_stride_b, out_stride_h, softmax_scale, causal, dropout_mode, dropout_p, dropout_mask, dropout_mask_out, dropout_bits, seed, offset, dtype, stream, nullptr, 0);
+  return flash_batched_fwd(q, k, v, out, key_padding_mask, key_info, time_mask, time_info, softmax_lse, batch, heads, head_dim, len_q, len_k, q_stride_t, q_stride_b, q_stride_h, k_stride_t, k_stride_b, k_stride_h, v_stride_t, v_stride_b, v_stride_h, out_stride_t, out_stride_b, out_stride_h, softmax_scale, causal, dropout_mode, dropout_p, dropout_mask, dropout_mask_out, dropout_bits, seed, offset, dtype, stream, false, nullptr, 0);
 }
 
 extern "C" int nmtg_flash_attn_batched_fwd_probs(const void* q, const void* k, const void* v, void* out, const uint8_t* key_padding_mask,
@@ -1918,8 +1918,7 @@ extern "C" int nmtg_flash_attn_batched_fwd_probs(const void* q, const void* k, c
                                                  const uint8_t* dropout_mask, uint8_t* dropout_mask_out, void* dropout_bits,
                                                  uint64_t seed, uint64_t offset, int dtype, void* stream,
                                                  void* probs, int probs_dropped) {
-  NMTG_REQUIRE(probs, "flash_attn_batched_fwd_probs: null pointer argument");
-  return flash_batched_fwd(q, k, v, out, key_padding_mask, key_info, time_mask, time_info, softmax_lse, batch, heads, head_dim, len_q, len_k, q_stride_t, q_stride_b, q_stride_h, k_stride_t, k_stride_b, k_stride_h, v_stride_t, v_stride_b, v_stride_h, out_stride_t, out_stride_b, out_stride_h, softmax_scale, causal, dropout_mode, dropout_p, dropout_mask, dropout_mask_out, dropout_bits, seed, offset, dtype, stream, probs, probs_dropped);
+  return flash_batched_fwd(q, k, v, out, key_padding_mask, key_info, time_mask, time_info, softmax_lse, batch, heads, head_dim, len_q, len_k, q_stride_t, q_stride_b, q_stride_h, k_stride_t, k_stride_b, k_stride_h, v_stride_t, v_stride_b, v_stride_h, out_stride_t, out_stride_b, out_stride_h, softmax_scale, causal, dropout_mode, dropout_p, dropout_mask, dropout_mask_out, dropout_bits, seed, offset, dtype, stream, true, probs, probs_dropped);
 }
 
 extern "C" int nmtg_flash_attn_batched_bwd(const void* dout, const void* q, const void* k, const void* v, const void* out,

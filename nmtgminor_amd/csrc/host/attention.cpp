@@ -67,9 +67,11 @@ struct SelfAttentionNode : Function<SelfAttentionNode> {
     LinearGrads i;
     if (o.dx.defined()) {
       Tensor dlin = new_like(lin);
-      flash_bwd_batched({cx.size(0), cx.size(0), cx.size(1), heads, d}, o.dx, slot_view(lin, heads, 3, 0), slot_view(lin, heads, 3, 1), slot_view(lin, heads, 3, 2), cx, lse,
-                        slot_view(dlin, heads, 3, 0), slot_view(dlin, heads, 3, 1), slot_view(dlin, heads, 3, 2), pad, time, ctx->saved_data["p"].toDouble(),
-                        1.0 / std::sqrt(static_cast<double>(d)), false, kept_bits(ctx, words));
+      if (cx.numel() > 0)
+        flash_bwd_batched({cx.size(0), cx.size(0), cx.size(1), heads, d}, o.dx, slot_view(lin, heads, 3, 0), slot_view(lin, heads, 3, 1),
+                          slot_view(lin, heads, 3, 2), cx, lse, slot_view(dlin, heads, 3, 0), slot_view(dlin, heads, 3, 1),
+                          slot_view(dlin, heads, 3, 2), pad, time, ctx->saved_data["p"].toDouble(), 1.0 / std::sqrt(static_cast<double>(d)),
+                          false, kept_bits(ctx, words));
       i = linear_bwd(dlin, x, wi, need(0), need(1), need_bi);
     }
     return {i.dx, i.dw, o.dw, i.db, o.db, Tensor()};
@@ -113,9 +115,11 @@ struct CrossAttentionNode : Function<CrossAttentionNode> {
     LinearGrads o = linear_bwd(contiguous(grads[0]), cx, wo, inner, need(4), need_bo), q, kv;
     if (inner) {
       Tensor dq = new_like(ql), dkv = new_like(kvl);
-      flash_bwd_batched({cx.size(0), kvl.size(0), cx.size(1), heads, d}, o.dx, head_view(ql, heads), slot_view(kvl, heads, 2, 0), slot_view(kvl, heads, 2, 1), cx, lse,
-                        head_view(dq, heads), slot_view(dkv, heads, 2, 0), slot_view(dkv, heads, 2, 1), pad, Tensor(), ctx->saved_data["p"].toDouble(),
-                        1.0 / std::sqrt(static_cast<double>(d)), false, kept_bits(ctx, words));
+      if (cx.numel() > 0)
+        flash_bwd_batched({cx.size(0), kvl.size(0), cx.size(1), heads, d}, o.dx, head_view(ql, heads), slot_view(kvl, heads, 2, 0),
+                          slot_view(kvl, heads, 2, 1), cx, lse, head_view(dq, heads), slot_view(dkv, heads, 2, 0), slot_view(dkv, heads, 2, 1), pad,
+                          Tensor(), ctx->saved_data["p"].toDouble(), 1.0 / std::sqrt(static_cast<double>(d)), false, kept_bits(ctx, words));
+      else dkv.zero_();                            // no query position looked at the keys
       q = linear_bwd(dq, xq, wq, need(0), need(2), need_bq);
       kv = linear_bwd(dkv, xkv, wkv, need(1), need(3), need_bkv);
     }

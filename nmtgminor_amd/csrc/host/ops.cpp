@@ -130,6 +130,10 @@ LinearGrads linear_bwd(const Tensor& dy, const Tensor& x, const Tensor& w, bool 
   if (want_x) { auto sizes = dy.sizes().vec(); sizes.back() = in; r.dx = empty_like_sized(dy, sizes); }
   if (want_w) r.dw = new_like(w);
   if (want_b) r.db = empty_like_sized(dy, {out});
+  if (rows == 0) {                                  // no rows contribute zero gradients
+    for (Tensor* t : {&r.dw, &r.db}) if (t->defined()) t->zero_();
+    return r;
+  }
   const Scratch ws = mlp_workspace(dy, 1, &out, rows, in);
   const void* weights[1] = {ptr(w)};
   void* dws[1] = {ptr(r.dw)};

@@ -40,3 +40,15 @@ def test_header_compiles_as_plain_c(tmp_path):
     inc = os.path.join(os.path.dirname(os.path.dirname(_lib.LIB_PATH)), "include")
     subprocess.run(["gcc", "-std=c99", "-Wall", "-Werror", "-I", inc, "-c", str(src), "-o", str(tmp_path / "t.o")],
                    check=True)
+
+
+def test_attention_of_an_empty_batch_needs_no_address():
+    """Sizes are looked at before pointers: torch gives a tensor without elements the null address."""
+    lib = _lib.load()
+    n, s = None, [_lib.i64(64)] * 12
+    for fn, extra in ((lib.nmtg_flash_attn_batched_fwd, ()), (lib.nmtg_flash_attn_batched_fwd_probs, (n, _lib.i32(1)))):
+        for batch, len_q in ((0, 6), (2, 0), (0, 0), (2, 6)):
+            rc = fn(n, n, n, n, n, n, n, n, n, _lib.i64(batch), _lib.i64(2), _lib.i64(64), _lib.i64(len_q), _lib.i64(6), *s, _lib.f32(0.125),
+                    _lib.i32(0), _lib.i32(0), _lib.f32(0.0), n, n, n, ctypes.c_uint64(0), ctypes.c_uint64(0), _lib.i32(_lib.BF16), n, *extra)
+            assert rc == (-1 if batch and len_q else 0)
+            assert rc == 0 or b"null pointer" in lib.nmtg_last_error()

@@ -4,6 +4,8 @@ The autograd modules must also survive them, so that a training step over an emp
 import pytest
 import torch
 
+from nmtgminor_amd.modules.encdec_attention_func import encdec_attn_func
+from nmtgminor_amd.modules.encdec_attention_func_bias import encdec_attn_bias_func
 from nmtgminor_amd.modules.feed_forward import PositionWiseFeedForward
 from nmtgminor_amd.modules.self_attention import SelfMultiheadAttn
 from nmtgminor_amd.native import (encdec_multihead_attn_bias_blaslt as ed, fast_layer_norm_cuda as ln, fused_dropout_add_cuda as da,
@@ -68,3 +70,28 @@ def test_modules_train_through_an_empty_batch(dev):
     assert x.grad.shape == x.shape
     for p in list(attn.parameters()) + list(ffn.parameters()):
         assert p.grad is not None and not p.grad.any()
+
+
+@pytest.mark.parametrize("tq,tk,b", [(3, 7, 0), (0, 7, 2), (0, 0, 0)])
+@pytest.mark.parametrize("bias", [True, False])
+def test_encoder_decoder_attention_trains_through_an_empty_batch(dev, tq, tk, b, bias):
+    """With the coverage (the tiled core of the host layer): zero gradients for the weights and for keys no query looked at."""
+    e, h = 128, 2
+    r = lambda *s: torch.randn(*s).to(BF).to(dev).requires_grad_()
+    ins = [r(tq, b, e), r(tk, b, e), r(e, e), r(2 * e, e), r(e, e)] + ([r(e), r(2 * e), r(e)] if bias else [])
+    mask = torch.zeros(b, tk, dtype=torch.bool, device=dev)
+    if bias:
+        y, cov = encdec_attn_bias_func(False, True, h, *ins, mask, 0.1, False, None, False, None, None, True, True)
+    else:
+        y, cov = encdec_attn_func(False, True, h, *ins, mask, 0.1, False, None, False, None, None, False, True)
+    assert y.shape == (tq, b, e) and cov.shape == (b * h, tq, tk)
+    for t, g in zip(ins, torch.autograd.grad(y, ins, torch.ones_like(y))):
+        assert g.shape == t.shape and not g.any()
+
+
+def test_self_attention_trains_without_positions(dev):
+    attn = SelfMultiheadAttn(128, 2, 0.1).to(dev).to(BF).train()
+    x = torch.randn(0, 3, 128).to(BF).to(dev).requires_grad_()
+    y, cov = attn(x, None, torch.zeros(3, 0, dtype=torch.bool, device=dev), None)
+    y.backward(torch.ones_like(y))
+    assert cov.shape == (6, 0, 0) and x.grad.shape == x.shape and not any(p.grad.any() for p in attn.parameters())
