@@ -61,9 +61,10 @@ struct MlpNode : Function<MlpNode> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     auto s = ctx->get_saved_variables();
-    const bool want_w = ctx->needs_input_grad(1) || ctx->needs_input_grad(2);
+    auto need = [&](int i) { return ctx->needs_input_grad(i); };   // counts the tensors among the arguments: an absent bias does not
+    const bool has_b1 = ctx->saved_data["b1"].toBool(), has_b2 = ctx->saved_data["b2"].toBool();
     MlpGrads r = mlp_bwd(contiguous(g[0]), s[0], s[1], s[2], s[3], s[4], s[5], ctx->saved_data["p"].toDouble(), ctx->saved_data["a"].toInt(),
-                         ctx->needs_input_grad(0), want_w, ctx->saved_data["b1"].toBool() && want_w, ctx->saved_data["b2"].toBool() && want_w);
+                         need(0), need(1) || need(2), has_b1 && need(3), has_b2 && need(has_b1 ? 4 : 3));
     return {r.dx, r.dw1, r.dw2, r.db1, r.db2, Tensor(), Tensor(), Tensor()};
   }
 };

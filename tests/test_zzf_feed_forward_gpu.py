@@ -10,6 +10,7 @@ pass through two to four tensors stored in the 16-bit type on their way back).
 import pytest
 import torch
 
+from nmtgminor_amd import _lib as L
 from nmtgminor_amd._rng import philox_keep_mask_reference
 from nmtgminor_amd.modules.feed_forward import PositionWiseFeedForward
 from nmtgminor_amd.native import glu_dropout
@@ -161,3 +162,31 @@ def test_sigmoid_needs_the_gate(dev):
         PositionWiseFeedForward(8, 8, activation="sigmoid")
     with pytest.raises(RuntimeError):
         glu_dropout.forward(torch.zeros(4, 7, device=dev), "relu", 0.0)          # odd width: no two halves
+
+
+@pytest.mark.parametrize("act", ["relu", "gelu", "silu", "agelu"])
+@pytest.mark.parametrize("rows", [21, 1100])                     # bias sums of one job; of partial rows
+@pytest.mark.parametrize("trained", [("b1", "b2"), ("b1",), ("b2",), ("x",), ("x", "b1", "b2"), ("w1",), ("x", "w1", "w2", "b1", "b2")])
+@pytest.mark.parametrize("absent", [None, "b1", "b2"])
+def test_every_choice_of_trained_parameters_gets_its_gradients(dev, act, rows, trained, absent):
+    dtype, dm, di = torch.float16, 64, 96
+    gen = torch.Generator().manual_seed(rows)
+    names, shapes = ("x", "w1", "w2", "b1", "b2"), ((rows, dm), (di, dm), (dm, di), (di,), (dm,))
+    host = {n: ((s[-1] ** -0.5 if n[0] == "w" else 1.0) * torch.randn(s, generator=gen)).to(dtype) for n, s in zip(names, shapes)}
+    go = torch.randn(rows, dm, generator=gen).to(dtype)
+    wanted = [n for n in trained if n != absent]
+    hip = {n: (None if n == absent else t.to(dev).requires_grad_(n in wanted)) for n, t in host.items()}
+    ref = {n: (torch.zeros_like(t) if n == absent else t).to(D).requires_grad_(n in wanted) for n, t in host.items()}
+    fn = L.host().mlp(hip["x"], hip["w1"], hip["w2"], hip["b1"], hip["b2"], None, 0.0, L.ACT_CODES[act])
+    want = off.feed_forward(ref["x"].view(rows, 1, dm), ref["w1"], ref["b1"], ref["w2"], ref["b2"], act, round_to=dtype)
+    assert_close(fn, want.view(rows, dm), dtype, "out", scale_atol=True)
+    if not wanted:
+        assert not fn.requires_grad
+        return
+    fn.backward(go.to(dev))
+    want.backward(go.to(D).view(rows, 1, dm))
+    for n in names:
+        if n in wanted:
+            assert_close(hip[n].grad, ref[n].grad, dtype, "d" + n, scale_atol=True, atol=2e-3)
+        else:
+            assert hip[n] is None or hip[n].grad is None
