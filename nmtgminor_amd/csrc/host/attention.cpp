@@ -145,7 +145,7 @@ void define_attention(pybind11::module_& m) {
     const int64_t t = x.size(0), b = x.size(1), e = x.size(2);
     check_projection(x, wi, bi, 3 * e);
     check_projection(x, wo, bo, e);
-    const Call call{time_mask ? Tensor() : pad_bytes(mask, b, t), time_mask ? pad_bytes(mask, t, t) : Tensor(), heads, p,
+    const Call call{time_mask ? Tensor() : pad_bytes(mask, x, b, t), time_mask ? pad_bytes(mask, x, t, t) : Tensor(), heads, p,
                     Coverage::dropped};
     return SelfAttentionNode::apply(contiguous(x), contiguous(wi), contiguous(wo), flat(bi), flat(bo), &call);
   });
@@ -159,7 +159,7 @@ void define_attention(pybind11::module_& m) {
     check_projection(xq, wq, bq, e);
     check_projection(xkv, wkv, bkv, 2 * e);
     check_projection(xq, wo, bo, e);
-    const Call call{pad_bytes(mask, xkv.size(1), xkv.size(0)), Tensor(), heads, p, dropped ? Coverage::dropped : Coverage::softmax};
+    const Call call{pad_bytes(mask, xq, xkv.size(1), xkv.size(0)), Tensor(), heads, p, dropped ? Coverage::dropped : Coverage::softmax};
     return CrossAttentionNode::apply(contiguous(xq), contiguous(xkv), contiguous(wq), contiguous(wkv), contiguous(wo), flat(bq), flat(bkv), flat(bo),
                                      &call);
   });

@@ -138,7 +138,11 @@ void flash_bwd_batched(const FlashShape& shape, const Tensor& dout, const View& 
                        bool causal, const Bits& bits);
 // q / k / v slots of a projection [T, B, H, parts, D]
 Tensor slot(const Tensor& lin, int64_t heads, int64_t parts, int64_t which);
-Tensor pad_bytes(const optional<Tensor>& mask, int64_t rows, int64_t cols);
+// a mask as contiguous bytes [rows, cols], on the device of the operand it belongs to (a kernel is handed its address)
+Tensor pad_bytes(const optional<Tensor>& mask, const Tensor& operand, int64_t rows, int64_t cols);
+inline void check_device(const Tensor& t, const Tensor& operand) {
+  TORCH_CHECK(!t.defined() || t.device() == operand.device(), "expected a tensor on ", operand.device(), ", got one on ", t.device());
+}
 
 void define_autograd(pybind11::module_& m);
 void define_layers(pybind11::module_& m);

@@ -284,8 +284,8 @@ void define_layers(pybind11::module_& m) {
       }
     return grad && at::GradMode::is_enabled() ? 2 : 1;
   });
-  m.def("mask_bytes", [](const optional<Tensor>& mask, int64_t rows, int64_t cols) {
-    Tensor t = pad_bytes(mask, rows, cols);
+  m.def("mask_bytes", [](const optional<Tensor>& mask, const Tensor& operand, int64_t rows, int64_t cols) {
+    Tensor t = pad_bytes(mask, operand, rows, cols);
     return t.defined() ? optional<Tensor>(t) : optional<Tensor>();
   });
   // the rest of an encoder layer, from the context of its attention core
@@ -304,6 +304,8 @@ void define_layers(pybind11::module_& m) {
   m.def("decoder_step", [](const Tensor& x, const Tensor& kbuf, const Tensor& vbuf, int64_t n, const Tensor& ck, const Tensor& cv,
                            const optional<Tensor>& pad, const Params& w, int64_t heads, int64_t act) {
     at::AutoDispatchBelowADInplaceOrView off;
+    for (const Tensor* t : {&kbuf, &vbuf, &ck, &cv}) check_device(*t, x);
+    check_device(defined_or(pad), x);
     auto r = decoder_step(contiguous(x), kbuf, vbuf, n, ck, cv, defined_or(pad), w, heads, act);
     return std::make_tuple(std::get<0>(r), std::get<1>(r), kbuf.narrow(0, 0, n + 1), vbuf.narrow(0, 0, n + 1));
   });

@@ -158,6 +158,7 @@ Mlp mlp_fwd(const Tensor& x, const Tensor& w1, const Tensor& w2, const Tensor& b
   if (p > 0.0) {
     if (mask.has_value()) {
       TORCH_CHECK(mask->scalar_type() == at::kByte && mask->numel() == hidden, "mlp: mask must be uint8 with one byte per hidden activation");
+      check_device(*mask, x);
       r.mask = contiguous(*mask);
       mode = 1;
     } else {
@@ -252,8 +253,9 @@ Tensor slot(const Tensor& lin, int64_t heads, int64_t parts, int64_t which) {
   return lin.as_strided({lin.size(0), lin.size(1), heads, d}, {lin.stride(0), lin.stride(1), parts * d, 1}, lin.storage_offset() + which * d);
 }
 
-Tensor pad_bytes(const optional<Tensor>& mask, int64_t rows, int64_t cols) {
+Tensor pad_bytes(const optional<Tensor>& mask, const Tensor& operand, int64_t rows, int64_t cols) {
   if (!mask.has_value() || !mask->defined() || mask->numel() == 0) return Tensor();
+  check_device(*mask, operand);
   TORCH_CHECK(mask->numel() == rows * cols, "mask must be [", rows, ", ", cols, "]");
   Tensor m = contiguous(*mask).view({rows, cols});
   if (m.scalar_type() == at::kBool) return m.view(at::kByte);          // a bool mask is its bytes

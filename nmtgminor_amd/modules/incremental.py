@@ -38,6 +38,7 @@ def _decode_core(heads, q_lin, keys, values, pad_mask):
         km = pad_mask.to(torch.uint8).contiguous()
         if km.shape != (b, tk):
             raise RuntimeError(f"incremental attention: key mask of shape {tuple(km.shape)}, expected {(b, tk)}")
+    L.require_cuda(q_lin, keys, values, km)
     probs = torch.empty(b * heads, 1, tk, dtype=q_lin.dtype, device=q_lin.device)
     context = torch.empty(1, b, e, dtype=q_lin.dtype, device=q_lin.device)
     L.call("nmtg_attn_decode", L.ptr(q_lin), L.i64(e), L.ptr(keys), L.i64(keys.stride(0)), L.i64(keys.stride(1)), L.ptr(values),

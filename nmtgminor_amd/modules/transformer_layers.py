@@ -177,7 +177,7 @@ class EncoderLayer(_Layer):
         heads = mh.num_heads
         p_attn, p_res, p_ffn = (mh.dropout, self._modules["postprocess_ffn"].dropout_p, ff.dropout) if train else (0.0, 0.0, 0.0)
         x = x.contiguous()
-        pad = host.mask_bytes(attn_mask, x.shape[1], x.shape[0])
+        pad = host.mask_bytes(attn_mask, x, x.shape[1], x.shape[0])
         z, stats, lin, q, k, v = host.layer_begin(x, *params[:4], heads)
         ctx, lse, state = flash_attn_cuda.fwd_batched(q, k, v, pad, p_attn, mh.head_dim ** -0.5, False)
         return host.encoder_end(x, z, stats, lin, ctx, lse, state, pad, params, heads, ff.activation_code, p_attn, p_res, p_ffn, mode == 2)
@@ -233,8 +233,9 @@ class DecoderLayer(_Layer):
         x = x.contiguous()
         time = None
         if mask_tgt is not None:
-            time = host.mask_bytes(mask_tgt if mask_tgt.dtype in (torch.bool, torch.uint8) else mask_tgt.to(torch.bool), x.shape[0], x.shape[0])
-        pad = host.mask_bytes(mask_src, context.shape[1], context.shape[0])
+            time = host.mask_bytes(mask_tgt if mask_tgt.dtype in (torch.bool, torch.uint8) else mask_tgt.to(torch.bool), x, x.shape[0],
+                                   x.shape[0])
+        pad = host.mask_bytes(mask_src, x, context.shape[1], context.shape[0])
         z, stats, lin, q, k, v = host.layer_begin(x, *params[:4], heads)
         ctx, lse, state = flash_attn_cuda.fwd_batched(q, k, v, None, p_attn, mh.head_dim ** -0.5, False, time_mask=time)
         return host.decoder_end(x, context, z, stats, lin, ctx, lse, state, time, pad, params, heads, ff.activation_code, p_attn, p_cross,

@@ -45,6 +45,7 @@ def _validate(x, weights, biases):
 def forward(act, p, inputs, mask=None, save_pre=True):
     x, weights, biases = _split_inputs(inputs)
     _validate(x, weights, biases)
+    L.require_cuda(mask)
     x2 = x.contiguous().view(-1, x.shape[-1])
     weights = [w.contiguous() for w in weights]
     biases = [b.contiguous() if b is not None else None for b in biases]

@@ -112,6 +112,36 @@ def test_decoding_step(dev, dtype, b, tk, prev, e):
     same(res, dtype)
 
 
+def test_a_mask_in_host_memory_is_refused(dev):
+    """Wherever a layer hands a mask's address to a kernel; on the native path and operator by operator."""
+    e, tq, tk, b = 128, 5, 8, 2
+    x, c = torch.randn(tq, b, e, device=dev).half(), torch.randn(tk, b, e, device=dev).half()
+    causal = torch.triu(torch.ones(tq, tq, device=dev), 1).bool()
+    good, bad = torch.zeros(b, tk, dtype=torch.bool, device=dev), torch.zeros(b, tk, dtype=torch.bool)
+    dec = randomised(DecoderLayer(options(e, 0.1, "relu")), dev, F16, 5)
+    enc = randomised(EncoderLayer(options(e, 0.1, "relu")), dev, F16, 5)
+    for by_operator in (False, True):
+        handles = [m.feedforward.register_forward_hook(lambda m, i, o: None) for m in (dec, enc) if by_operator]
+        for train in (True, False):
+            with torch.set_grad_enabled(train):
+                for call in (lambda: enc.train(train)(c, bad), lambda: dec.train(train)(x, c, causal, bad),
+                             lambda: dec.train(train)(x, c, causal.cpu(), good)):
+                    with pytest.raises(RuntimeError, match="expected a tensor|must be contiguous uint8"):
+                        call()
+        with torch.no_grad():
+            dec.eval()
+            cache = {}
+            dec(x, c, causal, good, incremental=True, incremental_cache=cache)
+            for mask in (bad, bad[:, None]):
+                with pytest.raises(RuntimeError, match="expected a tensor|key mask of shape"):
+                    dec(x[:1], c, None, mask, incremental=True, incremental_cache=dict(cache))
+            with pytest.raises(RuntimeError, match="expected a tensor"):
+                dec(x[:1], c, None, good, incremental=True, incremental_cache=dict(cache, c_k=cache["c_k"].cpu()))
+            assert torch.isfinite(dec(x[:1], c, None, good, incremental=True, incremental_cache=cache)[0]).all()
+        for h in handles:
+            h.remove()
+
+
 @pytest.mark.parametrize("dtype", [F16, BF16])
 @pytest.mark.parametrize("bad", [math.inf, -math.inf, math.nan])
 def test_a_stream_that_is_not_finite_is_clamped_and_its_gradient_stops(dev, dtype, bad):
