@@ -341,6 +341,11 @@ int nmtg_encdec_attn_fwd(const void* x_q, const void* x_kv, const void* w_q, con
                          float p, uint64_t seed, uint64_t offset, void* ctx, void* out, int64_t tq,
                          int64_t tk, int64_t b, int64_t e, int heads, int dtype, void* stream);
 
+/* Whether an inference call needs the score buffer (see above): 0 = scores may be NULL, for tensors of the library's own
+ * alignment (16 bytes; probabilities 8, mask 4). 1 for a form the one-kernel path does not take, and always with
+ * NMTG_ATTN_PROBS=0 in the environment. */
+int nmtg_attn_scores_needed(int64_t len_k, int64_t head_dim, int dtype);
+
 int64_t nmtg_encdec_attn_bwd_workspace_bytes(int64_t tq, int64_t tk, int64_t b, int64_t e, int heads);
 
 int nmtg_encdec_attn_bwd(const void* grad_out, const void* ctx, const void* dropped,

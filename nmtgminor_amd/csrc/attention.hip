@@ -310,6 +310,8 @@ extern "C" int nmtg_self_attn_bwd(const void* grad_out, const void* ctx, const v
   return linear_bwd(dtype, dlin, x, w_in, grad_x, grad_w_in, grad_b_in, rows, e, 3 * e, splitk_ws, ws.splitk, colsum_ws, st);
 }
 
+extern "C" int nmtg_attn_scores_needed(int64_t len_k, int64_t head_dim, int dtype) { return attn_probs_form(dtype, head_dim, len_k) ? 0 : 1; }
+
 extern "C" int nmtg_encdec_attn_fwd(const void* x_q, const void* x_kv, const void* w_q, const void* w_kv, const void* w_out,
                                     const void* b_q, const void* b_kv, const void* b_out, const uint8_t* pad_mask,
                                     void* q_lin, void* kv_lin, void* scores, void* softmax_out, void* dropped,

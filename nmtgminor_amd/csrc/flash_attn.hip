@@ -1737,13 +1737,16 @@ int probs_launch(const AttnProbsCall& c, dim3 grid, hipStream_t st) {
 
 }  // namespace
 
+bool attn_probs_form(int dtype, int64_t head_dim, int64_t len_k) {
+  return !switched_off("NMTG_ATTN_PROBS") && (dtype == NMTG_F16 || dtype == NMTG_BF16) && (head_dim == 64 || head_dim == 128) && len_k >= 1 &&
+         len_k % 4 == 0;
+}
+
 bool attn_probs_ok(const AttnProbsCall& c) {
-  if (switched_off("NMTG_ATTN_PROBS")) return false;
   auto view = [&](const void* p, int64_t st, int64_t sb, int64_t sh) {
     return aligned16(p) && st % 8 == 0 && sb % 8 == 0 && sh % 8 == 0 && st >= 0 && sb >= 0 && sh >= 0;
   };
-  return (c.dtype == NMTG_F16 || c.dtype == NMTG_BF16) && (c.d == 64 || c.d == 128) && c.tk >= 1 && c.tk % 4 == 0 && c.tq >= 1 &&
-         c.batch >= 1 && c.batch <= 65535 && c.heads >= 1 && c.heads <= 65535 && view(c.q, c.q_st, c.q_sb, c.q_sh) &&
+  return attn_probs_form(c.dtype, c.d, c.tk) && c.tq >= 1 && c.batch >= 1 && c.batch <= 65535 && c.heads >= 1 && c.heads <= 65535 && view(c.q, c.q_st, c.q_sb, c.q_sh) &&
          view(c.k, c.k_st, c.k_sb, c.k_sh) && view(c.v, c.v_st, c.v_sb, c.v_sh) && view(c.ctx, c.c_st, c.c_sb, c.c_sh) &&
          reinterpret_cast<uintptr_t>(c.probs) % 8 == 0 &&
          (c.mask == nullptr || c.mask_kind == 0 || reinterpret_cast<uintptr_t>(c.mask) % 4 == 0) && fabsf(c.scale) <= 1e6f;

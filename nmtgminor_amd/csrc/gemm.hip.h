@@ -994,7 +994,8 @@ struct AttnProbsCall {
   float scale;
   int dtype;
 };
-bool attn_probs_ok(const AttnProbsCall& c);    // NMTG_ATTN_PROBS=0 switches the kernel off
+bool attn_probs_form(int dtype, int64_t head_dim, int64_t len_k);    // NMTG_ATTN_PROBS=0 switches the kernel off
+bool attn_probs_ok(const AttnProbsCall& c);                          // a call of that form, with the alignment of its operands
 int attn_probs_run(const AttnProbsCall& c, hipStream_t st);
 
 // Fused Q K^T -> mask -> softmax -> dropout (EPI_SCORES_SOFTMAX) for rows of at most 512 keys. `a` is filled as

@@ -27,7 +27,8 @@ using std::optional;
 #define NMTG_HOST_API(X)                                                                                              \
   X(last_error) X(ln_fwd) X(ln_bwd_parts) X(ln_bwd) X(dropout_add_fwd) X(dropout_add_bwd) X(xentropy_fwd)             \
   X(add_ln_fwd) X(ln_bwd_add) X(dropout_add_guard_fwd) X(dropout_add_guard_bwd) X(encdec_attn_fwd)                    \
-  X(attn_decode) X(attn_decode_append) X(encdec_attn_bwd_workspace_bytes) X(encdec_attn_bwd_from_probs)                                                    \
+  X(attn_decode) X(attn_decode_append) X(encdec_attn_bwd_workspace_bytes) X(encdec_attn_bwd_from_probs)               \
+  X(attn_scores_needed)                                                                                               \
   X(xentropy_bwd) X(gemm) X(mlp_fwd) X(mlp_bwd_dtype_workspace_bytes) X(mlp_bwd) X(flash_attn_dropout_bits_bytes)     \
   X(flash_attn_fwd) X(flash_attn_bwd) X(flash_attn_key_info_bytes) X(flash_attn_time_info_bytes)                      \
   X(flash_attn_batched_fwd) X(flash_attn_batched_bwd) X(multi_tensor_adam) X(multi_tensor_clip)                       \

@@ -114,7 +114,7 @@ struct DecoderIn {
 };
 
 struct Cross { Tensor q_lin, kv_lin, softmax, dropped, mask, ctx, out; };
-Cross cross_fwd(const Tensor& xq, const Tensor& xkv, const Tensor& wq, const Tensor& wkv, const Tensor& wo, const Tensor& pad, int64_t heads,
+Cross cross_fwd(const Tensor& xq, const Tensor& xkv, const Tensor& wq, const Tensor& wkv, const Tensor& wo, const Tensor& mask, int64_t heads,
                 double p, bool grad) {
   const int64_t tq = xq.size(0), tk = xkv.size(0), b = xq.size(1), e = xq.size(2), d = e / heads;
   Launch on(xq);
@@ -124,8 +124,10 @@ Cross cross_fwd(const Tensor& xq, const Tensor& xkv, const Tensor& wq, const Ten
   r.ctx = new_like(xq);
   r.out = new_like(xq);
   r.dropped = empty_like_sized(xq, {b * heads, tq, tk});
+  // the kernels read mask bytes four or eight at a time: a view that starts at an odd address is copied
+  const Tensor pad = mask.defined() && reinterpret_cast<uintptr_t>(ptr(mask)) % 8 != 0 ? mask.clone() : mask;
   // an inference call writes the probabilities only where one kernel makes them and the context (nmtg_encdec_attn_fwd)
-  const bool probs_only = !grad && p == 0.0 && tk % 4 == 0 && (d == 64 || d == 128);
+  const bool probs_only = !grad && p == 0.0 && api.attn_scores_needed(tk, d, dtype_code(xq)) == 0;
   Scratch scores;
   if (!probs_only) scores = Scratch(xq, b * heads * tq * tk * static_cast<int64_t>(xq.element_size()));
   uint64_t seed = 0, offset = 0;

@@ -52,3 +52,13 @@ def test_attention_of_an_empty_batch_needs_no_address():
                     _lib.i32(0), _lib.i32(0), _lib.f32(0.0), n, n, n, ctypes.c_uint64(0), ctypes.c_uint64(0), _lib.i32(_lib.BF16), n, *extra)
             assert rc == (-1 if batch and len_q else 0)
             assert rc == 0 or b"null pointer" in lib.nmtg_last_error()
+
+
+def test_which_inference_calls_need_a_score_buffer(monkeypatch):
+    lib = _lib.load()
+    need = lambda tk, d, dtype=_lib.F16: lib.nmtg_attn_scores_needed(_lib.i64(tk), _lib.i64(d), _lib.i32(dtype))
+    monkeypatch.delenv("NMTG_ATTN_PROBS", raising=False)
+    assert [need(4, 64), need(1500, 128, _lib.BF16)] == [0, 0]
+    assert [need(61, 64), need(0, 64), need(64, 32), need(64, 64, _lib.F32)] == [1, 1, 1, 1]
+    monkeypatch.setenv("NMTG_ATTN_PROBS", "0")
+    assert need(4, 64) == 1

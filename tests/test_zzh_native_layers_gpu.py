@@ -112,6 +112,29 @@ def test_decoding_step(dev, dtype, b, tk, prev, e):
     same(res, dtype)
 
 
+@pytest.mark.parametrize("tk", [64, 61])                    # the one-kernel inference path; stored scores
+@pytest.mark.parametrize("shift", [0, 1, 2, 4])             # bytes the mask starts behind a multiple of eight
+@pytest.mark.parametrize("probs", ["1", "0"])
+@pytest.mark.parametrize("train", [True, False])
+def test_a_mask_at_any_address_and_with_the_inference_kernel_switched_off(dev, monkeypatch, tk, shift, probs, train):
+    e, tq, b, dtype = 128, 9, 3, F16
+    monkeypatch.setenv("NMTG_ATTN_PROBS", probs)
+    # gelu: the paths round the cross-attention at different points, and behind a relu a hidden element within that rounding of
+    # zero would pass its whole gradient on one path and none on the other: of 27 x 256 hidden elements half of them live, one
+    # is sqrt(1 / 3456) = 1.7e-2 of the gradient in front of it, beyond the 2e-3 that the roundings themselves are held to
+    layer = randomised(DecoderLayer(options(e, 0.1, "gelu")), dev, dtype, 7).train(train)
+    x = torch.randn(tq, b, e, device=dev).to(dtype).requires_grad_(train)
+    c = torch.randn(tk, b, e, device=dev).to(dtype).requires_grad_(train)
+    buf = torch.zeros(8 + b * tk, dtype=torch.uint8, device=dev)
+    pad = buf[shift:shift + b * tk].view(b, tk)
+    pad.copy_(torch.arange(tk, device=dev)[None] >= torch.tensor([tk, tk - 3, tk // 2], device=dev)[:, None])
+    assert pad.data_ptr() % 8 == shift
+    causal = torch.triu(torch.ones(tq, tq, device=dev), 1).bool()
+    dy = torch.randn(tq, b, e, device=dev).to(dtype)
+    with torch.set_grad_enabled(train):
+        same(both_paths(layer, layer.feedforward, lambda: layer(x, c, causal, pad), [x, c] if train else [], dy if train else None), dtype)
+
+
 def test_a_mask_in_host_memory_is_refused(dev):
     """Wherever a layer hands a mask's address to a kernel; on the native path and operator by operator."""
     e, tq, tk, b = 128, 5, 8, 2
