@@ -59,6 +59,8 @@ void check(int rc, const char* what);
 int dtype_code(const Tensor& t);
 inline void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 inline void* ptr(const optional<Tensor>& t) { return t.has_value() ? ptr(*t) : nullptr; }
+// A forward-mode dual: its tangent would be lost where the autograd node is passed by (the node itself refuses it).
+inline bool has_tangent(const Tensor& t) { return t.defined() && t._fw_grad(/*level=*/0).defined(); }
 inline Tensor contiguous(const Tensor& t) { return t.is_contiguous() ? t : t.contiguous(); }
 // Results. A small batch is bound by this host work, and a layer's pass makes some 60 tensors: the allocator's own entry
 // leaves out at::empty's way through the dispatcher. With it, Scratch and View (the six views of the attention's backward cost a

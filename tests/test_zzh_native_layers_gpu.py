@@ -135,6 +135,35 @@ def test_a_mask_at_any_address_and_with_the_inference_kernel_switched_off(dev, m
         same(both_paths(layer, layer.feedforward, lambda: layer(x, c, causal, pad), [x, c] if train else [], dy if train else None), dtype)
 
 
+@pytest.mark.parametrize("train", [True, False])
+def test_a_forward_mode_tangent_is_refused_and_not_dropped(dev, train):
+    import torch.autograd.forward_ad as fwd
+    e, t, b = 128, 6, 2
+    enc = randomised(EncoderLayer(options(e, 0.1, "gelu")), dev, F16, 8).train(train).requires_grad_(train)
+    dec = randomised(DecoderLayer(options(e, 0.1, "gelu")), dev, F16, 8).train(train).requires_grad_(train)
+    x = torch.randn(t, b, e, device=dev).half()
+    causal, pad = torch.triu(torch.ones(t, t, device=dev), 1).bool(), torch.zeros(b, t, dtype=torch.bool, device=dev)
+    cache = {}
+    with torch.no_grad():
+        dec.eval()(x, x, causal, pad, incremental=True, incremental_cache=cache)
+    dec.train(train)
+    with fwd.dual_level():
+        dual = fwd.make_dual(x, torch.ones_like(x))
+        for call in (lambda: enc(dual, pad), lambda: dec(dual, x, causal, pad), lambda: dec(x, dual, causal, pad), lambda: enc.feedforward(dual),
+                     lambda: enc.preprocess_ffn(dual), lambda: enc.multihead(dual, None, pad, None)):
+            with pytest.raises(RuntimeError, match="jvp"):
+                call()
+        if not train:
+            with torch.no_grad(), pytest.raises(RuntimeError, match="jvp"):
+                dec(dual[:1], x, None, pad, incremental=True, incremental_cache=dict(cache))
+        for name in ("in_proj_weight", "in_proj_bias", "out_proj_bias"):
+            w = getattr(enc.feedforward, name)
+            with pytest.raises(RuntimeError, match="jvp"):
+                torch.func.functional_call(enc.feedforward, {name: fwd.make_dual(w.detach(), torch.ones_like(w))}, (x,))
+            with pytest.raises(RuntimeError, match="jvp"):
+                torch.func.functional_call(enc, {"feedforward." + name: fwd.make_dual(w.detach(), torch.ones_like(w))}, (x, pad))
+
+
 def test_a_mask_in_host_memory_is_refused(dev):
     """Wherever a layer hands a mask's address to a kernel; on the native path and operator by operator."""
     e, tq, tk, b = 128, 5, 8, 2
