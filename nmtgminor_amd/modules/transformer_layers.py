@@ -113,7 +113,8 @@ class _Layer(nn.Module):
     _PRE, _POST = ["n"], ["d", "a"]
 
     def _sub_parameters(self, pre, mods):
-        """The parameters of the sub-modules in the order of the native layer, or None where one is not of the plain form."""
+        """The parameters of the sub-modules in the order of the native layer, or None where one is not of the plain form. (An
+        entry is None where a sub-module carries a plain tensor in a parameter's place: the native layer then declines.)"""
         t, out = self.training, []
         for name in mods:
             m = self._modules.get(name)
@@ -126,23 +127,24 @@ class _Layer(nn.Module):
                     n = n._modules["function"] if type(n) is Bottle else None
                     if type(n) is not LayerNorm or n.eps != 1e-5 or n.memory_efficient or n._forward_hooks or n._forward_pre_hooks:
                         return None
-                    out += [n._parameters["weight"], n._parameters["bias"]]
+                    p = n._parameters.get
+                    out += [p("weight"), p("bias")]
                 elif m.steps != self._POST or m.variational or type(m._modules["dropout"]) is not nn.Dropout \
                         or m._modules["dropout"].p != m.dropout_p or m.dropout_p != self.postprocess_ffn.dropout_p:
                     return None
             elif kind is SelfMultiheadAttn:
                 if m.rotary_pos_enc or m.head_dim not in (64, 128):
                     return None
-                p = m._parameters
-                out += [p["in_proj_weight"], p["in_proj_bias"], p["out_proj_weight"], p["out_proj_bias"]]
+                p = m._parameters.get
+                out += [p("in_proj_weight"), p("in_proj_bias"), p("out_proj_weight"), p("out_proj_bias")]
             elif kind is EncdecMultiheadAttn:
-                p = m._parameters
-                out += [p["in_proj_weight_q"], p["in_proj_weight_kv"], p["out_proj_weight"]]
+                p = m._parameters.get
+                out += [p("in_proj_weight_q"), p("in_proj_weight_kv"), p("out_proj_weight")]
             elif kind is PositionWiseFeedForward:
                 if m.glu or m.variational or m.dropout_residual or m.fused_function is None:
                     return None
-                p = m._parameters
-                out += [p["in_proj_weight"], p["in_proj_bias"], p["out_proj_weight"], p["out_proj_bias"]]
+                p = m._parameters.get
+                out += [p("in_proj_weight"), p("in_proj_bias"), p("out_proj_weight"), p("out_proj_bias")]
             else:
                 return None
         return out

@@ -164,6 +164,29 @@ def test_a_forward_mode_tangent_is_refused_and_not_dropped(dev, train):
                 torch.func.functional_call(enc, {"feedforward." + name: fwd.make_dual(w.detach(), torch.ones_like(w))}, (x, pad))
 
 
+@pytest.mark.parametrize("where", ["preprocess_attn.layer_norm.function.weight", "multihead_tgt.in_proj_bias", "multihead_src.out_proj_weight",
+                                   "feedforward.in_proj_weight"])
+@pytest.mark.parametrize("train", [True, False])
+def test_a_plain_tensor_in_the_place_of_a_parameter(dev, where, train):
+    """As a hyper-network or a weight computed from another leaves it: deleted as a parameter, set as a tensor."""
+    e, t, b = 128, 6, 2
+    layer = randomised(DecoderLayer(options(e, 0.0, "gelu")), dev, F16, 9).train(train)
+    x = torch.randn(t, b, e, device=dev).half().requires_grad_(train)
+    causal, pad = torch.triu(torch.ones(t, t, device=dev), 1).bool(), torch.zeros(b, t, dtype=torch.bool, device=dev)
+    with torch.set_grad_enabled(train):
+        want = layer(x, x, causal, pad)[0]
+        owner = layer.get_submodule(where.rsplit(".", 1)[0])
+        name = where.rsplit(".", 1)[1]
+        source = getattr(owner, name)
+        delattr(owner, name)
+        setattr(owner, name, source * 1.0)
+        got = layer(x, x, causal, pad)[0]
+        assert rel_err(got, want) < 2e-3
+        if train:
+            got.backward(torch.ones_like(got))
+            assert source.grad is not None and torch.isfinite(source.grad).all() and source.grad.any()
+
+
 def test_a_mask_in_host_memory_is_refused(dev):
     """Wherever a layer hands a mask's address to a kernel; on the native path and operator by operator."""
     e, tq, tk, b = 128, 5, 8, 2
