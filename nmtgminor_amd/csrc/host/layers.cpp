@@ -253,6 +253,23 @@ std::tuple<Tensor, Tensor> decoder_step(const Tensor& x, const Tensor& kbuf, con
   return {f.out, coverage};
 }
 
+// Whether an encoder layer's 12 or a decoder layer's 17 parameters (all present) have the shapes that x's last dimension asks
+// for: what follows hands their addresses to kernels. Anything else is left to the operators, whose checks name it.
+bool shapes_fit(int64_t e, const std::vector<optional<Tensor>>& p) {
+  const bool decoder = p.size() == 17;
+  if (!decoder && p.size() != 12) return false;
+  size_t i = 0;
+  auto vec = [&](int64_t n) { return p[i++]->numel() == n; };
+  auto mat = [&](int64_t rows, int64_t cols) {
+    const Tensor& t = *p[i++];
+    return t.dim() == 2 && t.size(0) == rows && t.size(1) == cols;
+  };
+  if (!(vec(e) && vec(e) && mat(3 * e, e) && vec(3 * e) && mat(e, e) && vec(e) && vec(e) && vec(e))) return false;
+  if (decoder && !(mat(e, e) && mat(2 * e, e) && mat(e, e) && vec(e) && vec(e))) return false;
+  const int64_t inner = p[i]->dim() == 2 ? p[i]->size(0) : -1;
+  return mat(inner, e) && vec(inner) && mat(e, inner) && vec(e);
+}
+
 using State = std::tuple<int64_t, uint64_t, uint64_t, optional<Tensor>, optional<Tensor>, optional<Tensor>>;
 using Params = std::vector<Tensor>;
 
@@ -262,6 +279,7 @@ void define_layers(pybind11::module_& m) {
   // LayerNorm and in-projection of the self-attention -> (z, stats, projection, q, k, v)
   m.def("layer_begin", [](const Tensor& input, const Tensor& g, const Tensor& b, const Tensor& wi, const Tensor& bi, int64_t heads) {
     at::AutoDispatchBelowADInplaceOrView off;
+    TORCH_CHECK(heads > 0 && input.size(2) % heads == 0, "layer: ", heads, " heads do not divide ", input.size(2));
     Tensor x = contiguous(input);
     Norm n = ln_fwd(x, g, b, kEps);
     Tensor lin = linear_fwd(n.z, wi, bi);
@@ -274,7 +292,7 @@ void define_layers(pybind11::module_& m) {
     return std::make_tuple(f.out, f.lse, State(f.bits.mode, f.bits.seed, f.bits.offset, {},
                                                f.bits.words.defined() ? optional<Tensor>(f.bits.words) : optional<Tensor>(), {}));
   });
-  // What the layers ask before they take this path: 0 = no (a parameter of another type, layout or device, or none, or a
+  // What the layers ask before they take this path: 0 = no (a parameter of another type, shape, layout or device, or none, or a
   // forward-mode tangent anywhere), 1 = yes, nothing will be back-propagated, 2 = yes, with gradients.
   m.def("layer_mode", [](const Tensor& x, const std::vector<optional<Tensor>>& inputs, const std::vector<optional<Tensor>>& params) {
     if (!x.is_cuda() || x.dim() != 3 || x.numel() == 0 || (x.scalar_type() != at::kHalf && x.scalar_type() != at::kBFloat16) ||
@@ -288,6 +306,7 @@ void define_layers(pybind11::module_& m) {
           return 0;
         grad = grad || p->requires_grad();
       }
+    if (!shapes_fit(x.size(2), params)) return 0;
     return grad && at::GradMode::is_enabled() ? 2 : 1;
   });
   m.def("mask_bytes", [](const optional<Tensor>& mask, const Tensor& operand, int64_t rows, int64_t cols) {

@@ -187,6 +187,33 @@ def test_a_plain_tensor_in_the_place_of_a_parameter(dev, where, train):
             assert source.grad is not None and torch.isfinite(source.grad).all() and source.grad.any()
 
 
+@pytest.mark.parametrize("train", [True, False])
+def test_shapes_that_do_not_fit_are_refused_before_a_kernel_sees_them(dev, train):
+    e, t, b = 128, 6, 2
+    enc = randomised(EncoderLayer(options(e, 0.1, "gelu")), dev, F16, 8).train(train)
+    dec = randomised(DecoderLayer(options(e, 0.1, "gelu")), dev, F16, 8).train(train)
+    causal, pad = torch.triu(torch.ones(t, t, device=dev), 1).bool(), torch.zeros(b, t, dtype=torch.bool, device=dev)
+    x, wide, slim = (torch.randn(t, b, n, device=dev).half() for n in (e, 2 * e, e // 2))
+    with torch.set_grad_enabled(train):
+        for bad in (wide, slim):
+            for call in (lambda: enc(bad, pad), lambda: dec(bad, bad, causal, pad), lambda: dec(x, bad, causal, pad)):
+                with pytest.raises(RuntimeError):
+                    call()
+        if not train:
+            cache = {}
+            dec(x, x, causal, pad, incremental=True, incremental_cache=cache)
+            with pytest.raises(RuntimeError):
+                dec(wide[:1], x, None, pad, incremental=True, incremental_cache=dict(cache))
+        for layer, call in ((enc, lambda: enc(x, pad)), (dec, lambda: dec(x, x, causal, pad))):
+            for name in ("in_proj_weight", "out_proj_weight", "in_proj_bias", "out_proj_bias"):
+                w = getattr(layer.feedforward, name)
+                setattr(layer.feedforward, name, torch.nn.Parameter(w[:-8].detach().contiguous()))
+                with pytest.raises(RuntimeError, match="mlp: (weight|bias) shape"):
+                    call()
+                setattr(layer.feedforward, name, w)
+            call()
+
+
 def test_a_mask_in_host_memory_is_refused(dev):
     """Wherever a layer hands a mask's address to a kernel; on the native path and operator by operator."""
     e, tq, tk, b = 128, 5, 8, 2
