@@ -62,6 +62,10 @@ def load():
 
 _host_module = None
 
+# Not None while torch.jit.trace records. The host layer's calls are invisible to it (their results would be baked in as
+# constants); a Python autograd function is recorded as an operator, so a traced call takes that.
+tracing = torch._C._get_tracing_state
+
 
 def host():
     """The native host layer (csrc/host): operators that take tensors, prepare the call and enqueue the kernels without the

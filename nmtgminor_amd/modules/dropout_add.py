@@ -35,7 +35,7 @@ class FusedDropoutAdd(torch.autograd.Function):
 
 
 def fused_dropout_add(*args):
-    if len(args) == 4 and args[0].is_cuda and not torch.is_autocast_enabled():
+    if len(args) == 4 and args[0].is_cuda and not torch.is_autocast_enabled() and not L.tracing():
         return L.host().dropout_add(*args)
     args = cast_if_autocast_enabled(*args)
     with no_autocast():

@@ -17,6 +17,7 @@ import os
 
 import torch
 
+from .. import _lib as L
 from ..native import flash_attn_cuda as fa
 from .rotary import _linear, _linear_bwd
 
@@ -36,9 +37,9 @@ def eligible(is_training, return_coverage, recompute, x, heads):
 
 def with_coverage(return_coverage, p, dropout_mask):
     """Whether a call that would be eligible without its coverage runs on the tiled core in the host layer, which writes the
-    coverage besides: on the GPU, with dropout and no explicit keep-mask. (A call without dropout stays on the extension's
+    coverage besides: on the GPU, with dropout, no explicit keep-mask and no trace being recorded. (A call without dropout stays on the extension's
     path, whose probabilities round where the reference's stored scores do; it has no mask to write or read either.)"""
-    return bool(return_coverage) and dropout_mask is None and p > 0.0
+    return bool(return_coverage) and dropout_mask is None and p > 0.0 and not L.tracing()
 
 
 def _pad(mask, batch, len_k):

@@ -91,7 +91,7 @@ class FlashAttnKVPackedFunc(torch.autograd.Function):
 def _host_takes(qkv, cu_seqlens, dropout_p, return_softmax):
     return (not return_softmax and qkv.is_cuda and cu_seqlens.is_cuda and qkv.dim() == 4 and qkv.shape[1] == 3
             and qkv.dtype in (torch.float16, torch.bfloat16) and qkv.stride(3) == 1 and qkv.shape[0] > 0
-            and cu_seqlens.dtype == torch.int32 and cu_seqlens.is_contiguous() and cu_seqlens.numel() > 1)
+            and cu_seqlens.dtype == torch.int32 and cu_seqlens.is_contiguous() and cu_seqlens.numel() > 1 and not L.tracing())
 
 
 def flash_bert_mha(*args):

@@ -45,11 +45,12 @@ class FastLayerNormFN(torch.autograd.Function):
 
 
 def fast_layer_norm_affine(input, weight, bias, normalized_shape, eps=1e-5, memory_efficient=False):
-    if input.is_cuda and not torch.is_autocast_enabled():
+    native = input.is_cuda and not L.tracing()
+    if native and not torch.is_autocast_enabled():
         return L.host().layer_norm(input, weight, bias, eps, memory_efficient)
     args = cast_if_autocast_enabled(input, weight, bias, eps, memory_efficient)
     with no_autocast():
-        return L.host().layer_norm(*args) if input.is_cuda else FastLayerNormFN.apply(*args)
+        return L.host().layer_norm(*args) if native else FastLayerNormFN.apply(*args)
 
 
 def _affine_or_identity(input, weight, bias, hidden):

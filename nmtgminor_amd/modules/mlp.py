@@ -97,7 +97,7 @@ def _callable(fn, act):
     act = L.ACT_CODES[act]
 
     def call(p, recompute, *args, mask=None):
-        if len(args) == 5 and not recompute and args[0].is_cuda and not torch.is_autocast_enabled():
+        if len(args) == 5 and not recompute and args[0].is_cuda and not torch.is_autocast_enabled() and not L.tracing():
             return L.host().mlp(*args, mask, p, act)          # the transformer's two layers
         args = cast_if_autocast_enabled(*args)
         with no_autocast():

@@ -151,7 +151,7 @@ class _Layer(nn.Module):
 
     def _native_mode(self, x, inputs, params):
         if params is None or self.macaron or self.death_rate > 0 or feed_forward.recompute or torch.is_autocast_enabled() \
-                or not flash_core.switched_on():
+                or not flash_core.switched_on() or L.tracing():
             return 0
         mode = L.host().layer_mode(x, inputs, params)
         return mode if (mode == 2) is self.training else 0

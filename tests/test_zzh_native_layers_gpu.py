@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from nmtgminor_amd import _lib as L
+from nmtgminor_amd.modules.softmax_xentropy import SoftmaxCrossEntropyLoss
 from nmtgminor_amd.modules.transformer_layers import DecoderLayer, EncoderLayer
 from nmtgminor_amd.native import fast_layer_norm_cuda as ln
 from util import assert_close, rel_err
@@ -212,6 +213,25 @@ def test_shapes_that_do_not_fit_are_refused_before_a_kernel_sees_them(dev, train
                     call()
                 setattr(layer.feedforward, name, w)
             call()
+
+
+def test_a_traced_module_computes_on_its_new_inputs(dev):
+    """torch.jit.trace records Python autograd functions and cannot see the host layer: what it cannot see would be a constant.
+    (A layer's dropout + add works in place, which a traced program refuses to run.)"""
+    e, t, b = 128, 6, 2
+    enc = randomised(EncoderLayer(options(e, 0.1, "gelu")), dev, F16, 8).eval().requires_grad_(False)
+    pad = torch.zeros(b, t, dtype=torch.bool, device=dev)
+    x, new = torch.randn(2, t, b, e, device=dev).half()
+    trace = lambda call, y: torch.jit.trace(call, (y,), check_trace=False)
+    with torch.no_grad():
+        for call in (enc.preprocess_ffn, enc.feedforward, lambda y: enc.multihead(y, None, pad)[0]):
+            assert rel_err(trace(call, x)(new), call(new)) < 2e-3
+        with pytest.raises(RuntimeError, match="not supported in the JIT"):
+            trace(lambda y: enc(y, pad), x)(new)
+    rows = torch.randn(2, 40, 100, device=dev).half()
+    labels = torch.randint(0, 100, (40,), device=dev)
+    loss = lambda z: SoftmaxCrossEntropyLoss.apply(z, labels, 0.1, 1, True)
+    assert rel_err(trace(loss, rows[0])(rows[1]), loss(rows[1])) < 1e-5
 
 
 def test_a_mask_in_host_memory_is_refused(dev):
