@@ -22,6 +22,8 @@ from .dropout_add import fused_dropout_add
 from .glu import gated_activation_dropout
 from .linear import linear_function
 
+FUNCTIONS = {"relu": fused.mlp_relu_function, "gelu": fused.mlp_gelu_function, "silu": fused.mlp_silu_function,
+             "swish": fused.mlp_silu_function, "agelu": fused.mlp_agelu_function}
 recompute = False  # process-wide switch, the counterpart of onmt.constants.recompute
 
 
@@ -29,17 +31,15 @@ class PositionWiseFeedForward(nn.Module):
     def __init__(self, model_size, inner_size, dropout=0., variational=False, activation="relu", glu=False,
                  weight_drop=0.0, dropout_residual=False, res_dropout=0.0):
         super().__init__()
-        fns = {"relu": fused.mlp_relu_function, "gelu": fused.mlp_gelu_function, "silu": fused.mlp_silu_function,
-               "swish": fused.mlp_silu_function, "agelu": fused.mlp_agelu_function}
         if activation == "sigmoid" and not glu:
             raise NotImplementedError("PositionWiseFeedForward: the sigmoid activation exists as a gate only (glu=True)")
-        if activation not in fns and activation != "sigmoid":
+        if activation not in FUNCTIONS and activation != "sigmoid":
             raise NotImplementedError(f"PositionWiseFeedForward: activation {activation!r} has no HIP kernel")
         self.model_size, self.inner_size = model_size, inner_size
         self.dropout, self.activation = dropout, activation
         self.bias, self.glu, self.variational, self.weight_drop = True, glu, variational, weight_drop
         self.dropout_residual, self.res_dropout = dropout_residual, res_dropout
-        self.fused, self.fused_function = not glu, fns.get(activation)
+        self.fused, self.fused_function = not glu, FUNCTIONS.get(activation)
         self.activation_code = L.ACT_CODES.get("silu" if activation == "swish" else activation)
         self.in_proj_weight = Parameter(torch.empty(inner_size * (2 if glu else 1), model_size))
         self.out_proj_weight = Parameter(torch.empty(model_size, inner_size))

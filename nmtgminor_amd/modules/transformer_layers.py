@@ -15,15 +15,18 @@ of this package and asking for them raises.
 """
 import torch
 from torch import nn
+from torch.nn.modules.module import _has_any_global_hook
 
 from .. import _lib as L
 from ..native import flash_attn_cuda
 from . import feed_forward, flash_core, incremental as incremental_steps
 from .encdec_attention import EncdecMultiheadAttn
+from .encdec_attention_func import encdec_attn_func
 from .feed_forward import PositionWiseFeedForward
 from .layer_norm import LayerNorm
 from .pre_post_processing import Bottle, PrePostProcessing
 from .self_attention import SelfMultiheadAttn
+from .self_attention_func import self_attn_func
 
 
 class Identity(nn.Module):
@@ -51,6 +54,12 @@ def _clamp_non_finite_(x):
         clamp_value = torch.finfo(x.dtype).max - 1000
         x.clamp_(min=-clamp_value, max=clamp_value)
     return x
+
+
+def _called_as_built(attributes):
+    """Whether calling the module of these instance attributes runs its class's forward and nothing else."""
+    return not (attributes["_forward_hooks"] or attributes["_forward_pre_hooks"] or attributes["_backward_hooks"]
+                or attributes["_backward_pre_hooks"] or "forward" in attributes)
 
 
 class _Layer(nn.Module):
@@ -108,43 +117,54 @@ class _Layer(nn.Module):
 
     # -- the layer as one node of the host layer (csrc/host/layers.cpp) -------------------------------------------------
     # Taken by the plain form: 16-bit tensors on the GPU, LayerNorm with affine parameters in front, dropout + add behind,
-    # no gate, no variational dropout, no stochastic depth, no macaron block, no hooks on the sub-modules, and either
-    # training with a backward to come or evaluation without one. Everything else runs operator by operator below.
+    # no gate, no variational dropout, no stochastic depth, no macaron block, nothing that listens to or replaces the call of
+    # a sub-module at any depth, and either training with a backward to come or evaluation without one. Everything else runs
+    # operator by operator below.
     _PRE, _POST = ["n"], ["d", "a"]
 
     def _sub_parameters(self, pre, mods):
         """The parameters of the sub-modules in the order of the native layer, or None where one is not of the plain form. (An
         entry is None where a sub-module carries a plain tensor in a parameter's place: the native layer then declines.)"""
-        t, out = self.training, []
+        if _has_any_global_hook():
+            return None
+        train, subs, out = self.training, self._modules, []
         for name in mods:
-            m = self._modules.get(name)
-            if m is None or m.training is not t or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks:
+            m = subs.get(name)
+            if m is None:
                 return None
-            kind = type(m)
+            kind, d = type(m), m.__dict__            # (instance attributes read from the dict: this runs on every call)
+            if d["training"] is not train or not _called_as_built(d):
+                return None
             if kind is PrePostProcessing:
                 if name in pre:
-                    n = m._modules["layer_norm"] if m.steps == self._PRE else None
-                    n = n._modules["function"] if type(n) is Bottle else None
-                    if type(n) is not LayerNorm or n.eps != 1e-5 or n.memory_efficient or n._forward_hooks or n._forward_pre_hooks:
+                    n = d["_modules"]["layer_norm"] if d["steps"] == self._PRE else None
+                    if type(n) is not Bottle or not _called_as_built(n.__dict__):
+                        return None
+                    n = n._modules["function"]
+                    if type(n) is not LayerNorm or n.eps != 1e-5 or n.memory_efficient or not _called_as_built(n.__dict__):
                         return None
                     p = n._parameters.get
-                    out += [p("weight"), p("bias")]
-                elif m.steps != self._POST or m.variational or type(m._modules["dropout"]) is not nn.Dropout \
-                        or m._modules["dropout"].p != m.dropout_p or m.dropout_p != self.postprocess_ffn.dropout_p:
-                    return None
+                    out += (p("weight"), p("bias"))
+                else:
+                    n = d["_modules"].get("dropout")
+                    if d["steps"] != self._POST or d["variational"] or type(n) is not nn.Dropout or n.training is not train \
+                            or not n.p == d["dropout_p"] == subs["postprocess_ffn"].dropout_p or not _called_as_built(n.__dict__):
+                        return None
             elif kind is SelfMultiheadAttn:
-                if m.rotary_pos_enc or m.head_dim not in (64, 128):
+                if d["rotary_pos_enc"] or d["head_dim"] not in (64, 128) or d["attn_func"] is not self_attn_func:
                     return None
-                p = m._parameters.get
-                out += [p("in_proj_weight"), p("in_proj_bias"), p("out_proj_weight"), p("out_proj_bias")]
+                p = d["_parameters"].get
+                out += (p("in_proj_weight"), p("in_proj_bias"), p("out_proj_weight"), p("out_proj_bias"))
             elif kind is EncdecMultiheadAttn:
-                p = m._parameters.get
-                out += [p("in_proj_weight_q"), p("in_proj_weight_kv"), p("out_proj_weight")]
-            elif kind is PositionWiseFeedForward:
-                if m.glu or m.variational or m.dropout_residual or m.fused_function is None:
+                if d["attn_func"] is not encdec_attn_func:
                     return None
-                p = m._parameters.get
-                out += [p("in_proj_weight"), p("in_proj_bias"), p("out_proj_weight"), p("out_proj_bias")]
+                p = d["_parameters"].get
+                out += (p("in_proj_weight_q"), p("in_proj_weight_kv"), p("out_proj_weight"))
+            elif kind is PositionWiseFeedForward:
+                if d["glu"] or d["variational"] or d["dropout_residual"] or d["fused_function"] is not feed_forward.FUNCTIONS.get(d["activation"]):
+                    return None
+                p = d["_parameters"].get
+                out += (p("in_proj_weight"), p("in_proj_bias"), p("out_proj_weight"), p("out_proj_bias"))
             else:
                 return None
         return out

@@ -1,8 +1,11 @@
 """What the native host layer (nmtgminor_amd/_host.so) decides before it touches a GPU: it loads and binds without one."""
+from types import SimpleNamespace
+
 import pytest
 import torch
 
 from nmtgminor_amd import _lib as L
+from nmtgminor_amd.modules.transformer_layers import DecoderLayer, EncoderLayer
 
 
 def test_the_host_layer_loads_and_finds_every_entry_point():
@@ -33,3 +36,66 @@ def test_operands_of_a_call_share_a_device():
         pad = torch.zeros(2, 4, dtype=torch.uint8, device="cpu" if at == 4 else "meta")
         with pytest.raises(RuntimeError, match="expected a tensor on meta, got one on cpu"):
             L.host().decoder_step(step[0], cache[0], cache[1], 3, cache[2], cache[3], pad, [], 1, L.ACT_RELU)
+
+
+def _layers():
+    opt = SimpleNamespace(model_size=128, inner_size=256, n_heads=2, dropout=0.1, attn_dropout=0.1, ffn_activation="swish")
+    yield EncoderLayer(opt), ("preprocess_attn", "preprocess_ffn"), 12
+    yield DecoderLayer(opt), ("preprocess_attn", "preprocess_src_attn", "preprocess_ffn"), 17
+
+
+LISTEN = {"forward_hook": lambda m: m.register_forward_hook(lambda *a: None),
+          "forward_pre_hook": lambda m: m.register_forward_pre_hook(lambda *a: None),
+          "backward_hook": lambda m: m.register_full_backward_hook(lambda *a: None),
+          "backward_pre_hook": lambda m: m.register_full_backward_pre_hook(lambda *a: None)}
+
+
+@pytest.mark.parametrize("kind", list(LISTEN) + ["forward", "mode"])
+def test_what_listens_to_a_sub_module_keeps_the_layer_off_the_native_form(kind):
+    """At any depth: the operators call every sub-module, the native form none."""
+    for layer, pre, count in _layers():
+        def native():
+            return layer._sub_parameters(pre, layer._SUB) is not None
+        assert native() and len(layer._sub_parameters(pre, layer._SUB)) == count
+        inner = [(n, m) for n, m in layer.named_modules() if n]
+        assert {type(m).__name__ for _, m in inner} >= {"PrePostProcessing", "Bottle", "LayerNorm", "Dropout", "SelfMultiheadAttn",
+                                                        "PositionWiseFeedForward"}
+        for name, m in inner:
+            if kind == "forward":
+                plain = m.forward
+                m.forward = lambda *a, **k: plain(*a, **k)
+                assert not native(), name
+                del m.forward
+            elif kind == "mode":
+                if type(m).__name__ in ("Bottle", "LayerNorm"):
+                    continue                              # no difference between their modes
+                m.train(not layer.training)
+                assert not native(), name
+                layer.train(layer.training)
+            else:
+                handle = LISTEN[kind](m)
+                assert not native(), name
+                handle.remove()
+            assert native(), name
+
+
+def test_hooks_on_every_module_and_replaced_functions_keep_the_layer_off_the_native_form():
+    from torch.nn.modules import module as mod
+    for layer, pre, _ in _layers():
+        def native():
+            return layer._sub_parameters(pre, layer._SUB) is not None
+        for register in (mod.register_module_forward_hook, mod.register_module_forward_pre_hook, mod.register_module_full_backward_hook,
+                         mod.register_module_full_backward_pre_hook):
+            handle = register(lambda *a: None)
+            assert not native()
+            handle.remove()
+            assert native()
+        for name, m in layer.named_modules():
+            for function in ("attn_func", "fused_function"):
+                if hasattr(m, function):
+                    plain = getattr(m, function)
+                    setattr(m, function, lambda *a, **k: plain(*a, **k))
+                    assert not native(), name
+                    setattr(m, function, plain)
+        layer.postprocess_attn.dropout.p = 0.3
+        assert not native()
