@@ -1,0 +1,249 @@
+"""The layers as one native node (csrc/host/layers.cpp) against the layer oracle in fp64 with nothing rounded, at odd key counts;
+and what such a node has to leave as it was: frozen parameters, strided inputs, another stream, a captured graph, a second
+backward of the projection + loss."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from nmtgminor_amd.modules.encdec_attention_func import encdec_attn_func
+from nmtgminor_amd.modules.generator_loss import GeneratorLoss
+from nmtgminor_amd.modules.self_attention_func import self_attn_func
+from nmtgminor_amd.modules.transformer_layers import DecoderLayer, EncoderLayer
+from oracle import transformer_layers as otl
+from util import rel_err
+
+pytestmark = pytest.mark.gpu
+D, F16, BF16 = torch.float64, torch.float16, torch.bfloat16
+# A result passes at most about 20 tensors stored in 16 bits on its way (forward and backward of a decoder layer). A stored
+# element is off by at most u = 2^-11 (fp16) or 2^-8 (bf16) of itself, u / sqrt(3) in the 2-norm, and 20 independent ones add up
+# to sqrt(20) times that: 1.3e-3 and 1e-2.
+BOUND = {F16: 1.3e-3, BF16: 1.0e-2}
+
+
+def options(e, p=0.0):
+    return SimpleNamespace(model_size=e, inner_size=2 * e, n_heads=e // 64, dropout=p, attn_dropout=p, variational_dropout=False,
+                           macaron=False, rezero=False, ffn_activation="gelu", ffn_glu=False, fast_self_attention=True,
+                           fast_xattention=True, fast_feed_forward=True, ignore_source=False)
+
+
+def randomised(layer, dev, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    with torch.no_grad():
+        for p in layer.parameters():
+            p.add_((0.1 if p.dim() == 1 else 0.02) * torch.randn(p.shape, generator=g))
+    return layer.to(dev).to(dtype)
+
+
+def on_the_native_node(out, train, name):
+    assert not train or out.grad_fn.name().find(name) >= 0
+
+
+def padding(b, t, seed):
+    n = torch.randint((t + 1) // 2, t + 1, (b,), generator=torch.Generator().manual_seed(seed))
+    return torch.arange(t)[None] >= n[:, None]
+
+
+def compare(what, got, want, dtype, factor=1):
+    err = rel_err(got, want)
+    assert got.shape == want.shape and err < factor * BOUND[dtype], f"{what}: {err:.2e}"
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("t,b,e", [(1, 1, 128), (37, 3, 128), (65, 2, 256)])
+@pytest.mark.parametrize("train", [True, False])
+def test_encoder_layer(dev, dtype, t, b, e, train):
+    layer = randomised(EncoderLayer(options(e)), dev, dtype, 1).train(train)
+    g = torch.Generator().manual_seed(t)
+    x, dy = torch.randn(2, t, b, e, generator=g).to(dtype)
+    pad = padding(b, t, 2)
+    p64 = {k: v.detach().cpu().to(D).requires_grad_() for k, v in layer.state_dict().items()}
+    x64 = x.to(D).requires_grad_()
+    want = otl.encoder_layer(x64, p64, e // 64, pad, act="gelu")
+    xin = x.to(dev).requires_grad_(train)
+    with torch.set_grad_enabled(train):
+        y = layer(xin, pad.to(dev))
+    on_the_native_node(y, train, "EncoderNode")
+    compare("output", y, want, dtype)
+    if train:
+        y.backward(dy.to(dev))
+        want.backward(dy.to(D))
+        compare("dx", xin.grad, x64.grad, dtype)
+        for name, p in layer.named_parameters():
+            compare("d " + name, p.grad, p64[name].grad, dtype)
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("tq,tk,b,e", [(1, 3, 1, 128), (24, 61, 3, 128), (61, 73, 2, 256), (17, 130, 2, 128), (9, 64, 2, 128)])
+@pytest.mark.parametrize("train", [True, False])
+def test_decoder_layer(dev, dtype, tq, tk, b, e, train):
+    layer = randomised(DecoderLayer(options(e)), dev, dtype, 3).train(train)
+    g = torch.Generator().manual_seed(tk)
+    x, dy = torch.randn(2, tq, b, e, generator=g).to(dtype)
+    c = torch.randn(tk, b, e, generator=g).to(dtype)
+    pad, causal = padding(b, tk, 4), torch.triu(torch.ones(tq, tq), 1).bool()
+    p64 = {k: v.detach().cpu().to(D).requires_grad_() for k, v in layer.state_dict().items()}
+    x64, c64 = x.to(D).requires_grad_(), c.to(D).requires_grad_()
+    want, cov = otl.decoder_layer(x64, c64, p64, e // 64, causal, pad, act="gelu")
+    xin, cin = x.to(dev).requires_grad_(train), c.to(dev).requires_grad_(train)
+    with torch.set_grad_enabled(train):
+        y, coverage, _ = layer(xin, cin, causal.to(dev), pad.to(dev))
+    on_the_native_node(y, train, "DecoderNode")
+    compare("output", y, want, dtype)
+    compare("coverage", coverage, cov.view(coverage.shape), dtype)
+    if train:
+        y.backward(dy.to(dev))
+        want.backward(dy.to(D))
+        compare("dx", xin.grad, x64.grad, dtype)
+        compare("dcontext", cin.grad, c64.grad, dtype)
+        # the gradient of a score is the difference of a rounded product and the mean of tk of them: of three products and one
+        # query the difference may well be half of what it is taken from, and carries their rounding
+        for name, p in layer.named_parameters():
+            compare("d " + name, p.grad, p64[name].grad, dtype, 2 if tq * tk < 4 else 1)
+
+
+def passes(dev, layer, inputs, masks, dy, trained):
+    """-> the output and the gradients of a training pass, as {name: tensor}, under one generator state"""
+    torch.manual_seed(3)
+    torch.cuda.manual_seed(5)
+    named = dict(layer.named_parameters(), **{f"input {i}": t for i, t in enumerate(inputs)})
+    for name, t in named.items():
+        t.grad = None
+        t.requires_grad_(trained(name))
+    out = layer(*inputs, *masks)
+    out = out[0] if isinstance(out, tuple) else out
+    out.backward(dy)
+    res = {name: t.grad for name, t in named.items()}
+    for t in named.values():
+        t.requires_grad_(True)
+    return dict(res, output=out.detach())
+
+
+def both_layers(dev, p, dtype=F16, e=128, tq=13, tk=21, b=3):
+    x = torch.randn(tq, b, e, device=dev).to(dtype)
+    c = torch.randn(tk, b, e, device=dev).to(dtype)
+    causal = torch.triu(torch.ones(tq, tq, device=dev), 1).bool()
+    yield randomised(EncoderLayer(options(e, p)), dev, dtype, 5).train(), [x.clone()], [padding(b, tq, 6).to(dev)]
+    yield randomised(DecoderLayer(options(e, p)), dev, dtype, 5).train(), [x.clone(), c], [causal, padding(b, tk, 6).to(dev)]
+
+
+CHOICES = {"no parameter": lambda n: n.startswith("input"), "no input": lambda n: not n.startswith("input"),
+           "biases": lambda n: n.endswith("bias"), "LayerNorms": lambda n: "layer_norm" in n,
+           "weights": lambda n: n.endswith(("proj_weight", "weight_q", "weight_kv")), "the context": lambda n: n == "input 1" or n == "input 0",
+           "one bias": lambda n: n == "feedforward.in_proj_bias", "the first projection": lambda n: n.endswith("in_proj_weight")}
+
+
+@pytest.mark.parametrize("choice", list(CHOICES))
+def test_frozen_parameters(dev, choice):
+    """What is frozen gets no gradient, and the rest the gradient that it has when nothing is frozen (a sum may run in another
+    order where the pass that it rode with is not needed: the roundings of one operator)."""
+    for layer, inputs, masks in both_layers(dev, 0.1):
+        dy = torch.randn_like(inputs[0])
+        full = passes(dev, layer, inputs, masks, dy, lambda n: True)
+        some = passes(dev, layer, inputs, masks, dy, CHOICES[choice])
+        assert all(t is not None for t in full.values()) and torch.equal(some["output"], full["output"])
+        for name, want in full.items():
+            if name == "output" or CHOICES[choice](name):
+                compare(name, some[name], want, F16)
+            else:
+                assert some[name] is None, name
+
+
+def test_strided_inputs(dev):
+    """A batch-first buffer seen time first, a slice of a wider one, and an upstream gradient that is neither."""
+    for layer, inputs, masks in both_layers(dev, 0.1):
+        dy = torch.randn_like(inputs[0])
+        want = passes(dev, layer, inputs, masks, dy, lambda n: True)
+        dy_t = dy.transpose(0, 1).contiguous().transpose(0, 1)
+        for view in (lambda t: t.transpose(0, 1).contiguous().transpose(0, 1),
+                     lambda t: torch.cat([t, t], 2)[:, :, :t.shape[2]]):
+            strided = [view(t.detach()) for t in inputs]
+            assert not strided[0].is_contiguous()
+            got = passes(dev, layer, strided, masks, dy_t, lambda n: True)
+            for name in want:
+                compare(name, got[name], want[name], F16)
+
+
+def test_an_empty_batch(dev):
+    for layer, inputs, masks in both_layers(dev, 0.1, b=0):
+        got = passes(dev, layer, inputs, masks, torch.empty_like(inputs[0]), lambda n: True)
+        assert got["output"].shape == inputs[0].shape and not any(t.any() for t in got.values())
+
+
+def test_another_stream(dev):
+    """A whole pass on a stream of its own, its memory given back and taken again between the passes: the same bits."""
+    for layer, inputs, masks in both_layers(dev, 0.1, tq=96, tk=120):
+        dy = torch.randn_like(inputs[0])
+        want = passes(dev, layer, inputs, masks, dy, lambda n: True)
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        for _ in range(3):
+            with torch.cuda.stream(side):
+                got = passes(dev, layer, inputs, masks, dy, lambda n: True)
+            torch.full((1 << 20,), float("nan"), device=dev)             # work of the first stream in between
+            torch.cuda.synchronize()
+            for name in want:
+                assert torch.equal(got[name], want[name]), name
+
+
+def test_an_evaluation_in_a_captured_graph(dev):
+    layer = randomised(EncoderLayer(options(128, 0.1)), dev, BF16, 7).eval()
+    x = torch.randn(40, 3, 128, device=dev).to(BF16)
+    pad = padding(3, 40, 8).to(dev)
+    with torch.no_grad():
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            layer(x, pad)
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = layer(x, pad)
+        for i in range(4):
+            x.copy_(torch.randn(40, 3, 128, device=dev))
+            graph.replay()
+            torch.cuda.synchronize()
+            want = layer(x, pad)                                        # eager work between the replays
+            assert torch.equal(out, want), i
+
+
+@pytest.mark.parametrize("first", [("x", "w", "b"), ("x",), ("w",), ("b",)])
+@pytest.mark.parametrize("loss_of", ["sum", "rows"])
+def test_a_second_backward_of_the_projection_and_loss(dev, first, loss_of):
+    """The first backward turns the kept logits into their gradient; the second one projects again."""
+    m = GeneratorLoss(64, 517, label_smoothing=0.1, padding_idx=1).to(dev).to(BF16).train()
+    with torch.no_grad():
+        m.linear.bias.normal_(0, 0.1)
+    x = torch.randn(80, 64, device=dev).to(BF16).requires_grad_()
+    y = torch.randint(0, 517, (80,), device=dev)
+    leaves = {"x": x, "w": m.linear.weight, "b": m.linear.bias}
+
+    def loss():
+        r = m(x, y, sum_loss=loss_of == "sum")["loss"]
+        return r if loss_of == "sum" else (r * torch.linspace(0.5, 1.5, 80, device=dev)).sum()
+    want = dict(zip(leaves, torch.autograd.grad(loss(), list(leaves.values()))))
+    out = loss()
+    assert "GeneratorNode" in (out.grad_fn.name() if loss_of == "sum" else out.grad_fn.next_functions[0][0].next_functions[0][0].name())
+    for names in (first, tuple(leaves), tuple(leaves)):
+        got = torch.autograd.grad(out, [leaves[n] for n in names], retain_graph=True)
+        for n, g in zip(names, got):
+            compare(n, g, want[n], BF16)
+
+
+@pytest.mark.parametrize("shift", [1, 2, 4, 7])
+def test_attention_with_coverage_under_a_mask_at_any_address(dev, shift):
+    tq, tk, b, e, h = 9, 21, 3, 128, 2
+    r = lambda *s: torch.randn(*s, device=dev).half().requires_grad_()
+    ins = [r(tq, b, e), r(tk, b, e), r(e, e), r(2 * e, e), r(e, e)]
+    own = [r(tk, b, e), r(3 * e, e), r(e, e), r(3 * e), r(e)]
+    mask = padding(b, tk, 9).to(dev)
+    odd = torch.zeros(8 + mask.numel(), dtype=torch.uint8, device=dev)[shift:shift + mask.numel()].view(b, tk)
+    odd.copy_(mask)
+    assert odd.data_ptr() % 8 == shift
+    res = []
+    for m in (mask, odd):
+        torch.cuda.manual_seed(5)
+        y, cov = encdec_attn_func(False, True, h, *ins, m, 0.1, False, None, False, None, None, False, True)
+        z, own_cov = self_attn_func(False, True, h, *own, m, 0.1, False, None, False, None, True, True, False)
+        res.append([y, cov, z, own_cov, *torch.autograd.grad(y, ins, torch.ones_like(y)), *torch.autograd.grad(z, own, torch.ones_like(z))])
+    assert all(torch.equal(a, w) for a, w in zip(*res))
