@@ -116,14 +116,13 @@ int gemm_launch_one(const GemmArgs& a, hipStream_t st) {
     }
     return gemm_launch_ring<T, TILE, A_KC, B_KC, EPI>(a, st);
   }
-  if constexpr (TILE == TILE_X) return fail(NMTG_ERR_UNSUPPORTED, "gemm: the 64x64 tile has a ring kernel only");
-  else if (a.vec == 8) return gemm_launch_vec<T, TILE, A_KC, B_KC, EPI, 8>(a, st);
-  if constexpr (TILE == TILE_X) return 0;
-  else if constexpr (TILE != TILE_L) {
-    if (a.vec == 4) return gemm_launch_vec<T, TILE, A_KC, B_KC, EPI, 4>(a, st);
-    return gemm_launch_vec<T, TILE, A_KC, B_KC, EPI, 1>(a, st);
+  if constexpr (TILE == TILE_X) {
+    return fail(NMTG_ERR_UNSUPPORTED, "gemm: the 64x64 tile has a ring kernel only");
   } else {
-    return fail(NMTG_ERR_UNSUPPORTED, "gemm: the 256x256 tile needs 16-byte aligned operands");
+    if (a.vec == 8) return gemm_launch_vec<T, TILE, A_KC, B_KC, EPI, 8>(a, st);
+    if constexpr (TILE == TILE_L) return fail(NMTG_ERR_UNSUPPORTED, "gemm: the 256x256 tile needs 16-byte aligned operands");
+    else if (a.vec == 4) return gemm_launch_vec<T, TILE, A_KC, B_KC, EPI, 4>(a, st);
+    else return gemm_launch_vec<T, TILE, A_KC, B_KC, EPI, 1>(a, st);
   }
 }
 

@@ -44,7 +44,6 @@ struct EncoderIn {
   uint64_t seed, offset;
   Rates p;
   bool grad;
-  Tensor out;
 };
 
 struct EncoderNode : Function<EncoderNode> {
@@ -318,7 +317,7 @@ void define_layers(pybind11::module_& m) {
                           const State& state, const optional<Tensor>& pad, const Params& w, int64_t heads, int64_t act, double p_attn,
                           double p_residual, double p_ffn, bool grad) {
     EncoderIn in{x, z1, stats1, lin, cx, lse, defined_or(std::get<4>(state)), defined_or(pad), heads, act, std::get<0>(state), std::get<1>(state),
-                 std::get<2>(state), {p_attn, p_residual, p_ffn}, grad, Tensor()};
+                 std::get<2>(state), {p_attn, p_residual, p_ffn}, grad};
     if (!grad) {
       at::AutoDispatchBelowADInplaceOrView off;
       Tensor keep;

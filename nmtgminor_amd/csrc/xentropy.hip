@@ -270,7 +270,7 @@ __global__ __launch_bounds__(XE_THREADS) void xentropy_bwd_kernel(
 }
 
 // The backward with the column sums of its result (the bias gradient of the output projection). A block owns XC_COLS
-// columns of `rows_per_block` rows and walks down the rows, a lane's eight columns summed in registers, so the gradient is
+// columns of XC_ROWS rows and walks down the rows, a lane's eight columns summed in registers, so the gradient is
 // not read again for the sums; per-row values are wavefront-uniform loads. 16-bit types, 16-byte aligned rows.
 // 4096 rows of 250 054 classes in bf16: 815 + 11 us (5.0 TB/s); the row kernel above took 795 and the column sums of its
 // result another 575.
@@ -282,10 +282,10 @@ constexpr int XC_ROWS = 128;            // rows per block; few enough that the p
 template <typename T>
 __global__ __launch_bounds__(XC_THREADS) void xentropy_bwd_colsum_kernel(
     const float* __restrict__ grad_loss, int64_t grad_stride, const T* logits, const float* __restrict__ lse_in,
-    const int64_t* __restrict__ labels, T* grad_logits, float* __restrict__ part, int rows, int rows_per_block, int64_t vocab,
+    const int64_t* __restrict__ labels, T* grad_logits, float* __restrict__ part, int rows, int64_t vocab,
     int64_t ld, int64_t ld_grad, float smoothing, int64_t padding_idx) {
   static_assert(sizeof(T) == 2, "a lane moves eight 16-bit elements");
-  const int r0 = blockIdx.y * rows_per_block, r1 = min(rows, r0 + rows_per_block);
+  const int r0 = blockIdx.y * XC_ROWS, r1 = min(rows, r0 + XC_ROWS);
   const int64_t c0 = static_cast<int64_t>(blockIdx.x) * XC_COLS + threadIdx.x * 8;
   if (c0 >= vocab) return;
   const int valid = static_cast<int>(min(static_cast<int64_t>(8), vocab - c0));   // the last lane's vector ends in the pitch
@@ -428,7 +428,7 @@ extern "C" int nmtg_xentropy_bwd_colsum(const float* grad_loss, int64_t grad_str
     auto go = [&](auto tag) {
       using T = decltype(tag);
       hipLaunchKernelGGL((xentropy_bwd_colsum_kernel<T>), grid, dim3(XC_THREADS), 0, st, grad_loss, grad_stride, static_cast<const T*>(logits),
-                         lse, labels, static_cast<T*>(grad_logits), part, static_cast<int>(rows), XC_ROWS, vocab, ld_logits, ld_grad,
+                         lse, labels, static_cast<T*>(grad_logits), part, static_cast<int>(rows), vocab, ld_logits, ld_grad,
                          smoothing, padding_idx);
     };
     if (dtype == NMTG_F16) go(f16_t{});
