@@ -654,7 +654,7 @@ int nmtg_rel_softmax_dropout_bwd(const void* grad_dropped, const void* scores, c
                                  int64_t len_q, int64_t len_k, int64_t heads, int dtype, void* stream);
 
 /* ------------------------------------------------------------------------------------------
- * Optimizer-side passes over a list of tensors (one launch per 48 tensors instead of one per tensor).
+ * Optimizer-side passes over a list of tensors (one launch per 84 to 160 tensors instead of one per tensor).
  * Reference: fused_optim.multi_tensor_adam / multi_tensor_scale / multi_tensor_axpby / multi_tensor_l2norm /
  *   multi_tensor_l2norm_scale
  *   (onmt/modules/extensions/fused_optim/frontend.cpp:45-53; multi_tensor_adam.cu:22-171,

@@ -73,8 +73,8 @@ __global__ __launch_bounds__(DA_THREADS) void dropout_add_fwd_kernel(
 // stands is the whole effect; for fp16 the bound (64504, stored as 64512) lies below the largest finite values, which are
 // clamped too once any element of the tensor is not finite: the kernel raises `flag`, and guard_clamp_f16_kernel, behind
 // it, returns at once unless it is raised. Bit 1 of an element's mask byte records that no gradient passes it (clamped or
-// NaN). Bandwidth bound like the plain form: 16.4 us at [512 x 32 x 1024] bf16 against 39 us for the two reductions it
-// replaces, and no host round trip.
+// NaN). Bandwidth bound like the plain form: 22 us at [512 x 32 x 1024] bf16 with the mask drawn here, and none of the 39 us
+// of the two reductions it replaces, nor a host round trip.
 // ---------------------------------------------------------------------------------------------------------------------
 template <typename T> __device__ __forceinline__ float guard_limit();
 template <> __device__ __forceinline__ float guard_limit<float>() { return INFINITY; }

@@ -1364,8 +1364,8 @@ __global__ __launch_bounds__(FA_THREADS * G, (D == 64 && G == 1) ? 2 : 1) void a
 // them): the one tensor of that size is written once and never read. Bound by those stores. A block owns 128 queries and
 // a run of key tiles (`tiles_per_block`); nothing is summed, so the keys are dealt out freely. [512 x 512] x 512 heads in
 // bf16: scores, probabilities after dropout and mask bytes in one kernel and their product with the values took 336 us; the
-// keep bits (75), the context (70) and these probabilities (76) take 221, and the backward, which read 670 MB of them in
-// 436 us, takes 245. (Keys straight from memory instead of through LDS, without the barrier: 102 us, bound by the vector
+// keep bits (64), the context (72) and these probabilities (78) take 214, and the backward, which read 670 MB of them in
+// 436 us, takes 259. (Keys straight from memory instead of through LDS, without the barrier: 102 us, bound by the vector
 // memory pipe. The lane masks through a pointer that may alias `probs`: 94 us, they come in vector registers then.)
 constexpr int FP_PITCH = FA_TILE * 2 + 16;   // bytes per row of a wavefront's strip
 template <typename T, int D, int DROP, int PAD>

@@ -3,8 +3,10 @@
 // autograd.cpp wraps them in autograd nodes, layers.cpp composes the transformer layers, attention.cpp the attention modules, loss.cpp the output
 // projection with its loss, optim.cpp prepares the optimizer's passes.
 //
-// Why it exists: a call through the Python stand-ins costs 25 to 80 us of interpreter, ctypes and autograd bookkeeping per
-// operator and direction, several times what the kernels of a small batch take. The same work here is 3 to 8 us.
+// Why it exists: interpreter, ctypes and autograd bookkeeping of a call through the Python functions take several times what
+// the kernels of a small batch take. Host time of a call on [64 x 512], LayerNorm / feed-forward block / dropout + add: forward
+// 20 / 27 / 20 us there and 6 / 12 / 11 here, forward and backward 146 / 190 / 118 and 66 / 90 / 61 (about 40 of those are the
+// autograd engine's way to its own thread and back).
 #pragma once
 #include <torch/extension.h>
 #include <ATen/hip/EmptyTensor.h>

@@ -1,12 +1,14 @@
 // The pre-norm encoder and decoder layers in their plain form (modules/transformer_layers.py decides which calls that is) as
-// one autograd node each. The forward is called in pieces: the attention core of the self-attention is the Python stand-in
-// flash_attn_cuda.fwd_batched, called between them; the backward runs here from end to end.
+// one autograd node each. The forward is called in pieces: the attention core of the self-attention is called between them
+// through its Python name, flash_attn_cuda.fwd_batched (which comes back to flash_fwd_batched here); the backward runs from end
+// to end.
 //
 // What the composition of single operators paid for and this does not: an autograd node, its saved tensors and an
 // interpreter round trip per operator; the additions and copies autograd makes to sum the two gradients of every residual
 // stream (the LayerNorm backward adds the stream's gradient to its own); a pass of its own for every
 // residual addition (the next LayerNorm makes it on the way in); two reductions and two host synchronisations per layer for
-// the clamp of non-finite values. Encoder layer [512 x 32 x 1024] bf16, forward + backward: 53 launches before, 29 now.
+// the clamp of non-finite values. Encoder layer [512 x 32 x 1024] bf16, forward + backward: 53 launches before, 33 now, six of
+// them reductions of products too large to carry them (28 at [37 x 13 x 512]).
 #include "host.h"
 
 namespace nmtg_host {
