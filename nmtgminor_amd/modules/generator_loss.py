@@ -236,8 +236,10 @@ class GeneratorLoss(nn.Module):
         else:
             smoothing = self.label_smoothing if self.training else 0.0
             w, c = self.linear.weight, self.linear.bias
-            kept = L.host().generator_loss(h, w, c, y, float(smoothing), int(self.padding_idx), DEFAULT_KEEP_LOGITS_BYTES) \
-                if h.is_cuda and not L.tracing() else None
+            kept = None
+            if h.is_cuda and self.chunk_rows > 0 and not L.tracing():
+                pad = xentropy_cuda.NO_PADDING if self.padding_idx is None else int(self.padding_idx)
+                kept = L.host().generator_loss(h, w, c, y, float(smoothing), pad, DEFAULT_KEEP_LOGITS_BYTES)
             if kept is not None:
                 rows, total_loss = kept
                 if sum_loss and not loss_constraint and loss_weights is None:

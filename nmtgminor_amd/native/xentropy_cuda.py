@@ -13,7 +13,7 @@ from .. import _lib as L
 
 __version__ = "0.1"
 
-_NO_PAD = -(1 << 63)
+NO_PADDING = -(1 << 63)          # no label is this one
 
 
 def _check(cond, msg):
@@ -44,7 +44,7 @@ def forward(logits, labels, smoothing, half_to_float=False, *, padding_idx=None,
     n, v = logits.shape
     losses = torch.empty(n, dtype=torch.float32, device=logits.device)
     lse = torch.empty(n, dtype=torch.float32, device=logits.device)
-    pad = L.i64(_NO_PAD if padding_idx is None else padding_idx)
+    pad = L.i64(NO_PADDING if padding_idx is None else padding_idx)
     best = None
     if want_argmax:
         best = torch.empty(n, dtype=torch.int64, device=logits.device)
@@ -83,7 +83,7 @@ def backward(grad_loss, logits, max_log_sum_exp, labels, smoothing, *, padding_i
     L.call("nmtg_xentropy_bwd", L.ptr(grad_loss), L.ptr(logits), L.ptr(lse), L.ptr(labels),
            L.ptr(grad_logits), L.i64(n), L.i64(v), L.i64(logits.stride(0)), L.i64(grad_logits.stride(0)),
            L.i64(class_offset), L.i64(v if total_classes is None else total_classes), L.f32(smoothing),
-           L.i64(_NO_PAD if padding_idx is None else padding_idx), L.i32(L.dtype_code(logits)), L.stream_of(logits))
+           L.i64(NO_PADDING if padding_idx is None else padding_idx), L.i32(L.dtype_code(logits)), L.stream_of(logits))
     return grad_logits
 
 
@@ -99,5 +99,5 @@ def backward_with_colsum(grad_loss, logits, lse, labels, smoothing, padding_idx,
     part = torch.empty(int(L.load().nmtg_xentropy_bwd_colsum_parts(L.i64(n))), v, dtype=torch.float32, device=logits.device)
     L.call("nmtg_xentropy_bwd_colsum", L.ptr(grad_loss), L.i64(int(grad_loss.numel() == n and n > 1)), L.ptr(logits), L.ptr(lse),
            L.ptr(labels), L.ptr(out), L.ptr(colsum), L.ptr(part), L.i64(n), L.i64(v), L.i64(logits.stride(0)), L.i64(out.stride(0)),
-           L.f32(smoothing), L.i64(_NO_PAD if padding_idx is None else padding_idx), L.i32(L.dtype_code(logits)), L.stream_of(logits))
+           L.f32(smoothing), L.i64(NO_PADDING if padding_idx is None else padding_idx), L.i32(L.dtype_code(logits)), L.stream_of(logits))
     return out, colsum

@@ -152,3 +152,20 @@ def test_argument_checks_and_empty_batch(dev):
     assert loss.shape == (0,)
     loss.sum().backward()
     assert hd.grad.shape == (0, 64) and float(wd.grad.abs().sum()) == 0.0
+
+
+def test_loss_without_a_padding_index_and_with_a_chunk_size_that_is_none(dev):
+    h, w, b, y, _ = _case(40, 64, 300, torch.bfloat16, True, 7)
+    m = GeneratorLoss(64, 300, label_smoothing=0.1, padding_idx=None).to(dev).to(torch.bfloat16).train()
+    with torch.no_grad():
+        m.linear.weight.copy_(w)
+        m.linear.bias.copy_(b)
+    x = h.to(dev).requires_grad_()
+    r = m(x, y.to(dev))
+    r["loss"].backward()
+    want = LinearSoftmaxCrossEntropy.apply(h.to(dev), w.to(dev), b.to(dev), y.to(dev), 0.1, None)
+    assert_close(r["loss"], want.double().sum().cpu(), torch.float32, "loss")
+    assert (want > 0).all() and x.grad.float().abs().sum(1).min().item() > 0          # every row counts
+    m.chunk_rows = 0
+    with pytest.raises(RuntimeError, match="chunk_rows must be positive"):
+        m(x, y.to(dev))
