@@ -72,8 +72,11 @@ class PrePostProcessing(nn.Module):
             return False
         if i > 0 and self.steps[i - 1] == "n":
             return False        # the LayerNorm output may be what its backward reads (memory-efficient form)
-        # autograd forbids writing into a view that a custom Function created itself (its backward would be bypassed)
-        if output.requires_grad and output._is_view() and isinstance(output.grad_fn, torch.autograd.function.BackwardCFunction):
+        # autograd forbids writing into a view that a custom Function created itself (its backward would be bypassed). The same
+        # training call without gradients, whose result names no Function, has to draw its mask in the same way: it may be the
+        # forward of a reentrant checkpoint, which is computed again with them
+        if output._is_view() and (isinstance(output.grad_fn, torch.autograd.function.BackwardCFunction)
+                                  or (self.training and not torch.is_grad_enabled())):
             return False
         return True
 

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from nmtgminor_amd import _lib as L
+from nmtgminor_amd.modules.pre_post_processing import PrePostProcessing
 from nmtgminor_amd.modules.transformer_layers import DecoderLayer, EncoderLayer
 
 
@@ -99,3 +100,24 @@ def test_hooks_on_every_module_and_replaced_functions_keep_the_layer_off_the_nat
                     setattr(m, function, plain)
         layer.postprocess_attn.dropout.p = 0.3
         assert not native()
+
+
+class _View(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x):
+        return (2 * x).view(2, 3, 4)
+
+    @staticmethod
+    def backward(ctx, g):
+        return 2 * g.view(24)
+
+
+def test_dropout_and_add_draw_alike_with_and_without_gradients():
+    """The forward of a reentrant checkpoint runs without gradients and its recomputation with them: a result that is a view of an
+    autograd function's own tensor takes torch's dropout in both."""
+    post = PrePostProcessing(4, 0.5, sequence="da").train()
+    x, residual = torch.ones(24, requires_grad=True), torch.zeros(2, 3, 4)
+    with_gradients = post._fusable(0, _View.apply(x), residual)
+    with torch.no_grad():
+        assert post._fusable(0, _View.apply(x), residual) is with_gradients is False
+        assert post._fusable(0, _View.apply(x).clone(), residual) is post.eval()._fusable(0, _View.apply(x), residual) is True

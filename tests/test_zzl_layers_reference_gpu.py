@@ -5,6 +5,7 @@ from types import SimpleNamespace
 
 import pytest
 import torch
+from torch.utils.checkpoint import checkpoint
 
 from nmtgminor_amd.modules.encdec_attention_func import encdec_attn_func
 from nmtgminor_amd.modules.generator_loss import GeneratorLoss
@@ -184,6 +185,39 @@ def test_another_stream(dev):
             torch.cuda.synchronize()
             for name in want:
                 assert torch.equal(got[name], want[name]), name
+
+
+@pytest.mark.parametrize("reentrant", [True, False])
+def test_a_checkpointed_layer(dev, reentrant):
+    """The recomputation draws the masks of the forward. (The reentrant form runs its forward without gradients, where a training
+    layer goes operator by operator: the same masks, other roundings.)"""
+    for layer, inputs, masks in both_layers(dev, 0.1):
+        def run(x):
+            out = layer(x, *inputs[1:], *masks)
+            return out[0] if isinstance(out, tuple) else out
+        res = []
+        for call in (run, lambda x: checkpoint(run, x, use_reentrant=reentrant)):
+            torch.manual_seed(3)
+            torch.cuda.manual_seed(5)
+            x = inputs[0].clone().requires_grad_()
+            y = call(x)
+            y.backward(inputs[0])
+            res.append((y.detach(), x.grad, *(p.grad.clone() for p in layer.parameters())))
+            layer.zero_grad()
+        for want, got in zip(*res):
+            if reentrant:
+                compare("checkpointed", got, want, F16)
+            else:
+                assert torch.equal(got, want)
+
+
+def test_saved_tensors_kept_on_the_host(dev):
+    for layer, inputs, masks in both_layers(dev, 0.1):
+        dy = torch.randn_like(inputs[0])
+        want = passes(dev, layer, inputs, masks, dy, lambda n: True)
+        with torch.autograd.graph.save_on_cpu():
+            got = passes(dev, layer, inputs, masks, dy, lambda n: True)
+        assert all(torch.equal(got[n], want[n]) for n in want)
 
 
 def test_an_evaluation_in_a_captured_graph(dev):
