@@ -185,7 +185,7 @@ void define_autograd(pybind11::module_& m) {
       }
     const bool grad = at::GradMode::is_enabled() && (x.requires_grad() || w1.requires_grad() || w2.requires_grad() ||
                                                      (b1 && b1->requires_grad()) || (b2 && b2->requires_grad()));
-    const bool dual = has_tangent(x) || has_tangent(w1) || has_tangent(w2) || has_tangent(saved(b[0])) || has_tangent(saved(b[1]));
+    const bool dual = forward_mode() && (has_tangent(x) || has_tangent(w1) || has_tangent(w2) || has_tangent(saved(b[0])) || has_tangent(saved(b[1])));
     if (!grad && !dual)                              // nothing will be back-propagated: the pre-activations are not written
       return mlp_fwd(contiguous(x), contiguous(w1), contiguous(w2), saved(b[0]), saved(b[1]), p, act, mask, false).out;
     return MlpNode::apply(contiguous(x), contiguous(w1), contiguous(w2), b[0], b[1], mask, p, act);

@@ -9,6 +9,7 @@
 // autograd engine's way to its own thread and back).
 #pragma once
 #include <torch/extension.h>
+#include <torch/csrc/autograd/forward_grad.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/CPUAllocator.h>
 #include <c10/core/DeviceGuard.h>
@@ -61,7 +62,9 @@ void check(int rc, const char* what);
 int dtype_code(const Tensor& t);
 inline void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 inline void* ptr(const optional<Tensor>& t) { return t.has_value() ? ptr(*t) : nullptr; }
-// A forward-mode dual: its tangent would be lost where the autograd node is passed by (the node itself refuses it).
+// A forward-mode dual: its tangent would be lost where the autograd node is passed by (the node itself refuses it). Duals exist
+// while a level is open, which is asked first: a look at one tensor takes a lock of its own.
+inline bool forward_mode() { return torch::autograd::ForwardADLevel::try_get_by_idx(0) != nullptr; }
 inline bool has_tangent(const Tensor& t) { return t.defined() && t._fw_grad(/*level=*/0).defined(); }
 inline Tensor contiguous(const Tensor& t) { return t.is_contiguous() ? t : t.contiguous(); }
 // Results. A small batch is bound by this host work, and a layer's pass makes some 60 tensors: the allocator's own entry

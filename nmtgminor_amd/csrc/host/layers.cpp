@@ -296,14 +296,15 @@ void define_layers(pybind11::module_& m) {
   // What the layers ask before they take this path: 0 = no (a parameter of another type, shape, layout or device, or none, or a
   // forward-mode tangent anywhere), 1 = yes, nothing will be back-propagated, 2 = yes, with gradients.
   m.def("layer_mode", [](const Tensor& x, const std::vector<optional<Tensor>>& inputs, const std::vector<optional<Tensor>>& params) {
+    const bool forward = forward_mode();
     if (!x.is_cuda() || x.dim() != 3 || x.numel() == 0 || (x.scalar_type() != at::kHalf && x.scalar_type() != at::kBFloat16) ||
-        has_tangent(x))
+        (forward && has_tangent(x)))
       return 0;
     bool grad = x.requires_grad();
     for (const auto* list : {&inputs, &params})
       for (const auto& p : *list) {
         if (!p.has_value() || !p->defined() || p->device() != x.device() || p->scalar_type() != x.scalar_type() || !p->is_contiguous() ||
-            has_tangent(*p))
+            (forward && has_tangent(*p)))
           return 0;
         grad = grad || p->requires_grad();
       }
