@@ -9,7 +9,8 @@
 //   lane's accumulators, so the running maximum and sum of the online softmax are per-lane scalars;
 //   the probabilities are rounded to the 16-bit type, moved from accumulator to operand layout with two
 //   v_permlane32_swap per 16 keys, and multiplied with V^T, read from LDS with the transposing read.
-// Backward, two kernels with the same tiling, both recomputing S from Q, K and the saved log-sum-exp:
+// Backward, recomputing S from Q, K and the saved log-sum-exp: one kernel for sequences of up to 512 positions
+// (flash_bwd_kernel), otherwise two with the forward's tiling:
 //   dQ kernel  (block = 128 queries, loop over key tiles): D = rowsum(dO * O), dP^T = V dO^T, dS = P (dP - D),
 //              dQ^T += K^T dS^T;
 //   dK/dV kernel (block = 128 keys, loop over query tiles of 64): the mirror image with one key per lane pair:
@@ -26,7 +27,7 @@
 // key's word per group of queries and tests bits. An explicit byte mask is turned into the same words, and so are the
 // decisions of the extension modules' numbering (mode 3: element (i, j) uses word e % 4 of the Philox block e / 4,
 // e = ((b H + h) max_q + i) max_k + j, and is kept when word / 2^32 < 1 - p), for calls that return the probabilities.
-#include "gemm.hip.h"
+#include "gemm_ring.hip.h"
 
 namespace nmtg {
 namespace {
@@ -1045,6 +1046,375 @@ __global__ __launch_bounds__(FA_THREADS, D == 64 ? 2 : 1) void flash_bwd_dkv_ker
 }
 
 // -------------------------------------------------------------------------------------------------------------------
+// backward of short sequences: dQ, dK and dV in one kernel, one block per (sequence, head)
+// -------------------------------------------------------------------------------------------------------------------
+// NW wavefronts hold all the sequence's keys (at most 64 NW), two groups of 32 each: group `wave` and group `wave + NW`, so
+// that a short sequence leaves every wavefront something. The dK / dV accumulators of the 64 keys and their V operands
+// stay in registers, the keys in one LDS image that is read both by rows (S = Q K^T) and transposed (dQ^T = K^T dS^T).
+// Queries come in steps of 32: the scores, exponentials and dP of the step are computed once, dS goes through LDS as
+// [key][query], and behind a barrier the wavefronts share out dQ's 64 x 32 results as eight 16 x 16 tiles that each sum
+// over all keys (v_mfma_f32_16x16x32): nothing is added up between wavefronts, no atomics, results do not depend on
+// scheduling. The two kernels make scores, exponentials and dP twice each: [512 x 512], 512 heads in bf16 with dropout 205 us
+// (91 + 114), here 152; [256 x 256] 78 and 50; [61 x 73], 384 heads 20 and 14. What bounds it: nothing alone. Vector instructions are 45 %
+// of the time, LDS reads 30 %, MFMA 22 %, with two wavefronts per SIMD to overlap them (all 256 registers are taken: 128 of
+// accumulators, 32 of V, 32 of scores).
+// Images of 128-byte rows: chunk c of row r at c ^ fb_swz(r). LDS serves 256 bytes per clock from 64 banks, so 16 lanes of a
+// row read (16 rows, one chunk) and 32 lanes of a transposing read (4 rows x 64 bytes for the 32 x 32 operands, 8 rows x 32
+// bytes for the 16 x 16 ones) must not meet: even and odd rows lie in different halves, rows that differ in bit 1 must
+// differ by four chunks, in bits 2 and 3 by one and two.
+constexpr int FB_STEP = 32;                      // queries per step
+constexpr int FB_QIMG = FB_STEP * 128;           // Q or dO of a step
+constexpr int FB_MAX_Q = 512;                    // the statistics of every query lie in LDS
+template <int NW> constexpr int fb_ds_images() { return NW == 8 ? 2 : 1; }
+template <int NW> constexpr int fb_lds(int max_q) {
+  return 64 * NW * 128 + fb_ds_images<NW>() * 64 * NW * FB_STEP * 2 + 4 * FB_QIMG + 2 * 4 * ((max_q + FB_STEP - 1) / FB_STEP * FB_STEP);
+}
+__device__ __forceinline__ int fb_swz(int r) { return ((r & 2) << 1) | ((r >> 2) & 1) | ((r >> 2) & 2); }
+
+typedef float acc4_t __attribute__((ext_vector_type(4)));
+template <typename T> __device__ __forceinline__ void mfma16(const uint4& a, const uint4& b, acc4_t& c);
+template <> __device__ __forceinline__ void mfma16<f16_t>(const uint4& a, const uint4& b, acc4_t& c) {
+  c = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(mfma<f16_t>::vec, a), __builtin_bit_cast(mfma<f16_t>::vec, b), c, 0, 0, 0);
+}
+template <> __device__ __forceinline__ void mfma16<bf16_t>(const uint4& a, const uint4& b, acc4_t& c) {
+  c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(mfma<bf16_t>::vec, a), __builtin_bit_cast(mfma<bf16_t>::vec, b), c, 0, 0, 0);
+}
+// two transposing reads as one operand: rows at `lo` are elements 0..3, rows at `hi` elements 4..7
+__device__ __forceinline__ uint4 read_tr_pair(const uint8_t* lo, const uint8_t* hi) {
+  union { s16x4_t s[2]; uint4 u; } cv;
+  cv.s[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(lo));
+  cv.s[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(hi));
+  return cv.u;
+}
+
+// TM: the call has a time mask; without it none of that code is compiled in.
+template <typename T, int DROP, int TM, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void flash_bwd_kernel(FaArgs a) {
+  constexpr int D = 64, CH = D / 8, NT = 64 * NW, NDS = fb_ds_images<NW>();
+  constexpr int KIMG = 64 * NW * 128, DSIMG = 64 * NW * FB_STEP * 2;
+  extern __shared__ __align__(16) uint8_t lds_raw[];
+  uint8_t* const kimg = lds_raw;
+  uint8_t* const ds_images = lds_raw + KIMG;
+  uint8_t* const q_images = ds_images + NDS * DSIMG;          // two of Q, dO
+  float* const lse2s = reinterpret_cast<float*>(q_images + 4 * FB_QIMG);
+  float* const deltas = lse2s + (a.max_q + FB_STEP - 1) / FB_STEP * FB_STEP;
+  const int h = blockIdx.x, b = blockIdx.y, bh = b * a.heads + h;
+  const SeqSpan sp = seq_span(a, b);
+  const int qs = sp.qs, lq = sp.lq, ks = sp.ks, lk = sp.lk;
+  const int lk_out = a.cu_q != nullptr ? lk : a.max_k;      // rows of dK / dV to write, see flash_bwd_dkv_kernel
+  const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const T* qb = static_cast<const T*>(a.q) + static_cast<int64_t>(qs) * a.q_st + static_cast<int64_t>(b) * a.q_sb + static_cast<int64_t>(h) * a.q_sh;
+  const T* gb = static_cast<const T*>(a.d_o) + static_cast<int64_t>(qs) * a.do_st + static_cast<int64_t>(b) * a.do_sb + static_cast<int64_t>(h) * a.do_sh;
+  T* dqb = static_cast<T*>(a.dq) + static_cast<int64_t>(qs) * a.dq_st + static_cast<int64_t>(b) * a.dq_sb + static_cast<int64_t>(h) * a.dq_sh;
+  const int nsteps = (lq + FB_STEP - 1) / FB_STEP, groups = (lk + 31) / 32;
+
+  // The registers are full: what is cheap to make again from the lane is not kept across the loop (the compiler would move it
+  // out of the loop and then to scratch, whose reloads wait behind the transfers).
+  auto again = [&]() {
+    int l = lane;
+    asm volatile("" : "+v"(l));
+    return l;
+  };
+  // A step's rows come by direct transfers of 8 rows: four of Q, four of dO, dealt out to the wavefronts; rows past the end
+  // repeat the last one and are cleared when they have landed.
+  constexpr int TPW = 8 / NW;   // transfers (and tiles of dQ) per wavefront
+  const uint32_t q_lds = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(q_images)));
+  auto request = [&](int t) {
+    const int lane = again();
+#pragma unroll
+    for (int i = 0; i < TPW; ++i) {
+      const int x = wave * TPW + i, r = 8 * (x & 3) + (lane >> 3);
+      const int64_t stride = x < 4 ? a.q_st : a.do_st;
+      const T* base = (x < 4 ? qb : gb) + static_cast<int64_t>(FB_STEP * t) * stride;
+      const uint32_t off = static_cast<uint32_t>(min(r, lq - FB_STEP * t - 1)) * static_cast<uint32_t>(stride * 2) +
+                           static_cast<uint32_t>(((lane & 7) ^ fb_swz(r)) * 16);
+      dma16(off, base, q_lds + static_cast<uint32_t>((t & 1) * 2 * FB_QIMG + x * 1024));
+    }
+  };
+  auto landed = [&](int t) {
+    const int left = lq - FB_STEP * t;
+    if (left < FB_STEP) {
+      const int lane = again();
+#pragma unroll
+      for (int i = 0; i < TPW; ++i) {
+        const int x = wave * TPW + i;
+        if (8 * (x & 3) + (lane >> 3) >= left)
+          *reinterpret_cast<uint4*>(q_images + (t & 1) * 2 * FB_QIMG + x * 1024 + lane * 16) = make_uint4(0, 0, 0, 0);
+      }
+    }
+  };
+  if (nsteps > 0) request(0);
+
+  // the keys of the whole sequence (rows past its end are zeros) and the V operands of this wavefront's two groups
+  int krow[2];
+  bool kdead[2], group_dead[2];
+  uint4 vf[2][D / 16];
+  acc16_t dk[2][D / 32], dv[2][D / 32];
+  {
+    const T* kb = static_cast<const T*>(a.k) + static_cast<int64_t>(ks) * a.k_st + static_cast<int64_t>(b) * a.k_sb + static_cast<int64_t>(h) * a.k_sh;
+    const T* vb = static_cast<const T*>(a.v) + static_cast<int64_t>(ks) * a.v_st + static_cast<int64_t>(b) * a.v_sb + static_cast<int64_t>(h) * a.v_sh;
+    uint4 kv[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = (tid + NT * i) / CH, c = tid % CH;
+      kv[i] = make_uint4(0, 0, 0, 0);
+      if (r < lk) kv[i] = *reinterpret_cast<const uint4*>(kb + static_cast<int64_t>(r) * a.k_st + 8 * c);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = (tid + NT * i) / CH, c = tid % CH;
+      *reinterpret_cast<uint4*>(kimg + r * 128 + ((c ^ fb_swz(r)) * 16)) = kv[i];
+    }
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      krow[g] = 32 * (wave + NW * g) + (lane & 31);
+      kdead[g] = krow[g] >= lk || (a.pad != nullptr && a.pad[static_cast<int64_t>(b) * a.max_k + krow[g]] != 0);
+      group_dead[g] = __builtin_amdgcn_ballot_w64(kdead[g]) != 0;
+      load_resident<T, D>(vf[g], vb, a.v_st, krow[g], lk, lane);
+#pragma unroll
+      for (int i = 0; i < D / 32; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) { dk[g][i][r] = 0.f; dv[g][i][r] = 0.f; }
+    }
+  }
+  // D = rowsum(dO * O) and the log-sum-exp in units of log2; a row without a live key (or past the end) gets the large value
+  // that makes its probabilities zero. Eight lanes per row.
+  {
+    const T* ob = static_cast<const T*>(a.o) + static_cast<int64_t>(qs) * a.o_st + static_cast<int64_t>(b) * a.o_sb + static_cast<int64_t>(h) * a.o_sh;
+    const int c = tid & 7;
+    for (int row0 = tid >> 3; row0 < FB_STEP * nsteps; row0 += 4 * (NT / 8)) {
+      uint4 x[4], y[4];
+      float lse[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = row0 + i * (NT / 8);
+        x[i] = y[i] = make_uint4(0, 0, 0, 0);
+        lse[i] = -INFINITY;
+        if (row < lq) {
+          x[i] = *reinterpret_cast<const uint4*>(ob + static_cast<int64_t>(row) * a.o_st + 8 * c);
+          y[i] = *reinterpret_cast<const uint4*>(gb + static_cast<int64_t>(row) * a.do_st + 8 * c);
+          lse[i] = a.lse[static_cast<int64_t>(bh) * a.max_q + row];
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = row0 + i * (NT / 8);
+        const T *xe = reinterpret_cast<const T*>(&x[i]), *ye = reinterpret_cast<const T*>(&y[i]);
+        float sum = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sum += elem<T>::to_float(xe[e]) * elem<T>::to_float(ye[e]);
+        for (int off = 1; off < 8; off *= 2) sum += __shfl_xor(sum, off, 64);
+        if (c == 0 && row < FB_STEP * nsteps) {
+          deltas[row] = sum;
+          lse2s[row] = lse[i] == -INFINITY ? -FA_NEG : lse[i] * FA_LOG2E;
+          if (row < lq) a.delta[static_cast<int64_t>(bh) * a.max_q + row] = sum;
+        }
+      }
+    }
+  }
+  // keep bits of the two keys for a step's queries, and their packed time-mask words: one step ahead, like the tile itself
+  [[maybe_unused]] uint32_t keep_next[2] = {0, 0}, tdead_next[2] = {0, 0};
+  auto load_words = [&](int t) {
+    const int lane = again();
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const int key = 32 * (wave + NW * g) + (lane & 31);
+      if constexpr (DROP != 0) {
+        const uint32_t* row = a.bits + (static_cast<int64_t>(bh) * a.q32 + t) * a.kp;
+        if (key < lk) keep_next[g] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(row) + 4u * static_cast<uint32_t>(bit_slot(key)));
+      }
+      if constexpr (TM != 0)
+        tdead_next[g] = a.tk_bits[(static_cast<int64_t>(min(key, a.max_k - 1)) * a.query_tiles + t / 2) * 2 + (lane >> 5)];
+    }
+  };
+  // Lane t keeps what step t asks for by scalar (there are at most FB_MAX_Q / 32 steps): the number of key groups that some query
+  // of the step sees, and whether the time mask hides any of the wavefront's groups. Loads of such values inside the loop
+  // would be vector loads behind the transfers.
+  int live_at = groups, masked_at = 0;
+  if (a.causal) live_at = min(live_at, lane + 1);
+  if constexpr (TM != 0) {
+    const int t = min(lane, nsteps - 1), last = (a.max_k + 31) / 32 - 1;
+    if (nsteps > 0) {
+      live_at = min(live_at, 2 * a.qinfo[static_cast<int64_t>(t) * a.qinfo_pitch]);
+      for (int g = 0; g < 2; ++g)
+        masked_at |= (a.kqinfo[static_cast<int64_t>(min(wave + NW * g, last)) * a.kqinfo_pitch + 2 + t / 2] != 0 ? 1 : 0) << g;
+    }
+  }
+  auto live_groups = [&](int t) { return __builtin_amdgcn_readlane(live_at, t); };
+
+  const float dead_raw = FA_NEG / a.scale_log2;   // the raw score that the scale turns into -1e30
+  // lane offsets of the transposed 32 x 32 read (columns 32 i .., rows 16 kk + 8 half + tr_r and + 4)
+  uint32_t tr_lo[2], tr_hi[2];
+  const int tr_r = (lane >> 2) & 3;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int r = 8 * half + tr_r, c = 4 * i + 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1);
+    tr_lo[i] = static_cast<uint32_t>(r * 128 + ((c ^ fb_swz(r)) * 16) + (lane & 1) * 8);
+    tr_hi[i] = static_cast<uint32_t>((r + 4) * 128 + ((c ^ fb_swz(r + 4)) * 16) + (lane & 1) * 8);
+  }
+
+  // dQ^T of a step: tile `id` is columns 16 (id % 4) .. of queries 16 (id / 4) ..; lane (query, four columns)
+  auto dq_tile = [&](int id, const uint8_t* ds, int live) {
+    const int lane = again();
+    const int r = 8 * (lane >> 4) + ((lane >> 2) & 3), in = (lane & 1) * 8;
+    const int kc = 2 * (id & 3) + ((lane >> 1) & 1), qc = 2 * (id >> 2) + ((lane >> 1) & 1);
+    const uint8_t* k_lo = kimg + r * 128 + ((kc ^ fb_swz(r)) * 16) + in;
+    const uint8_t* k_hi = kimg + (r + 4) * 128 + ((kc ^ fb_swz(r + 4)) * 16) + in;
+    const uint8_t* s_lo = ds + r * 64 + ((qc ^ ((r >> 2) & 3)) * 16) + in;
+    const uint8_t* s_hi = ds + (r + 4) * 64 + ((qc ^ (((r + 4) >> 2) & 3)) * 16) + in;
+    acc4_t z[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    int n = 0;
+    for (; n + 4 <= live; n += 4) {
+      uint4 kf[4], sf[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        kf[u] = read_tr_pair(k_lo + u * 4096, k_hi + u * 4096);
+        sf[u] = read_tr_pair(s_lo + u * 2048, s_hi + u * 2048);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) mfma16<T>(kf[u], sf[u], z[u & 1]);
+      k_lo += 4 * 4096; k_hi += 4 * 4096; s_lo += 4 * 2048; s_hi += 4 * 2048;
+    }
+    for (; n < live; ++n) {
+      mfma16<T>(read_tr_pair(k_lo, k_hi), read_tr_pair(s_lo, s_hi), z[0]);
+      k_lo += 4096; k_hi += 4096; s_lo += 2048; s_hi += 2048;
+    }
+    uint2 w;
+    w.x = pack2<T>((z[0][0] + z[1][0]) * a.scale, (z[0][1] + z[1][1]) * a.scale);
+    w.y = pack2<T>((z[0][2] + z[1][2]) * a.scale, (z[0][3] + z[1][3]) * a.scale);
+    return w;
+  };
+  auto dq_store = [&](int id, int t, const uint2& w) {
+    const int lane = again();
+    char* base = reinterpret_cast<char*>(dqb + static_cast<int64_t>(FB_STEP * t + 16 * (id >> 2)) * a.dq_st + 16 * (id & 3));
+    if ((lane & 15) < lq - FB_STEP * t - 16 * (id >> 2))
+      *reinterpret_cast<uint2*>(base + (static_cast<uint32_t>(lane & 15) * static_cast<uint32_t>(a.dq_st * 2) + 8u * static_cast<uint32_t>(lane >> 4))) = w;
+  };
+
+  // scores, probabilities, dS of a step for the wavefront's two groups; dS into LDS, dV and dK accumulated
+  auto compute = [&](int t, uint8_t* ds, int live) {
+    const uint8_t* const qimg = q_images + (t & 1) * 2 * FB_QIMG;
+    const uint8_t* const gimg = qimg + FB_QIMG;
+    [[maybe_unused]] const uint32_t keep[2] = {keep_next[0], keep_next[1]}, tdead[2] = {tdead_next[0], tdead_next[1]};
+    if (t + 1 < nsteps) load_words(t + 1);
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const int group = wave + NW * g;
+      if (group >= live) continue;
+      const uint8_t* krows = kimg + group * 32 * 128;
+      const int lane = again();
+      acc16_t s, dp;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) { s[r] = 0.f; dp[r] = 0.f; }
+#pragma unroll
+      for (int ss = 0; ss < D / 16; ++ss) {
+        const uint32_t at = static_cast<uint32_t>((lane & 31) * 128 + (((2 * ss + half) ^ fb_swz(lane & 31)) * 16));
+        mfma<T>::run(*reinterpret_cast<const uint4*>(qimg + at), *reinterpret_cast<const uint4*>(krows + at), s);
+        mfma<T>::run(*reinterpret_cast<const uint4*>(gimg + at), vf[g][ss], dp);
+      }
+      // s[r], dp[r]: query 8 (r / 4) + 4 half + r % 4 of the step, key krow[g]
+      // One bit per register, then a select each. (With the conditions written out per element, short-circuited, the compiler
+      // branched around each of them and lost the write of one of the paths.)
+      bool tmt = false;
+      if constexpr (TM != 0) tmt = ((__builtin_amdgcn_readlane(masked_at, t) >> g) & 1) != 0;
+      const bool diagonal = a.causal != 0 && group == t;
+      if (group_dead[g] || diagonal || tmt) {
+        uint32_t dead = kdead[g] ? 0xffffu : 0u;
+        if constexpr (TM != 0) dead |= tdead[g] >> (16 * (t & 1));
+        if (diagonal) {   // the registers whose query 8 (r / 4) + 4 half + r % 4 comes before the lane's key: the first n
+          const int x = max((lane & 31) - 4 * half, 0);
+          dead |= (1u << (4 * (x >> 3) + min(x & 7, 4))) - 1u;
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = ((dead >> r) & 1u) != 0 ? dead_raw : s[r];
+      }
+      [[maybe_unused]] const uint32_t kbits = DROP != 0 ? keep[g] >> (4 * half) : 0;   // bit 8 q + c is register 4 q + c
+      const float* const l_at = lse2s + FB_STEP * t + 4 * half;
+      const float* const d_at = deltas + FB_STEP * t + 4 * half;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float4 l4 = *reinterpret_cast<const float4*>(l_at + 8 * q);
+        const float4 d4 = *reinterpret_cast<const float4*>(d_at + 8 * q);
+        const float lse2[4] = {l4.x, l4.y, l4.z, l4.w}, dl[4] = {d4.x, d4.y, d4.z, d4.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int r = 4 * q + e;
+          const float pr = fast_exp2(__builtin_fmaf(s[r], a.scale_log2, -lse2[e]));
+          // all ones where the element is kept
+          const uint32_t kept = DROP != 0 ? static_cast<uint32_t>(static_cast<int32_t>(kbits << (31 - (8 * q + e))) >> 31) : ~0u;
+          const float kscale = DROP != 0 ? __uint_as_float(__float_as_uint(a.drop_scale) & kept) : 1.f;
+          s[r] = pr * __builtin_fmaf(dp[r], kscale, -dl[e]);   // dS
+          dp[r] = __uint_as_float(__float_as_uint(pr) & kept); // kept probabilities; their scale waits for the end
+        }
+      }
+      uint8_t* const ds_row = ds + (32 * group + (lane & 31)) * (2 * FB_STEP);
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {
+        float pv[8], dsv[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) { pv[e] = dp[8 * kk + e]; dsv[e] = s[8 * kk + e]; }
+        const uint4 pf = acc_to_operand<T>(pv), df = acc_to_operand<T>(dsv);
+        *reinterpret_cast<uint4*>(ds_row + (((2 * kk + half) ^ ((lane >> 2) & 3)) * 16)) = df;
+#pragma unroll
+        for (int i = 0; i < D / 32; ++i) {
+          mfma<T>::run(read_tr_pair(gimg + tr_lo[i] + kk * 2048, gimg + tr_hi[i] + kk * 2048), pf, dv[g][i]);
+          mfma<T>::run(read_tr_pair(qimg + tr_lo[i] + kk * 2048, qimg + tr_hi[i] + kk * 2048), df, dk[g][i]);
+        }
+      }
+    }
+  };
+
+  if (nsteps > 0) load_words(0);
+  wait_vmcnt<0>();   // on every path: or the wait for the V operands would be repeated inside the loop
+  if (nsteps > 0) landed(0);
+  ring_barrier();
+  if constexpr (NDS == 2) {
+    // One barrier per step. Between two barriers a wavefront owes dQ of the step before and the next step's own work, in
+    // any order: the two wavefronts of a SIMD take them in opposite order, so that one multiplies while the other is in
+    // its exponentials. The stores of the second kind wait for the next step (the wait for the transfers would include them).
+    const bool early = wave < NW / 2;
+    uint2 w = make_uint2(0, 0);
+    for (int t = 0; t < nsteps; ++t) {
+      if (t >= 2 && !early) dq_store(wave, t - 2, w);
+      if (t + 1 < nsteps) request(t + 1);
+      if (t >= 1 && early) dq_store(wave, t - 1, dq_tile(wave, ds_images + ((t - 1) & 1) * DSIMG, live_groups(t - 1)));
+      compute(t, ds_images + (t & 1) * DSIMG, live_groups(t));
+      if (t >= 1 && !early) w = dq_tile(wave, ds_images + ((t - 1) & 1) * DSIMG, live_groups(t - 1));
+      wait_vmcnt<0>();
+      if (t + 1 < nsteps) landed(t + 1);
+      ring_barrier();
+    }
+    if (nsteps >= 2 && !early) dq_store(wave, nsteps - 2, w);
+    if (nsteps >= 1) dq_store(wave, nsteps - 1, dq_tile(wave, ds_images + ((nsteps - 1) & 1) * DSIMG, live_groups(nsteps - 1)));
+  } else {
+    // One dS image and two barriers: the smaller block leaves room for a second one on the CU.
+    for (int t = 0; t < nsteps; ++t) {
+      const int live = live_groups(t);
+      if (t + 1 < nsteps) request(t + 1);
+      compute(t, ds_images, live);
+      wait_vmcnt<0>();
+      if (t + 1 < nsteps) landed(t + 1);
+      ring_barrier();
+#pragma unroll
+      for (int u = 0; u < TPW; ++u) dq_store(wave + NW * u, t, dq_tile(wave + NW * u, ds_images, live));
+      ring_barrier();
+    }
+  }
+  __syncthreads();   // every wavefront is done with the keys: the results leave through their image
+  T* dkb = static_cast<T*>(a.dk) + static_cast<int64_t>(ks) * a.dk_st + static_cast<int64_t>(b) * a.dk_sb + static_cast<int64_t>(h) * a.dk_sh;
+  T* dvb = static_cast<T*>(a.dv) + static_cast<int64_t>(ks) * a.dv_st + static_cast<int64_t>(b) * a.dv_sb + static_cast<int64_t>(h) * a.dv_sh;
+  uint8_t* patch = kimg + wave * (32 * D * 2);
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    store_rows_out<T, D>(dk[g], a.scale, patch, dkb, a.dk_st, 32 * (wave + NW * g), lk_out, lane);
+    __syncthreads();
+    store_rows_out<T, D>(dv[g], a.drop_scale, patch, dvb, a.dv_st, 32 * (wave + NW * g), lk_out, lane);
+    __syncthreads();
+  }
+}
+
+// -------------------------------------------------------------------------------------------------------------------
 // inference: probabilities and context in one kernel, two passes over the keys
 // -------------------------------------------------------------------------------------------------------------------
 // The reference's inference calls return the probabilities (its coverage), so they have to be written once; the scores
@@ -1531,6 +1901,37 @@ int fwd_launch(const FaArgs& a, int drop, dim3 grid, hipStream_t st) {
   return drop == 0 ? launch(flash_fwd_kernel<T, D, 0, 0>, "flash_attn_fwd", grid, fwd_lds<D>(), st, a)
                    : launch(flash_fwd_kernel<T, D, 1, 0>, "flash_attn_fwd", grid, fwd_lds<D>(), st, a);
 }
+// The kernel that makes all three gradients.
+template <typename T, int NW>
+int bwd_one_launch(const FaArgs& a, int drop, int64_t batch, hipStream_t st) {
+  TraceScope trace("flash_attn_bwd", st);
+  auto go = [&](auto kern) {
+    const int lds = fb_lds<NW>(a.max_q);
+    if (lds > 64 * 1024) {
+      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+      if (e != hipSuccess) return fail(NMTG_ERR_LAUNCH, "flash_attn_bwd: cannot reserve %d bytes of LDS: %s", lds, hipGetErrorString(e));
+    }
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(a.heads), static_cast<unsigned>(batch)), dim3(64 * NW), lds, st, a);
+    return 0;
+  };
+  if (a.tmask != nullptr) return drop == 0 ? go(flash_bwd_kernel<T, 0, 1, NW>) : go(flash_bwd_kernel<T, 1, 1, NW>);
+  return drop == 0 ? go(flash_bwd_kernel<T, 0, 0, NW>) : go(flash_bwd_kernel<T, 1, 0, NW>);
+}
+// Which calls take it: head dimension 64, keys that eight wavefronts hold, queries whose statistics fit the LDS, row strides
+// that 32-bit lane offsets reach over a step's rows. A block walks all queries of its head, so where queries are many and
+// heads few the two kernels' many short blocks are done first: [512 x 512], 64 / 128 / 192 / 256 heads: two kernels 53 / 67 / 101 /
+// 119 us, one 71 / 75 / 77 / 80; [512 x 128]: 39 / 44 / 52 / 58 against 42 / 46 / 49 / 49. With at most 256 queries the one kernel is
+// level or ahead at any number of heads ([128 x 512], 8 heads: 25 against 24; [256 x 256], 64 heads: 30 against 27; [256 x 64], 64
+// heads: 23 and 24).
+bool bwd_in_one(const FaArgs& a, int64_t batch, int64_t d) {
+  constexpr int64_t far = 1 << 25;
+  if (d != 64 || a.max_q <= 0 || a.max_k <= 0 || a.max_q > FB_MAX_Q || a.max_k > 512) return false;
+  if (a.q_st > far || a.do_st > far || a.dq_st > far) return false;
+  if (a.max_q > 256 && 5 * batch * a.heads < 3 * num_cus()) return false;
+  const char* off = getenv("NMTG_ATTN_BWD_ONE");
+  return off == nullptr || off[0] != '0';
+}
+
 template <typename T, int D>
 int bwd_launch(const FaArgs& a, int drop, dim3 grid_q, dim3 grid_k, hipStream_t st) {
   int rc = 0;
@@ -1631,6 +2032,19 @@ int bwd_run(const char* what, FaArgs& a, int64_t batch, int64_t d, int drop_mode
   const dim3 grid_k(static_cast<unsigned>((a.max_k + FA_ROWS - 1) / FA_ROWS), static_cast<unsigned>(a.heads), static_cast<unsigned>(batch));
   int rc = bits_launch(what, a, drop_mode, batch, bits, bits_ready, st);
   if (rc) return rc;
+  if (bwd_in_one(a, batch, d)) {
+    auto pick = [&](auto t) {
+      using T = decltype(t);
+      // Four wavefronts hold up to 256 keys, and two such blocks share a CU; while the heads do not fill the CUs twice eight
+      // wavefronts of one group each are done sooner ([256 x 256]: 512 heads 50 us with four and 57 with eight, 256 heads 38 and 33).
+      const int four = a.heads * batch > num_cus() ? 256 : 128;
+      return a.max_k <= four ? bwd_one_launch<T, 4>(a, drop_mode, batch, st) : bwd_one_launch<T, 8>(a, drop_mode, batch, st);
+    };
+    rc = dtype == NMTG_F16 ? pick(f16_t{}) : pick(bf16_t{});
+    if (rc) return rc;
+    NMTG_CHECK_LAUNCH(what);
+    return 0;
+  }
   if (dtype == NMTG_F16) rc = d == 64 ? bwd_launch<f16_t, 64>(a, drop_mode, grid_q, grid_k, st) : bwd_launch<f16_t, 128>(a, drop_mode, grid_q, grid_k, st);
   else rc = d == 64 ? bwd_launch<bf16_t, 64>(a, drop_mode, grid_q, grid_k, st) : bwd_launch<bf16_t, 128>(a, drop_mode, grid_q, grid_k, st);
   if (rc) return rc;

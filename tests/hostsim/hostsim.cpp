@@ -278,6 +278,19 @@ uint64_t shfl_xor_bits(uint64_t bits, int mask) {
   return s.bits;
 }
 
+struct ReadLane { uint32_t bits; int lane; };
+static void resolve_readlane(void** payloads, int lanes) {
+  const int from = static_cast<ReadLane*>(payloads[0])->lane;
+  if (from < 0 || from >= lanes) fail("v_readlane of a lane outside the wavefront");
+  const uint32_t bits = static_cast<ReadLane*>(payloads[from])->bits;
+  for (int l = 0; l < lanes; ++l) static_cast<ReadLane*>(payloads[l])->bits = bits;
+}
+uint32_t readlane_bits(uint32_t bits, int lane) {
+  ReadLane r{bits, lane};
+  wave_collective(resolve_readlane, &r);
+  return r.bits;
+}
+
 void dma_issue(const void* src, uint32_t lds_offset, int bytes) {
   const Transfer t{src, lds_offset, bytes};
   if (dma_early) land(t);
@@ -341,6 +354,28 @@ static void resolve_mfma(void** payloads, int lanes) {
     }
   }
 }
+template <bool BF16>
+static void resolve_mfma16(void** payloads, int lanes) {
+  if (lanes != 64) fail("MFMA in a partial wavefront");
+  float A[16][32], B[32][16];
+  for (int l = 0; l < 64; ++l) {
+    const Mfma* m = static_cast<const Mfma*>(payloads[l]);
+    for (int t = 0; t < 8; ++t) {
+      A[l & 15][8 * (l >> 4) + t] = widen<BF16>(m->a[t]);
+      B[8 * (l >> 4) + t][l & 15] = widen<BF16>(m->b[t]);
+    }
+  }
+  for (int l = 0; l < 64; ++l) {
+    float* c = static_cast<Mfma*>(payloads[l])->c;
+    for (int r = 0; r < 4; ++r) {
+      float s = c[r];
+      for (int k = 0; k < 32; ++k) s += A[4 * (l >> 4) + r][k] * B[k][l & 15];
+      c[r] = s;
+    }
+  }
+}
+void resolve_mfma16_f16(void** payloads, int lanes) { resolve_mfma16<false>(payloads, lanes); }
+void resolve_mfma16_bf16(void** payloads, int lanes) { resolve_mfma16<true>(payloads, lanes); }
 // v_mfma_f32_32x32x2_f32: lane l holds A[l & 31][l >> 5] and B[l >> 5][l & 31]
 void resolve_mfma_f32(void** payloads, int lanes) {
   if (lanes != 64) fail("MFMA in a partial wavefront");

@@ -50,6 +50,7 @@ void wave_collective(Resolver resolver, void* payload);
 [[noreturn]] void fail(const char* what);
 unsigned lane_id();
 uint64_t shfl_xor_bits(uint64_t bits, int mask);
+uint32_t readlane_bits(uint32_t bits, int lane);
 uint64_t gather_bits(uint64_t bits, int source_lane);   // every lane names the lane whose value it reads
 void sync_block();
 // direct global -> LDS transfers (asynchronous; see hostsim.cpp for the two timing models)
@@ -238,4 +239,30 @@ static inline hostsim_float16 __builtin_amdgcn_mfma_f32_32x32x16_f16(hostsim_hal
 }
 static inline hostsim_float16 __builtin_amdgcn_mfma_f32_32x32x16_bf16(hostsim_bf16x8 a, hostsim_bf16x8 b, hostsim_float16 c, int, int, int) {
   return hostsim::mfma<true>(a, b, c);
+}
+// v_mfma_f32_16x16x32_{f16,bf16}: 16 x 16 x 32. Lane l holds A[l & 15][8 (l >> 4) + t] and B[8 (l >> 4) + t][l & 15] for
+// t = 0..7, and D[4 (l >> 4) + r][l & 15] in accumulator register r = 0..3.
+typedef float hostsim_float4 __attribute__((ext_vector_type(4)));
+namespace hostsim {
+void resolve_mfma16_f16(void** payloads, int lanes);
+void resolve_mfma16_bf16(void** payloads, int lanes);
+template <bool BF16, typename V>
+static inline hostsim_float4 mfma16(V a, V b, hostsim_float4 c) {
+  uint16_t av[8], bv[8];
+  float cv[4];
+  std::memcpy(av, &a, 16);
+  std::memcpy(bv, &b, 16);
+  std::memcpy(cv, &c, 16);
+  Mfma m{av, bv, cv};
+  wave_collective(BF16 ? resolve_mfma16_bf16 : resolve_mfma16_f16, &m);
+  hostsim_float4 d;
+  std::memcpy(&d, cv, 16);
+  return d;
+}
+}  // namespace hostsim
+static inline hostsim_float4 __builtin_amdgcn_mfma_f32_16x16x32_f16(hostsim_half8 a, hostsim_half8 b, hostsim_float4 c, int, int, int) {
+  return hostsim::mfma16<false>(a, b, c);
+}
+static inline hostsim_float4 __builtin_amdgcn_mfma_f32_16x16x32_bf16(hostsim_bf16x8 a, hostsim_bf16x8 b, hostsim_float4 c, int, int, int) {
+  return hostsim::mfma16<true>(a, b, c);
 }

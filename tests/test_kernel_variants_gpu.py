@@ -4,6 +4,7 @@ for shapes the default does not take, forced here by its switch (NAME=0 in the e
   NMTG_ATTN_FUSED=0    Q K^T -> mask, then softmax -> dropout as two kernels instead of one (rows of up to 512 keys)
   NMTG_GEMM_SKINNY=0   a product with at most 32 rows against a row-major weight on the tiled kernels instead of the
                        kernel that gives every wavefront one output column
+  NMTG_ATTN_BWD_ONE=0  the backward of tiled attention as two kernels (dQ; dK and dV) instead of one (the form beyond 512 keys)
   NMTG_ATTN_DECODE=0   a one-position decoding step as one-row batched GEMMs and a softmax instead of the kernel that
                        streams the cached keys and values once
 
@@ -273,3 +274,41 @@ def test_few_row_products_match_the_tiled_kernels(dev, dtype, m, n, k):
     pitched = torch.full((m, k + 24), float("nan"), dtype=dtype, device=dev)      # rows with a pitch, NaN in the padding
     pitched[:, :k] = x
     assert torch.equal(gemm(pitched[:, :k], w, False, True, alpha=0.5, bias=bias), got)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("mask", ["none", "padding", "time", "causal"])
+@pytest.mark.parametrize("p", [0.0, 0.2])
+def test_attention_backward_in_one_kernel_matches_the_two_kernels(dev, dtype, mask, p):
+    """At the edges of the one kernel's steps (32 queries), groups (32 keys) and block sizes (128 and 256 keys), and with heads
+    next to each other or in the slots of a projection. Both forms sum the same products in fp32, in another order: a result
+    differs where the two sums (relative distance d) fall on either side of a rounding boundary, which befalls a share d / eps
+    of the elements with eps each, sqrt(d eps) in the 2-norm; the same holds for the rounded operand dS. d: one unit of fp32 per
+    term. Few of a small tensor's elements decide, hence the factor."""
+    from nmtgminor_amd.native import flash_attn_cuda as fa
+    eps = torch.finfo(dtype).eps
+    for n, (tq, tk, b, h) in enumerate([(1, 1, 1, 1), (31, 33, 2, 3), (33, 65, 1, 2), (64, 128, 2, 2), (65, 129, 1, 2), (40, 300, 2, 1), (256, 257, 1, 2),
+                                        (96, 512, 1, 2), (512, 64, 1, 1)]):
+        g = torch.Generator().manual_seed(700 + n)
+        qs = torch.randn(tq, b, h, 3, 64, generator=g).to(dtype).to(dev)
+        ks = torch.randn(tk, b, h, 3, 64, generator=g).to(dtype).to(dev)
+        q, k, v = qs[..., 0, :], ks[..., 1, :], ks[..., 2, :]
+        dout = torch.randn(tq, b, h, 64, generator=g).to(dtype).to(dev)
+        pad = (torch.rand(b, tk, generator=g) < 0.3).to(torch.uint8).to(dev) if mask == "padding" else None
+        time = (torch.rand(tq, tk, generator=g) < 0.3).to(torch.uint8).to(dev) if mask == "time" else None
+        out, lse, state = fa.fwd_batched(q, k, v, pad, p, 0.125, mask == "causal", time_mask=time)
+
+        def grads():
+            dqs, dks = torch.full_like(qs, 7.0), torch.full_like(ks, 7.0)
+            delta = fa.bwd_batched(dout, q, k, v, out, lse, dqs[..., 0, :], dks[..., 1, :], dks[..., 2, :], pad, p, 0.125, mask == "causal", state,
+                                   time_mask=time)
+            return [x.double().cpu() for x in (dqs, dks, delta)]
+        one = grads()
+        with off("NMTG_ATTN_BWD_ONE"):
+            two = grads()
+        for x, y, name in zip(one, two, ("dq", "dk / dv", "rowsum(dO O)")):
+            what = f"{name} {tq} x {tk}"
+            assert torch.isfinite(x).all(), what
+            e = eps if x.dim() == 5 else 2.0 ** -24
+            bound = 4 * (2.0 ** -24 * max(64, tq, tk) * e) ** 0.5
+            assert (x - y).norm() <= bound * y.norm().clamp_min(1e-6), (what, float((x - y).norm() / y.norm()))
