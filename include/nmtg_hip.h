@@ -226,6 +226,19 @@ int nmtg_gemm(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float a
 int nmtg_linear_step(int64_t rows, int64_t out, int64_t in, const void* x, const void* w, const void* bias, void* y,
                      int dtype, void* stream);
 
+/* The same with what stands around a product in a layer's step, in one launch (rows <= 64, in a multiple of 8, dense tensors,
+ * x and w 16-byte aligned; fp16 / bf16):
+ *   gamma, beta (may be NULL; in <= 1024): the product takes LayerNorm(x), or with `residual` LayerNorm(h), where h = x + residual
+ *     is written. clear: a device int set to 0, or NULL;
+ *   act (an nmtg_act code): y = act(product + bias), or
+ *   add (without gamma and act): y = add + (product + bias), clamped as nmtg_dropout_add_guard_fwd does. fp16 needs `guard`: a
+ *     device int that is 0 (see clear).
+ * nmtg_step_linear_ok: whether all products of a layer with `rows` rows are of this form (1) or take the separate calls (0). */
+int nmtg_step_linear_ok(int64_t rows, int64_t model, int64_t inner);
+int nmtg_step_linear(int64_t rows, int64_t out, int64_t in, const void* x, const void* residual, const void* gamma,
+                     const void* beta, float eps, void* h, int* clear, const void* w, const void* bias, int act,
+                     const void* add, int* guard, void* y, int dtype, void* stream);
+
 /* nmtg_gemm without a workspace argument, for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc). No counterpart in the reference. The split-K
  * partial sums go to an array of nmtg_gemm_static_max_workspace_bytes() (32 MiB) that the library keeps in device

@@ -245,6 +245,34 @@ __device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
 #endif
 }
 
+// A value that exists in fp32 before it is rounded to 16 bits: the compiler may otherwise fold the last multiply-add and the
+// conversion into one rounding (v_fma_mixlo_f16) in one kernel and not in the next, and z would differ from nmtg_ln_fwd's in
+// the last place here and there, which a relu behind the next product turns into a gradient that differs visibly.
+__device__ __forceinline__ float as_fp32(float v) {
+  uint32_t w = __float_as_uint(v);
+  asm volatile("" : "+v"(w));
+  return __uint_as_float(w);
+}
+
+// The guard at the end of a layer (dropout_add.hip): whether a value needs a closer look, and one that is not finite made finite
+// where the clamp is elementwise. -> whether it was not finite
+template <typename T> __device__ __forceinline__ float guard_limit();
+template <> __device__ __forceinline__ float guard_limit<float>() { return INFINITY; }
+template <> __device__ __forceinline__ float guard_limit<bf16_t>() { return 3.3895313892515355e38f; }
+template <> __device__ __forceinline__ float guard_limit<f16_t>() { return 65504.f; }
+__device__ __forceinline__ bool guard_element(bf16_t& o) {
+  if ((o.bits & 0x7f80u) != 0x7f80u) return false;
+  if ((o.bits & 0x7fu) == 0) o.bits = static_cast<uint16_t>((o.bits & 0x8000u) | 0x7f7fu);
+  return true;
+}
+__device__ __forceinline__ bool guard_element(float& o) {
+  const uint32_t b = __float_as_uint(o);
+  if ((b & 0x7f800000u) != 0x7f800000u) return false;
+  if ((b & 0x7fffffu) == 0) o = __uint_as_float((b & 0x80000000u) | 0x7f7fffffu);
+  return true;
+}
+__device__ __forceinline__ bool guard_element(f16_t& o) { return (o.bits & 0x7c00u) == 0x7c00u; }
+
 struct Philox {
   uint32_t key0, key1;
   __device__ __forceinline__ Philox(uint64_t seed) : key0(static_cast<uint32_t>(seed)), key1(static_cast<uint32_t>(seed >> 32)) {}

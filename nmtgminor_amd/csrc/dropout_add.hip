@@ -76,23 +76,6 @@ __global__ __launch_bounds__(DA_THREADS) void dropout_add_fwd_kernel(
 // NaN). Bandwidth bound like the plain form: 22 us at [512 x 32 x 1024] bf16 with the mask drawn here, and none of the 39 us
 // of the two reductions it replaces, nor a host round trip.
 // ---------------------------------------------------------------------------------------------------------------------
-template <typename T> __device__ __forceinline__ float guard_limit();
-template <> __device__ __forceinline__ float guard_limit<float>() { return INFINITY; }
-template <> __device__ __forceinline__ float guard_limit<bf16_t>() { return 3.3895313892515355e38f; }
-template <> __device__ __forceinline__ float guard_limit<f16_t>() { return 65504.f; }
-__device__ __forceinline__ bool guard_element(bf16_t& o) {
-  if ((o.bits & 0x7f80u) != 0x7f80u) return false;
-  if ((o.bits & 0x7fu) == 0) o.bits = static_cast<uint16_t>((o.bits & 0x8000u) | 0x7f7fu);
-  return true;
-}
-__device__ __forceinline__ bool guard_element(float& o) {
-  const uint32_t b = __float_as_uint(o);
-  if ((b & 0x7f800000u) != 0x7f800000u) return false;
-  if ((b & 0x7fffffu) == 0) o = __uint_as_float((b & 0x80000000u) | 0x7f7fffffu);
-  return true;
-}
-__device__ __forceinline__ bool guard_element(f16_t& o) { return (o.bits & 0x7c00u) == 0x7c00u; }
-
 template <typename T, int EPV, int MODE>
 __device__ __forceinline__ void guard_pack(T* __restrict__ x, const T* __restrict__ residual, uint8_t* __restrict__ mask, int64_t first,
                                            float keep_p, float scale, uint64_t seed, uint64_t offset, int* __restrict__ flag) {
@@ -240,6 +223,14 @@ int guard_launch(void* x, const void* residual, uint8_t* mask, int64_t n, float 
 }
 
 }  // namespace
+// Behind the kernel that raises `flag`: the clamp of an fp16 stream that is not finite everywhere (also behind the decoding step's
+// last product, gemm_skinny.hip).
+void guard_clamp_f16(void* x, uint8_t* mask, int64_t n, const int* flag, hipStream_t st) {
+  const int64_t blocks = (n + DA_THREADS * 8 - 1) / (DA_THREADS * 8), cap = num_cus();
+  hipLaunchKernelGGL(guard_clamp_f16_kernel, dim3(static_cast<unsigned>(blocks < cap ? blocks : cap)), dim3(DA_THREADS), 0, st,
+                     static_cast<f16_t*>(x), mask, n, flag);
+}
+
 }  // namespace nmtg
 
 using namespace nmtg;
@@ -256,11 +247,7 @@ extern "C" int nmtg_dropout_add_guard_fwd(void* x, const void* residual, uint8_t
   int rc = 0;
   NMTG_DISPATCH_DTYPE(dtype, T, rc = guard_launch<T>(x, residual, mask, n, p, mask_mode, seed, offset, flag, st));
   if (rc) return rc;
-  if (dtype == NMTG_F16) {
-    const int64_t blocks = (n + DA_THREADS * 8 - 1) / (DA_THREADS * 8), cap = num_cus();
-    hipLaunchKernelGGL(guard_clamp_f16_kernel, dim3(static_cast<unsigned>(blocks < cap ? blocks : cap)), dim3(DA_THREADS), 0, st,
-                       static_cast<f16_t*>(x), mask, n, flag);
-  }
+  if (dtype == NMTG_F16) guard_clamp_f16(x, mask, n, flag, st);
   NMTG_CHECK_LAUNCH("dropout_add_guard_fwd");
   return 0;
 }

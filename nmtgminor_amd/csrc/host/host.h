@@ -35,7 +35,7 @@ using std::optional;
   X(xentropy_bwd) X(gemm) X(mlp_fwd) X(mlp_bwd_dtype_workspace_bytes) X(mlp_bwd) X(flash_attn_dropout_bits_bytes)     \
   X(flash_attn_fwd) X(flash_attn_bwd) X(flash_attn_key_info_bytes) X(flash_attn_time_info_bytes)                      \
   X(flash_attn_batched_fwd) X(flash_attn_batched_bwd) X(multi_tensor_adam) X(multi_tensor_clip)                       \
-  X(multi_tensor_l2norm) X(multi_tensor_l2norm_workspace_bytes) X(flash_attn_batched_fwd_probs) X(linear_step) X(gemm_workspace_bytes)            \
+  X(multi_tensor_l2norm) X(multi_tensor_l2norm_workspace_bytes) X(flash_attn_batched_fwd_probs) X(linear_step) X(step_linear) X(step_linear_ok) X(gemm_workspace_bytes) \
   X(xentropy_bwd_colsum) X(xentropy_bwd_colsum_parts)
 
 struct Api {
@@ -105,6 +105,11 @@ AddNormGrads ln_bwd_add(const Tensor& dz, const Tensor& x, const Tensor& stats, 
 
 Tensor linear_fwd(const Tensor& x, const Tensor& w, const Tensor& b);
 Tensor linear_step(const Tensor& x, const Tensor& w, const Tensor& b);          // of a decoding step: few rows, no gradient
+// the same on LayerNorm(x), or with a residual on LayerNorm(h), h = x + residual (see nmtg_step_linear)
+struct StepNorm { Tensor y, h; };
+StepNorm norm_step(const Tensor& x, const Tensor& residual, const Tensor& gamma, const Tensor& beta, double eps, const Tensor& clear, const Tensor& w,
+                   const Tensor& b, int64_t act);
+Tensor linear_add_step(const Tensor& x, const Tensor& w, const Tensor& b, const Tensor& add, const Tensor& guard);
 struct LinearGrads { Tensor dx, dw, db; };
 LinearGrads linear_bwd(const Tensor& dy, const Tensor& x, const Tensor& w, bool want_x, bool want_w, bool want_b);
 

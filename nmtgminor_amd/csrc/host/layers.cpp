@@ -239,19 +239,35 @@ std::tuple<Tensor, Tensor> decoder_step(const Tensor& x, const Tensor& kbuf, con
   const int64_t b = x.size(1), e = x.size(2), d = e / heads, tk = ck.size(0);
   const float scale = static_cast<float>(1.0 / std::sqrt(static_cast<double>(d)));
   Launch on(x);
-  Norm n1 = ln_fwd(x, w[0], w[1], kEps);
-  Tensor lin = linear_step(n1.z, w[2], w[3]);
+  // few rows: LayerNorms, activation and last addition go with the products (8 launches and the clamp of fp16 instead of 13)
+  auto whole = [](const Tensor& t) { return reinterpret_cast<uintptr_t>(ptr(t)) % 16 == 0; };
+  bool fused = api.step_linear_ok(b, e, w[13].size(0)) != 0 && whole(x);
+  for (int i : {0, 1, 2, 6, 7, 8, 11, 12, 13, 15}) fused = fused && whole(w[i]);
+  Tensor lin = fused ? norm_step(x, Tensor(), w[0], w[1], kEps, Tensor(), w[2], w[3], NMTG_ACT_NONE).y : linear_step(ln_fwd(x, w[0], w[1], kEps).z, w[2], w[3]);
   Tensor cx = new_like(x);
   check(api.attn_decode_append(ptr(lin), 3 * e, ptr(kbuf), kbuf.stride(0), kbuf.stride(1), ptr(vbuf), vbuf.stride(0), vbuf.stride(1), ptr(cx), e, b,
                                heads, d, n, scale, dtype_code(x), on.stream), "nmtg_attn_decode_append");
-  AddNorm n2 = add_ln_fwd(linear_step(cx, w[4], w[5]), x, 0.0, Tensor(), w[6], w[7], kEps);
-  Tensor q = linear_step(n2.z, w[8], Tensor());
+  Tensor y = linear_step(cx, w[4], w[5]), q, h;
+  if (fused) {
+    StepNorm s = norm_step(y, x, w[6], w[7], kEps, Tensor(), w[8], Tensor(), NMTG_ACT_NONE);
+    q = s.y;
+    h = s.h;
+  } else {
+    AddNorm n2 = add_ln_fwd(y, x, 0.0, Tensor(), w[6], w[7], kEps);
+    q = linear_step(n2.z, w[8], Tensor());
+    h = n2.h;
+  }
   Tensor coverage = empty_like_sized(x, {b * heads, 1, tk});
   check(api.attn_decode(ptr(q), e, ptr(ck), ck.stride(0), ck.stride(1), ptr(cv), cv.stride(0), cv.stride(1),
                         static_cast<const uint8_t*>(ptr(pad)), ptr(coverage), ptr(cx), e, b, heads, d, tk, scale, dtype_code(x), on.stream),
         "nmtg_attn_decode");
-  FfnState f = ffn_fwd(linear_step(cx, w[10], Tensor()), n2.h, 0.0, w[11], w[12], w[13], w[14], w[15], w[16], act, 0.0, 0.0, false);
-  return {f.out, coverage};
+  y = linear_step(cx, w[10], Tensor());
+  if (fused) {
+    Tensor guard = guard_flag(x);
+    StepNorm s = norm_step(y, h, w[11], w[12], kEps, guard, w[13], w[14], act);
+    return {linear_add_step(s.y, w[15], w[16], s.h, guard), coverage};
+  }
+  return {ffn_fwd(y, h, 0.0, w[11], w[12], w[13], w[14], w[15], w[16], act, 0.0, 0.0, false).out, coverage};
 }
 
 // Whether an encoder layer's 12 or a decoder layer's 17 parameters (all present) have the shapes that x's last dimension asks

@@ -119,6 +119,26 @@ Tensor linear_step(const Tensor& x, const Tensor& w, const Tensor& b) {
   return y;
 }
 
+StepNorm norm_step(const Tensor& x, const Tensor& residual, const Tensor& gamma, const Tensor& beta, double eps, const Tensor& clear, const Tensor& w,
+                   const Tensor& b, int64_t act) {
+  const int64_t in = w.size(1), out = w.size(0);
+  Launch on(x);
+  StepNorm r{linear_result(x, out), residual.defined() ? new_like(x) : Tensor()};
+  check(api.step_linear(x.numel() / in, out, in, ptr(x), ptr(residual), ptr(gamma), ptr(beta), static_cast<float>(eps), ptr(r.h),
+                        static_cast<int*>(ptr(clear)), ptr(w), ptr(b), static_cast<int>(act), nullptr, nullptr, ptr(r.y), dtype_code(x), on.stream),
+        "nmtg_step_linear");
+  return r;
+}
+
+Tensor linear_add_step(const Tensor& x, const Tensor& w, const Tensor& b, const Tensor& add, const Tensor& guard) {
+  const int64_t in = w.size(1), out = w.size(0);
+  Launch on(x);
+  Tensor y = linear_result(x, out);
+  check(api.step_linear(x.numel() / in, out, in, ptr(x), nullptr, nullptr, nullptr, 0.f, nullptr, nullptr, ptr(w), ptr(b), NMTG_ACT_NONE, ptr(add),
+                        static_cast<int*>(ptr(guard)), ptr(y), dtype_code(x), on.stream), "nmtg_step_linear");
+  return y;
+}
+
 static Scratch mlp_workspace(const Tensor& x, int layers, const int64_t* outs, int64_t rows, int64_t in) {
   return Scratch(x, std::max<int64_t>(api.mlp_bwd_dtype_workspace_bytes(layers, outs, rows, in, dtype_code(x)), 256));
 }

@@ -73,15 +73,6 @@ template <typename TI> struct LnAdd {
   int* clear;                // set to 0 (the flag of a guard further down the stream), or null
 };
 
-// A value that exists in fp32 before it is rounded to 16 bits: the compiler may otherwise fold the last multiply-add and the
-// conversion into one rounding (v_fma_mixlo_f16) in one kernel and not in the next, and z would differ from nmtg_ln_fwd's in
-// the last place here and there, which a relu behind the next product turns into a gradient that differs visibly.
-__device__ __forceinline__ float as_fp32(float v) {
-  uint32_t w = __float_as_uint(v);
-  asm volatile("" : "+v"(w));
-  return __uint_as_float(w);
-}
-
 template <typename TI, int EPV, int ADD>
 __device__ __forceinline__ void ln_add_row(const LnAdd<TI>& add, int64_t first, const pack<TI, EPV>& res, float (&xf)[EPV]) {
   float rf[EPV];
