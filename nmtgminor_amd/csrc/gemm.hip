@@ -180,6 +180,12 @@ int gemm_run(int dtype, int layout, int epi, GemmArgs a, void* workspace, size_t
   const bool can_ride = (tile == TILE_M || tile == TILE_X) && a.vec == 8 && a.ring && a.batch == 1 && layout == LAYOUT_NN && epi == EPI_PLAIN;
   a.riders_taken = (a.riders != nullptr && a.rider_blocks > 0 && can_ride) ? 1 : 0;
   if (!a.riders_taken) { a.riders = nullptr; a.rider_blocks = 0; }
+  if (layout == LAYOUT_TN) {
+    const int64_t rows = static_cast<int64_t>(a.splits) * a.n_tiles;
+    const bool carry = a.colsum_part != nullptr && epi == EPI_SPLITK && a.ring && a.batch == 1 && rows <= a.colsum_cap;
+    a.colsum_rows = carry ? static_cast<int>(rows) : 0;
+    if (!carry) a.colsum_part = nullptr;
+  }
   if (planned_out) *planned_out = a;
   int rc;
   if (layout == LAYOUT_NT) rc = gemm_launch_nt(dtype, tile, epi, a, st);

@@ -83,7 +83,11 @@ struct GemmArgs {
   const void* riders;
   int rider_blocks;
   int riders_taken;
+  // Partial column sums [rows][M or N] in fp32. EPI_ACT_BWD: of the result, one row per row tile. Split-K calls of the TN layout:
+  // of A over its rows (dY^T 1 beside dW = dY^T X), one row per column tile and split; host: up to colsum_cap rows fit, and
+  // gemm_run reports in colsum_rows how many were written (0: the kernel of this call does not carry them).
   float* colsum_part;
+  int colsum_cap, colsum_rows;
   const uint8_t* kmask;
   int kmask_kind, heads;
   float* ws;

@@ -192,20 +192,24 @@ extern "C" int nmtg_mlp_bwd(int num_layers, const void* x, const void* const* we
     const int64_t in_i = i == 0 ? in_features : out_features[i - 1];
     const void* input_i = i == 0 ? x : static_cast<const uint8_t*>(post_acts) + offs[i - 1] * esz;
     int rc;
-    // bias gradient (its partial rows: written by the data-gradient GEMM of the layer above, or by a kernel of its own)
+    // bias gradient (its partial rows: written by the data-gradient GEMM of the layer above, by this layer's weight-gradient GEMM,
+    // or by a kernel of its own)
     float* colsum_ws = colsum_region(i);
+    auto own_partials = [&]() -> int {
+      const int parts = colsum_parts(static_cast<int>(batch));
+      if (int rc2 = tail_add_colsum_partial(head, dtype, g_cur, out_i, static_cast<int>(batch), static_cast<int>(out_i), colsum_ws)) return rc2;
+      head_pending = true;
+      return tail_add_colsum(tail, colsum_ws, parts, static_cast<int>(out_i), grad_biases[i]);
+    };
+    bool bias_with_weight = false;
     if (grad_biases && grad_biases[i]) {
       if (!bias_from_parts && tail_add_colsum_whole(tail, dtype, g_cur, out_i, static_cast<int>(batch), static_cast<int>(out_i), grad_biases[i])) {
         rc = 0;
-      } else if (!tail.full()) {
-        int parts = parts_rows;
+      } else if (!bias_from_parts && dtype != NMTG_F32 && grad_weights && grad_weights[i]) {
+        bias_with_weight = true;
         rc = 0;
-        if (!bias_from_parts) {
-          parts = colsum_parts(static_cast<int>(batch));
-          rc = tail_add_colsum_partial(head, dtype, g_cur, out_i, static_cast<int>(batch), static_cast<int>(out_i), colsum_ws);
-          head_pending = !rc;
-        }
-        if (!rc) rc = tail_add_colsum(tail, colsum_ws, parts, static_cast<int>(out_i), grad_biases[i]);
+      } else if (!tail.full()) {
+        rc = bias_from_parts ? tail_add_colsum(tail, colsum_ws, parts_rows, static_cast<int>(out_i), grad_biases[i]) : own_partials();
       } else if (bias_from_parts) {
         rc = colsum_finish(dtype, colsum_ws, parts_rows, static_cast<int>(out_i), grad_biases[i], st);
       } else {
@@ -222,6 +226,10 @@ extern "C" int nmtg_mlp_bwd(int num_layers, const void* x, const void* const* we
       g.M = static_cast<int>(out_i); g.N = static_cast<int>(in_i); g.K = static_cast<int>(batch);
       g.batch = 1; g.alpha = 1.f;
       g.defer_reduce = !tail.full() ? 1 : 0;
+      if (bias_with_weight) {
+        g.colsum_part = colsum_ws;
+        g.colsum_cap = static_cast<int>(plan.colsum_bytes / (out_i * sizeof(float)));
+      }
       // (the partial column sums do not ride with this product: a split-K launch repeats the rider blocks in every
       // split, and the tiles then share CUs unevenly; measured slower than the launch of their own)
       if (int rc2 = flush_head()) return rc2;
@@ -230,6 +238,13 @@ extern "C" int nmtg_mlp_bwd(int num_layers, const void* x, const void* const* we
       if (!rc && planned.defer_reduce && planned.splits > 1)
         rc = tail_add_splitk(tail, planned.tile_used, planned.ws, planned.C, planned.ldc, planned.M, planned.N, planned.m_tiles,
                              planned.n_tiles, planned.batch, planned.sC, planned.splits, planned.alpha, planned.vec);
+      if (!rc && bias_with_weight) {
+        if (planned.colsum_rows > 0)
+          rc = !tail.full() ? tail_add_colsum(tail, colsum_ws, planned.colsum_rows, static_cast<int>(out_i), grad_biases[i])
+                            : colsum_finish(dtype, colsum_ws, planned.colsum_rows, static_cast<int>(out_i), grad_biases[i], st);
+        else
+          rc = !tail.full() ? own_partials() : colsum_run(dtype, g_cur, out_i, static_cast<int>(batch), static_cast<int>(out_i), colsum_ws, grad_biases[i], st);
+      }
       if (rc) return rc;
     }
     // data gradient

@@ -312,3 +312,23 @@ def test_attention_backward_in_one_kernel_matches_the_two_kernels(dev, dtype, ma
             e = eps if x.dim() == 5 else 2.0 ** -24
             bound = 4 * (2.0 ** -24 * max(64, tq, tk) * e) ** 0.5
             assert (x - y).norm() <= bound * y.norm().clamp_min(1e-6), (what, float((x - y).norm() / y.norm()))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("tokens,out,inner", [(1025, 64, 64), (1100, 264, 72), (1500, 512, 512), (2064, 136, 1096), (4100, 1024, 256), (1088, 2048, 2048)])
+def test_bias_gradient_beside_the_weight_gradient(dev, dtype, tokens, out, inner):
+    """Column sums of dY from the weight gradient's LDS tiles: every k-step counted once, whichever column tile and split adds it,
+    at ragged token counts and rows beyond the last tile, and calls with more partial rows than fit, which sum dY in a launch of
+    their own. fp32 sums of rounded numbers: tokens units of fp32 of the sum of magnitudes, then one rounding."""
+    g = torch.Generator().manual_seed(tokens)
+    x = torch.randn(tokens, inner, generator=g).to(dtype).to(dev).requires_grad_()
+    w = (0.05 * torch.randn(out, inner, generator=g)).to(dtype).to(dev)
+    b = torch.zeros(out, dtype=dtype, device=dev)
+    dy = (torch.randn(tokens, out, generator=g) + 0.5).to(dtype)
+    saved = fused_mlp_gelu.forward(0.0, [x, w, b])
+    _, dw, db = fused_mlp_gelu.backward(0.0, dy.to(dev), saved, [x, w, b])
+    d64 = dy.double()
+    want = d64.sum(0)
+    bound = torch.finfo(dtype).eps * want.abs() + tokens * 2.0 ** -24 * d64.abs().sum(0)
+    assert bool(((db.double().cpu() - want).abs() <= bound).all()), float((db.double().cpu() - want).abs().max())
+    assert_close(dw, d64.t() @ x.detach().double().cpu(), dtype, "dw", scale_atol=True)
