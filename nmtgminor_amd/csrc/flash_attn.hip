@@ -360,8 +360,22 @@ __global__ __launch_bounds__(256) void flash_key_info_kernel(const uint8_t* pad,
   }
 }
 
+// Bit 7 of each byte: whether that byte of w is below a threshold t < 256, given low = t & 127 in every byte and
+// top = ~0 where t >= 128, 0 otherwise. The other bits are undefined. Three instructions for four comparisons: bit 7 of
+// (w | 128) - low says whether the low seven bits reach the threshold's, and the two tests' majority with top is the answer.
+__device__ __forceinline__ uint32_t bytes_below(uint32_t w, uint32_t low, uint32_t top) {
+  const uint32_t reach = (w | 0x80808080u) - low;
+#if __has_builtin(__builtin_amdgcn_bitop3_b32)
+  return static_cast<uint32_t>(__builtin_amdgcn_bitop3_b32(static_cast<int>(w), static_cast<int>(reach), static_cast<int>(top), 0x2b));
+#else
+  return (~w & ~reach) | (top & (~w | ~reach));
+#endif
+}
+
 // Keep bits from the generator: one thread per (head of a sequence, group of 32 queries, group of four keys) runs the
-// eight generator calls of its 32 x 4 elements (one call per 4 x 4 patch) and writes the four keys' words.
+// eight generator calls of its 32 x 4 elements (one call per 4 x 4 patch) and writes the four keys' words. Vector
+// instructions bound it. With one comparison, select and shift per element, forming the bits took as long as the generator; four
+// bytes of a generator word are compared at once instead (512 x [512 x 512] elements: 27.2 -> 23.2 us).
 __global__ __launch_bounds__(256) void flash_bits_rng_kernel(FaArgs a, int64_t total) {
   const int64_t id = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   if (id >= total) return;
@@ -375,17 +389,24 @@ __global__ __launch_bounds__(256) void flash_bits_rng_kernel(FaArgs a, int64_t t
   if (32 * grp >= lq || 4 * j4 >= lk) return;        // never read: every element there is masked or not stored
   const Philox gen(a.seed);
   const uint64_t q4 = static_cast<uint64_t>((a.max_q + 3) / 4), k4 = static_cast<uint64_t>((a.max_k + 3) / 4);
-  uint32_t word[4] = {0, 0, 0, 0};
+  // eight queries by four keys per word, a key per byte; a threshold of 256 keeps everything
+  const uint32_t low = (a.thr & 0x7fu) * 0x01010101u, top = (a.thr & 0x80u) != 0 ? ~0u : 0u, all = a.thr > 0xffu ? ~0u : 0u;
+  uint32_t eight[4] = {all, all, all, all};
 #pragma unroll
   for (int u = 0; u < 8; ++u) {
     const uint4 r = gen((static_cast<uint64_t>(bh) * q4 + static_cast<uint64_t>(8 * grp + u)) * k4 + static_cast<uint64_t>(j4), a.offset);
     const uint32_t w[4] = {r.x, r.y, r.z, r.w};
 #pragma unroll
-    for (int qi = 0; qi < 4; ++qi)
-#pragma unroll
-      for (int kj = 0; kj < 4; ++kj)
-        word[kj] |= (((w[qi] >> (8 * kj)) & 0xffu) < a.thr ? 1u : 0u) << (4 * u + qi);
+    for (int qi = 0; qi < 4; ++qi) {
+      const int bit = 4 * (u & 1) + qi;
+      eight[u / 2] |= (bytes_below(w[qi], low, top) >> (7 - bit)) & (0x01010101u << bit);
+    }
   }
+  uint32_t word[4];
+#pragma unroll
+  for (int kj = 0; kj < 4; ++kj)
+    word[kj] = ((eight[0] >> (8 * kj)) & 0xffu) | (((eight[1] >> (8 * kj)) & 0xffu) << 8) | (((eight[2] >> (8 * kj)) & 0xffu) << 16) |
+               (((eight[3] >> (8 * kj)) & 0xffu) << 24);
   uint32_t* out = a.bits + row * a.kp;
 #pragma unroll
   for (int kj = 0; kj < 4; ++kj) out[bit_slot(4 * j4 + kj)] = word[kj];

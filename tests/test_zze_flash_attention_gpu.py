@@ -214,3 +214,28 @@ def test_unsupported_inputs_are_refused(dev):
     q = torch.zeros(4, 2, 72, device=dev, dtype=torch.float16)[:, :, 4:68]          # 8-byte aligned view
     with pytest.raises(RuntimeError, match="16-byte aligned"):
         flash_attn_cuda.fwd(q, q, q, torch.empty(4, 2, 64, device=dev, dtype=torch.float16), cu, cu, 4, 4, 0.0, 1.0, False, False, False)
+
+
+@pytest.mark.parametrize("p", [0.0005, 1 / 256, 0.3, 127 / 256, 0.5, 129 / 256, 0.9, 254 / 256, 0.998])
+def test_every_keep_bit_of_the_byte_thresholds_edges(dev, p):
+    """All elements of a drawn mask against the documented stream where the four-bytes-at-once comparison can go wrong: a
+    threshold of 256 (keep all), 255, 129, 128, 127, 2 and 1; an odd number of keys and queries beyond whole groups."""
+    lens, heads, d = [37, 6], 2, 64
+    q, k, v, _ = _inputs(lens, lens, heads, d, torch.bfloat16, seed=29)
+    cu = _cu(lens).to(dev)
+    torch.cuda.manual_seed(77)
+    res = flash_attn_cuda.fwd(q.to(dev), k.to(dev), v.to(dev), torch.empty_like(q).to(dev), cu, cu, 37, 37, p, 0.125, False,
+                              False, True, 0, None)
+    mode, seed, offset = flash_attn_cuda.last_rng[:3]
+    assert mode == 2
+    mask, thr, n4 = res[1].cpu(), min(256, max(1, round(256 * (1 - p)))), 10
+    for b, n in enumerate(lens):
+        for h in range(heads):
+            for i4 in range((n + 3) // 4):
+                for j4 in range((n + 3) // 4):
+                    block = ((b * heads + h) * n4 + i4) * n4 + j4
+                    words = philox4x32_10([offset, offset >> 32, block, block >> 32], [seed, seed >> 32])
+                    for i in range(4 * i4, min(n, 4 * i4 + 4)):
+                        for j in range(4 * j4, min(n, 4 * j4 + 4)):
+                            byte = (words[i % 4] >> (8 * (j % 4))) & 0xFF
+                            assert int(mask[b, h, i, j]) == int(byte < thr), (b, h, i, j, byte, thr)
