@@ -8,6 +8,7 @@
 namespace nmtg {
 
 bool gemm_has(int layout, int tile, int epi) {
+  if (tile == TILE_X && epi == EPI_SCORES) return layout == LAYOUT_NT;
   if (tile == TILE_X) return epi == EPI_PLAIN || epi == (layout == LAYOUT_NT ? EPI_ACT_FWD : layout == LAYOUT_NN ? EPI_ACT_BWD : EPI_PLAIN);
   if (layout == LAYOUT_NT)
     return (tile == TILE_L || tile == TILE_M) && (epi == EPI_PLAIN || epi == EPI_ACT_FWD || epi == EPI_SCORES);
@@ -95,23 +96,21 @@ int gemm_run(int dtype, int layout, int epi, GemmArgs a, void* workspace, size_t
   // enter: a ragged M / N / K ends in a predicated last vector (loads stay inside the row's pitch, which is a multiple
   // of the vector; the K tail is zeroed; the stores of a partial vector and the bias of a ragged last tile go element
   // by element). Byte masks are addressed as row * N + n, so there N is the pitch and does count.
-  int vec = 8;
-  auto narrow = [&](const void* p, int64_t ld, int64_t stride, int batch) {
-    vec = std::min(vec, vec_of(p, ld, stride, batch));
-  };
-  narrow(a.A, a.lda, a.sA, a.batch);
-  narrow(a.B, a.ldb, a.sB, a.batch);
-  narrow(a.C, a.ldc, a.sC, a.batch);
-  if (a.aux_out) narrow(a.aux_out, a.ldc, a.sC, a.batch);
-  if (a.bias) narrow(a.bias, 8, 0, 1);
-  if (a.aux_in) narrow(a.aux_in, a.ld_aux, 0, 1);
+  auto narrow = [](int& vec, const void* p, int64_t ld, int64_t stride, int batch) { vec = std::min(vec, vec_of(p, ld, stride, batch)); };
+  a.vec_a = vec_of(a.A, a.lda, a.sA, a.batch);
+  a.vec_b = vec_of(a.B, a.ldb, a.sB, a.batch);
+  a.vec_c = vec_of(a.C, a.ldc, a.sC, a.batch);
+  if (a.aux_out) narrow(a.vec_c, a.aux_out, a.ldc, a.sC, a.batch);
+  if (a.bias) narrow(a.vec_c, a.bias, 8, 0, 1);
+  if (a.aux_in) narrow(a.vec_c, a.aux_in, a.ld_aux, 0, 1);
   auto narrow_bytes = [&](const uint8_t* p) {
     int v = 8;
     while (v > 1 && (reinterpret_cast<uintptr_t>(p) % v != 0 || a.N % v != 0)) v = v == 8 ? 4 : 1;
-    vec = std::min(vec, v);
+    a.vec_c = std::min(a.vec_c, v);
   };
   if (a.dmask) narrow_bytes(a.dmask);
   if (a.kmask && a.kmask_kind != 0) narrow_bytes(a.kmask);
+  const int vec = std::min(std::min(a.vec_a, a.vec_b), a.vec_c);
   a.vec = vec;
 
   int tile = -1;
@@ -151,7 +150,7 @@ int gemm_run(int dtype, int layout, int epi, GemmArgs a, void* workspace, size_t
   }
   // 64x64 tiles where 128x128 ones would leave more than half of the chip idle: four times the blocks, each a quarter of the
   // work, and the same sums in the same order. Chosen below, once the call is known to suit the ring kernel.
-  const bool few_tiles = tile == TILE_M && forced_tile < 0 && gemm_has(layout, TILE_X, epi) &&
+  const bool few_tiles = tile == TILE_M && forced_tile < 0 && epi != EPI_SCORES && gemm_has(layout, TILE_X, epi) &&
                          static_cast<int64_t>(ceil_div(a.M, 128)) * ceil_div(a.N, 128) * a.batch * 2 <= num_cus();
   if (!gemm_has(layout, tile, epi))
     return fail(NMTG_ERR_UNSUPPORTED, "gemm: layout %d has no kernel for epilogue %d", layout, epi);
@@ -163,6 +162,17 @@ int gemm_run(int dtype, int layout, int epi, GemmArgs a, void* workspace, size_t
   const bool whole = a.K % GEMM_BK == 0 || (layout != LAYOUT_NT && (epi == EPI_PLAIN || epi == EPI_SPLITK));
   a.ring = (a.K > 0 && whole && vec == 8 && a_span < (int64_t{1} << 32) && b_span < (int64_t{1} << 32)) ? 1 : 0;
   if (few_tiles && a.ring) tile = TILE_X;
+  // Outputs that fill at most half of their tile's area, in calls outside the ring kernel (the heads of a ragged batch: an odd
+  // number of keys is an odd pitch of the probabilities): a 64x64 tile stages and multiplies half or a quarter as much per output,
+  // leaves room for four blocks on a CU and reads the operands whose own rows are aligned in 16-byte accesses. Measured against
+  // the larger tile: P V 61x64x73 of 384 heads 16.4 -> 7.1 us, 128x64x73 of 4096 114 -> 52, 127x64x1501 of 256 104 -> 53;
+  // dS^T Q 127x64x999 of 256 68 -> 42; scores 61x301x64 of 384 30 -> 19, 61x73x64 16.8 -> 11.6 (never slower).
+  if (!a.ring && forced_tile < 0 && (epi == EPI_PLAIN || epi == EPI_SCORES) && gemm_has(layout, TILE_X, epi)) {
+    int bm0, bn0;
+    tile_dims(tile, bm0, bn0);
+    auto padded = [&](int m, int n) { return static_cast<int64_t>(ceil_div(a.M, m)) * m * ceil_div(a.N, n) * n; };
+    if (2 * padded(64, 64) <= padded(bm0, bn0)) tile = TILE_X;
+  }
   // gelu and gelu' of the activation epilogues come from a table in LDS in the ring kernels (they have the LDS room)
   a.act_lut = (a.ring && (epi == EPI_ACT_FWD || epi == EPI_ACT_BWD)) ? 1 : 0;
   int bm, bn;

@@ -62,6 +62,7 @@ struct GemmArgs {
   int splits, k_per_split;
   float alpha;
   int vec;                  // widest access (elements: 8, 4 or 1) every operand and extent allows
+  int vec_a, vec_b, vec_c;  // the same of A, of B, and of C with all that the epilogue reads
   int ring;                 // the call meets the requirements of the slot-ring kernel (gemm_ring.hip.h)
   const void* bias;
   void* aux_out;
@@ -859,7 +860,8 @@ constexpr int gemm_lds_bytes() {
   return main_loop > c_tile ? main_loop : c_tile;
 }
 
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, bool A_KC, bool B_KC, int EPI, int VEC>
+// VEC: accesses of the output and what the epilogue reads with it; VEC_A, VEC_B: of the operands
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, bool A_KC, bool B_KC, int EPI, int VEC, int VEC_A = VEC, int VEC_B = VEC>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_kernel(const GemmArgs g) {
   constexpr int NT = 64 * WAVES_M * WAVES_N;
   constexpr int BK = GEMM_BK;
@@ -902,8 +904,8 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_kernel(const Gemm
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-  TileStage<T, BM, NT, A_KC, VEC> stA;
-  TileStage<T, BN, NT, B_KC, VEC> stB;
+  TileStage<T, BM, NT, A_KC, VEC_A> stA;
+  TileStage<T, BN, NT, B_KC, VEC_B> stB;
 
   NMTG_PROF_MARK(0);
   if (nk > 0) {

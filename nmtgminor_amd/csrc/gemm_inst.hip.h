@@ -3,7 +3,8 @@
 //   L: 256x256 tile, 2x4 wavefronts (each 128x64), 512 threads  — large outputs
 //   M: 128x128 tile, 2x2 wavefronts (each 64x64),  256 threads  — outputs too small to fill the chip with L
 //   S: 256x64  tile, 4x1 wavefronts (each 64x64),  256 threads  — N <= 64 (per-head attention products)
-//   X: 64x64 tile, 2x2 wavefronts (each 32x32),    256 threads  — outputs too small to fill the chip with M (ring kernel only)
+//   X: 64x64 tile, 2x2 wavefronts (each 32x32),    256 threads  — outputs too small to fill the chip with M (ring kernel), or to fill a
+//      larger tile (two-buffer kernel, plain and score products)
 //   R: 128x512 tile, 4x2 wavefronts (each 32x256), 512 threads  — whole score rows (fused softmax epilogue only)
 #pragma once
 #include "gemm.hip.h"
@@ -22,10 +23,10 @@ inline void tile_dims(int tile, int& bm, int& bn) {
   else { bm = 256; bn = 64; }
 }
 
-template <typename T, int TILE, bool A_KC, bool B_KC, int EPI, int VEC>
+template <typename T, int TILE, bool A_KC, bool B_KC, int EPI, int VEC, int VEC_A = VEC, int VEC_B = VEC>
 int gemm_launch_vec(const GemmArgs& a, hipStream_t st) {
   using C = tile_cfg<TILE>;
-  auto kern = gemm_kernel<T, C::BM, C::BN, C::WM, C::WN, A_KC, B_KC, EPI, VEC>;
+  auto kern = gemm_kernel<T, C::BM, C::BN, C::WM, C::WN, A_KC, B_KC, EPI, VEC, VEC_A, VEC_B>;
   constexpr int lds = gemm_lds_bytes<C::BM, C::BN>();
   static bool attr_done = false;
   if (!attr_done) {
@@ -35,7 +36,7 @@ int gemm_launch_vec(const GemmArgs& a, hipStream_t st) {
   }
   dim3 grid(a.m_tiles * a.n_tiles, a.batch, a.splits);
   static const std::string name = std::string("gemm_") + (A_KC ? (B_KC ? "nt" : "nn") : "tn") + "_" +
-                                  (TILE == TILE_L ? "256x256" : TILE == TILE_M ? "128x128" : TILE == TILE_R ? "128x512" : "256x64") + "_" +
+                                  (TILE == TILE_L ? "256x256" : TILE == TILE_M ? "128x128" : TILE == TILE_R ? "128x512" : TILE == TILE_X ? "64x64" : "256x64") + "_" +
                                   (EPI == EPI_PLAIN ? "plain" : EPI == EPI_ACT_FWD ? "actfwd" : EPI == EPI_ACT_BWD ? "actbwd"
                                    : EPI == EPI_SCORES ? "scores" : (EPI == EPI_SCORES_SOFTMAX || EPI == EPI_SCORES_SOFTMAX_RNG) ? "scores_softmax" : EPI == EPI_DSOFTMAX ? "dsoftmax"
                                    : "splitk") +
@@ -101,9 +102,27 @@ int gemm_launch_ring(const GemmArgs& a, hipStream_t st) {
   return 0;
 }
 
+// Two-buffer kernel of the 64x64 tile. The product of a head with an odd number of positions has one operand or the output of
+// odd pitch (scores and probabilities, [queries][keys]) and the rest in rows of the head dimension, which keep 16-byte accesses.
+template <typename T, bool A_KC, bool B_KC, int EPI>
+int gemm_launch_small(const GemmArgs& a, hipStream_t st) {
+  if (a.vec == 8) return gemm_launch_vec<T, TILE_X, A_KC, B_KC, EPI, 8>(a, st);
+  if constexpr (B_KC) {
+    if (a.vec_a == 8 && a.vec_b == 8)
+      return a.vec_c == 4 ? gemm_launch_vec<T, TILE_X, A_KC, B_KC, EPI, 4, 8, 8>(a, st) : gemm_launch_vec<T, TILE_X, A_KC, B_KC, EPI, 1, 8, 8>(a, st);
+  } else {
+    if (a.vec_b == 8 && a.vec_c == 8)
+      return a.vec_a == 4 ? gemm_launch_vec<T, TILE_X, A_KC, B_KC, EPI, 8, 4, 8>(a, st) : gemm_launch_vec<T, TILE_X, A_KC, B_KC, EPI, 8, 1, 8>(a, st);
+  }
+  return a.vec == 4 ? gemm_launch_vec<T, TILE_X, A_KC, B_KC, EPI, 4>(a, st) : gemm_launch_vec<T, TILE_X, A_KC, B_KC, EPI, 1>(a, st);
+}
+
 // The 256x256 tile exists for 16-byte accesses only; narrower calls are routed to the smaller tiles.
 template <typename T, int TILE, bool A_KC, bool B_KC, int EPI>
 int gemm_launch_one(const GemmArgs& a, hipStream_t st) {
+  if constexpr (TILE == TILE_X && EPI == EPI_SCORES) {
+    return gemm_launch_small<T, A_KC, B_KC, EPI>(a, st);
+  } else {
   if (a.vec == 8 && a.ring) {
     // more 256x256 tiles than compute units: one block per unit walks its share of them (at least three steps of k, the ring's
     // worth of transfers)
@@ -116,13 +135,16 @@ int gemm_launch_one(const GemmArgs& a, hipStream_t st) {
     }
     return gemm_launch_ring<T, TILE, A_KC, B_KC, EPI>(a, st);
   }
-  if constexpr (TILE == TILE_X) {
-    return fail(NMTG_ERR_UNSUPPORTED, "gemm: the 64x64 tile has a ring kernel only");
+  if constexpr (TILE == TILE_X && EPI == EPI_PLAIN) {
+    return gemm_launch_small<T, A_KC, B_KC, EPI>(a, st);
+  } else if constexpr (TILE == TILE_X) {
+    return fail(NMTG_ERR_UNSUPPORTED, "gemm: the 64x64 tile has a ring kernel only for this epilogue");
   } else {
     if (a.vec == 8) return gemm_launch_vec<T, TILE, A_KC, B_KC, EPI, 8>(a, st);
     if constexpr (TILE == TILE_L) return fail(NMTG_ERR_UNSUPPORTED, "gemm: the 256x256 tile needs 16-byte aligned operands");
     else if (a.vec == 4) return gemm_launch_vec<T, TILE, A_KC, B_KC, EPI, 4>(a, st);
     else return gemm_launch_vec<T, TILE, A_KC, B_KC, EPI, 1>(a, st);
+  }
   }
 }
 

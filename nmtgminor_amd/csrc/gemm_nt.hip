@@ -6,7 +6,7 @@ namespace nmtg {
 template <typename T> static int run(int tile, int epi, const GemmArgs& a, hipStream_t st) {
   CASE(TILE_L, EPI_PLAIN) CASE(TILE_M, EPI_PLAIN)
   CASE(TILE_L, EPI_ACT_FWD) CASE(TILE_M, EPI_ACT_FWD) CASE(TILE_X, EPI_PLAIN) CASE(TILE_X, EPI_ACT_FWD)
-  CASE(TILE_L, EPI_SCORES) CASE(TILE_M, EPI_SCORES)
+  CASE(TILE_L, EPI_SCORES) CASE(TILE_M, EPI_SCORES) CASE(TILE_X, EPI_SCORES)
   // whole-row tile with the fused softmax epilogue: 16-byte accesses only, two-buffer loop (K is one or two steps)
   if (tile == TILE_R && epi == EPI_SCORES_SOFTMAX) return gemm_launch_vec<T, TILE_R, true, true, EPI_SCORES_SOFTMAX, 8>(a, st);
   if (tile == TILE_R && epi == EPI_SCORES_SOFTMAX_RNG) return gemm_launch_vec<T, TILE_R, true, true, EPI_SCORES_SOFTMAX_RNG, 8>(a, st);

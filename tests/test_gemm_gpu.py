@@ -174,3 +174,37 @@ def test_transposed_product_without_workspace_runs_unsplit(dev):
     c, tr = _traced(lambda: gemm(a, b, True, False, split_k=False))
     assert not any("splitk" in k for k in tr), tr
     assert_close(c, _ref(a, b, True, False).cpu(), torch.float16, "unsplit", scale_atol=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(61, 73, 64), (64, 65, 63), (1, 129, 7), (61, 300, 40), (128, 64, 73), (127, 33, 1500), (37, 500, 130), (64, 64, 61)])
+@pytest.mark.parametrize("layout,pitched", [("nt", "ab"), ("nn", "bc"), ("tn", "bc"), ("nt", ""), ("nn", ""), ("tn", ""), ("nt", "abc"), ("nn", "ac")])
+def test_small_outputs_in_64x64_tiles(dev, monkeypatch, dtype, m, n, k, layout, pitched):
+    """Outputs that leave half of a larger tile empty, batched as attention batches heads: each operand and the output in rows
+    of 16-byte multiples or not. The same sums in the same order as the 128x128 tile: equal bit for bit, and right. Nothing
+    beside the output's columns is written."""
+    monkeypatch.delenv("NMTG_GEMM_TILE", raising=False)
+    ta, tb, batch = layout[0] == "t", layout[1] == "t", 3
+
+    def mk(rows, cols, wide, seed):
+        w = (cols + 7) // 8 * 8 + 8 if wide else cols
+        return _mk((batch, rows, w), dev, dtype, seed)[:, :, :cols]
+    a = mk(*((k, m) if ta else (m, k)), "a" in pitched, 41)
+    b = mk(*((n, k) if tb else (k, n)), "b" in pitched, 42)
+
+    def product():
+        w = (n + 7) // 8 * 8 + 8 if "c" in pitched else n
+        c = torch.full((batch, m, w), float("nan"), dtype=dtype, device=dev)
+        _, tr = _traced(lambda: gemm(a, b, ta, tb, alpha=0.5, out=c[:, :, :n], split_k=False))
+        assert torch.isnan(c[:, :, n:]).all()
+        (name,) = tr
+        return c[:, :, :n], name
+    small, name = product()
+    aligned = all(x.stride(0) % 8 == 0 and x.stride(1) % 8 == 0 for x in (a, b, small))
+    assert "_64x64_" in name or (aligned and name.endswith("_ring")), name
+    want = 0.5 * (a.double().cpu().transpose(1, 2) if ta else a.double().cpu()) @ (b.double().cpu().transpose(1, 2) if tb else b.double().cpu())
+    assert_close(small, want, dtype, f"{layout} {m}x{n}x{k}", scale_atol=True)
+    monkeypatch.setenv("NMTG_GEMM_TILE", "1")
+    large, name = product()
+    assert "_128x128_" in name, name
+    assert torch.equal(small, large)
