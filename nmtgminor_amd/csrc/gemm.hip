@@ -162,16 +162,24 @@ int gemm_run(int dtype, int layout, int epi, GemmArgs a, void* workspace, size_t
   const bool whole = a.K % GEMM_BK == 0 || (layout != LAYOUT_NT && (epi == EPI_PLAIN || epi == EPI_SPLITK));
   a.ring = (a.K > 0 && whole && vec == 8 && a_span < (int64_t{1} << 32) && b_span < (int64_t{1} << 32)) ? 1 : 0;
   if (few_tiles && a.ring) tile = TILE_X;
-  // Outputs that fill at most half of their tile's area, in calls outside the ring kernel (the heads of a ragged batch: an odd
-  // number of keys is an odd pitch of the probabilities): a 64x64 tile stages and multiplies half or a quarter as much per output,
-  // leaves room for four blocks on a CU and reads the operands whose own rows are aligned in 16-byte accesses. Measured against
-  // the larger tile: P V 61x64x73 of 384 heads 16.4 -> 7.1 us, 128x64x73 of 4096 114 -> 52, 127x64x1501 of 256 104 -> 53;
-  // dS^T Q 127x64x999 of 256 68 -> 42; scores 61x301x64 of 384 30 -> 19, 61x73x64 16.8 -> 11.6 (never slower).
+  // Calls outside the ring kernel, most of them heads of a ragged batch: an odd number of keys is an odd pitch of scores and
+  // probabilities. A 64x64 tile leaves room for four blocks on a CU and reads the operands whose own rows are aligned in 16-byte
+  // accesses (`wide`; the larger tiles read all as the narrowest). It takes over
+  // - outputs that leave half of the larger tile empty: P V 61x64x73 of 384 heads 16.4 -> 7.1 us, 128x64x73 of 4096 114 -> 52,
+  //   127x64x1501 of 256 104 -> 53, scores 61x301x64 of 384 30 -> 19;
+  // - a quarter, with wide accesses: dS^T Q 190x64x250 of 256 24.4 -> 17.0, scores 190x77x64 15.5 -> 12.4;
+  // - with wide accesses outputs of more than one tile that fill their 64x64 tiles: scores 511x499x64 of 256 142 -> 117,
+  //   16384x8001x512 1040 -> 412, P V 250x64x301 of 512 53 -> 40. Not where blocks of mostly empty tiles outnumber the larger ones
+  //   (scores 70x77x64 of 1024 20 -> 32, 100x127 32 -> 36), not the weight-gradient form (500x64x512 53 -> 67), and not a
+  //   row-contiguous B read by many row tiles (4096x4096x4097 903 -> 915).
   if (!a.ring && forced_tile < 0 && (epi == EPI_PLAIN || epi == EPI_SCORES) && gemm_has(layout, TILE_X, epi)) {
     int bm0, bn0;
     tile_dims(tile, bm0, bn0);
     auto padded = [&](int m, int n) { return static_cast<int64_t>(ceil_div(a.M, m)) * m * ceil_div(a.N, n) * n; };
-    if (2 * padded(64, 64) <= padded(bm0, bn0)) tile = TILE_X;
+    const int64_t small = padded(64, 64), large = padded(bm0, bn0), used = static_cast<int64_t>(a.M) * a.N;
+    const bool wide = vec < 8 && a.vec_b == 8 && (layout == LAYOUT_NT ? a.vec_a : a.vec_c) == 8;
+    const bool several = layout == LAYOUT_NT ? large > static_cast<int64_t>(bm0) * bn0 : layout == LAYOUT_NN && small <= 2048 * 4096;
+    if (2 * small <= large || (wide && (4 * small <= 3 * large || (several && 5 * used >= 4 * small)))) tile = TILE_X;
   }
   // gelu and gelu' of the activation epilogues come from a table in LDS in the ring kernels (they have the LDS room)
   a.act_lut = (a.ring && (epi == EPI_ACT_FWD || epi == EPI_ACT_BWD)) ? 1 : 0;

@@ -208,3 +208,22 @@ def test_small_outputs_in_64x64_tiles(dev, monkeypatch, dtype, m, n, k, layout, 
     large, name = product()
     assert "_128x128_" in name, name
     assert torch.equal(small, large)
+
+
+@pytest.mark.parametrize("layout,m,n,k,batch,small", [
+    ("nt", 140, 150, 64, 3, True), ("nt", 190, 77, 64, 2, True), ("nt", 127, 301, 72, 2, True), ("nt", 511, 499, 64, 1, True),
+    ("nt", 70, 77, 64, 3, False), ("nt", 100, 127, 64, 2, False), ("nt", 333, 333, 333, 2, False), ("nn", 250, 64, 301, 2, True),
+    ("nn", 140, 64, 129, 2, True), ("nn", 260, 128, 333, 2, True), ("nn", 333, 333, 333, 2, False), ("tn", 301, 64, 127, 2, True),
+    ("tn", 190, 64, 250, 2, True), ("tn", 500, 64, 132, 2, False)])
+def test_where_64x64_tiles_take_over(dev, monkeypatch, layout, m, n, k, batch, small):
+    """Both sides of the rule, contiguous operands; either tile gives the same bits."""
+    monkeypatch.delenv("NMTG_GEMM_TILE", raising=False)
+    ta, tb = layout[0] == "t", layout[1] == "t"
+    a = _mk((batch, k, m) if ta else (batch, m, k), dev, torch.bfloat16, 43)
+    b = _mk((batch, n, k) if tb else (batch, k, n), dev, torch.bfloat16, 44)
+    c, tr = _traced(lambda: gemm(a, b, ta, tb, split_k=False))
+    (name,) = tr
+    assert ("_64x64_" in name) == small, name
+    assert_close(c, _ref(a, b, ta, tb).cpu(), torch.bfloat16, layout, scale_atol=True)
+    monkeypatch.setenv("NMTG_GEMM_TILE", "1")
+    assert torch.equal(c, gemm(a, b, ta, tb, split_k=False))
