@@ -66,14 +66,14 @@ template <bool B_KC, int EPI> struct gemm_ring_ragged {
   static constexpr bool value = !B_KC && (EPI == EPI_PLAIN || EPI == EPI_SPLITK);
 };
 
-template <typename T, int TILE, bool A_KC, bool B_KC, int EPI, bool RAGGED = false, bool STREAM = false>
+template <typename T, int TILE, bool A_KC, bool B_KC, int EPI, bool RAGGED = false, bool STREAM = false, bool SUMS = false>
 int gemm_launch_ring(const GemmArgs& a, hipStream_t st) {
   using C = tile_cfg<TILE>;
   constexpr int RING = ring_slots<TILE>::value;
   constexpr bool RIDER = ring_rider<TILE, A_KC, B_KC, EPI>::value;
   auto kern = [] {
     if constexpr (RIDER) return gemm_ring_rider_kernel<T, C::BM, C::BN, C::WM, C::WN, A_KC, B_KC, EPI, RING, ring_stepbuf<TILE>::value, RAGGED, STREAM>;
-    else return gemm_ring_kernel<T, C::BM, C::BN, C::WM, C::WN, A_KC, B_KC, EPI, RING, ring_stepbuf<TILE>::value, RAGGED, STREAM>;
+    else return gemm_ring_kernel<T, C::BM, C::BN, C::WM, C::WN, A_KC, B_KC, EPI, RING, ring_stepbuf<TILE>::value, RAGGED, STREAM, SUMS>;
   }();
   constexpr int lds = gemm_ring_lds_bytes<C::BM, C::BN, RING>();
   static bool attr_done = false;
@@ -129,6 +129,12 @@ int gemm_launch_one(const GemmArgs& a, hipStream_t st) {
     if constexpr (TILE == TILE_L && EPI == EPI_PLAIN) {
       if (a.K % GEMM_BK == 0 && a.K >= 3 * GEMM_BK && a.batch == 1 && a.splits == 1 && a.m_tiles * a.n_tiles > num_cus())
         return gemm_launch_ring<T, TILE, A_KC, B_KC, EPI, false, true>(a, st);
+    }
+    // partial column sums of A on the way (gemm_run clears colsum_part in calls that do not carry them)
+    if constexpr (EPI == EPI_SPLITK && !A_KC) {
+      if (a.colsum_part != nullptr)
+        return a.K % GEMM_BK != 0 ? gemm_launch_ring<T, TILE, A_KC, B_KC, EPI, true, false, true>(a, st)
+                                  : gemm_launch_ring<T, TILE, A_KC, B_KC, EPI, false, false, true>(a, st);
     }
     if constexpr (gemm_ring_ragged<B_KC, EPI>::value) {
       if (a.K % GEMM_BK != 0) return gemm_launch_ring<T, TILE, A_KC, B_KC, EPI, true>(a, st);

@@ -187,7 +187,7 @@ struct StreamEpilogue {
 // out between the MFMAs of the remaining k-groups. The matrix pipe has work on both sides of the barrier. Phase 0
 // only reads, one more phase without reads follows the last stage; the ring positions and the vmcnt bookkeeping are
 // those of the plain loop.
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, bool A_KC, bool B_KC, int EPI, int RING, bool STEPBUF = false, bool RAGGED = false, bool STREAM = false>
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, bool A_KC, bool B_KC, int EPI, int RING, bool STEPBUF = false, bool RAGGED = false, bool STREAM = false, bool SUMS = false>
 __device__ __forceinline__ void gemm_ring_body(const GemmArgs& g, int block_x) {
   constexpr int NT = 64 * WAVES_M * WAVES_N, NW = NT / 64;
   constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N;
@@ -362,16 +362,16 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs& g, int block_x) {
   };
   zero_past_end(0, 0);
 
-  // Sums of A's columns over this block's k (EPI_SPLITK of the row-contiguous layout, g.colsum_part): the operand is in LDS
-  // anyway. The column tiles of a row of tiles read the same A, so each of them adds up every n_tiles-th stage, by all threads,
+  // SUMS: sums of A's columns over this block's k (EPI_SPLITK of the row-contiguous layout, g.colsum_part): the operand is in LDS
+  // anyway. An instantiation of its own, since the code alone made calls without sums 0.7 % slower (ffn of 513 tokens). The column tiles of a row of tiles read the same A, so each of them adds up every n_tiles-th stage, by all threads,
   // eight columns and a few k-rows each. As passes of their own over dY these sums took 34 us of a large encoder layer's
   // backward (1024 wide, 16384 tokens) and 5 of the base model's feed-forward block. Measured, whole forward and backward:
   // feed-forward 512 -> 2048, 8192 tokens, 185 -> 182 us; attention block of 1024, 16384 tokens, 807 -> 785 us.
-  constexpr bool COLSUM = EPI == EPI_SPLITK && !A_KC && !STREAM;
+  static_assert(!SUMS || (EPI == EPI_SPLITK && !A_KC && !STREAM), "column sums go with the weight gradients");
   [[maybe_unused]] float csum[8] = {};
-  [[maybe_unused]] int turn = COLSUM && g.colsum_part != nullptr ? tile_n : nk;
+  [[maybe_unused]] int turn = tile_n;
   auto column_sums = [&](int st, int pos) {
-    if constexpr (COLSUM) {
+    if constexpr (SUMS) {
       if (st != turn) return;
       turn += g.n_tiles;
       constexpr int CPK = SR / 8, CPR = BM / 8, KROWS = NT / CPR;
@@ -659,29 +659,27 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs& g, int block_x) {
     }
   }
 
-  if constexpr (COLSUM) {
-    if (g.colsum_part != nullptr) {
-      constexpr int CPR = BM / 8, KROWS = NT / CPR;
-      float* red = reinterpret_cast<float*>(lds_raw);   // [KROWS][BM]
+  if constexpr (SUMS) {
+    constexpr int CPR = BM / 8, KROWS = NT / CPR;
+    float* red = reinterpret_cast<float*>(lds_raw);   // [KROWS][BM]
 #pragma unroll
-      for (int e = 0; e < 8; ++e) red[(tid / CPR) * BM + (tid % CPR) * 8 + e] = csum[e];
-      __syncthreads();
-      for (int col = tid; col < BM; col += NT) {
-        float s = 0.f;
+    for (int e = 0; e < 8; ++e) red[(tid / CPR) * BM + (tid % CPR) * 8 + e] = csum[e];
+    __syncthreads();
+    for (int col = tid; col < BM; col += NT) {
+      float s = 0.f;
 #pragma unroll
-        for (int r = 0; r < KROWS; ++r) s += red[r * BM + col];
-        if (m0 + col < g.M) g.colsum_part[static_cast<int64_t>(split * g.n_tiles + tile_n) * g.M + m0 + col] = s;
-      }
-      __syncthreads();
+      for (int r = 0; r < KROWS; ++r) s += red[r * BM + col];
+      if (m0 + col < g.M) g.colsum_part[static_cast<int64_t>(split * g.n_tiles + tile_n) * g.M + m0 + col] = s;
     }
+    __syncthreads();
   }
   NMTG_PROF_MARK(2);
   gemm_epilogue<T, BM, BN, WAVES_M, WAVES_N, EPI, 8, true>(g, acc, lds_raw, tile_m, tile_n, bz, split);
 }
 
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, bool A_KC, bool B_KC, int EPI, int RING, bool STEPBUF = false, bool RAGGED = false, bool STREAM = false>
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, bool A_KC, bool B_KC, int EPI, int RING, bool STEPBUF = false, bool RAGGED = false, bool STREAM = false, bool SUMS = false>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_ring_kernel(const GemmArgs g) {
-  gemm_ring_body<T, BM, BN, WAVES_M, WAVES_N, A_KC, B_KC, EPI, RING, STEPBUF, RAGGED, STREAM>(g, static_cast<int>(blockIdx.x));
+  gemm_ring_body<T, BM, BN, WAVES_M, WAVES_N, A_KC, B_KC, EPI, RING, STEPBUF, RAGGED, STREAM, SUMS>(g, static_cast<int>(blockIdx.x));
 }
 
 // The same kernel with riders: the first g.rider_blocks blocks of the grid's x extent (first batch and split only) run
