@@ -62,3 +62,20 @@ def test_which_inference_calls_need_a_score_buffer(monkeypatch):
     assert [need(61, 64), need(0, 64), need(64, 32), need(64, 64, _lib.F32)] == [1, 1, 1, 1]
     monkeypatch.setenv("NMTG_ATTN_PROBS", "0")
     assert need(4, 64) == 1
+
+
+def test_build_needs_nothing_under_tests(monkeypatch):
+    """build() compiles and checks the two libraries. The CPU build of the kernels under tests/ may lack an instruction of theirs, or
+    not be there at all."""
+    import sys
+    import types
+    import __graft_entry__ as entry
+
+    def broken():
+        raise RuntimeError("hostsim: compilation failed")
+    ran = []
+    monkeypatch.setattr(entry.subprocess, "run", lambda cmd, **kw: ran.append(cmd))      # the libraries themselves are built
+    monkeypatch.setitem(sys.modules, "hostsim_build", types.SimpleNamespace(available=lambda: True, build=broken, ensure=broken))
+    monkeypatch.setattr(sys, "path", list(sys.path))
+    entry.build()
+    assert len(ran) == 1 and ran[0][0] == "make"
