@@ -233,6 +233,7 @@ int nmtg_linear_step(int64_t rows, int64_t out, int64_t in, const void* x, const
  *   act (an nmtg_act code): y = act(product + bias), or
  *   add (without gamma and act): y = add + (product + bias), clamped as nmtg_dropout_add_guard_fwd does. fp16 needs `guard`: a
  *     device int that is 0 (see clear).
+ * y and h may not overlap each other or anything that is read, except y = add.
  * nmtg_step_linear_ok: whether all products of a layer with `rows` rows are of this form (1) or take the separate calls (0). */
 int nmtg_step_linear_ok(int64_t rows, int64_t model, int64_t inner);
 int nmtg_step_linear(int64_t rows, int64_t out, int64_t in, const void* x, const void* residual, const void* gamma,

@@ -310,6 +310,19 @@ extern "C" int nmtg_step_linear(int64_t rows, int64_t out, int64_t in, const voi
   NMTG_REQUIRE(residual == nullptr || (h && aligned16(residual) && aligned16(h)), "step_linear: 16-byte aligned residual and h required");
   NMTG_REQUIRE(add == nullptr || (gamma == nullptr && act == NMTG_ACT_NONE && (guard || dtype != NMTG_F16)),
                "step_linear: the addition follows a plain product, and in fp16 needs its guard");
+  // Blocks write their columns of y, and those of the first columns h, while others still read the rows: in place only y = add,
+  // whose elements are read and written by one thread.
+  struct Span { const void* at; int64_t bytes; };
+  const Span outs[2] = {{y, rows * out * 2}, {residual != nullptr ? h : nullptr, rows * in * 2}};
+  const Span ins[7] = {{x, rows * in * 2}, {residual, rows * in * 2}, {w, out * in * 2}, {bias, out * 2}, {gamma, in * 2}, {gamma != nullptr ? beta : nullptr, in * 2},
+                       {add != y ? add : nullptr, rows * out * 2}};
+  auto meet = [](const Span& a, const Span& b) {
+    const uintptr_t p = reinterpret_cast<uintptr_t>(a.at), q = reinterpret_cast<uintptr_t>(b.at);
+    return p != 0 && q != 0 && p < q + static_cast<uintptr_t>(b.bytes) && q < p + static_cast<uintptr_t>(a.bytes);
+  };
+  for (const Span& o : outs)
+    for (const Span& i : ins) NMTG_REQUIRE(!meet(o, i), "step_linear: y and h may not overlap what is read (y = add excepted)");
+  NMTG_REQUIRE(!meet(outs[0], outs[1]), "step_linear: y and h may not overlap");
   StepArgs g{x, residual, gamma, beta, w, bias, add, h, y, clear, guard, static_cast<int>(rows), static_cast<int>(out), static_cast<int>(in), act, sk_cols(static_cast<int>(rows), static_cast<int>(in)), eps};
   hipStream_t st = static_cast<hipStream_t>(stream);
   auto run = [&](auto t) {

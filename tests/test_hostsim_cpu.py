@@ -46,6 +46,7 @@ import test_zzd_fused_optim_gpu as topt  # noqa: E402
 import test_zze_flash_attention_gpu as tfl  # noqa: E402
 import test_zzf_feed_forward_gpu as tff  # noqa: E402
 import test_zzg_attention_no_coverage_gpu as tnc  # noqa: E402
+import test_zzm_step_linear_gpu as tsl  # noqa: E402
 
 pytestmark = pytest.mark.skipif(not hostsim_build.available(), reason="no host C++ compiler with __bf16 (ROCm clang++)")
 CPU = torch.device("cpu")
@@ -743,6 +744,10 @@ def test_split_k_epilogue_without_a_workspace_is_refused_before_any_launch(hosts
 def test_few_row_products(monkeypatch, mi355x, m, n, k):
     monkeypatch.delenv("NMTG_GEMM_SKINNY")
     tst.test_few_row_products_match_the_tiled_kernels(CPU, BF16, m, n, k)
+
+
+def test_step_products_refuse_outputs_over_inputs(mi355x):
+    tsl.test_outputs_over_inputs_are_refused(CPU)
 
 
 @pytest.mark.parametrize("dtype", HALVES)

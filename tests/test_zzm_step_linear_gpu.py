@@ -12,11 +12,11 @@ pytestmark = pytest.mark.gpu
 ACTS = {"none": lambda v: v, "relu": torch.relu, "gelu": lambda v: 0.5 * v * (1 + torch.erf(v / math.sqrt(2))), "silu": lambda v: v * torch.sigmoid(v)}
 
 
-def step(x, w, bias, dtype, *, residual=None, gamma=None, beta=None, act="none", add=None):
+def step(x, w, bias, dtype, *, residual=None, gamma=None, beta=None, act="none", add=None, y=None, h=None):
     rows, out = x.shape[0], w.shape[0]
     dev = x.device
-    y = torch.full((rows, out), 7.0, dtype=dtype, device=dev)
-    h = torch.full_like(x, 7.0) if residual is not None else None
+    y = torch.full((rows, out), 7.0, dtype=dtype, device=dev) if y is None else y
+    h = torch.full_like(x, 7.0) if residual is not None and h is None else h
     clear = torch.full((1,), 5, dtype=torch.int32, device=dev) if gamma is not None else None
     guard = torch.zeros(1, dtype=torch.int32, device=dev) if add is not None else None
     L.call("nmtg_step_linear", L.i64(rows), L.i64(out), L.i64(x.shape[1]), L.ptr(x), L.ptr(residual), L.ptr(gamma), L.ptr(beta), L.f32(1e-5),
@@ -82,3 +82,21 @@ def test_product_and_guarded_addition(dev, dtype, rows, out, k, spoilt):
             keep[at] = False
         y, want = y[keep], want[keep.to(want.device)]
     close(y, want, dtype, f"{rows} x {out} x {k}")
+
+
+def test_outputs_over_inputs_are_refused(dev):
+    """One block's outputs are other blocks' inputs: such calls are refused whatever their size, whole or in part. y = add stays."""
+    dtype = torch.bfloat16
+    t = tensors(dev, dtype, 5, 512, 512, 1)
+    norm = dict(gamma=t["gamma"], beta=t["beta"])
+    both = torch.zeros(8, 512, dtype=dtype, device=dev)                       # two overlapping tensors of five rows
+    low, high = both[:5], both[3:]
+    for kw in (dict(residual=t["residual"], h=t["residual"], **norm), dict(residual=t["residual"], h=t["x"], **norm),
+               dict(residual=t["residual"], y=t["residual"], **norm), dict(residual=t["residual"], y=t["x"], **norm), dict(y=t["x"], **norm), dict(y=t["x"]),
+               dict(residual=low, h=high, **norm), dict(residual=t["residual"], y=low, h=high, **norm), dict(add=low, y=high), dict(y=t["w"][:5]),
+               dict(residual=t["residual"], h=t["w"][-5:], **norm)):
+        with pytest.raises(RuntimeError, match="overlap"):
+            step(t["x"], t["w"], t["bias"], dtype, **kw)
+    want = t["add"].double() + (t["x"].double() @ t["w"].double().t()).to(dtype).double()
+    y, _ = step(t["x"], t["w"], None, dtype, add=t["add"], y=t["add"])
+    close(y, want, dtype, "y = add")
