@@ -96,17 +96,17 @@ int gemm_run(int dtype, int layout, int epi, GemmArgs a, void* workspace, size_t
   // enter: a ragged M / N / K ends in a predicated last vector (loads stay inside the row's pitch, which is a multiple
   // of the vector; the K tail is zeroed; the stores of a partial vector and the bias of a ragged last tile go element
   // by element). Byte masks are addressed as row * N + n, so there N is the pitch and does count.
-  auto narrow = [](int& vec, const void* p, int64_t ld, int64_t stride, int batch) { vec = std::min(vec, vec_of(p, ld, stride, batch)); };
-  a.vec_a = vec_of(a.A, a.lda, a.sA, a.batch);
-  a.vec_b = vec_of(a.B, a.ldb, a.sB, a.batch);
-  a.vec_c = vec_of(a.C, a.ldc, a.sC, a.batch);
+  auto narrow = [](int8_t& vec, const void* p, int64_t ld, int64_t stride, int batch) { vec = static_cast<int8_t>(std::min<int>(vec, vec_of(p, ld, stride, batch))); };
+  a.vec_a = static_cast<int8_t>(vec_of(a.A, a.lda, a.sA, a.batch));
+  a.vec_b = static_cast<int8_t>(vec_of(a.B, a.ldb, a.sB, a.batch));
+  a.vec_c = static_cast<int8_t>(vec_of(a.C, a.ldc, a.sC, a.batch));
   if (a.aux_out) narrow(a.vec_c, a.aux_out, a.ldc, a.sC, a.batch);
   if (a.bias) narrow(a.vec_c, a.bias, 8, 0, 1);
   if (a.aux_in) narrow(a.vec_c, a.aux_in, a.ld_aux, 0, 1);
   auto narrow_bytes = [&](const uint8_t* p) {
     int v = 8;
     while (v > 1 && (reinterpret_cast<uintptr_t>(p) % v != 0 || a.N % v != 0)) v = v == 8 ? 4 : 1;
-    a.vec_c = std::min(a.vec_c, v);
+    a.vec_c = static_cast<int8_t>(std::min<int>(a.vec_c, v));
   };
   if (a.dmask) narrow_bytes(a.dmask);
   if (a.kmask && a.kmask_kind != 0) narrow_bytes(a.kmask);
@@ -192,7 +192,7 @@ int gemm_run(int dtype, int layout, int epi, GemmArgs a, void* workspace, size_t
     return fail(NMTG_ERR_UNSUPPORTED, "gemm: grid too large (tiles %d x %d, batch %d)", a.m_tiles, a.n_tiles, a.batch);
   if (epi == EPI_SPLITK && a.ws == nullptr)
     return fail(NMTG_ERR_INVALID, "gemm: the split-K epilogue needs a workspace");
-  a.tile_used = tile;
+  a.tile_used = static_cast<int8_t>(tile);
   if (epi != EPI_SPLITK) a.defer_reduce = 0;
   // riders travel with the kernels that ring_rider<> (gemm_inst.hip.h) names, and only in an unbatched launch
   const bool can_ride = (tile == TILE_M || tile == TILE_X) && a.vec == 8 && a.ring && a.batch == 1 && layout == LAYOUT_NN && epi == EPI_PLAIN;

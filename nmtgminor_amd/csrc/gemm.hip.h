@@ -62,7 +62,6 @@ struct GemmArgs {
   int splits, k_per_split;
   float alpha;
   int vec;                  // widest access (elements: 8, 4 or 1) every operand and extent allows
-  int vec_a, vec_b, vec_c;  // the same of A, of B, and of C with all that the epilogue reads
   int ring;                 // the call meets the requirements of the slot-ring kernel (gemm_ring.hip.h)
   const void* bias;
   void* aux_out;
@@ -75,20 +74,21 @@ struct GemmArgs {
   uint64_t seed, offset;
   int act;
   int act_lut;              // gelu / gelu' through the LDS table (ring kernels only; set by the host on request)
-  int defer_reduce;         // host only: a split-K call leaves its reduction to the caller (who queues it in a ReduceTail)
-  int tile_used;            // host only, filled by gemm_run: the tile the call ran with
-  int skinny_rows;          // host only: the largest row count for the few-row kernel (0: its own block of 32)
+  int8_t defer_reduce;      // host only: a split-K call leaves its reduction to the caller (who queues it in a ReduceTail)
+  int8_t tile_used;         // host only, filled by gemm_run: the tile the call ran with
+  int8_t skinny_rows;       // host only: the largest row count for the few-row kernel (0: its own block of 32)
+  int8_t riders_taken;      // host only, see riders
+  int colsum_cap, colsum_rows;   // host only, see colsum_part
   // host only: a list of small reduction jobs (TailArgs, reduce.hip.h) that `rider_blocks` extra blocks of this launch
   // run beside the GEMM's own blocks (they have no part in the product; what they read must be complete before the
   // launch). Kernels that cannot carry them leave riders_taken at 0 and the caller launches the list itself.
   const void* riders;
   int rider_blocks;
-  int riders_taken;
+  int8_t vec_a, vec_b, vec_c;    // host only: `vec` of A, of B, and of C with all that the epilogue reads
   // Partial column sums [rows][M or N] in fp32. EPI_ACT_BWD: of the result, one row per row tile. Split-K calls of the TN layout:
-  // of A over its rows (dY^T 1 beside dW = dY^T X), one row per column tile and split; host: up to colsum_cap rows fit, and
-  // gemm_run reports in colsum_rows how many were written (0: the kernel of this call does not carry them).
+  // of A over its rows (dY^T 1 beside dW = dY^T X), one row per column tile and split; up to colsum_cap rows fit, and gemm_run
+  // reports in colsum_rows how many were written (0: the kernel of this call does not carry them).
   float* colsum_part;
-  int colsum_cap, colsum_rows;
   const uint8_t* kmask;
   int kmask_kind, heads;
   float* ws;
@@ -97,6 +97,11 @@ struct GemmArgs {
   long long* prof;          // per-block phase timestamps (tuning builds only)
 #endif
 };
+#ifndef NMTG_GEMM_PROF
+// Every block fetches these from memory that the host wrote, and a launch with riders the job list behind them: with 24 bytes more,
+// in fields that no kernel reads, a feed-forward block of 513 tokens (1024 to 4096, fp16) took 136.7 us and not 136.1.
+static_assert(sizeof(GemmArgs) == 272, "host-only fields go into bytes that are there");
+#endif
 
 #ifdef NMTG_GEMM_PROF
 // slots 0..4: shader-clock stamps of the phases; slots 5 and 6: constant-rate (100 MHz) stamps of the block's start and end

@@ -258,7 +258,7 @@ int step_launch(const StepArgs& g, hipStream_t st) {
 bool gemm_skinny_ok(int dtype, int layout, int epi, const GemmArgs& a) {
   if (switched_off("NMTG_GEMM_SKINNY")) return false;
   return (dtype == NMTG_F16 || dtype == NMTG_BF16) && layout == LAYOUT_NT && epi == EPI_PLAIN && a.batch == 1 && a.M >= 1 &&
-         a.M <= (a.skinny_rows != 0 ? std::min(a.skinny_rows, SK_MAX_ROWS) : SK_ROWS) && a.N >= 64 && a.K >= 8 && a.K % 8 == 0 && a.lda % 8 == 0 && a.ldb % 8 == 0 && aligned16(a.A) &&
+         a.M <= (a.skinny_rows != 0 ? std::min<int>(a.skinny_rows, SK_MAX_ROWS) : SK_ROWS) && a.N >= 64 && a.K >= 8 && a.K % 8 == 0 && a.lda % 8 == 0 && a.ldb % 8 == 0 && aligned16(a.A) &&
          aligned16(a.B);
 }
 
