@@ -169,16 +169,23 @@ int gemm_run(int dtype, int layout, int epi, GemmArgs a, void* workspace, size_t
   //   127x64x1501 of 256 104 -> 53, scores 61x301x64 of 384 30 -> 19;
   // - a quarter, with wide accesses: dS^T Q 190x64x250 of 256 24.4 -> 17.0, scores 190x77x64 15.5 -> 12.4;
   // - with wide accesses outputs of more than one tile that fill their 64x64 tiles: scores 511x499x64 of 256 142 -> 117,
-  //   16384x8001x512 1040 -> 412, P V 250x64x301 of 512 53 -> 40. Not where blocks of mostly empty tiles outnumber the larger ones
-  //   (scores 70x77x64 of 1024 20 -> 32, 100x127 32 -> 36), not the weight-gradient form (500x64x512 53 -> 67), and not a
-  //   row-contiguous B read by many row tiles (4096x4096x4097 903 -> 915).
+  //   16384x8001x512 1040 -> 400, P V 250x64x301 of 512 53 -> 40. Not where blocks of mostly empty tiles outnumber the larger ones
+  //   (scores 70x77x64 of 1024 20 -> 32, 100x127 32 -> 36), and not the weight-gradient form (500x64x512 53 -> 67).
+  // With a row-contiguous B (the last form in the layout NN) 128x128 tiles that come out even on the CUs, at least two on each,
+  // are ahead in long reductions: 2048x4096 outputs (two each), 64x64 / 128x128: k 301 37 / 44 us, 1001 103 / 112, 1501 166 / 168, 2001
+  // 220 / 217, 6001 655 / 617, 8001 933 / 897. One on each (2048x2048: 1001 56 / 69, 6001 347 / 393), an uneven last round (3072x2048:
+  // 1501 129 / 165, 6001 506 / 613) and 256x64 tiles (2000x64x4001 of 64 538 / 619) lose at any k. Above 2048x4096 outputs the
+  // larger tile stays: 16384x1024x1501 321 / 323, 4096x8192x1501 635 / 625, x4097 1824 / 1773.
   if (!a.ring && forced_tile < 0 && (epi == EPI_PLAIN || epi == EPI_SCORES) && gemm_has(layout, TILE_X, epi)) {
     int bm0, bn0;
     tile_dims(tile, bm0, bn0);
     auto padded = [&](int m, int n) { return static_cast<int64_t>(ceil_div(a.M, m)) * m * ceil_div(a.N, n) * n; };
     const int64_t small = padded(64, 64), large = padded(bm0, bn0), used = static_cast<int64_t>(a.M) * a.N;
     const bool wide = vec < 8 && a.vec_b == 8 && (layout == LAYOUT_NT ? a.vec_a : a.vec_c) == 8;
-    const bool several = layout == LAYOUT_NT ? large > static_cast<int64_t>(bm0) * bn0 : layout == LAYOUT_NN && small <= 2048 * 4096;
+    const int64_t blocks = static_cast<int64_t>(ceil_div(a.M, bm0)) * ceil_div(a.N, bn0) * a.batch, cus = num_cus();
+    const bool even = tile == TILE_M && blocks > cus && 10 * blocks > 9 * ((blocks + cus - 1) / cus * cus);
+    const bool several = layout == LAYOUT_NT ? large > static_cast<int64_t>(bm0) * bn0
+                                             : layout == LAYOUT_NN && small <= 2048 * 4096 && !(even && a.K > 1536);
     if (2 * small <= large || (wide && (4 * small <= 3 * large || (several && 5 * used >= 4 * small)))) tile = TILE_X;
   }
   // gelu and gelu' of the activation epilogues come from a table in LDS in the ring kernels (they have the LDS room)

@@ -214,7 +214,10 @@ def test_small_outputs_in_64x64_tiles(dev, monkeypatch, dtype, m, n, k, layout, 
     ("nt", 140, 150, 64, 3, True), ("nt", 190, 77, 64, 2, True), ("nt", 127, 301, 72, 2, True), ("nt", 511, 499, 64, 1, True),
     ("nt", 70, 77, 64, 3, False), ("nt", 100, 127, 64, 2, False), ("nt", 333, 333, 333, 2, False), ("nn", 250, 64, 301, 2, True),
     ("nn", 140, 64, 129, 2, True), ("nn", 260, 128, 333, 2, True), ("nn", 333, 333, 333, 2, False), ("tn", 301, 64, 127, 2, True),
-    ("tn", 190, 64, 250, 2, True), ("tn", 500, 64, 132, 2, False)])
+    ("tn", 190, 64, 250, 2, True), ("tn", 500, 64, 132, 2, False),
+    # 128x128 tiles, two for each of 256 compute units, at either side of k = 1536; one each; an uneven second round; 256x64 tiles
+    ("nn", 2048, 4096, 1535, 1, True), ("nn", 2048, 4096, 1537, 1, False), ("nn", 512, 512, 1601, 32, False), ("nn", 2048, 2048, 1601, 1, True),
+    ("nn", 3072, 2048, 1601, 1, True), ("nn", 2000, 64, 1601, 4, True)])
 def test_where_64x64_tiles_take_over(dev, monkeypatch, layout, m, n, k, batch, small):
     """Both sides of the rule, contiguous operands; either tile gives the same bits."""
     monkeypatch.delenv("NMTG_GEMM_TILE", raising=False)
