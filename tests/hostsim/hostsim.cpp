@@ -403,6 +403,15 @@ int compute_units() {
   return n > 0 ? n : 4;
 }
 
+int device() {
+  static std::vector<int> seen;
+  const int n = compute_units();
+  for (size_t i = 0; i < seen.size(); ++i)
+    if (seen[i] == n) return static_cast<int>(i);
+  seen.push_back(n);
+  return static_cast<int>(seen.size()) - 1;
+}
+
 void launch(dim3 grid, dim3 block, size_t dynamic_lds_bytes, const std::function<void()>& body) {
   const uint64_t nthreads = static_cast<uint64_t>(block.x) * block.y * block.z;
   if (nthreads == 0 || nthreads > MAX_THREADS) { std::fprintf(stderr, "hostsim: block of %llu threads\n", (unsigned long long)nthreads); std::abort(); }

@@ -57,6 +57,7 @@ void sync_block();
 void dma_issue(const void* src, uint32_t lds_offset, int bytes);
 void dma_wait(int may_stay_outstanding);
 uint32_t lds_offset_of(uint32_t low_address_bits);   // LDS byte offset from the low 32 bits of a pointer into LDS
+int device();            // another one for every number of compute units: the library asks a device for it once
 int compute_units();     // HOSTSIM_CUS (default 4): small, so that grid-stride loops take several trips
 extern unsigned char* dynamic_lds;   // at least dynamic_lds_bytes of the current launch
 }  // namespace hostsim
@@ -69,7 +70,7 @@ static inline long long clock64() { return 0; }
 static inline long long wall_clock64() { return 0; }
 static inline hipError_t hipGetLastError() { return hipSuccess; }
 static inline const char* hipGetErrorString(hipError_t) { return "host simulation"; }
-static inline hipError_t hipGetDevice(int* dev) { *dev = 0; return hipSuccess; }
+static inline hipError_t hipGetDevice(int* dev) { *dev = hostsim::device(); return hipSuccess; }
 static inline hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { *v = hostsim::compute_units(); return hipSuccess; }
 
 #define HIP_SYMBOL(x) x
