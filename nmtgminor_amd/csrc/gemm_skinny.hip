@@ -24,14 +24,18 @@ constexpr int SK_ROWS = 32, SK_WAVES = 8, SK_THREADS = 64 * SK_WAVES, SK_CHUNK =
 // with the other.
 constexpr int SK_MAX_ROWS = 64;
 
-// Columns per block: 32, and fewer of long rows of W, which one compute unit fetches slowly ([512 x 2048]: 16 blocks take 7.4 us, 64
-// blocks 3.5). More blocks read (and normalise, below) the same rows of X again, so the more rows the fewer. Steps of a
+// Columns per block: 32, and fewer of long rows of W, which one compute unit fetches slowly, while there is a compute unit for each
+// block. More blocks read (and normalise, below) the same rows of X again, so the more rows the fewer. Steps of a
 // decoder layer as a graph with at most 8192 / 16384 / 32768 elements of W per block: 5 rows, E = 512: 35.3 / 36.9 / 37.1 us (38.9 with 32
 // columns throughout); 20 rows, E = 1024: 64.0 / 63.2 / 67.2 (70.6); 64 rows, E = 1024: 99.7 / 82.9 / 74.5 (77.7). The sums are the same.
-inline int sk_cols(int rows, int k) {
+// Products alone, each call on a weight that is in no cache, us with 32 / 16 / 8 columns on 256 compute units: [512 x 2048], 8 rows:
+// 8.1 / 6.3 / 5.8; [2048 x 1024]: 5.5 / 4.7 / 4.5 (256 blocks of 8); [4096 x 1024]: 5.6 / 5.0 / 6.1 (512 of 8); [8192 x 1024]: 6.6 / 7.1 / 9.6;
+// [32000 x 1024]: 20 / 23 / 29, 32 rows 28 / 38 / 59.
+inline int sk_cols(int rows, int n, int k) {
   const int64_t most = rows <= 8 ? 8192 : rows <= SK_ROWS ? 16384 : 32768;
+  const int64_t cus = num_cus(), row_blocks = (rows + SK_ROWS - 1) / SK_ROWS;
   int cols = 32;
-  while (cols > 8 && static_cast<int64_t>(cols) * k > most) cols /= 2;
+  while (cols > 8 && static_cast<int64_t>(cols) * k > most && (n + static_cast<int64_t>(cols) / 2 - 1) / (cols / 2) * row_blocks <= cus) cols /= 2;
   return cols;
 }
 
@@ -263,7 +267,7 @@ bool gemm_skinny_ok(int dtype, int layout, int epi, const GemmArgs& a) {
 }
 
 int gemm_skinny_run(int dtype, const GemmArgs& a, hipStream_t st) {
-  const int cols = sk_cols(a.M, a.K);
+  const int cols = sk_cols(a.M, a.N, a.K);
   const dim3 grid(static_cast<unsigned>((a.N + cols - 1) / cols), static_cast<unsigned>((a.M + SK_ROWS - 1) / SK_ROWS));
   TraceScope trace("gemm_nt_skinny", st);
   if (dtype == NMTG_F16) hipLaunchKernelGGL((gemm_skinny_kernel<f16_t>), grid, dim3(SK_THREADS), 0, st, a, cols);
@@ -323,7 +327,8 @@ extern "C" int nmtg_step_linear(int64_t rows, int64_t out, int64_t in, const voi
   for (const Span& o : outs)
     for (const Span& i : ins) NMTG_REQUIRE(!meet(o, i), "step_linear: y and h may not overlap what is read (y = add excepted)");
   NMTG_REQUIRE(!meet(outs[0], outs[1]), "step_linear: y and h may not overlap");
-  StepArgs g{x, residual, gamma, beta, w, bias, add, h, y, clear, guard, static_cast<int>(rows), static_cast<int>(out), static_cast<int>(in), act, sk_cols(static_cast<int>(rows), static_cast<int>(in)), eps};
+  StepArgs g{x, residual, gamma, beta, w, bias, add, h, y, clear, guard, static_cast<int>(rows), static_cast<int>(out), static_cast<int>(in), act,
+             sk_cols(static_cast<int>(rows), static_cast<int>(out), static_cast<int>(in)), eps};
   hipStream_t st = static_cast<hipStream_t>(stream);
   auto run = [&](auto t) {
     using T = decltype(t);

@@ -43,6 +43,9 @@ extern "C" int64_t nmtg_trace_end(char* out, int64_t capacity) {
 
 using namespace nmtg;
 
+// blocks of the last launch
+extern "C" int64_t hostsim_last_blocks(void) { return static_cast<int64_t>(gridDim.x) * gridDim.y * gridDim.z; }
+
 extern "C" int hostsim_colsum_parts(int M) { return colsum_parts(M); }
 
 extern "C" int hostsim_colsum(int dtype, const void* X, int64_t ld, int M, int N, float* part, void* out) {

@@ -746,6 +746,22 @@ def test_few_row_products(monkeypatch, mi355x, m, n, k):
     tst.test_few_row_products_match_the_tiled_kernels(CPU, BF16, m, n, k)
 
 
+@pytest.mark.parametrize("rows,n,k,cus,blocks", [(5, 64, 1024, 8, 8), (5, 64, 1024, 7, 4), (5, 256, 1024, 8, 8), (5, 100, 512, 8, 7), (32, 64, 1024, 8, 4),
+                                                 (33, 64, 4096, 16, 16), (33, 64, 4096, 15, 8), (64, 128, 128, 64, 8)])
+def test_few_row_products_narrow_their_blocks_only_while_the_chip_is_not_full(hostsim_lib, monkeypatch, rows, n, k, cus, blocks):
+    """Blocks of 8 or 16 columns where rows of W are long, and no more blocks than compute units unless 32 columns need them."""
+    from nmtgminor_amd import _lib as L
+    monkeypatch.delenv("NMTG_GEMM_SKINNY")
+    monkeypatch.setenv("HOSTSIM_CUS", str(cus))
+    g = torch.Generator().manual_seed(rows + n)
+    x, w = torch.randn(rows, k, generator=g).to(BF16), (torch.randn(n, k, generator=g) * k ** -0.5).to(BF16)
+    y = torch.empty(rows, n, dtype=BF16)
+    L.call("nmtg_linear_step", L.i64(rows), L.i64(n), L.i64(k), L.ptr(x), L.ptr(w), None, L.ptr(y), L.i32(L.dtype_code(x)), None)
+    hostsim_lib.hostsim_last_blocks.restype = ctypes.c_int64
+    assert hostsim_lib.hostsim_last_blocks() == blocks
+    tat.assert_close(y, x.double() @ w.double().t(), BF16, "few rows")
+
+
 def test_step_products_refuse_outputs_over_inputs(mi355x):
     tsl.test_outputs_over_inputs_are_refused(CPU)
 
