@@ -17,6 +17,7 @@ import os
 import pytest
 import torch
 
+from nmtgminor_amd import _lib
 from nmtgminor_amd.native import encdec_multihead_attn_bias_blaslt as ed_native, fused_mlp_gelu, self_multihead_attn_blaslt as sa_native
 from nmtgminor_amd.native.linear_gemm import gemm
 from oracle import attention as oat, inputs, mlp as omlp
@@ -276,36 +277,51 @@ def test_few_row_products_match_the_tiled_kernels(dev, dtype, m, n, k):
     assert torch.equal(gemm(pitched[:, :k], w, False, True, alpha=0.5, bias=bias), got)
 
 
+def _attention_backward(dev, dtype, tq, tk, b, h, mask, p, seed):
+    """-> a function that runs the backward of one call with heads in the slots of a projection: ([dq, dk / dv, rowsum(dO O)], kernels)"""
+    from nmtgminor_amd.native import flash_attn_cuda as fa
+    g = torch.Generator().manual_seed(seed)
+    qs = torch.randn(tq, b, h, 3, 64, generator=g).to(dtype).to(dev)
+    ks = torch.randn(tk, b, h, 3, 64, generator=g).to(dtype).to(dev)
+    q, k, v = qs[..., 0, :], ks[..., 1, :], ks[..., 2, :]
+    dout = torch.randn(tq, b, h, 64, generator=g).to(dtype).to(dev)
+    pad = (torch.rand(b, tk, generator=g) < 0.3).to(torch.uint8).to(dev) if mask == "padding" else None
+    time = (torch.rand(tq, tk, generator=g) < 0.3).to(torch.uint8).to(dev) if mask == "time" else None
+    out, lse, state = fa.fwd_batched(q, k, v, pad, p, 0.125, mask == "causal", time_mask=time)
+
+    def grads():
+        dqs, dks = torch.full_like(qs, 7.0), torch.full_like(ks, 7.0)
+        _lib.trace_begin()
+        delta = fa.bwd_batched(dout, q, k, v, out, lse, dqs[..., 0, :], dks[..., 1, :], dks[..., 2, :], pad, p, 0.125, mask == "causal", state,
+                               time_mask=time)
+        names = {n for n in _lib.trace_end() if n.startswith("flash_attn_bwd")}
+        return [x.double().cpu() for x in (dqs, dks, delta)], names
+    return grads
+
+
+ONE, TWO = {"flash_attn_bwd"}, {"flash_attn_bwd_dq", "flash_attn_bwd_dkv"}
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("mask", ["none", "padding", "time", "causal"])
 @pytest.mark.parametrize("p", [0.0, 0.2])
-def test_attention_backward_in_one_kernel_matches_the_two_kernels(dev, dtype, mask, p):
-    """At the edges of the one kernel's steps (32 queries), groups (32 keys) and block sizes (128 and 256 keys), and with heads
-    next to each other or in the slots of a projection. Both forms sum the same products in fp32, in another order: a result
+def test_attention_backward_in_one_kernel_matches_the_two_kernels(dev, dtype, mask, p, shapes=None):
+    """At the edges of the one kernel's steps (32 queries, up to 16 of them), groups (32 keys) and block sizes (128 keys, 256 with more
+    heads than compute units, 512), and with heads next to each other or in the slots of a projection. Both forms sum the same
+    products in fp32, in another order: a result
     differs where the two sums (relative distance d) fall on either side of a rounding boundary, which befalls a share d / eps
     of the elements with eps each, sqrt(d eps) in the 2-norm; the same holds for the rounded operand dS. d: one unit of fp32 per
     term. Few of a small tensor's elements decide, hence the factor."""
-    from nmtgminor_amd.native import flash_attn_cuda as fa
     eps = torch.finfo(dtype).eps
-    for n, (tq, tk, b, h) in enumerate([(1, 1, 1, 1), (31, 33, 2, 3), (33, 65, 1, 2), (64, 128, 2, 2), (65, 129, 1, 2), (40, 300, 2, 1), (256, 257, 1, 2),
-                                        (96, 512, 1, 2), (512, 64, 1, 1)]):
-        g = torch.Generator().manual_seed(700 + n)
-        qs = torch.randn(tq, b, h, 3, 64, generator=g).to(dtype).to(dev)
-        ks = torch.randn(tk, b, h, 3, 64, generator=g).to(dtype).to(dev)
-        q, k, v = qs[..., 0, :], ks[..., 1, :], ks[..., 2, :]
-        dout = torch.randn(tq, b, h, 64, generator=g).to(dtype).to(dev)
-        pad = (torch.rand(b, tk, generator=g) < 0.3).to(torch.uint8).to(dev) if mask == "padding" else None
-        time = (torch.rand(tq, tk, generator=g) < 0.3).to(torch.uint8).to(dev) if mask == "time" else None
-        out, lse, state = fa.fwd_batched(q, k, v, pad, p, 0.125, mask == "causal", time_mask=time)
-
-        def grads():
-            dqs, dks = torch.full_like(qs, 7.0), torch.full_like(ks, 7.0)
-            delta = fa.bwd_batched(dout, q, k, v, out, lse, dqs[..., 0, :], dks[..., 1, :], dks[..., 2, :], pad, p, 0.125, mask == "causal", state,
-                                   time_mask=time)
-            return [x.double().cpu() for x in (dqs, dks, delta)]
-        one = grads()
+    for n, (tq, tk, b, h) in enumerate(shapes or [
+            (1, 1, 1, 1), (31, 33, 2, 3), (33, 65, 1, 2), (64, 128, 2, 2), (65, 129, 1, 2), (40, 300, 2, 1), (256, 257, 1, 2), (96, 512, 1, 2),
+            (257, 129, 33, 8), (300, 200, 20, 16), (512, 256, 18, 16), (257, 257, 10, 16), (512, 500, 10, 16)]):
+        grads = _attention_backward(dev, dtype, tq, tk, b, h, mask, p, 700 + n)
+        one, names = grads()
+        assert names == ONE, (tq, tk, b, h, names)
         with off("NMTG_ATTN_BWD_ONE"):
-            two = grads()
+            two, names = grads()
+        assert names == TWO, (tq, tk, b, h, names)
         for x, y, name in zip(one, two, ("dq", "dk / dv", "rowsum(dO O)")):
             what = f"{name} {tq} x {tk}"
             assert torch.isfinite(x).all(), what
