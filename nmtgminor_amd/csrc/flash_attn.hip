@@ -28,6 +28,7 @@
 // decisions of the extension modules' numbering (mode 3: element (i, j) uses word e % 4 of the Philox block e / 4,
 // e = ((b H + h) max_q + i) max_k + j, and is kept when word / 2^32 < 1 - p), for calls that return the probabilities.
 #include "gemm_ring.hip.h"
+#include <algorithm>
 
 namespace nmtg {
 namespace {
@@ -1940,17 +1941,32 @@ int bwd_one_launch(const FaArgs& a, int drop, int64_t batch, hipStream_t st) {
 }
 // Which calls take it: head dimension 64, keys that eight wavefronts hold, queries whose statistics fit the LDS, row strides
 // that 32-bit lane offsets reach over a step's rows. A block walks all queries of its head, so where queries are many and
-// heads few the two kernels' many short blocks are done first: [512 x 512], 64 / 128 / 192 / 256 heads: two kernels 53 / 67 / 101 /
-// 119 us, one 71 / 75 / 77 / 80; [512 x 128]: 39 / 44 / 52 / 58 against 42 / 46 / 49 / 49. With at most 256 queries the one kernel is
-// level or ahead at any number of heads ([128 x 512], 8 heads: 25 against 24; [256 x 256], 64 heads: 30 against 27; [256 x 64], 64
-// heads: 23 and 24).
-bool bwd_in_one(const FaArgs& a, int64_t batch, int64_t d) {
+// heads few the two kernels' many short blocks are done first. Measured in bf16, us as two kernels / one:
+// - more than 256 queries: [512 x 512], 64 / 128 / 192 / 256 heads, dropout: 53 / 71, 67 / 75, 101 / 77, 119 / 80.
+// Sequences that fill their tiles have no masked tile, which the two kernels pay for; for them also
+// - [256 x 256], dropout: 8 heads 22 / 25, 64 23 / 26, 128 28 / 28; without: 19 / 23, 21 / 25, 128 heads 24 / 26, 152 31 / 26;
+//   [256 x 512], dropout: 8 heads 28 / 38, 64 36 / 39, 128 44 / 43; [192 x 128]: 64 heads 18 / 20; but [160 x 256], 8 heads: 20 / 19, [200 x
+//   200]: 27 / 23, and with a causal flag [256 x 256], 8 heads: 26 / 23, with two or more padded sequences, 64 heads: 31 / 29;
+// - many queries on 97 to 128 keys (four wavefronts per block): [384 x 128], dropout: 160 heads 31 / 36, 192 38 / 37;
+// - without dropout, a second round of blocks that few heads reach: [512 x 512], 256 / 320 / 384 heads: 95 / 75, 116 / 136, 135 / 138.
+bool bwd_in_one(const FaArgs& a, int64_t batch, int64_t d, bool drop) {
   constexpr int64_t far = 1 << 25;
   if (d != 64 || a.max_q <= 0 || a.max_k <= 0 || a.max_q > FB_MAX_Q || a.max_k > 512) return false;
-  if (a.q_st > far || a.do_st > far || a.dq_st > far) return false;
-  if (a.max_q > 256 && 5 * batch * a.heads < 3 * num_cus()) return false;
-  const char* off = getenv("NMTG_ATTN_BWD_ONE");
-  return off == nullptr || off[0] != '0';
+  if (a.q_st > far || a.do_st > far || a.dq_st > far || switched_off("NMTG_ATTN_BWD_ONE")) return false;
+  const int64_t heads = batch * a.heads, cus = num_cus();
+  if (a.max_q > 256 && 5 * heads < 3 * cus) return false;
+  if (a.causal || a.tmask != nullptr) return true;
+  const bool uniform = batch == 1 || (a.pad == nullptr && a.cu_q == nullptr);
+  if (a.max_q > 256) {
+    if (!uniform) return true;
+    if (a.max_k > 96 && a.max_k <= 128) return drop ? 8 * heads > 5 * cus : 4 * heads > 3 * cus;
+    return drop || a.max_k <= 320 || heads <= cus || 4 * heads > 5 * cus;
+  }
+  const int key_blocks = (a.max_k + FA_ROWS - 1) / FA_ROWS, unit = a.max_q > 224 && key_blocks != 2 ? FA_TILE : FA_ROWS;
+  if (a.max_q <= 160 || (a.max_k - 1) % unit < unit - 16) return true;   // the last tile of keys is not full
+  if (!uniform) return a.max_q <= 224 || key_blocks != 4 || a.pad == nullptr || 8 * heads > cus;   // [256 x 512] padded: 32 heads 36 / 42, 64 44 / 42
+  const int weight = key_blocks == 4 && a.max_q > 224 ? 2 : key_blocks;
+  return heads * (drop ? 2 * weight : std::max(weight, 2)) > cus;
 }
 
 template <typename T, int D>
@@ -2053,7 +2069,7 @@ int bwd_run(const char* what, FaArgs& a, int64_t batch, int64_t d, int drop_mode
   const dim3 grid_k(static_cast<unsigned>((a.max_k + FA_ROWS - 1) / FA_ROWS), static_cast<unsigned>(a.heads), static_cast<unsigned>(batch));
   int rc = bits_launch(what, a, drop_mode, batch, bits, bits_ready, st);
   if (rc) return rc;
-  if (bwd_in_one(a, batch, d)) {
+  if (bwd_in_one(a, batch, d, drop_mode != 0)) {
     auto pick = [&](auto t) {
       using T = decltype(t);
       // Four wavefronts hold up to 256 keys, and two such blocks share a CU; while the heads do not fill the CUs twice eight

@@ -330,6 +330,20 @@ def test_attention_backward_in_one_kernel_matches_the_two_kernels(dev, dtype, ma
             assert (x - y).norm() <= bound * y.norm().clamp_min(1e-6), (what, float((x - y).norm() / y.norm()))
 
 
+@pytest.mark.parametrize("tq,tk,b,h,mask,p,one", [
+    (256, 256, 1, 8, "none", 0.1, False), (256, 256, 8, 8, "none", 0.1, False), (256, 256, 9, 8, "none", 0.1, True), (256, 256, 16, 8, "none", 0.0, False),
+    (256, 256, 17, 8, "none", 0.0, True), (256, 256, 1, 8, "padding", 0.1, False), (256, 256, 2, 4, "padding", 0.1, True), (256, 256, 1, 8, "causal", 0.1, True),
+    (256, 256, 1, 2, "time", 0.0, True), (200, 200, 1, 8, "none", 0.1, True), (160, 256, 1, 8, "none", 0.1, True), (161, 256, 1, 8, "none", 0.1, False),
+    (256, 320, 1, 8, "none", 0.1, False), (224, 320, 1, 8, "none", 0.1, True), (256, 512, 4, 8, "padding", 0.1, False), (256, 512, 5, 8, "padding", 0.1, True),
+    (384, 128, 20, 8, "none", 0.1, False), (384, 128, 21, 8, "none", 0.1, True), (384, 128, 20, 8, "padding", 0.1, True), (384, 96, 20, 8, "none", 0.1, True),
+    (512, 64, 1, 1, "none", 0.1, False), (512, 512, 32, 8, "none", 0.0, True), (512, 512, 36, 8, "none", 0.0, False), (512, 512, 36, 8, "none", 0.1, True),
+    (512, 512, 41, 8, "none", 0.0, True), (513, 64, 20, 8, "none", 0.1, False), (64, 513, 1, 1, "none", 0.1, False)])
+def test_where_the_attention_backward_takes_one_kernel(dev, tq, tk, b, h, mask, p, one):
+    """Both sides of the rule, on 256 compute units."""
+    _, names = _attention_backward(dev, torch.bfloat16, tq, tk, b, h, mask, p, tq)()
+    assert names == (ONE if one else TWO)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("tokens,out,inner", [(1025, 64, 64), (1100, 264, 72), (1500, 512, 512), (2064, 136, 1096), (4100, 1024, 256), (1088, 2048, 2048)])
 def test_bias_gradient_beside_the_weight_gradient(dev, dtype, tokens, out, inner):
