@@ -75,6 +75,13 @@ size_t gemm_splitk_workspace_bytes(int M, int N, int K, int batch) {
   return splitk_ws_bytes(p, M, N, batch);
 }
 
+int64_t gemm_splitk_colsum_rows(int M, int N, int K) {
+  const SplitPlan p = plan_splitk(M, N, K, 1);
+  int bm, bn;
+  tile_dims(p.tile, bm, bn);
+  return p.splits > 1 ? static_cast<int64_t>(p.splits) * ceil_div(N, bn) : 0;
+}
+
 int gemm_run(int dtype, int layout, int epi, GemmArgs a, void* workspace, size_t workspace_bytes, hipStream_t st,
              int* m_tiles_out, GemmArgs* planned_out) {
   if (m_tiles_out) *m_tiles_out = 0;

@@ -976,6 +976,8 @@ enum GemmLayout { LAYOUT_NT = 0 /* A KC, B KC */, LAYOUT_NN = 1 /* A KC, B MC */
 
 // Workspace bytes a split-K call of this shape needs (0 if it would not split).
 size_t gemm_splitk_workspace_bytes(int M, int N, int K, int batch);
+// Partial rows of column sums that come out of such a call on 16-byte aligned operands (0 if it would not split).
+int64_t gemm_splitk_colsum_rows(int M, int N, int K);
 
 // Runs one GEMM. `epi` is a GemmEpi; for LAYOUT_TN with epi == EPI_PLAIN and a workspace the call
 // may split K. Returns 0 or a negative nmtg_status; *m_tiles_out receives the number of row tiles

@@ -10,8 +10,8 @@
 //             last layer adds its bias.
 //   backward: per layer one weight-gradient GEMM (token dimension split over the chip, fp32
 //             partials) and one data-gradient GEMM whose epilogue applies act'(h) * mask / (1-p)
-//             and produces the bias-gradient column sums; one column-sum kernel for the last
-//             layer's bias.
+//             and produces the bias-gradient column sums. The last layer's are taken whole by the final
+//             reduction (up to 1024 tokens), or come out of its weight-gradient product, or of a kernel of their own.
 // The reference runs a GEMM and then separate element-wise kernels over the [tokens, inner]
 // tensors; here those tensors cross HBM once per direction.
 #include "gemm.hip.h"
@@ -177,8 +177,8 @@ extern "C" int nmtg_mlp_bwd(int num_layers, const void* x, const void* const* we
   bool bias_from_parts = false;      // colsum_ws holds the partial column sums of g_cur
   int parts_rows = 0;
   // The final reductions (split-K sums, bias-gradient sums) ride along with the last data-gradient product, which
-  // leaves room on the CUs (GemmArgs::riders); where there is no such product they are one launch at the end. The
-  // partial column sums of the output gradient, which those read, are a launch of their own ahead of the GEMMs.
+  // leaves room on the CUs (GemmArgs::riders); where there is no such product they are one launch at the end. Partial
+  // column sums of the output gradient that no product carries are a launch of their own ahead of what reads them.
   const int max_riders = num_cus();   // one rider per CU, whatever the number of jobs' blocks
   ReduceTail head;                   // partial column sums of grad_out, owed before the tail's final sums
   bool head_pending = false;
@@ -201,11 +201,20 @@ extern "C" int nmtg_mlp_bwd(int num_layers, const void* x, const void* const* we
       head_pending = true;
       return tail_add_colsum(tail, colsum_ws, parts, static_cast<int>(out_i), grad_biases[i]);
     };
+    // Beside the weight gradient where its product splits K and the partial rows fit. Elsewhere the kernel of its own goes first:
+    // behind the product it comes between the products' partial sums and their reduction, which then reads them out of the caches
+    // (1280 tokens, 1024 to 1024: 22.7 us, 21.2 with the sums first; 3000, 512 to 2000: 25.7 and 24.2).
+    const int colsum_cap = static_cast<int>(plan.colsum_bytes / (out_i * sizeof(float)));
+    auto carried = [&]() {
+      if (dtype == NMTG_F32 || !grad_weights || !grad_weights[i] || out_i % 8 != 0 || in_i % 8 != 0) return false;
+      const int64_t rows = gemm_splitk_colsum_rows(static_cast<int>(out_i), static_cast<int>(in_i), static_cast<int>(batch));
+      return rows > 0 && rows <= colsum_cap && aligned16(g_cur) && aligned16(input_i) && aligned16(grad_weights[i]);
+    };
     bool bias_with_weight = false;
     if (grad_biases && grad_biases[i]) {
       if (!bias_from_parts && tail_add_colsum_whole(tail, dtype, g_cur, out_i, static_cast<int>(batch), static_cast<int>(out_i), grad_biases[i])) {
         rc = 0;
-      } else if (!bias_from_parts && dtype != NMTG_F32 && grad_weights && grad_weights[i]) {
+      } else if (!bias_from_parts && carried()) {
         bias_with_weight = true;
         rc = 0;
       } else if (!tail.full()) {
@@ -228,7 +237,7 @@ extern "C" int nmtg_mlp_bwd(int num_layers, const void* x, const void* const* we
       g.defer_reduce = !tail.full() ? 1 : 0;
       if (bias_with_weight) {
         g.colsum_part = colsum_ws;
-        g.colsum_cap = static_cast<int>(plan.colsum_bytes / (out_i * sizeof(float)));
+        g.colsum_cap = colsum_cap;
       }
       // (the partial column sums do not ride with this product: a split-K launch repeats the rider blocks in every
       // split, and the tiles then share CUs unevenly; measured slower than the launch of their own)

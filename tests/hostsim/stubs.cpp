@@ -11,12 +11,14 @@
 namespace {
 bool g_trace = false;
 std::map<std::string, int> g_launches;
+std::string g_order;
 }  // namespace
 
 namespace nmtg {
 bool trace_on() { return g_trace; }
 void trace_open(const char* name, hipStream_t, int* slot) {
   ++g_launches[name];
+  g_order += std::string(name) + "\n";
   *slot = -1;
 }
 void trace_close(hipStream_t, int) {}
@@ -24,6 +26,7 @@ void trace_close(hipStream_t, int) {}
 
 extern "C" int nmtg_trace_begin(void) {
   g_launches.clear();
+  g_order.clear();
   g_trace = true;
   return 0;
 }
@@ -42,6 +45,9 @@ extern "C" int64_t nmtg_trace_end(char* out, int64_t capacity) {
 }
 
 using namespace nmtg;
+
+// names of the launches since nmtg_trace_begin, in order, one a line
+extern "C" const char* hostsim_trace_order(void) { return g_order.c_str(); }
 
 // blocks of the last launch
 extern "C" int64_t hostsim_last_blocks(void) { return static_cast<int64_t>(gridDim.x) * gridDim.y * gridDim.z; }

@@ -683,6 +683,15 @@ def test_three_layer_mlp_backward_with_one_reduction_launch(mi355x):
     tst.test_three_layer_mlp_backward_with_one_reduction_launch(CPU)
 
 
+@pytest.mark.parametrize("tokens,out,inner,carried", [(1025, 64, 64, True), (1100, 264, 72, True), (1100, 64, 1096, False), (1100, 72, 132, False)])
+def test_bias_gradient_beside_the_weight_gradient(mi355x, dma, hostsim_lib, tokens, out, inner, carried):
+    tst.test_bias_gradient_beside_the_weight_gradient(CPU, BF16, tokens, out, inner, carried)
+    hostsim_lib.hostsim_trace_order.restype = ctypes.c_char_p
+    order = hostsim_lib.hostsim_trace_order().decode().split()
+    assert [n for n in order if not n.startswith("gemm_tn")] == ["reduce_tail"] * len(order[1:])
+    assert order[0].startswith("gemm_tn") == carried, order                   # sums of their own come ahead of the product
+
+
 # ----------------------------------------------------------------------------- attention over packed sequences
 @pytest.mark.parametrize("dtype", HALVES)
 @pytest.mark.parametrize("d,causal", [(64, False), (64, True), pytest.param(128, True, marks=long_case)])

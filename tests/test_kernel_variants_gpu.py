@@ -345,11 +345,13 @@ def test_where_the_attention_backward_takes_one_kernel(dev, tq, tk, b, h, mask, 
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("tokens,out,inner", [(1025, 64, 64), (1100, 264, 72), (1500, 512, 512), (2064, 136, 1096), (4100, 1024, 256), (1088, 2048, 2048)])
-def test_bias_gradient_beside_the_weight_gradient(dev, dtype, tokens, out, inner):
-    """Column sums of dY from the weight gradient's LDS tiles: every k-step counted once, whichever column tile and split adds it,
-    at ragged token counts and rows beyond the last tile, and calls with more partial rows than fit, which sum dY in a launch of
-    their own. fp32 sums of rounded numbers: tokens units of fp32 of the sum of magnitudes, then one rounding."""
+@pytest.mark.parametrize("tokens,out,inner,carried", [
+    (1025, 64, 64, True), (1100, 264, 72, True), (1500, 512, 512, True), (2064, 136, 1096, False), (4100, 1024, 256, True), (1088, 2048, 2048, False),
+    (4096, 3072, 1024, True), (4100, 3072, 1024, True), (1280, 1024, 1024, False), (1100, 72, 132, False)])
+def test_bias_gradient_beside_the_weight_gradient(dev, dtype, tokens, out, inner, carried):
+    """Column sums of dY from the weight gradient's LDS tiles (128 x 128 and, from 3072 x 1024 on, 256 x 256): every k-step counted
+    once, whichever column tile and split adds it, at whole and ragged token counts and rows beyond the last tile. Calls with more
+    partial rows than fit or rows of no multiple of 16 bytes sum dY in a launch of their own, the first of two reductions. fp32 sums of rounded numbers: tokens units of fp32 of the sum of magnitudes, then one rounding."""
     g = torch.Generator().manual_seed(tokens)
     x = torch.randn(tokens, inner, generator=g).to(dtype).to(dev).requires_grad_()
     w = (0.05 * torch.randn(out, inner, generator=g)).to(dtype).to(dev)
@@ -362,3 +364,6 @@ def test_bias_gradient_beside_the_weight_gradient(dev, dtype, tokens, out, inner
     bound = torch.finfo(dtype).eps * want.abs() + tokens * 2.0 ** -24 * d64.abs().sum(0)
     assert bool(((db.double().cpu() - want).abs() <= bound).all()), float((db.double().cpu() - want).abs().max())
     assert_close(dw, d64.t() @ x.detach().double().cpu(), dtype, "dw", scale_atol=True)
+    _lib.trace_begin()
+    fused_mlp_gelu.backward(0.0, dy.to(dev), saved, [x.detach(), w, b])       # no data gradient for the last reduction to ride with
+    assert _lib.trace_end()["reduce_tail"][0] == (1 if carried else 2)
