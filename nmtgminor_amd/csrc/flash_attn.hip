@@ -1077,9 +1077,10 @@ __global__ __launch_bounds__(FA_THREADS, D == 64 ? 2 : 1) void flash_bwd_dkv_ker
 // [key][query], and behind a barrier the wavefronts share out dQ's 64 x 32 results as eight 16 x 16 tiles that each sum
 // over all keys (v_mfma_f32_16x16x32): nothing is added up between wavefronts, no atomics, results do not depend on
 // scheduling. The two kernels make scores, exponentials and dP twice each: [512 x 512], 512 heads in bf16 with dropout 205 us
-// (91 + 114), here 152; [256 x 256] 78 and 50; [61 x 73], 384 heads 20 and 14. What bounds it: nothing alone. Vector instructions are 45 %
-// of the time, LDS reads 30 %, MFMA 22 %, with two wavefronts per SIMD to overlap them (all 256 registers are taken: 128 of
-// accumulators, 32 of V, 32 of scores).
+// (91 + 114), here 152; [256 x 256] 78 and 50; [61 x 73], 384 heads 20 and 14. What bounds it: nothing alone. On 32
+// packed sequences of 256 to 512 (154 us) the SIMDs issue vector instructions 37 % of the time, the matrix units work 16 %, and 1.5
+// of two possible wavefronts per SIMD are there to overlap them (all 256 registers are taken: 128 of accumulators, 32 of V, 32 of
+// scores).
 // Images of 128-byte rows: chunk c of row r at c ^ fb_swz(r). LDS serves 256 bytes per clock from 64 banks, so 16 lanes of a
 // row read (16 rows, one chunk) and 32 lanes of a transposing read (4 rows x 64 bytes for the 32 x 32 operands, 8 rows x 32
 // bytes for the 16 x 16 ones) must not meet: even and odd rows lie in different halves, rows that differ in bit 1 must
@@ -1336,8 +1337,7 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_bwd_kernel(FaArgs a) {
         mfma<T>::run(*reinterpret_cast<const uint4*>(gimg + at), vf[g][ss], dp);
       }
       // s[r], dp[r]: query 8 (r / 4) + 4 half + r % 4 of the step, key krow[g]
-      // One bit per register, then a select each. (With the conditions written out per element, short-circuited, the compiler
-      // branched around each of them and lost the write of one of the paths.)
+      // One bit per register, then a select each: no branch per element, and no load waits inside one.
       bool tmt = false;
       if constexpr (TM != 0) tmt = ((__builtin_amdgcn_readlane(masked_at, t) >> g) & 1) != 0;
       const bool diagonal = a.causal != 0 && group == t;

@@ -363,8 +363,9 @@ __device__ __forceinline__ void gemm_ring_body(const GemmArgs& g, int block_x) {
   zero_past_end(0, 0);
 
   // SUMS: sums of A's columns over this block's k (EPI_SPLITK of the row-contiguous layout, g.colsum_part): the operand is in LDS
-  // anyway. An instantiation of its own, since the code alone made calls without sums 0.7 % slower (ffn of 513 tokens). The column tiles of a row of tiles read the same A, so each of them adds up every n_tiles-th stage, by all threads,
-  // eight columns and a few k-rows each. As passes of their own over dY these sums took 34 us of a large encoder layer's
+  // anyway. An instantiation of its own, since the code alone made calls without sums 0.2 to 0.7 % slower (ffn of 513 tokens). The
+  // column tiles of a row of tiles read the same A, so each of them adds up every n_tiles-th stage, by all threads, eight columns
+  // and a few k-rows each. As passes of their own over dY these sums took 34 us of a large encoder layer's
   // backward (1024 wide, 16384 tokens) and 5 of the base model's feed-forward block. Measured, whole forward and backward:
   // feed-forward 512 -> 2048, 8192 tokens, 185 -> 182 us; attention block of 1024, 16384 tokens, 807 -> 785 us.
   static_assert(!SUMS || (EPI == EPI_SPLITK && !A_KC && !STREAM), "column sums go with the weight gradients");

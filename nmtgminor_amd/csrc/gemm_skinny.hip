@@ -8,7 +8,8 @@
 // columns (sk_cols) and all (at most 32) rows, its eight wavefronts each take an eighth of k, load their slices of X and W
 // straight into matrix-core operand layout (a lane's 16 bytes of its row: no LDS staging, every load of a 128-k chunk in
 // flight at once), run v_mfma_f32_32x32x16 over them, and leave their 32 x 32 partial sums in LDS, where the block adds
-// the eight of them up in a fixed order. A [1024 x 1024] weight is 32 blocks of one load latency each.
+// the eight of them up in a fixed order. A [1024 x 1024] weight is 128 blocks (8 columns) for up to 8 rows, 64 for more, of one
+// load latency each.
 #include "gemm.hip.h"
 
 #include <algorithm>
@@ -91,8 +92,10 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_skinny_kernel(const GemmArgs 
 // A step is a chain of launches of a few microseconds that depend on each other, so what counts is their number. In front:
 // LayerNorm of x, or of h = x + residual, computed by every block for its rows (5 rows x 512: one row per wavefront) while its
 // weights are on their way from memory; block 0 writes h. Behind: the activation, or the layer's last addition with its guard.
-// Rounding points are those of the separate kernels (h, the normalised row, the product with its bias), and the sums are in
-// the same order. A beam of 5 at E = 512 in fp16: 13 launches and 50 us of kernels for a step, 9 and 40 with these.
+// Rounding points are those of the separate kernels (h, the normalised row, the product with its bias). The sums are in the same
+// order but for the product in front of an activation, which the separate calls run on the tiled kernels and this one as eight
+// partial sums over k: a step is evaluation, where no gradient depends on the side of a gate that a value rounds to. A beam of 5 at
+// E = 512 in fp16: 13 launches and 50 us of kernels for a step, 9 and 39 with these.
 enum { STEP_PRE_NONE = 0, STEP_PRE_NORM = 1, STEP_PRE_ADD_NORM = 2 };
 enum { STEP_POST_ACT = 0, STEP_POST_ADD = 1 };
 constexpr int STEP_MAX_NORM = 1024;                      // columns that a wavefront normalises out of its registers

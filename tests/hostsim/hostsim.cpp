@@ -278,19 +278,6 @@ uint64_t shfl_xor_bits(uint64_t bits, int mask) {
   return s.bits;
 }
 
-struct ReadLane { uint32_t bits; int lane; };
-static void resolve_readlane(void** payloads, int lanes) {
-  const int from = static_cast<ReadLane*>(payloads[0])->lane;
-  if (from < 0 || from >= lanes) fail("v_readlane of a lane outside the wavefront");
-  const uint32_t bits = static_cast<ReadLane*>(payloads[from])->bits;
-  for (int l = 0; l < lanes; ++l) static_cast<ReadLane*>(payloads[l])->bits = bits;
-}
-uint32_t readlane_bits(uint32_t bits, int lane) {
-  ReadLane r{bits, lane};
-  wave_collective(resolve_readlane, &r);
-  return r.bits;
-}
-
 void dma_issue(const void* src, uint32_t lds_offset, int bytes) {
   const Transfer t{src, lds_offset, bytes};
   if (dma_early) land(t);

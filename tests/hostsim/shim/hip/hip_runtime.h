@@ -50,7 +50,6 @@ void wave_collective(Resolver resolver, void* payload);
 [[noreturn]] void fail(const char* what);
 unsigned lane_id();
 uint64_t shfl_xor_bits(uint64_t bits, int mask);
-uint32_t readlane_bits(uint32_t bits, int lane);
 uint64_t gather_bits(uint64_t bits, int source_lane);   // every lane names the lane whose value it reads
 void sync_block();
 // direct global -> LDS transfers (asynchronous; see hostsim.cpp for the two timing models)

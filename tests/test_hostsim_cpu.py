@@ -319,6 +319,18 @@ def test_gemm_unaligned_extents(mi355x, dtype):
     tg.test_gemm_unaligned_extents(CPU, dtype)
 
 
+@pytest.mark.parametrize("m,n,k", [(61, 73, 64), (64, 65, 63), (1, 129, 7), (128, 64, 73)])
+@pytest.mark.parametrize("layout,pitched", [("nt", "ab"), ("nn", "bc"), ("tn", "bc"), ("nt", ""), ("nn", "ac")])
+def test_gemm_small_outputs_in_64x64_tiles(mi355x, monkeypatch, m, n, k, layout, pitched):
+    tg.test_small_outputs_in_64x64_tiles(CPU, monkeypatch, BF16, m, n, k, layout, pitched)
+
+
+@pytest.mark.parametrize("layout,m,n,k,batch,small", [("nt", 140, 150, 64, 3, True), ("nt", 70, 77, 64, 3, False), ("nn", 250, 64, 301, 2, True),
+                                                      ("nn", 333, 333, 333, 2, False), ("tn", 190, 64, 250, 2, True), ("tn", 500, 64, 132, 2, False)])
+def test_where_64x64_tiles_take_over(mi355x, monkeypatch, layout, m, n, k, batch, small):
+    tg.test_where_64x64_tiles_take_over(CPU, monkeypatch, layout, m, n, k, batch, small)
+
+
 def test_gemm_bias_and_batched_strided_views(mi355x):
     tg.test_gemm_bias_and_batched_strided_views(CPU)
 
@@ -714,6 +726,26 @@ def test_packed_attention_dropout_philox_and_autograd_functions():
     tfl.test_packed_kv_function_with_dropout_repeats_its_mask_in_the_backward(CPU)
 
 
+@pytest.mark.parametrize("p", [0.0005, 127 / 256, 0.998])
+def test_every_keep_bit(p):
+    tfl.test_every_keep_bit_of_the_byte_thresholds_edges(CPU, p)
+
+
+@pytest.mark.parametrize("dtype,mask,p", [(BF16, "none", 0.0), (BF16, "padding", 0.2), (BF16, "time", 0.2), (BF16, "causal", 0.2),
+                                          pytest.param(F16, "time", 0.0, marks=long_case), pytest.param(F16, "none", 0.2, marks=long_case)])
+def test_attention_backward_in_one_kernel(monkeypatch, dma, dtype, mask, p):
+    monkeypatch.setenv("HOSTSIM_CUS", "2")               # with three heads the smaller block holds up to 256 keys
+    tst.test_attention_backward_in_one_kernel_matches_the_two_kernels(
+        CPU, dtype, mask, p, [(1, 1, 1, 2), (31, 33, 2, 3), (65, 129, 1, 3), (40, 300, 2, 1), (257, 130, 1, 3), (290, 257, 1, 2)])
+
+
+@pytest.mark.parametrize("tq,tk,b,h,mask,p,one", [(256, 256, 1, 4, "none", 0.1, False), (200, 200, 1, 4, "none", 0.1, True), (160, 256, 1, 4, "none", 0.1, True),
+                                                  (256, 256, 1, 2, "padding", 0.1, False), (256, 256, 2, 2, "padding", 0.1, True),
+                                                  (256, 256, 1, 2, "causal", 0.0, True), (512, 64, 1, 1, "none", 0.1, False)])
+def test_where_the_attention_backward_takes_one_kernel(mi355x, tq, tk, b, h, mask, p, one):
+    tst.test_where_the_attention_backward_takes_one_kernel(CPU, tq, tk, b, h, mask, p, one)
+
+
 # ----------------------------------------------------------------------------- the same kernels over a padded batch
 def test_training_attention_without_coverage(mi355x, monkeypatch):
     tnc.test_self_attention_with_masked_keys_anywhere(CPU, BF16)
@@ -769,6 +801,18 @@ def test_few_row_products_narrow_their_blocks_only_while_the_chip_is_not_full(ho
     hostsim_lib.hostsim_last_blocks.restype = ctypes.c_int64
     assert hostsim_lib.hostsim_last_blocks() == blocks
     tat.assert_close(y, x.double() @ w.double().t(), BF16, "few rows")
+
+
+@pytest.mark.parametrize("rows,out,k", [(5, 100, 512), (33, 64, 1024), (8, 64, 1016)])
+@pytest.mark.parametrize("pre,act", [("none", "gelu"), ("norm", "none"), ("add", "relu"), ("add", "silu")])
+def test_step_products_with_what_stands_around_them(mi355x, rows, out, k, pre, act):
+    tsl.test_normalisation_product_activation(CPU, BF16, rows, out, k, pre, act)
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("spoilt", [False, True])
+def test_step_product_and_guarded_addition(mi355x, dtype, spoilt):
+    tsl.test_product_and_guarded_addition(CPU, dtype, 40, 72, 136, spoilt)
 
 
 def test_step_products_refuse_outputs_over_inputs(mi355x):
